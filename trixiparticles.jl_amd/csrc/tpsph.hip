@@ -722,7 +722,7 @@ __device__ __forceinline__ void
             int *__restrict__ nwtargets, int *__restrict__ noverflow,
             const unsigned char *__restrict__ wall_near, const int *__restrict__ brow_gb,
             const int *__restrict__ brow_lds, int *__restrict__ bntot,
-            unsigned long long *__restrict__ nbr16)
+            unsigned long long *__restrict__ nbr16, int2 *__restrict__ thead)
 {
     if (skip(flag)) return;
     for (int t = bx * kBlock + threadIdx.x; t < P.nf; t += gx * kBlock) {
@@ -730,7 +730,7 @@ __device__ __forceinline__ void
         const int c0 = cell_1d(F.x[s], P.lo[0], P.inv_cs[0], P.n[0]);
         const int c1 = cell_1d(F.y[s], P.lo[1], P.inv_cs[1], P.n[1]);
         const int c2 = (ND == 3) ? cell_1d(F.z[s], P.lo[2], P.inv_cs[2], P.n[2]) : 0;
-        int b = -1;
+        int b = -1, self = 0;
         if (nbr16) {
             const int bxi = c0 / P.bc[0], byi = c1 / P.bc[1], bzi = c2 / P.bc[2];
             b = bxi + P.nb[0] * (byi + P.nb[1] * bzi);
@@ -741,8 +741,14 @@ __device__ __forceinline__ void
             const BrickRows br{brow_gb + (size_t)b * P.maxr, brow_lds + (size_t)b * (P.maxr + 1),
                                byi * P.bc[1] - P.ur[1], (ND == 3) ? bzi * P.bc[2] - P.ur[2] : 0,
                                P.bc[1] + 2 * P.ur[1]};
-            bool ok = true;
-            build_list<ND, false, true>(P, F, Wv, s, t, ls, cap_f, nbr, cnt, br, nbr16, &ok);
+            // the target's own record in the union
+            const int row = (c1 - br.uy0) + br.nuy * (((ND == 3) ? c2 : 0) - br.uz0);
+            self = br.lds[row] + (s - br.gb[row]);
+            bool ok = self >= br.lds[row] && self < br.lds[row + 1] && self < P.brick_cap - 1;
+            if (!ok) self = 0;
+            bool in_union = true;
+            build_list<ND, false, true>(P, F, Wv, s, t, ls, cap_f, nbr, cnt, br, nbr16, &in_union);
+            ok = ok && in_union;
             if (!ok) bntot[b] = INT_MAX;
         } else {
             build_list<ND, false>(P, F, Wv, s, t, ls, cap_f, nbr, cnt);
@@ -757,6 +763,9 @@ __device__ __forceinline__ void
                 wcnt[t] = 0;
             }
         }
+        if (thead)
+            thead[t] = make_int2(F.perm[s], self | max(cnt[t], 0) << kHeadCount |
+                                                (P.nw > 0 && wcnt[t] != 0 ? kHeadWalls : 0));
     }
 }
 
@@ -1045,6 +1054,7 @@ struct ListsArgs {
     const int *brow_gb, *brow_lds;
     int *bntot;
     unsigned long long *nbr16;  // nullptr without bricks
+    int2 *thead;                // nullptr without bricks
 };
 struct UnionArgs {
     const int *start, *bstart;
@@ -1087,46 +1097,85 @@ __global__ void __launch_bounds__(kBlock, 6)
 {
     lists_body<ND>(blockIdx.x, gridDim.x, flag, P, F, Wv, a.ord, a.ls, a.cap_f, a.nbr, a.cnt,
                    a.cap_w, a.wnbr, a.wcnt, a.wtargets, a.nwtargets, a.noverflow, a.wall_near,
-                   a.brow_gb, a.brow_lds, a.bntot, a.nbr16);
+                   a.brow_gb, a.brow_lds, a.bntot, a.nbr16, a.thead);
 }
+
+// Header and union row tables of one brick in LDS.
+template <int ROWS>
+struct BrickTables {
+    int gb[ROWS], lds[ROWS + 1];
+    int4 head;  // {brick or -1, first target, one past the last, union size}
+
+    // Those of brick nel[item] (none past ne), read by one wave.
+    __device__ __forceinline__ void read(const DevParams &P, const int *__restrict__ nel,
+                                         const int *__restrict__ bstart,
+                                         const int *__restrict__ bntot,
+                                         const int *__restrict__ brow_gb,
+                                         const int *__restrict__ brow_lds, int item, int ne,
+                                         int lane)
+    {
+        int4 h = make_int4(-1, 0, 0, 0);
+        if (item < ne) {
+            const int b = nel[item];
+            for (int r = lane; r <= P.maxr; r += 64) {
+                if (r < P.maxr) gb[r] = brow_gb[(size_t)b * P.maxr + r];
+                lds[r] = brow_lds[(size_t)b * (P.maxr + 1) + r];
+            }
+            h = make_int4(b, bstart[b], bstart[b + 1], bntot[b]);
+        }
+        if (lane == 0) head = h;
+    }
+};
 
 // Staged union: one record per particle as four 16-byte fields and one 8-byte field, each in
 // an array of its own, read with one ds_read_b128 (ds_read_b64) per field.  The 16-byte
 // stride spreads random candidates over all banks; 72- or 64-byte records made the lanes of
 // a read collide on fewer bank groups (measured 2% and 12% slower).  The last record is the
-// far record that pads the list groups (finite values, zero volume).  With a global brick
-// the same bytes hold the lanes' int lists.
+// far record that pads the list groups (finite values, zero volume).
 // ANT (DensityDiffusionAntuono): also the renormalised density gradient, g0 {gx, gy} and in
 // 3D g1 {gz}, in CAP = kBrickCapGrad records there (96 bytes each: the LDS holds fewer).
 template <int ND, bool ANT = false>
 struct BrickSmem {
     static constexpr int CAP = (ANT && ND == 3) ? kBrickCapGrad : kBrickCap;
+    static constexpr int ROWS = (ANT && ND == 3) ? kBrickMaxRowsGrad : kBrickMaxRows;
     // 3D: p0 {x, y}, p1 {z, rho}, p2 {vx, vy}, p3 {vz, p};  2D: p0 {x, y}, p1 {rho, vx},
-    // p2 {vy, p} (p3 unused); vol: V = m / rho
+    // p2 {vy, p} (p3 unused); vol: V = m / rho (SummationDensity: m)
     double2 p0[CAP], p1[CAP], p2[CAP], p3[ND == 3 ? CAP : 1];
     double vol[CAP];
     double2 g0[ANT ? CAP : 1];
     double g1[(ANT && ND == 3) ? CAP : 1];
-    int row_gb[kBrickMaxRows], row_lds[kBrickMaxRows + 1];
-    int item;
+    BrickTables<ROWS> tab[2];  // this brick's and the next one's
+};
+
+// A staged record in registers.
+struct BrickRec {
+    double x[3], rho, v[3], p, V;
 };
 
 template <int ND, bool ANT>
-__device__ __forceinline__ FluidNbr lds_fluid(const BrickSmem<ND, ANT> &S, int e)
+__device__ __forceinline__ BrickRec lds_rec(const BrickSmem<ND, ANT> &S, int e)
 {
-    FluidNbr n;
+    BrickRec n;
     const double2 a = S.p0[e], b = S.p1[e], c = S.p2[e];
-    const double V = S.vol[e];
+    n.x[0] = a.x;
+    n.x[1] = a.y;
     if constexpr (ND == 3) {
         const double2 d = S.p3[e];
-        n.a = make_double4(a.x, a.y, b.x, b.y);
-        n.b = make_double4(c.x, c.y, d.x, d.y);
-        n.v = make_double2(V, V * b.y);
+        n.x[2] = b.x;
+        n.rho = b.y;
+        n.v[0] = c.x;
+        n.v[1] = c.y;
+        n.v[2] = d.x;
+        n.p = d.y;
     } else {
-        n.a = make_double4(a.x, a.y, 0.0, b.x);
-        n.b = make_double4(b.y, c.x, 0.0, c.y);
-        n.v = make_double2(V, V * b.x);
+        n.x[2] = 0.0;
+        n.rho = b.x;
+        n.v[0] = b.y;
+        n.v[1] = c.x;
+        n.v[2] = 0.0;
+        n.p = c.y;
     }
+    n.V = S.vol[e];
     return n;
 }
 
@@ -1140,207 +1189,385 @@ __device__ __forceinline__ void lds_grad(const BrickSmem<ND, ANT> &S, int e, dou
     g[2] = (ND == 3) ? S.g1[e] : 0.0;
 }
 
-// Fluid-fluid kernel over the bricks (one block of kBrickThreads per non-empty brick, taken
-// from a work counter that k_gather<0> resets).  Targets with wall candidates are completed
-// by k_fluid_walls.
-// GLOBAL_ONLY: only the bricks that do not stage, which the mixed-precision pass
-// (tpsph_mixed.hip) leaves to this kernel: the work[1] bricks it listed in bfall, taken by
-// blocks in turn.  VISC: visc_mode(P), the viscosity form of the staged pair loop.  ANT:
-// DensityDiffusionAntuono (P.ddgrad), whose gradients are staged beside the records.  SUM:
-// SummationDensity (pressure slot staged as p / rho^2, no density rate, dv of ND rows).
-template <int ND, bool GLOBAL_ONLY = false, int VISC = kViscAlpha, bool ANT = false,
-          bool SUM = false>
+// The pair constants of the staged pair loop (scalar registers).
+struct BrickConsts {
+    double az2, minus_half_h_inv, eps_h2, two_av_c, dd2, h, two_beta, kgrad_c;
+
+    __device__ __forceinline__ explicit BrickConsts(const DevParams &P)
+        : az2(P.az2), minus_half_h_inv(-0.5 * P.h_inv), eps_h2(P.eps_h2), two_av_c(2.0 * P.av_c),
+          dd2(P.dd2), h(P.h), two_beta(2.0 * P.beta), kgrad_c(P.kgrad_c)
+    {
+    }
+};
+
+// A target of the staged pair loop and its fluid-fluid terms (pair_fluid's) without branches.
+// With k = (1 - r / 2h)^3 of a pair the sums are
+//   acc  += V_b k [-(p_a + p_b) + 2 alpha c h rho_a rho_b min(v_ab.r_ab, 0) /
+//                  ((r^2 + eps h^2)(rho_a + rho_b)) + ...beta] r_ab
+//   drho += V_b k [2 delta h c (rho_a - rho_b) + rho_a v_ab.r_ab]
+// and what is common to all pairs of the target, kgrad_c / rho_a and kgrad_c, multiplies the
+// finished sums: 8 instructions fewer per candidate than with the factors in every term.
+// SUM (SummationDensity): acc += m_b k [-(p_a/rho_a^2 + p_b/rho_b^2) + 2 alpha c h ...], with
+// p / rho^2 staged in the pressure slot and m in the volume slot, and no density rate.
+//
+// The range test is the kernel factor itself: max(1 - r / 2h, 0) is zero for every candidate
+// beyond R (up to rounding at exactly R, where (1 - r / 2h)^3 is below 1e-46), for the far
+// record (whose volume is zero too) and, as max(NaN, 0), for a pair at d^2 < az2, whose
+// high word is replaced by a NaN's.
+template <int ND, int VISC, bool ANT, bool SUM>
+struct BrickTarget {
+    double x[3], v[3], rho, p, visc, g[ANT ? 3 : 1];
+
+    __device__ __forceinline__ BrickTarget(const BrickConsts &C, const BrickRec &me)
+    {
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            x[d] = me.x[d];
+            v[d] = me.v[d];
+        }
+        rho = me.rho;
+        p = me.p;
+        visc = SUM ? C.two_av_c : C.two_av_c * me.rho;
+    }
+
+    // gb: the candidate's renormalised density gradient (ANT)
+    __device__ __forceinline__ void add(const BrickConsts &C, const BrickRec &n, double *acc,
+                                        double &drho, const double *gb) const
+    {
+        const double p0 = x[0] - n.x[0], p1 = x[1] - n.x[1];
+        const double p2 = (ND == 3) ? x[2] - n.x[2] : 0.0;
+        double d2 = dist2<ND>(p0, p1, p2);
+        const double near = __hiloint2double(d2 >= C.az2 ? __double2hiint(d2) : 0x7ff80000,
+                                             __double2loint(d2));
+        const double w = fmax(fma(C.minus_half_h_inv, sqrt_pos(near), 1.0), 0.0);
+        const double Vk = n.V * (w * w * w);
+        const double v0 = v[0] - n.v[0], v1 = v[1] - n.v[1];
+        const double v2 = (ND == 3) ? v[2] - n.v[2] : 0.0;
+        double vr = v0 * p0 + v1 * p1;
+        if constexpr (ND == 3) vr += v2 * p2;
+        double f = -(p + n.p);
+        if constexpr (VISC != kViscNone) {
+            const double q = d2 + C.eps_h2;
+            const double sum_rho = rho + n.rho;
+            const double vn = fmin(vr, 0.0);
+            const double num = SUM ? visc * vn : visc * (n.rho * vn);
+            f = fma(num, rcp_pos(q * sum_rho), f);
+            if constexpr (VISC == kViscAlphaBeta) {
+                const double mu = C.h * vn * rcp_pos(q);
+                const double b = C.two_beta * (mu * mu) * rcp_pos(sum_rho);
+                f += SUM ? b : (rho * n.rho) * b;
+            }
+        }
+        f *= Vk;
+        acc[0] = fma(f, p0, acc[0]);
+        acc[1] = fma(f, p1, acc[1]);
+        if constexpr (ND == 3) acc[2] = fma(f, p2, acc[2]);
+        if constexpr (!SUM) {
+            double drr = rho - n.rho;
+            if constexpr (ANT) {
+                double gr = (g[0] + gb[0]) * p0 + (g[1] + gb[1]) * p1;
+                if constexpr (ND == 3) gr += (g[2] + gb[2]) * p2;
+                drr = fma(-0.5, gr, drr);
+            }
+            drho = fma(Vk, fma(C.dd2, drr, rho * vr), drho);
+        }
+    }
+
+    // the factors common to all pairs of the target
+    __device__ __forceinline__ void scale(const BrickConsts &C, double *acc, double &drho) const
+    {
+        const double f = SUM ? C.kgrad_c : C.kgrad_c / rho;
+#pragma unroll
+        for (int d = 0; d < 3; d++) acc[d] *= f;
+        drho *= C.kgrad_c;
+    }
+};
+
+// One thread's share of a union on its way from global memory to LDS: records tid and
+// tid + kBrickThreads (a union holds fewer than 2 kBrickThreads).
+template <int ND, bool ANT, bool SUM>
+struct UnionShare {
+    double4 a[2], c[2];
+    double V[2], g[2][ANT ? ND : 1];
+
+    __device__ __forceinline__ void load(const DevParams &P, const FluidView &F,
+                                         const int *row_gb, const int *row_lds, int ntot)
+    {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int i = (int)threadIdx.x + h * kBrickThreads;
+            const int r = bsearch_le(row_lds, P.maxr + 1, i);
+            const int s = i < ntot ? row_gb[r] + (i - row_lds[r]) : 0;
+            a[h] = F.rec[2 * (size_t)s];
+            c[h] = F.rec[2 * (size_t)s + 1];
+            V[h] = SUM ? F.vol[s].y : F.vol[s].x;
+            if constexpr (ANT) {
+#pragma unroll
+                for (int d = 0; d < ND; d++) g[h][d] = P.ddgrad[(size_t)s * ND + d];
+            }
+        }
+    }
+
+    __device__ __forceinline__ void store(BrickSmem<ND, ANT> &S, int ntot) const
+    {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int i = (int)threadIdx.x + h * kBrickThreads;
+            if (i >= ntot) continue;
+            const double pslot = SUM ? c[h].w / (a[h].w * a[h].w) : c[h].w;
+            S.p0[i] = make_double2(a[h].x, a[h].y);
+            if constexpr (ND == 3) {
+                S.p1[i] = make_double2(a[h].z, a[h].w);
+                S.p2[i] = make_double2(c[h].x, c[h].y);
+                S.p3[i] = make_double2(c[h].z, pslot);
+            } else {
+                S.p1[i] = make_double2(a[h].w, c[h].x);
+                S.p2[i] = make_double2(c[h].y, pslot);
+            }
+            S.vol[i] = V[h];
+            if constexpr (ANT) {
+                S.g0[i] = make_double2(g[h][0], g[h][1]);
+                if constexpr (ND == 3) S.g1[i] = g[h][2];
+            }
+        }
+    }
+};
+
+// The fluid-fluid sums of the targets of a brick that does not stage (four lanes per target):
+// the int Verlet lists, or the cell walk (lane 0) of an overflowed list.
+template <int ND, bool SUM, typename Args>
+__device__ __forceinline__ void brick_from_global(const DevParams &P, const FluidView &F,
+                                                  const Args &A, int t0, int t1)
+{
+    const int q = (int)threadIdx.x & 3;
+    for (int base = t0; base < t1; base += kBrickThreads / 4) {
+        const int t = base + (int)threadIdx.x / 4;
+        const bool active = t < t1;
+        const int col = active ? t : t0;
+        const int s = A.ord[col];
+        const double4 a = F.rec[2 * (size_t)s], c = F.rec[2 * (size_t)s + 1];
+        const double xa[3] = {a.x, a.y, a.z}, va[3] = {c.x, c.y, c.z};
+        const double rho_a = a.w, inv_rho_a = 1.0 / a.w;
+        const double p_a = SUM ? c.w / (rho_a * rho_a) : c.w;
+        double ga[3] = {0.0, 0.0, 0.0};  // DensityDiffusionAntuono: the target's gradient
+        const bool ant = !SUM && P.ddgrad;
+        if (ant) {
+#pragma unroll
+            for (int d = 0; d < ND; d++) ga[d] = P.ddgrad[(size_t)s * ND + d];
+        }
+        double acc[3] = {0.0, 0.0, 0.0}, drho = 0.0;
+        auto pair = [&](int j) {
+            const FluidNbr nb = load_fluid(F, j);
+            const double p0 = xa[0] - nb.a.x, p1 = xa[1] - nb.a.y;
+            const double p2 = (ND == 3) ? xa[2] - nb.a.z : 0.0;
+            const double d2 = dist2<ND>(p0, p1, p2);
+            if (d2 <= P.R2 && d2 >= P.az2)
+                pair_fluid<ND, SUM>(P, nb, xa, va, rho_a, p_a, inv_rho_a, acc, drho, ant ? ga : nullptr);
+        };
+        const int n = active ? A.cnt[col] : 0;
+        if (n >= 0) {
+            for (int k = q; k < n; k += 4) pair(A.nbr[(size_t)k * A.ls + col]);
+        } else if (q == 0) {
+            Pencils<ND> it;
+            it.init(P, xa[0], xa[1], xa[2], P.hs_fluid);
+            int jb, je;
+            while (it.next(P, F.start, jb, je))
+                for (int j = jb; j < je; j++) pair(j);
+        }
+#pragma unroll
+        for (int o = 1; o < 4; o <<= 1) {
+#pragma unroll
+            for (int d = 0; d < 3; d++) acc[d] += __shfl_xor(acc[d], o);
+            drho += __shfl_xor(drho, o);
+        }
+        if (active && q == 0) {
+            constexpr int rows = SUM ? ND : ND + 1;
+            const bool walls = P.nw > 0 && A.wcnt[col] != 0;
+            const int i = F.perm[s];
+#pragma unroll
+            for (int d = 0; d < ND; d++)
+                A.dv[(size_t)i * rows + d] = walls ? acc[d] : acc[d] + P.g[d];
+            if constexpr (!SUM) A.dv[(size_t)i * rows + ND] = drho;
+        }
+    }
+}
+
+struct BrickArgs {
+    const int *ord, *bstart, *nel, *nne;
+    int *work;
+    const int *brow_gb, *brow_lds, *bntot;
+    const unsigned short *nbr16;
+    const int2 *thead;
+    const int *nbr, *cnt, *wcnt;
+    int ls;
+    double *dv;
+    const int *bfall;
+};
+
+// Fluid-fluid kernel over the bricks, one block of kBrickThreads per compute unit.  Targets
+// with wall candidates are completed by k_fluid_walls.
+//
+// What bounds it: 1024 threads with one 147 KB union leave a compute unit one block, so
+// nothing hides a brick's chain of dependent loads (claim, brick header, row tables, records,
+// target headers: 24k of 57k cycles per brick at 1.02M particles) but the block itself.  So
+// the chain runs one brick ahead: while a brick's pair loop runs, wave 0 claims the brick
+// after the next one and reads its header and row tables; every wave that has finished its
+// targets loads its share of the next union into registers before it waits for the others;
+// and the targets' own records come from the staged union (thead).  Measured at 1.02M
+// particles, with the pair terms of BrickTarget: 299 -> 247 us per launch.
+// Bricks: the first gridDim.x in the order of the blocks, then from the work counter (which
+// k_gather<0> and the stage kernel reset).
+// VISC: visc_mode(P), the viscosity form of the pair loop.  ANT: DensityDiffusionAntuono
+// (P.ddgrad), whose gradients are staged beside the records.  SUM: SummationDensity
+// (pressure slot staged as p / rho^2, no density rate, dv of ND rows).
+template <int ND, int VISC = kViscAlpha, bool ANT = false, bool SUM = false>
 __global__ void __launch_bounds__(kBrickThreads)
-    k_fluid_brick(int *flag, DevParams P, FluidView F, WallView Wv, const int *__restrict__ ord,
-                  const int *__restrict__ bstart, const int *__restrict__ nel,
-                  const int *__restrict__ nne, int *__restrict__ work,
-                  const int *__restrict__ brow_gb, const int *__restrict__ brow_lds,
-                  const int *__restrict__ bntot, const unsigned short *__restrict__ nbr16,
-                  const int *__restrict__ nbr, const int *__restrict__ cnt,
-                  const int *__restrict__ wnbr, const int *__restrict__ wcnt, int ls,
-                  double *__restrict__ dv, const int *__restrict__ bfall = nullptr)
+    k_fluid_brick(int *flag, DevParams P, FluidView F, BrickArgs A)
 {
     P = with_sound(P);
-    // cell-walk fallback lists of a global brick: as many entries per lane as the staging
-    // area holds (at most kCap)
     using Smem = BrickSmem<ND, ANT>;
-    constexpr int kCapB = Smem::CAP;
-    constexpr int kFallbackCap = std::min<int>(kCap, sizeof(Smem) / (sizeof(int) * kBrickThreads));
-    static_assert(kFallbackCap >= 8, "the fallback lists must fit the staging area");
     __shared__ Smem S;
     const int tid = threadIdx.x;
+    const bool wave0 = tid < 64;
     if (blockIdx.x == 0 && tid == 0) *flag = 0;  // the rebuild (if any) is done
-    int *lst = reinterpret_cast<int *>(&S) + tid;  // fallback lists, stride kBrickThreads
-    const int ne = GLOBAL_ONLY ? work[1] : *nne;
-    for (int turn = blockIdx.x;; turn += gridDim.x) {
-        int item = turn;
-        if (!GLOBAL_ONLY) {
-            if (tid == 0) S.item = atomicAdd(work, 1);
-            __syncthreads();
-            item = S.item;
+    const int ne = *A.nne;
+    if ((int)blockIdx.x >= ne) return;  // uniform: a block without a brick
+    constexpr int kFarSlot = Smem::CAP - 1;
+    if (tid == 0) {  // the far record: coordinates kFar, rho 1, the rest 0
+        if constexpr (ANT) {
+            S.g0[kFarSlot] = make_double2(0.0, 0.0);
+            if constexpr (ND == 3) S.g1[kFarSlot] = 0.0;
         }
-        if (item >= ne) break;
-        const int b = GLOBAL_ONLY ? bfall[item] : nel[item];
-        const int t0 = bstart[b], t1 = bstart[b + 1];
-        const int ntot = bntot[b];
-        const bool staged = ntot <= kCapB - 1;
-        if (GLOBAL_ONLY && staged) continue;  // uniform per block; no LDS is touched
-        if (staged) {
-            for (int r = tid; r <= P.maxr; r += kBrickThreads) {
-                if (r < P.maxr) S.row_gb[r] = brow_gb[(size_t)b * P.maxr + r];
-                S.row_lds[r] = brow_lds[(size_t)b * (P.maxr + 1) + r];
-            }
-            if (tid == 0) {  // the far record: coordinates kFar, rho 1, the rest 0
-                constexpr int f = kCapB - 1;
-                if constexpr (ANT) {
-                    S.g0[f] = make_double2(0.0, 0.0);
-                    if constexpr (ND == 3) S.g1[f] = 0.0;
-                }
-                S.p0[f] = make_double2(kFar, kFar);
-                if constexpr (ND == 3) {
-                    S.p1[f] = make_double2(kFar, 1.0);
-                    S.p2[f] = make_double2(0.0, 0.0);
-                    S.p3[f] = make_double2(0.0, 0.0);
-                } else {
-                    S.p1[f] = make_double2(1.0, 0.0);
-                    S.p2[f] = make_double2(0.0, 0.0);
-                }
-                S.vol[f] = 0.0;
-            }
-            __syncthreads();
-            for (int i = tid; i < ntot; i += kBrickThreads) {
-                const int r = bsearch_le(S.row_lds, P.maxr + 1, i);
-                const int g = S.row_gb[r] + (i - S.row_lds[r]);
-                const double4 a = F.rec[2 * (size_t)g];
-                const double4 c = F.rec[2 * (size_t)g + 1];
-                const double pslot = SUM ? c.w / (a.w * a.w) : c.w;
-                if constexpr (ND == 3) {
-                    S.p0[i] = make_double2(a.x, a.y);
-                    S.p1[i] = make_double2(a.z, a.w);
-                    S.p2[i] = make_double2(c.x, c.y);
-                    S.p3[i] = make_double2(c.z, pslot);
-                } else {
-                    S.p0[i] = make_double2(a.x, a.y);
-                    S.p1[i] = make_double2(a.w, c.x);
-                    S.p2[i] = make_double2(c.y, pslot);
-                }
-                S.vol[i] = F.vol[g].x;
-                if constexpr (ANT) {
-                    const double *gg = P.ddgrad + (size_t)g * ND;
-                    S.g0[i] = make_double2(gg[0], gg[1]);
-                    if constexpr (ND == 3) S.g1[i] = gg[2];
-                }
-            }
-            __syncthreads();
+        S.p0[kFarSlot] = make_double2(kFar, kFar);
+        S.p2[kFarSlot] = make_double2(0.0, 0.0);
+        if constexpr (ND == 3) {
+            S.p1[kFarSlot] = make_double2(kFar, 1.0);
+            S.p3[kFarSlot] = make_double2(0.0, 0.0);
+        } else {
+            S.p1[kFarSlot] = make_double2(1.0, 0.0);
         }
-        // Four lanes per target: lane q of target i takes every fourth group of four list
-        // slots, starting at group q (every fourth slot of the global lists); the four
-        // partial sums are added across the lanes (a fixed butterfly) and lane 0 writes.
-        // With four lanes a brick's targets (about 385) take two passes of 256 whose waves
-        // spread evenly over the four SIMDs; two lanes left a quarter of the waves idle and
-        // one SIMD with the most work (8% slower).
-        constexpr int kL = 4;
-        const int half = tid & (kL - 1);
-        for (int base = t0; base < t1; base += kBrickThreads / kL) {
-            const int t = base + (tid / kL);
-            const bool active = t < t1;
-            const int col = active ? t : t0;
-            const int s = ord[col];
-            double xa[3] = {0.0, 0.0, 0.0}, va[3] = {0.0, 0.0, 0.0}, rho_a = 1.0, p_a = 0.0;
-            int n = 0, nw = 0;
-            if (active) {
-                const double4 a = F.rec[2 * (size_t)s];
-                const double4 c = F.rec[2 * (size_t)s + 1];
-                xa[0] = a.x;
-                xa[1] = a.y;
-                xa[2] = a.z;
-                rho_a = a.w;
-                va[0] = c.x;
-                va[1] = c.y;
-                va[2] = c.z;
-                p_a = c.w;
-                n = cnt[col];
-                if (P.nw > 0) nw = wcnt[col];
+        S.vol[kFarSlot] = 0.0;
+    }
+    auto read_tables = [&](int item, int k) {  // wave 0
+        S.tab[k].read(P, A.nel, A.bstart, A.bntot, A.brow_gb, A.brow_lds, item, ne, tid);
+    };
+    if (wave0) read_tables(blockIdx.x, 0);
+    __syncthreads();
+    int4 hd = S.tab[0].head;  // {brick or -1, first target, one past the last, union size}
+    {
+        UnionShare<ND, ANT, SUM> share;
+        const int nstage = hd.w <= kFarSlot ? hd.w : 0;
+        share.load(P, F, S.tab[0].gb, S.tab[0].lds, nstage);
+        if (wave0) {
+            int item = ne;
+            if ((int)gridDim.x < ne) {
+                if (tid == 0) item = (int)gridDim.x + atomicAdd(A.work, 1);
+                item = __builtin_amdgcn_readfirstlane(item);
             }
-            const double inv_rho_a = 1.0 / rho_a;
-            if constexpr (SUM) p_a = p_a / (rho_a * rho_a);  // the target's p / rho^2
-            double acc[3] = {0.0, 0.0, 0.0}, drho = 0.0;
-            double ga[3] = {0.0, 0.0, 0.0};  // DensityDiffusionAntuono: the target's gradient
-            if constexpr (ANT) {
-                if (active) {
-#pragma unroll
-                    for (int d = 0; d < ND; d++) ga[d] = P.ddgrad[(size_t)s * ND + d];
-                }
-            }
-            const double *gap = ANT ? ga : nullptr;
-            const int m = max(n, 0);
-            if (staged) {
+            read_tables(item, 1);
+        }
+        share.store(S, nstage);
+    }
+    __syncthreads();
+    // Four lanes per target: lane q of target i takes every fourth group of four list
+    // slots, starting at group q; the four partial sums are added across the lanes (a fixed
+    // butterfly) and lane 0 writes.  With four lanes a brick's targets (about 385) take two
+    // passes of 256 whose waves spread evenly over the four SIMDs; two lanes left a quarter
+    // of the waves idle and one SIMD with the most work (8% slower).
+    constexpr int kL = 4;
+    const int q = tid & (kL - 1);
+    const ushort4 *l4 = reinterpret_cast<const ushort4 *>(A.nbr16);
+    const BrickConsts C(P);
+    for (int cur = 0;; cur ^= 1) {
+        const int4 nx = S.tab[cur ^ 1].head;
+        int item = ne;  // the brick after the next one: its number arrives during the pair loop
+        if (tid == 0 && nx.x >= 0) item = (int)gridDim.x + atomicAdd(A.work, 1);
+        if (hd.w <= kFarSlot) {
+            for (int base = hd.y; base < hd.z; base += kBrickThreads / kL) {
+                const int t = base + (tid / kL);
+                const bool active = t < hd.z;
+                const int col = active ? t : hd.y;
+                // the target: where its rates go, its record in the union, its list length
+                // and whether it has wall candidates
+                const int2 th = A.thead[col];
+                ushort4 cur4 = l4[(size_t)q * A.ls + col];
+                const BrickRec me = lds_rec<ND>(S, th.y & (kBrickCap - 1));
+                const int m = active ? (th.y >> kHeadCount) & kHeadCountMask : 0;
+                BrickTarget<ND, VISC, ANT, SUM> T(C, me);
+                if constexpr (ANT) lds_grad<ND>(S, th.y & (kBrickCap - 1), T.g);
+                double acc[3] = {0.0, 0.0, 0.0}, drho = 0.0;
                 // four LDS indices per 8-byte load, one group ahead of the pair terms
-                const ushort4 *l4 = reinterpret_cast<const ushort4 *>(nbr16);
                 const int ng = (m + 3) >> 2;
-                // rows clamped into the list (row 0 always exists) rather than a select between
-                // a load and a register: the select made the compiler keep cur4 in scratch
-                // and issue a flat load, whose wait also held up every LDS read
-                ushort4 cur4 = l4[(size_t)min(half, max(ng - 1, 0)) * ls + col];
-                for (int g = half; g < ng; g += kL) {
-                    const ushort4 nxt4 = l4[(size_t)min(g + kL, ng - 1) * ls + col];
+                for (int g = q; g < ng; g += kL) {
+                    // rows clamped into the list rather than a select between a load and a
+                    // register: the select made the compiler keep cur4 in scratch and issue
+                    // a flat load, whose wait also held up every LDS read
+                    const ushort4 nxt4 = l4[(size_t)min(g + kL, ng - 1) * A.ls + col];
                     // the candidates are independent chains without branches: two at a time
                     // interleave within the register budget of four waves per SIMD
 #pragma unroll 1
                     for (int h2 = 0; h2 < 2; h2++) {
                         // slots past the end of the list read the far record: exact zeros
                         const int ea = h2 ? cur4.z : cur4.x, eb = h2 ? cur4.w : cur4.y;
-                        const FluidNbr na = lds_fluid<ND>(S, ea);
-                        const FluidNbr nb = lds_fluid<ND>(S, eb);
+                        const BrickRec na = lds_rec<ND>(S, ea);
+                        const BrickRec nb = lds_rec<ND>(S, eb);
+                        double gna[3], gnb[3];
                         if constexpr (ANT) {
-                            double gna[3], gnb[3];
                             lds_grad<ND>(S, ea, gna);
                             lds_grad<ND>(S, eb, gnb);
-                            pair_fluid_masked<ND, VISC, true>(P, na, true, xa, va, rho_a, p_a,
-                                                              inv_rho_a, acc, drho, ga, gna);
-                            pair_fluid_masked<ND, VISC, true>(P, nb, true, xa, va, rho_a, p_a,
-                                                              inv_rho_a, acc, drho, ga, gnb);
-                        } else {
-                            pair_fluid_masked<ND, VISC, false, SUM>(P, na, true, xa, va, rho_a, p_a,
-                                                                    inv_rho_a, acc, drho);
-                            pair_fluid_masked<ND, VISC, false, SUM>(P, nb, true, xa, va, rho_a, p_a,
-                                                                    inv_rho_a, acc, drho);
                         }
+                        T.add(C, na, acc, drho, gna);
+                        T.add(C, nb, acc, drho, gnb);
                     }
                     cur4 = nxt4;
                 }
-            } else {
-                for (int k = half; k < m; k += kL) {
-                    const FluidNbr nb = load_fluid(F, nbr[(size_t)k * ls + col]);
-                    const double p0 = xa[0] - nb.a.x, p1 = xa[1] - nb.a.y;
-                    const double p2 = (ND == 3) ? xa[2] - nb.a.z : 0.0;
-                    const double d2 = dist2<ND>(p0, p1, p2);
-                    if (d2 <= P.R2 && d2 >= P.az2)
-                        pair_fluid<ND, SUM>(P, nb, xa, va, rho_a, p_a, inv_rho_a, acc, drho, gap);
+                T.scale(C, acc, drho);
+#pragma unroll
+                for (int o = 1; o < kL; o <<= 1) {
+#pragma unroll
+                    for (int d = 0; d < 3; d++) acc[d] += __shfl_xor(acc[d], o);
+                    drho += __shfl_xor(drho, o);
                 }
-                if (__any(n < 0))
-                    neighbour_sweep<ND, false, kFallbackCap, kBrickThreads, SUM>(
-                        P, F.start, F.x, F.y, F.z, P.hs_fluid, n < 0 && half == 0, F, Wv, lst, xa,
-                        va, rho_a, p_a, inv_rho_a, acc, drho, 0.0, gap);
-            }
+                if (active && q == 0) {
+                    // with wall candidates k_fluid_walls adds the wall sum and then gravity
+                    constexpr int rows = SUM ? ND : ND + 1;
+                    const bool walls = (th.y & kHeadWalls) != 0;
+                    double *o = A.dv + (size_t)th.x * rows;
 #pragma unroll
-            for (int o = 1; o < kL; o <<= 1) {
-#pragma unroll
-                for (int d = 0; d < 3; d++) acc[d] += __shfl_xor(acc[d], o);
-                drho += __shfl_xor(drho, o);
+                    for (int d = 0; d < ND; d++) o[d] = walls ? acc[d] : acc[d] + P.g[d];
+                    if constexpr (!SUM) o[ND] = drho;
+                }
             }
-            if (active && half == 0) {
-                // with wall candidates k_fluid_walls adds the wall sum and then gravity
-                constexpr int rows = SUM ? ND : ND + 1;
-                const int i = F.perm[s];
-                const bool walls = nw != 0;
-#pragma unroll
-                for (int d = 0; d < ND; d++)
-                    dv[(size_t)i * rows + d] = walls ? acc[d] : acc[d] + P.g[d];
-                if constexpr (!SUM) dv[(size_t)i * rows + ND] = drho;
-            }
+        } else {
+            brick_from_global<ND, SUM>(P, F, A, hd.y, hd.z);
         }
-        __syncthreads();  // the LDS is staged again for the next brick
+        if (nx.x < 0) break;  // uniform: no brick after this one
+        // (of a brick that does not stage, some record of its first row: a load without a
+        // branch around it keeps the share in registers)
+        const int nstage = nx.w <= kFarSlot ? nx.w : 0;
+        UnionShare<ND, ANT, SUM> share;
+        share.load(P, F, S.tab[cur ^ 1].gb, S.tab[cur ^ 1].lds, nstage);
+        // wave 0 is the first to finish (the oldest wave wins the issue): the tables of this
+        // brick are no longer read, so it fills them with those of the brick after the next
+        if (wave0) read_tables(__builtin_amdgcn_readfirstlane(item), cur);
+        __syncthreads();  // every wave has finished with the staged union
+        hd = nx;
+        share.store(S, nstage);
+        __syncthreads();
+    }
+}
+
+// The bricks that do not stage, which the mixed-precision pass (tpsph_mixed.hip) leaves to
+// FP64: the work[1] bricks it listed in bfall, taken by blocks in turn.
+template <int ND>
+__global__ void __launch_bounds__(kBrickThreads)
+    k_fluid_brick_global(DevParams P, FluidView F, BrickArgs A)
+{
+    P = with_sound(P);
+    const int ne = A.work[1];
+    for (int k = blockIdx.x; k < ne; k += gridDim.x) {
+        const int b = A.bfall[k];
+        brick_from_global<ND, false>(P, F, A, A.bstart[b], A.bstart[b + 1]);
     }
 }
 
@@ -2169,7 +2396,7 @@ int update_fluid(tpsph_handle *h, const double *v, const double *u, bool gathere
                 ListsArgs{h->ord, h->ls, h->cap_f, h->nbr, h->cnt, h->cap_w, h->wnbr, h->wcnt,
                           h->wtargets, h->counters + 2, h->counters + 3, h->wall_near,
                           h->brow_gb, h->brow_lds, h->bntot,
-                          h->bricks ? reinterpret_cast<unsigned long long *>(h->nbr16) : nullptr});
+                          h->bricks ? reinterpret_cast<unsigned long long *>(h->nbr16) : nullptr, h->thead});
             TRY(launch_check(h, "k_lists"));
         }
         // the fluid kernel of this kick lowers the flag
@@ -2233,6 +2460,12 @@ int prepare_impl(tpsph_handle *h, const double *v, const double *u, bool gathere
     return TPSPH_OK;
 }
 
+BrickArgs brick_args(const tpsph_handle *h, double *dv)
+{
+    return {h->ord, h->bstart, h->nel, h->counters, h->bwork, h->brow_gb, h->brow_lds, h->bntot,
+            h->nbr16, h->thead, h->nbr, h->cnt, h->wcnt, h->ls, dv, h->bfall};
+}
+
 template <int ND>
 int kick_impl(tpsph_handle *h, double *dv, const double *v, const double *u, bool gathered)
 {
@@ -2255,10 +2488,8 @@ int kick_impl(tpsph_handle *h, double *dv, const double *v, const double *u, boo
         }
         if (h->search == TPSPH_SEARCH_LISTS && h->bricks && h->mixed) {
             TRY(launch_fluid_brick_mixed(h, dv));
-            hipLaunchKernelGGL((k_fluid_brick<ND, true>), dim3(std::max(1, std::min(h->nbricks, h->n_cu))),
-                dim3(kBrickThreads), 0, h->stream, h->flag, h->P, h->fluid_view(), h->wall_view(),
-                h->ord, h->bstart, h->nel, h->counters, h->bwork, h->brow_gb, h->brow_lds, h->bntot,
-                h->nbr16, h->nbr, h->cnt, h->wnbr, h->wcnt, h->ls, dv, h->bfall);
+            hipLaunchKernelGGL((k_fluid_brick_global<ND>), dim3(std::max(1, std::min(h->nbricks, h->n_cu))),
+                dim3(kBrickThreads), 0, h->stream, h->P, h->fluid_view(), brick_args(h, dv));
             if (nw > 0)
                 hipLaunchKernelGGL((k_fluid_walls<ND>), dim3(gate_blocks(4 * (int64_t)nf)), dim3(kBlock), 0, h->stream,
                     h->P, h->fluid_view(), h->wall_view(), h->ord, h->wtargets, h->counters + 2,
@@ -2267,19 +2498,17 @@ int kick_impl(tpsph_handle *h, double *dv, const double *v, const double *u, boo
             const int vm = visc_mode(h->P);
             const bool ant = h->P.ddgrad != nullptr, sum = h->P.summation != 0;
             const auto brick =
-                ant   ? (vm == kViscNone    ? k_fluid_brick<ND, false, kViscNone, true>
-                         : vm == kViscAlpha ? k_fluid_brick<ND, false, kViscAlpha, true>
-                                            : k_fluid_brick<ND, false, kViscAlphaBeta, true>)
-                : sum ? (vm == kViscNone    ? k_fluid_brick<ND, false, kViscNone, false, true>
-                         : vm == kViscAlpha ? k_fluid_brick<ND, false, kViscAlpha, false, true>
-                                            : k_fluid_brick<ND, false, kViscAlphaBeta, false, true>)
-                      : (vm == kViscNone    ? k_fluid_brick<ND, false, kViscNone>
-                         : vm == kViscAlpha ? k_fluid_brick<ND, false, kViscAlpha>
-                                            : k_fluid_brick<ND, false, kViscAlphaBeta>);
+                ant   ? (vm == kViscNone    ? k_fluid_brick<ND, kViscNone, true>
+                         : vm == kViscAlpha ? k_fluid_brick<ND, kViscAlpha, true>
+                                            : k_fluid_brick<ND, kViscAlphaBeta, true>)
+                : sum ? (vm == kViscNone    ? k_fluid_brick<ND, kViscNone, false, true>
+                         : vm == kViscAlpha ? k_fluid_brick<ND, kViscAlpha, false, true>
+                                            : k_fluid_brick<ND, kViscAlphaBeta, false, true>)
+                      : (vm == kViscNone    ? k_fluid_brick<ND, kViscNone>
+                         : vm == kViscAlpha ? k_fluid_brick<ND, kViscAlpha>
+                                            : k_fluid_brick<ND, kViscAlphaBeta>);
             hipLaunchKernelGGL(brick, dim3(std::max(1, std::min(h->nbricks, h->n_cu))),
-                dim3(kBrickThreads), 0, h->stream, h->flag, h->P, h->fluid_view(), h->wall_view(),
-                h->ord, h->bstart, h->nel, h->counters, h->bwork, h->brow_gb, h->brow_lds, h->bntot,
-                h->nbr16, h->nbr, h->cnt, h->wnbr, h->wcnt, h->ls, dv, nullptr);
+                dim3(kBrickThreads), 0, h->stream, h->flag, h->P, h->fluid_view(), brick_args(h, dv));
             const auto walls = sum ? k_fluid_walls<ND, true> : k_fluid_walls<ND, false>;
             if (nw > 0)
                 hipLaunchKernelGGL(walls, dim3(gate_blocks(4 * (int64_t)nf)), dim3(kBlock), 0, h->stream,
@@ -2981,7 +3210,7 @@ int tpsph_create(const tpsph_params *params, int64_t n_fluid, int64_t n_wall,
         CTRY(dalloc(h, &h->counters, 4));
         // the brick kernel (with DensityDiffusionAntuono its records also carry the density
         // gradients) whenever every brick's union rows fit one scan block
-        h->bricks = P.maxr <= kBrickMaxRows;
+        h->bricks = P.maxr <= (P.brick_cap == kBrickCapGrad ? kBrickMaxRowsGrad : kBrickMaxRows);
         if (h->bricks) {
             CTRY(dalloc(h, &h->brow_gb, (size_t)h->nbricks * P.maxr));
             CTRY(dalloc(h, &h->brow_lds, (size_t)h->nbricks * (P.maxr + 1)));
@@ -2994,6 +3223,7 @@ int tpsph_create(const tpsph_params *params, int64_t n_fluid, int64_t n_wall,
             CTRY(dalloc(h, &h->bwork, 3));
             if (h->mixed) CTRY(dalloc(h, &h->bfall, (size_t)h->nbricks));
             CTRY(dalloc(h, &h->nbr16, (size_t)h->cap_f * h->ls));
+            CTRY(dalloc(h, &h->thead, (size_t)h->ls));
         }
         CTRY(dalloc(h, &h->bcount, (size_t)h->nbricks + 1));
         CTRY(dalloc(h, &h->bstart, (size_t)h->nbricks + 1));
@@ -3560,7 +3790,7 @@ void tpsph_destroy(tpsph_handle *h)
                     h->rhow, h->st_v, h->st_u, h->st_dv, h->st_du, h->sol_dv, h->sol_tv,
                     h->sol_tu, h->integ, h->nrebuild, h->adj_kb, h->adj_coef, h->adj_th,
                     h->adj_gw, h->adj_red, h->adj_vb, h->adj_ub, h->adj_tvb, h->adj_tub,
-                    h->adj_ck, h->adj_st, h->sum_rho, h->bfall};
+                    h->adj_ck, h->adj_st, h->sum_rho, h->bfall, h->thead};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     for (hipEvent_t e : h->event_pool) (void)hipEventDestroy(e);

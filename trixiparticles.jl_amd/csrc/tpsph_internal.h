@@ -30,6 +30,11 @@ constexpr int kBrickCapGrad = 1664;   // the same with DensityDiffusionAntuono's
                                       // gradients in the records (3D: 96 instead of 72 bytes)
 constexpr double kFar = 1e100;        // coordinate of the far record (never within R)
 constexpr int kBrickMaxRows = 256;    // union rows per brick (one scan block)
+constexpr int kBrickMaxRowsGrad = 144;  // the same beside the records of kBrickCapGrad
+// target header of the brick kernels (thead): {index in the caller's order, union record |
+// list length << kHeadCount | kHeadWalls with wall candidates}; a record needs 11 bits
+// (kBrickCap) and a length 13 (at most 4096)
+constexpr int kHeadCount = 11, kHeadCountMask = (1 << 13) - 1, kHeadWalls = 1 << 24;
 constexpr int kGateBlocks = 1024;     // grid-stride kernels behind the rebuild flag: a small
                                       // grid keeps the launch cheap when the flag is down
 constexpr int kPad = 4;               // NaN entries after the SoA coordinate arrays
@@ -857,6 +862,7 @@ struct tpsph_handle {
     int *brow_gb = nullptr, *brow_lds = nullptr, *bntot = nullptr, *nel = nullptr, *bwork = nullptr;
     int *bfall = nullptr;  // mixed precision: the bricks left to the FP64 pass
     unsigned short *nbr16 = nullptr;
+    int2 *thead = nullptr;  // target headers of the brick kernels, in the order of ord
     double *dyn = nullptr;       // adaptive sound speed: {c, B, av_c, dd2}
     double *wvel = nullptr;      // no-slip wall velocities (3 per wall particle)
     double *ddgrad = nullptr;    // DensityDiffusionAntuono: renormalised density gradients
