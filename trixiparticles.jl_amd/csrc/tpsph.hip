@@ -5,10 +5,10 @@
 //                    permutation, fluid state equation, and flag a rebuild if any particle
 //                    moved by more than half the skin since the last cell-list build;
 //   2. rebuild, only when flagged (every kernel reads the flag and returns otherwise; the
-//      fluid kernel of step 4 lowers the flag again):
-//      k_cells + k_scan_* + k_scatter + k_sort_cells (a stable counting sort on the linear
-//      cell index), k_gather<1> (gather again, snapshot of the build positions) and, with
-//      Verlet lists, k_lists (fluid and wall candidates within R + skin);
+//      fluid kernel of step 4 lowers the flag again): k_cells + k_scan + k_scatter (a counting
+//      sort on the linear cell index), k_gather<1> (makes the sort stable, gathers again,
+//      snapshot of the build positions) and, with Verlet lists, k_brick_lists (bricks, unions,
+//      fluid and wall candidates within R + skin);
 //   3. k_wall        Adami pressure extrapolation + inverse state equation per wall particle;
 //   4. the fused fluid-fluid + fluid-wall interaction + gravity, results scattered back to
 //      the caller's particle order: k_fluid_brick + k_fluid_walls (Verlet lists with the
@@ -51,9 +51,13 @@ namespace {
 
 template <int ND>
 __global__ void k_cells(const int *flag, DevParams P, int n, const double *__restrict__ x,
-                        int *__restrict__ cell, int *__restrict__ rank, int *__restrict__ count)
+                        int *__restrict__ cell, int *__restrict__ rank, int *__restrict__ count,
+                        unsigned long long *__restrict__ state, int words,
+                        int *__restrict__ zero, int nzero)
 {
     if (skip(flag)) return;
+    clear_scan_state(state, words);
+    if (zero && blockIdx.x == 0 && (int)threadIdx.x < nzero) zero[threadIdx.x] = 0;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const double *xi = x + (size_t)i * ND;
         int c0 = cell_1d(xi[0], P.lo[0], P.inv_cs[0], P.n[0]);
@@ -65,23 +69,6 @@ __global__ void k_cells(const int *flag, DevParams P, int n, const double *__res
     }
 }
 
-// Processing order of the list kernels: the cell-sorted particles grouped by bricks of cells
-// (counted by k_gather<1>), so the targets of a block are a compact cluster and the union of
-// their neighbourhoods is small.  The order inside a brick follows the histogram atomics; it
-// only decides which lane handles which particle, never a result.
-// ord[t] = sorted index of the t-th particle in brick order; clears the brick histogram.
-__global__ void k_brick_scatter(const int *flag, int n, const int *__restrict__ bid,
-                                const int *__restrict__ rank, const int *__restrict__ bstart,
-                                int *__restrict__ ord, int *__restrict__ bcount)
-{
-    if (skip(flag)) return;
-    for (int s = blockIdx.x * blockDim.x + threadIdx.x; s < n; s += gridDim.x * blockDim.x) {
-        const int b = bid[s];
-        ord[bstart[b] + rank[s]] = s;
-        bcount[b] = 0;
-    }
-}
-
 // ------------------------------------------------------------------------------------------
 // gather into cell-sorted order + fluid state equation (wcsph/system.jl:426-438)
 //   MODE 0: runs when no rebuild is pending; flags one if a particle left its skin.  A block
@@ -89,9 +76,11 @@ __global__ void k_brick_scatter(const int *flag, int n, const int *__restrict__ 
 //           follows gathers everything again.
 //   MODE 1: runs after a rebuild; stores the build positions.
 // ------------------------------------------------------------------------------------------
-// MODE 1 with bcount also counts the particles of every brick of cells (the processing
-// order of the list kernels: see k_brick_scatter), recording each particle's brick and rank,
-// and zeroes the `nzero` counters of the list build.
+// MODE 1 takes the members of every cell in the order the histogram's atomics gave (permu) and
+// orders them by particle index on the way (the stable counting sort, whatever order the
+// atomics were served in): a particle's place is the number of members with a smaller index.
+// With bcount it also counts the particles of every brick of cells and lists the bricks that
+// hold any (nel, nne of them; k_cells cleared it).
 // FP32 position for the pre-test of the list build: relative to the grid origin, NaN
 // outside the grid box (the list build then leaves the particle to the FP64 test)
 template <int ND>
@@ -127,8 +116,9 @@ __global__ void k_gather(int *flag, int *work, DevParams P, const int *__restric
                          double *__restrict__ ys, double *__restrict__ zs,
                          double4 *__restrict__ rec, double2 *__restrict__ vol,
                          double *__restrict__ snap, int *__restrict__ iperm,
-                         int *__restrict__ bid, int *__restrict__ rank,
-                         int *__restrict__ bcount, int *__restrict__ zero, int nzero,
+                         const int *__restrict__ cell, const int *__restrict__ start,
+                         int *__restrict__ perm_out, int *__restrict__ bcount,
+                         int *__restrict__ nel, int *__restrict__ nne,
                          const int *__restrict__ noverflow, int *__restrict__ nrebuild,
                          float4 *__restrict__ xf)
 {
@@ -144,12 +134,20 @@ __global__ void k_gather(int *flag, int *work, DevParams P, const int *__restric
     // the loop bound is uniform per wavefront (blockDim is a multiple of 64): the brick
     // counting below works on whole wavefronts
     for (int s0 = blockIdx.x * blockDim.x; s0 < P.nf; s0 += gridDim.x * blockDim.x) {
-        const int s = s0 + (int)threadIdx.x;
+        int s = s0 + (int)threadIdx.x;
         const bool in = s < P.nf;
         int b = -1;          // brick of the particle (MODE 1 with bcount)
         bool moved = false;  // left its skin (MODE 0)
         if (in) {
             const int i = perm[s];
+            if constexpr (MODE == 1) {
+                const int c = cell[i];
+                const int c_end = start[c + 1];
+                int k = start[c];
+                s = k;
+                for (; k < c_end; k++) s += perm[k] < i ? 1 : 0;
+                perm_out[s] = i;
+            }
             double x[3] = {0.0, 0.0, 0.0}, vv[3] = {0.0, 0.0, 0.0};
 #pragma unroll
             for (int d = 0; d < ND; d++) {
@@ -192,27 +190,19 @@ __global__ void k_gather(int *flag, int *work, DevParams P, const int *__restric
         }
         if constexpr (MODE == 0) raise_rebuild_flag(flag, moved);
         if (MODE == 1 && bcount) {
-            // a wavefront holds consecutive cell-sorted particles, so equal bricks come in runs:
-            // the first lane of a run takes ranks for the whole run with one atomic, and lane l
-            // of the run gets base + l (a rank only decides which lane handles which particle)
+            // a wavefront holds consecutive cell-sorted particles, so equal bricks come in
+            // runs: the first lane of a run adds the run with one atomic, and whoever finds a
+            // brick empty lists it
             const int lane = (int)threadIdx.x & 63;
             const int prev = __shfl_up(b, 1);
             const bool head = lane == 0 || b != prev;
             const unsigned long long heads = __ballot(head);
-            const unsigned long long upto = (2ull << lane) - 1;  // lanes 0..lane (all for 63)
-            const int first = 63 - __clzll((long long)(heads & upto));
-            const unsigned long long after = heads & ~upto;
+            const unsigned long long after = heads & ~((2ull << lane) - 1);
             const int end = after ? __ffsll((long long)after) - 1 : 64;
-            int base = 0;
-            if (head && b >= 0) base = atomicAdd(&bcount[b], end - first);
-            base = __shfl(base, first);
-            if (b >= 0) {
-                bid[s] = b;
-                rank[s] = base + (lane - first);
-            }
+            if (head && b >= 0 && atomicAdd(&bcount[b], end - lane) == 0)
+                nel[atomicAdd(nne, 1)] = b;
         }
     }
-    if (MODE == 1 && zero && blockIdx.x == 0 && (int)threadIdx.x < nzero) zero[threadIdx.x] = 0;
     if (MODE == 1 && nrebuild && blockIdx.x == 0 && threadIdx.x == 0) *nrebuild += 1;
 }
 
@@ -434,6 +424,30 @@ __global__ void __launch_bounds__(kBlock)
     if (active && q == 0) rho[s] = sum;
 }
 
+// Arguments of the brick kernels (see tpsph_handle).
+struct BrickArgs {
+    const int *ord, *nne;
+    int *work;
+    const int4 *bhead;
+    const int *uidx;
+    const unsigned short *nbr16;
+    const int2 *thead;
+    const int *nbr, *cnt, *wcnt;
+    int ls;
+    double *dv;
+    const int *bfall;
+};
+
+// The 16-byte (8-byte) field of the record at byte offset e16 (16 times its number).
+__device__ __forceinline__ double2 lds_at(const double2 *p, int e16)
+{
+    return *reinterpret_cast<const double2 *>(reinterpret_cast<const char *>(p) + e16);
+}
+__device__ __forceinline__ double lds_at(const double *p, int e16)
+{
+    return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(p) + (e16 >> 1));
+}
+
 // The fluid part of the sums brick by brick: the union staged in LDS as {x, y} and {z, m}
 // fields (the far record: far away, zero mass), each target summing m W over its list's LDS
 // indices, four lanes per target; the particle itself (m W(0)) and the wall part as in
@@ -442,47 +456,33 @@ __global__ void __launch_bounds__(kBlock)
 template <int ND>
 struct SumSmem {
     double2 p0[kBrickCap], p1[kBrickCap];  // {x, y}, {z, m} (2D: {0, m})
-    int row_gb[kBrickMaxRows], row_lds[kBrickMaxRows + 1];
     int item;
 };
 
 template <int ND>
 __global__ void __launch_bounds__(kBrickThreads)
-    k_sum_density_brick(DevParams P, FluidView F, WallView Wv, const int *__restrict__ ord,
-                        const int *__restrict__ bstart, const int *__restrict__ nel,
-                        const int *__restrict__ nne, int *__restrict__ work,
-                        const int *__restrict__ brow_gb, const int *__restrict__ brow_lds,
-                        const int *__restrict__ bntot, const unsigned short *__restrict__ nbr16,
-                        const int *__restrict__ nbr, const int *__restrict__ cnt,
-                        const int *__restrict__ wnbr, const int *__restrict__ wcnt, int ls,
-                        double *__restrict__ rho)
+    k_sum_density_brick(DevParams P, FluidView F, WallView Wv, BrickArgs A,
+                        const int *__restrict__ wnbr, double *__restrict__ rho)
 {
     __shared__ SumSmem<ND> S;
     const int tid = threadIdx.x;
-    const int ne = *nne;
+    const int ne = *A.nne, ls = A.ls;
     const int cap = P.brick_cap;
     while (true) {
-        if (tid == 0) S.item = atomicAdd(&work[2], 1);
+        if (tid == 0) S.item = atomicAdd(&A.work[2], 1);
         __syncthreads();
         const int item = S.item;
         if (item >= ne) break;
-        const int b = nel[item];
-        const int t0 = bstart[b], t1 = bstart[b + 1];
-        const int ntot = bntot[b];
+        const int4 hd = A.bhead[item];
+        const int t0 = hd.x, t1 = hd.y, ntot = hd.z;
         const bool staged = ntot <= cap - 1;
         if (staged) {
-            for (int r = tid; r <= P.maxr; r += kBrickThreads) {
-                if (r < P.maxr) S.row_gb[r] = brow_gb[(size_t)b * P.maxr + r];
-                S.row_lds[r] = brow_lds[(size_t)b * (P.maxr + 1) + r];
-            }
             if (tid == 0) {  // the far record
                 S.p0[cap - 1] = make_double2(kFar, kFar);
                 S.p1[cap - 1] = make_double2(kFar, 0.0);
             }
-            __syncthreads();
             for (int i = tid; i < ntot; i += kBrickThreads) {
-                const int r = bsearch_le(S.row_lds, P.maxr + 1, i);
-                const int g = S.row_gb[r] + (i - S.row_lds[r]);
+                const int g = A.uidx[hd.w + i];
                 const double4 a = F.rec[2 * (size_t)g];
                 S.p0[i] = make_double2(a.x, a.y);
                 S.p1[i] = make_double2(ND == 3 ? a.z : 0.0, F.vol[g].y);
@@ -494,14 +494,14 @@ __global__ void __launch_bounds__(kBrickThreads)
             const int t = base + tid / 4;
             const bool active = t < t1;
             const int col = active ? t : t0;
-            const int s = ord[col];
+            const int s = A.ord[col];
             const double4 a = F.rec[2 * (size_t)s];
             const double x0 = a.x, x1 = a.y, x2 = (ND == 3) ? a.z : 0.0;
             double sum = (q == 0) ? F.vol[s].y * wendland_c2(P, 0.0) : 0.0;
-            const int n = active ? cnt[col] : 0;
+            const int n = active ? A.cnt[col] : 0;
             if (staged) {
-                const ushort4 *l4 = reinterpret_cast<const ushort4 *>(nbr16);
-                const int ng = (max(n, 0) + 3) >> 2;
+                const ushort4 *l4 = reinterpret_cast<const ushort4 *>(A.nbr16);
+                const int ng = list_rows(max(n, 0));
                 // rows clamped into the list rather than a select between a load and a
                 // register (which made the compiler issue flat loads)
                 ushort4 cur4 = l4[(size_t)min(q, max(ng - 1, 0)) * ls + col];
@@ -510,7 +510,7 @@ __global__ void __launch_bounds__(kBrickThreads)
                     const unsigned short e4[4] = {cur4.x, cur4.y, cur4.z, cur4.w};
 #pragma unroll
                     for (int k = 0; k < 4; k++) {
-                        const double2 b0 = S.p0[e4[k]], b1 = S.p1[e4[k]];
+                        const double2 b0 = lds_at(S.p0, e4[k]), b1 = lds_at(S.p1, e4[k]);
                         const double d2 = dist2<ND>(x0 - b0.x, x1 - b0.y, (ND == 3) ? x2 - b1.x : 0.0);
                         // the far record (and the slots past the list) add zero mass
                         if (d2 <= P.R2) sum += b1.y * wendland_c2(P, sqrt(d2));
@@ -519,7 +519,7 @@ __global__ void __launch_bounds__(kBrickThreads)
                 }
             } else if (n >= 0) {
                 for (int k = q; k < n; k += 4) {
-                    const int j = nbr[(size_t)k * ls + col];
+                    const int j = A.nbr[(size_t)k * ls + col];
                     const double4 c = F.rec[2 * (size_t)j];
                     const double d2 = dist2<ND>(x0 - c.x, x1 - c.y, (ND == 3) ? x2 - c.z : 0.0);
                     if (d2 <= P.R2) sum += F.vol[j].y * wendland_c2(P, sqrt(d2));
@@ -534,7 +534,7 @@ __global__ void __launch_bounds__(kBrickThreads)
                         if (d2 <= P.R2 && j != s) sum += F.vol[j].y * wendland_c2(P, sqrt(d2));
                     }
             }
-            const int nw = (active && P.nw > 0) ? wcnt[col] : 0;
+            const int nw = (active && P.nw > 0) ? A.wcnt[col] : 0;
             if (nw > 0) {
                 for (int k = q; k < nw; k += 4) {
                     const double4 xw = Wv.pos[wnbr[(size_t)k * ls + col]];
@@ -607,26 +607,19 @@ __global__ void k_wall_near(DevParams P, int nw, const double4 *__restrict__ wpo
 // lanes of a wavefront read one contiguous 256-byte row per slot.  A particle with more
 // candidates than the capacity stores count -1 and walks the cells in the kick instead.
 // ------------------------------------------------------------------------------------------
-// The union rows of the brick of a target, for the LDS indices of its list (the records the
-// brick kernel stages): row r of the union covers the cells (uy0 + r % nuy, uz0 + r / nuy)
-// and holds the cell-sorted particles gb[r] ... in LDS slots lds[r] .. lds[r + 1] - 1.
-struct BrickRows {
-    const int *gb, *lds;
-    int uy0, uz0, nuy;
-};
+// Broadcast of lane I of each quad (four consecutive lanes) to the whole quad (DPP).
+template <int I>
+__device__ __forceinline__ int quad_bcast(int v)
+{
+    return __builtin_amdgcn_mov_dpp(v, I * 0x55, 0xF, 0xF, false);
+}
 
 // Verlet list of fluid particle s (sorted index) in column col: the candidates within the
-// list radius, in the pencils' order.  BRICK: also the 16-bit LDS indices of the entries in
-// the union of the target's brick, four per 8-byte group (the slots past the end of the list
-// point at the far record); ok turns false if an entry lies outside the union (the brick
-// then does not stage).
-template <int ND, bool WALL, bool BRICK = false>
+// list radius, in the pencils' order (the walls' lists and the bricks that do not stage).
+template <int ND, bool WALL>
 __device__ __forceinline__ void build_list(const DevParams &P, const FluidView &F,
                                            const WallView &Wv, int s, int col, int ls, int cap,
-                                           int *__restrict__ nbr, int *__restrict__ cnt,
-                                           const BrickRows &br = BrickRows{},
-                                           unsigned long long *__restrict__ nbr16 = nullptr,
-                                           bool *ok = nullptr)
+                                           int *__restrict__ nbr, int *__restrict__ cnt)
 {
     const double xa = F.x[s], ya = F.y[s], za = (ND == 3) ? F.z[s] : 0.0;
     const int *start = WALL ? Wv.start : F.start;
@@ -643,22 +636,7 @@ __device__ __forceinline__ void build_list(const DevParams &P, const FluidView &
     Pencils<ND> it;
     it.init(P, xa, ya, za, WALL ? P.hs_list_wall : P.hs_list_fluid);
     int n = 0, j, je;
-    int rg = 0, rl = 0, rl1 = 0;      // BRICK: the union row of the current pencil
-    bool row_ok = false, good = true;
-    unsigned long long pack = 0ull;    // BRICK: the LDS indices of the open group
-    const unsigned long long kFarSlot = (unsigned long long)(P.brick_cap - 1);
     while (it.next(P, start, j, je)) {
-        if constexpr (BRICK) {
-            // the pencil is the cell row (iy - 1, iz) of the fluid grid
-            const int ry = (it.iy - 1) - br.uy0, rz = ((ND == 3) ? it.iz : 0) - br.uz0;
-            const int r = ry + br.nuy * rz;
-            row_ok = ry >= 0 && ry < br.nuy && rz >= 0 && r < P.maxr;
-            if (row_ok) {
-                rg = br.gb[r];
-                rl = br.lds[r];
-                rl1 = br.lds[r + 1];
-            }
-        }
         // four candidates per step, their loads in flight together: the SoA arrays carry
         // kPad entries past their end, so the loads stay in bounds, and j + k < je masks the
         // candidates past the range (the list order is the candidates' order)
@@ -680,107 +658,26 @@ __device__ __forceinline__ void build_list(const DevParams &P, const FluidView &
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 if (j + k < je && hit[k] && (WALL || j + k != s)) {
-                    if (n < cap) {
-                        nbr[(size_t)n * ls + col] = j + k;
-                        if constexpr (BRICK) {
-                            const int e = rl + (j + k - rg);
-                            const bool in = row_ok && j + k >= rg && e < rl1 && e < P.brick_cap - 1;
-                            good = good && in;
-                            pack |= (in ? (unsigned long long)e : kFarSlot) << (16 * (n & 3));
-                            if ((n & 3) == 3) {
-                                nbr16[(size_t)(n >> 2) * ls + col] = pack;
-                                pack = 0ull;
-                            }
-                        }
-                    }
+                    if (n < cap) nbr[(size_t)n * ls + col] = j + k;
                     n++;
                 }
             }
         }
     }
-    if constexpr (BRICK) {
-        if (n <= cap && (n & 3) != 0) {  // pad the last group with the far record
-            for (int k = n & 3; k < 4; k++) pack |= kFarSlot << (16 * k);
-            nbr16[(size_t)(n >> 2) * ls + col] = pack;
-        }
-        *ok = good && n <= cap;
-    }
     cnt[col] = n <= cap ? n : -1;
-}
-
-// Fluid and wall lists of every fluid particle, stored in column t for the particle ord[t].
-// The wall lists only for particles in cells flagged near a wall (wall_near, whose reach
-// covers the wall list radius).  With bricks (nbr16 != nullptr) the fluid lists also get
-// their LDS indices in the union of the particle's brick (brick_union_body ran before), and
-// a brick with an entry outside its union, or with an overflowed list, is marked not to
-// stage (bntot = INT_MAX).
-template <int ND>
-__device__ __forceinline__ void
-    lists_body(int bx, int gx, const int *flag, DevParams P, FluidView F, WallView Wv, const int *__restrict__ ord,
-            int ls, int cap_f, int *__restrict__ nbr, int *__restrict__ cnt, int cap_w,
-            int *__restrict__ wnbr, int *__restrict__ wcnt, int *__restrict__ wtargets,
-            int *__restrict__ nwtargets, int *__restrict__ noverflow,
-            const unsigned char *__restrict__ wall_near, const int *__restrict__ brow_gb,
-            const int *__restrict__ brow_lds, int *__restrict__ bntot,
-            unsigned long long *__restrict__ nbr16, int2 *__restrict__ thead)
-{
-    if (skip(flag)) return;
-    for (int t = bx * kBlock + threadIdx.x; t < P.nf; t += gx * kBlock) {
-        const int s = ord[t];
-        const int c0 = cell_1d(F.x[s], P.lo[0], P.inv_cs[0], P.n[0]);
-        const int c1 = cell_1d(F.y[s], P.lo[1], P.inv_cs[1], P.n[1]);
-        const int c2 = (ND == 3) ? cell_1d(F.z[s], P.lo[2], P.inv_cs[2], P.n[2]) : 0;
-        int b = -1, self = 0;
-        if (nbr16) {
-            const int bxi = c0 / P.bc[0], byi = c1 / P.bc[1], bzi = c2 / P.bc[2];
-            b = bxi + P.nb[0] * (byi + P.nb[1] * bzi);
-            if (bntot[b] > P.brick_cap - 1) b = -1;  // the brick's union does not stage
-        }
-        if (b >= 0) {
-            const int byi = c1 / P.bc[1], bzi = c2 / P.bc[2];
-            const BrickRows br{brow_gb + (size_t)b * P.maxr, brow_lds + (size_t)b * (P.maxr + 1),
-                               byi * P.bc[1] - P.ur[1], (ND == 3) ? bzi * P.bc[2] - P.ur[2] : 0,
-                               P.bc[1] + 2 * P.ur[1]};
-            // the target's own record in the union
-            const int row = (c1 - br.uy0) + br.nuy * (((ND == 3) ? c2 : 0) - br.uz0);
-            self = br.lds[row] + (s - br.gb[row]);
-            bool ok = self >= br.lds[row] && self < br.lds[row + 1] && self < P.brick_cap - 1;
-            if (!ok) self = 0;
-            bool in_union = true;
-            build_list<ND, false, true>(P, F, Wv, s, t, ls, cap_f, nbr, cnt, br, nbr16, &in_union);
-            ok = ok && in_union;
-            if (!ok) bntot[b] = INT_MAX;
-        } else {
-            build_list<ND, false>(P, F, Wv, s, t, ls, cap_f, nbr, cnt);
-        }
-        // an overflowed list walks the cells, which need the SoA coordinates every kick
-        if (cnt[t] < 0) atomicAdd(noverflow, 1);
-        if (P.nw > 0) {
-            if (wall_near[c0 + P.n[0] * (c1 + P.n[1] * c2)]) {
-                build_list<ND, true>(P, F, Wv, s, t, ls, cap_w, wnbr, wcnt);
-                if (wtargets && wcnt[t] != 0) wtargets[atomicAdd(nwtargets, 1)] = t;
-            } else {
-                wcnt[t] = 0;
-            }
-        }
-        if (thead)
-            thead[t] = make_int2(F.perm[s], self | max(cnt[t], 0) << kHeadCount |
-                                                (P.nw > 0 && wcnt[t] != 0 ? kHeadWalls : 0));
-    }
 }
 
 // Verlet lists of the wall particles (wall-sorted order w) over the fluid: candidates within
 // R + skin/2 of the static wall particle, for the Adami pass.
 template <int ND>
 __device__ __forceinline__ void
-    wall_lists_body(int bx, int gx, const int *flag, DevParams P, FluidView F, const double4 *__restrict__ wpos,
+    wall_lists_body(int bx, int gx, DevParams P, FluidView F, const double4 *__restrict__ wpos,
                  int lw, int cap, int *__restrict__ nbr, int *__restrict__ cnt,
                  int *__restrict__ active, int *__restrict__ nactive, double *__restrict__ pw,
                  double *__restrict__ rhow, double2 *__restrict__ wpv, double *__restrict__ wvel)
 {
     P = with_sound(P);
-    if (skip(flag)) return;
-    for (int w = bx * kBlock + threadIdx.x; w < P.nw; w += gx * kBlock) {
+    for (int w = bx * kListThreads + threadIdx.x; w < P.nw; w += gx * kListThreads) {
         const double4 xw = wpos[w];
         const float4 xwf = list_f32<ND>(P, xw.x, xw.y, xw.z);
         Pencils<ND> it;
@@ -809,13 +706,6 @@ __device__ __forceinline__ void
         else
             active[atomicAdd(nactive, 1)] = w;
     }
-}
-
-// Broadcast of lane I of each quad (four consecutive lanes) to the whole quad (DPP).
-template <int I>
-__device__ __forceinline__ int quad_bcast(int v)
-{
-    return __builtin_amdgcn_mov_dpp(v, I * 0x55, 0xF, 0xF, false);
 }
 
 // Fluid kernel over the Verlet lists.
@@ -953,113 +843,32 @@ __global__ void __launch_bounds__(kBlock)
 
 // ------------------------------------------------------------------------------------------
 // Bricks in LDS.  A brick is a block of bc[0] x bc[1] x bc[2] cells; its targets are the
-// fluid particles in those cells (ord[bstart[b] .. bstart[b+1])).  Its union is every fluid
+// fluid particles in those cells (ord[t0 .. t1), columns of the lists).  Its union is every fluid
 // particle in a cell row (y, z) near the brick, trimmed in x: the cells within the list radius
 // R + skin of the brick box, as contiguous ranges of the cell-sorted arrays.  Every Verlet list
-// entry of a target lies in the union of its brick, so after one coalesced staging pass of the
-// union into LDS the pair terms read every candidate from LDS.  The lists also store the
-// candidate's LDS index (u16, four slots per ushort4; the slots past the end of a list hold
-// the index of the far record, kBrickCap - 1, which no target reaches).  A brick whose union
+// entry of a target lies in the union of its brick, so after one staging pass of the union
+// into LDS the pair terms read every candidate from LDS, and the list of a target holds record
+// numbers of the union (16 bits, list_place; the places past the end of a list in its last
+// rows hold the far record, brick_cap - 1, which no target reaches).  uidx holds the sorted
+// index of every union record, the union of a brick from bhead.w on.  A brick whose union
 // does not leave room for the far record, or with a target whose list overflowed, is marked
-// (bntot = INT_MAX) and its targets read their candidates from global memory.
+// (union size INT_MAX) and its targets have int lists and read their candidates from global
+// memory.
+//
+// Without staging (h->bricks false: the union rows of a brick exceed kBrickMaxRows) every brick
+// takes the int lists.
 // ------------------------------------------------------------------------------------------
-
-// Union rows of every brick (one block per brick, grid-stride) and, in the first block, the
-// list of non-empty bricks.  Row r = (cy - (by bc[1] - ur[1])) + nuy (cz - (bz bc[2] - ur[2])).
-template <int ND>
-__device__ __forceinline__ void
-    brick_union_body(int bx, int gx, const int *flag, DevParams P, const int *__restrict__ start,
-                  const int *__restrict__ bstart, int nbricks, int *__restrict__ brow_gb,
-                  int *__restrict__ brow_lds, int *__restrict__ bntot, int *__restrict__ nel,
-                  int *__restrict__ nne)
-{
-    if (skip(flag)) return;
-    __shared__ int scan_buf[kBlock];
-    const int tid = threadIdx.x;
-    if (bx == 0) {
-        // the non-empty bricks in brick order (the order the brick kernel takes them in;
-        // neighbouring bricks in flight share their unions in L2)
-        int carry = 0;
-        for (int c = 0; c < nbricks; c += kScanTile) {
-            const int b0 = c + tid * kScanItems;
-            int f[kScanItems], n = 0;
-#pragma unroll
-            for (int k = 0; k < kScanItems; k++) {
-                const int b = b0 + k;
-                f[k] = (b < nbricks && bstart[b + 1] > bstart[b]) ? 1 : 0;
-                n += f[k];
-            }
-            int tot;
-            int pos = carry + block_exclusive_scan(n, scan_buf, tot);
-#pragma unroll
-            for (int k = 0; k < kScanItems; k++)
-                if (f[k]) nel[pos++] = b0 + k;
-            carry += tot;
-        }
-        if (tid == 0) *nne = carry;
-    }
-    const int nuy = P.bc[1] + 2 * P.ur[1];
-    for (int b = bx; b < nbricks; b += gx) {
-        // only the bricks with targets are staged or looked up (most of a tank's bricks hold
-        // no fluid); the condition is uniform over the block
-        if (bstart[b + 1] == bstart[b]) continue;
-        const int bx = b % P.nb[0], by = (b / P.nb[0]) % P.nb[1], bz = b / (P.nb[0] * P.nb[1]);
-        const int X0 = bx * P.bc[0], X1 = min(X0 + P.bc[0], P.n[0]) - 1;
-        const int Y0 = by * P.bc[1], Y1 = min(Y0 + P.bc[1], P.n[1]) - 1;
-        const int Z0 = (ND == 3) ? bz * P.bc[2] : 0;
-        const int Z1 = (ND == 3) ? min(Z0 + P.bc[2], P.n[2]) - 1 : 0;
-        const double m = P.hs_union;
-        const double bxlo = cell_lo(P, 0, X0, m), bxhi = cell_hi(P, 0, X1, m);
-        const double bylo = cell_lo(P, 1, Y0, m), byhi = cell_hi(P, 1, Y1, m);
-        const double bzlo = (ND == 3) ? cell_lo(P, 2, Z0, m) : 0.0;
-        const double bzhi = (ND == 3) ? cell_hi(P, 2, Z1, m) : 0.0;
-        int cntr = 0, gb = 0;
-        if (tid < P.maxr) {
-            const int cy = Y0 - P.ur[1] + tid % nuy;
-            const int cz = (ND == 3) ? Z0 - P.ur[2] + tid / nuy : 0;
-            if (cy >= 0 && cy < P.n[1] && cz >= 0 && cz < P.n[2]) {
-                const double dy = fmax(0.0, fmax(cell_lo(P, 1, cy, m) - byhi, bylo - cell_hi(P, 1, cy, m)));
-                double dz = 0.0;
-                if constexpr (ND == 3)
-                    dz = fmax(0.0, fmax(cell_lo(P, 2, cz, m) - bzhi, bzlo - cell_hi(P, 2, cz, m)));
-                const double r2 = P.rl_union2 - (dy * dy + dz * dz);
-                if (r2 >= 0.0) {
-                    const double rx = sqrt(r2) * (1.0 + 1e-9) + m;
-                    const int x0 = cell_1d(bxlo - rx, P.lo[0], P.inv_cs[0], P.n[0]);
-                    const int x1 = cell_1d(bxhi + rx, P.lo[0], P.inv_cs[0], P.n[0]);
-                    const int row = P.n[0] * (cy + P.n[1] * cz);
-                    gb = start[row + x0];
-                    cntr = start[row + x1 + 1] - gb;
-                }
-            }
-            brow_gb[(size_t)b * P.maxr + tid] = gb;
-        }
-        int tot;
-        const int lds0 = block_exclusive_scan(cntr, scan_buf, tot);
-        if (tid < P.maxr) brow_lds[(size_t)b * (P.maxr + 1) + tid] = lds0;
-        if (tid == 0) {
-            brow_lds[(size_t)b * (P.maxr + 1) + P.maxr] = tot;
-            bntot[b] = tot;
-        }
-    }
-}
-
 struct ListsArgs {
-    const int *ord;
-    int ls, cap_f;
-    int *nbr, *cnt;
-    int cap_w;
-    int *wnbr, *wcnt, *wtargets, *nwtargets, *noverflow;
+    const int *nel;
+    int *nne;  // counters (see tpsph_handle): [0] bricks ... [6] work counter
+    int *bcount, *ord, *tbase, *uidx;
+    int uidx_cap;
+    int4 *bhead;
+    int ls, cap_f, cap_w;
+    int *nbr, *cnt, *wnbr, *wcnt, *wtargets;
     const unsigned char *wall_near;
-    const int *brow_gb, *brow_lds;
-    int *bntot;
-    unsigned long long *nbr16;  // nullptr without bricks
-    int2 *thead;                // nullptr without bricks
-};
-struct UnionArgs {
-    const int *start, *bstart;
-    int nbricks;
-    int *brow_gb, *brow_lds, *bntot, *nel, *nne;
+    unsigned short *nbr16;  // nullptr: no brick stages
+    int2 *thead;
 };
 struct WallListsArgs {
     const double4 *wpos;
@@ -1070,62 +879,344 @@ struct WallListsArgs {
     double *wvel;
 };
 
-// The rebuild's union tables of the bricks (first nblocks_union blocks) beside the Verlet
-// lists of the wall particles (the Adami pass): both read only the new cell-sorted order.
-template <int ND>
-__global__ void __launch_bounds__(kBlock)
-    k_brick_union_and_walls(const int *flag, DevParams P, FluidView F, UnionArgs b,
-                            WallListsArgs w, int nblocks_union)
-{
-    if ((int)blockIdx.x < nblocks_union)
-        brick_union_body<ND>(blockIdx.x, nblocks_union, flag, P, b.start, b.bstart, b.nbricks,
-                             b.brow_gb, b.brow_lds, b.bntot, b.nel, b.nne);
-    else
-        wall_lists_body<ND>(blockIdx.x - nblocks_union, gridDim.x - nblocks_union, flag, P, F,
-                            w.wpos, w.lw, w.cap, w.nbr, w.cnt, w.active, w.nactive, w.pw, w.rhow,
-                            w.wpv, w.wvel);
-}
-
-// The fluid particles' Verlet lists (with their LDS indices when the bricks stage) and wall
-// lists, after the union tables.  Its candidate loads wait on L2 latency: a grid of one
-// particle per thread with registers bounded for six waves per SIMD (80 VGPRs, a few
-// spilled outside the candidate loop) builds the lists 9% faster than four waves per SIMD
-// at 92 VGPRs; eight waves (64 VGPRs) spill inside the loop and are slower.
-template <int ND>
-__global__ void __launch_bounds__(kBlock, 6)
-    k_lists(const int *flag, DevParams P, FluidView F, WallView Wv, ListsArgs a)
-{
-    lists_body<ND>(blockIdx.x, gridDim.x, flag, P, F, Wv, a.ord, a.ls, a.cap_f, a.nbr, a.cnt,
-                   a.cap_w, a.wnbr, a.wcnt, a.wtargets, a.nwtargets, a.noverflow, a.wall_near,
-                   a.brow_gb, a.brow_lds, a.bntot, a.nbr16, a.thead);
-}
-
-// Header and union row tables of one brick in LDS.
-template <int ROWS>
-struct BrickTables {
-    int gb[ROWS], lds[ROWS + 1];
-    int4 head;  // {brick or -1, first target, one past the last, union size}
-
-    // Those of brick nel[item] (none past ne), read by one wave.
-    __device__ __forceinline__ void read(const DevParams &P, const int *__restrict__ nel,
-                                         const int *__restrict__ bstart,
-                                         const int *__restrict__ bntot,
-                                         const int *__restrict__ brow_gb,
-                                         const int *__restrict__ brow_lds, int item, int ne,
-                                         int lane)
-    {
-        int4 h = make_int4(-1, 0, 0, 0);
-        if (item < ne) {
-            const int b = nel[item];
-            for (int r = lane; r <= P.maxr; r += 64) {
-                if (r < P.maxr) gb[r] = brow_gb[(size_t)b * P.maxr + r];
-                lds[r] = brow_lds[(size_t)b * (P.maxr + 1) + r];
-            }
-            h = make_int4(b, bstart[b], bstart[b + 1], bntot[b]);
-        }
-        if (lane == 0) head = h;
-    }
+struct ListsSmem {
+    // FP32 positions of the union (relative to the grid origin) and their padding
+    float x[kBrickCap + 4], y[kBrickCap + 4], z[kBrickCap + 4];
+    unsigned short list[kListArea];
+    unsigned short ctab[kCellTab];
+    int row_gb[kBrickMaxRows], row_lds[kBrickMaxRows + 1];
+    short row_x0[kBrickMaxRows], row_x1[kBrickMaxRows];
+    int trow_s[kBrickMaxRows], trow_t[kBrickMaxRows + 1];
+    int scan[kListThreads / 64];
+    int item, col0, ubase, bad;
 };
+
+// Exclusive scan over the kListThreads threads of a block.
+__device__ __forceinline__ int lists_scan(int value, int *s, int &total)
+{
+    const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+    int x = value;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int y = __shfl_up(x, off);
+        if (lane >= off) x += y;
+    }
+    if (lane == 63) s[wave] = x;
+    __syncthreads();
+    int below = 0;
+    total = 0;
+#pragma unroll
+    for (int w = 0; w < kListThreads / 64; w++) {
+        const int y = s[w];
+        below += w < wave ? y : 0;
+        total += y;
+    }
+    __syncthreads();  // s is free again
+    return below + x - value;
+}
+
+// Target `k` of the brick: its sorted index.
+__device__ __forceinline__ int lists_target(const ListsSmem &S, int nrows, int k)
+{
+    const int r = bsearch_le(S.trow_t, nrows, k);
+    return S.trow_s[r] + (k - S.trow_t[r]);
+}
+
+// Wall list of fluid particle s in column col, four lanes (q) to the particle: the pencils'
+// candidates four at a time, the hits placed by the quad's ballot.  Returns the count.
+template <int ND>
+__device__ __forceinline__ int wall_list_quad(const DevParams &P, const FluidView &F,
+                                              const WallView &Wv, int s, int col, int ls, int cap,
+                                              int q, int *__restrict__ nbr)
+{
+    const double xa = F.x[s], ya = F.y[s], za = (ND == 3) ? F.z[s] : 0.0;
+    const float4 xaf = F.xf[s];
+    const int quad = (int)threadIdx.x & 60;
+    Pencils<ND> it;
+    it.init(P, xa, ya, za, P.hs_list_wall);
+    int n = 0, j, je;
+    while (it.next(P, Wv.start, j, je)) {  // uniform over the quad
+        for (; j < je; j += 4) {
+            const int k = j + q;  // kPad entries follow the arrays
+            const float4 c = Wv.xf[k];
+            const float ex = xaf.x - c.x, ey = xaf.y - c.y, ez = (ND == 3) ? xaf.z - c.z : 0.f;
+            const float d2f = ex * ex + ey * ey + ez * ez;
+            bool hit = d2f <= P.wlist_in2;
+            if (!hit && !(d2f > P.wlist_out2) && k < je)
+                hit = dist2<ND>(xa - Wv.x[k], ya - Wv.y[k], (ND == 3) ? za - Wv.z[k] : 0.0) <= P.rl2_wall;
+            hit = hit && k < je;
+            const int hits = (int)(__ballot(hit) >> quad) & 15;
+            const int place = n + __popc(hits & ((1 << q) - 1));
+            if (hit && place < cap) nbr[(size_t)place * ls + col] = k;
+            n += __popc(hits);
+        }
+    }
+    return n <= cap ? n : -1;
+}
+
+// The lists of one brick's targets by quads: four lanes share a target, lane q testing the
+// candidates q, q + 4, ... of each union row near it, from LDS.  Returns false through S.bad
+// when a list overflowed (the brick then does not stage).
+template <int ND>
+__device__ __forceinline__ void brick_lists(const DevParams &P, const FluidView &F,
+                                            const WallView &Wv, const ListsArgs &A, ListsSmem &S,
+                                            int ntargets, int nrows, int uy0, int uz0, int nuy)
+{
+    const int tid = threadIdx.x, q = tid & 3, quad = tid & 60;
+    const int cap16 = (A.cap_f + 15) & ~15;
+    const int batch = max(1, min(kListThreads / 4, kListArea / cap16));
+    const int nry = 2 * P.lr[1] + 1, nr = nry * (ND == 3 ? 2 * P.lr[2] + 1 : 1);
+    constexpr int kRanges = (ND == 3 ? 25 : 9) / 4 + 1;  // rows per lane
+    const unsigned short far16 = (unsigned short)((P.brick_cap - 1) * 16);
+    for (int base = 0; base < ntargets; base += batch) {
+        const int tl = tid >> 2, k = base + tl;
+        const bool active = tl < batch && k < ntargets;
+        const int s = lists_target(S, nrows, active ? k : 0);
+        const double xa = F.x[s], ya = F.y[s], za = (ND == 3) ? F.z[s] : 0.0;
+        const float4 xaf = F.xf[s];
+        const int c0 = cell_1d(xa, P.lo[0], P.inv_cs[0], P.n[0]);
+        const int c1 = cell_1d(ya, P.lo[1], P.inv_cs[1], P.n[1]);
+        const int c2 = (ND == 3) ? cell_1d(za, P.lo[2], P.inv_cs[2], P.n[2]) : 0;
+        const int own = (c1 - uy0) + nuy * (c2 - uz0);
+        const int self = S.row_lds[own] + (s - S.row_gb[own]);
+        // the record ranges of the rows near the target (pencils): lane q has rows q, q + 4, ...
+        int range[kRanges];
+        const double hs = P.hs_list_fluid;
+#pragma unroll
+        for (int i = 0; i < kRanges; i++) {
+            const int r = 4 * i + q;
+            range[i] = 0;
+            const int cy = c1 + (ND == 3 ? r % nry : r) - P.lr[1];
+            const int cz = (ND == 3) ? c2 + r / nry - P.lr[2] : 0;
+            if (!active || r >= nr || cy < 0 || cy >= P.n[1] || cz < 0 || cz >= P.n[2]) continue;
+            const double dy = transverse(P, 1, cy, ya, hs);
+            const double dz = (ND == 3) ? transverse(P, 2, cz, za, hs) : 0.0;
+            const double r2 = P.R2 - fma(dy, dy, dz * dz);
+            if (r2 < 0.0) continue;
+            const double rx = (double)(__builtin_amdgcn_sqrtf((float)r2) * 1.000001f) + hs;
+            const int u = (cy - uy0) + nuy * (cz - uz0);
+            const int x0 = max(cell_1d(xa - rx, P.lo[0], P.inv_cs[0], P.n[0]), (int)S.row_x0[u]);
+            const int x1 = min(cell_1d(xa + rx, P.lo[0], P.inv_cs[0], P.n[0]), (int)S.row_x1[u]);
+            if (x0 > x1) continue;
+            const unsigned short *ct = S.ctab + u * P.ctab - S.row_x0[u];
+            range[i] = (int)ct[x0] | (int)ct[x1 + 1] << 16;
+        }
+        unsigned short *list = S.list + (active ? tl * cap16 : 0);
+        int n = 0;
+#pragma unroll
+        for (int r = 0; r < 4 * kRanges; r++) {
+            const int rg = r % 4 == 0   ? quad_bcast<0>(range[r / 4])
+                           : r % 4 == 1 ? quad_bcast<1>(range[r / 4])
+                           : r % 4 == 2 ? quad_bcast<2>(range[r / 4])
+                                        : quad_bcast<3>(range[r / 4]);
+            const int e = (int)((unsigned)rg >> 16);
+#pragma unroll 1
+            for (int b = rg & 0xffff; b < e; b += 4) {
+                const int k2 = b + q;
+                const float ex = xaf.x - S.x[k2], ey = xaf.y - S.y[k2];
+                const float ez = (ND == 3) ? xaf.z - S.z[k2] : 0.f;
+                const float d2f = ex * ex + ey * ey + ez * ez;
+                const bool valid = k2 < e && k2 != self;
+                bool hit = d2f <= P.list_in2;
+                if (!hit && !(d2f > P.list_out2) && valid) {  // the FP32 test's band (or NaN)
+                    const int u = bsearch_le(S.row_lds, P.maxr + 1, k2);
+                    const int j = S.row_gb[u] + (k2 - S.row_lds[u]);
+                    hit = dist2<ND>(xa - F.x[j], ya - F.y[j], (ND == 3) ? za - F.z[j] : 0.0) <= P.rl2_fluid;
+                }
+                hit = hit && valid;
+                const int hits = (int)(__ballot(hit) >> quad) & 15;
+                const int place = n + __popc(hits & ((1 << q) - 1));
+                if (hit && place < A.cap_f) list[list_place(place)] = (unsigned short)(k2 * 16);
+                n += __popc(hits);
+            }
+        }
+        if (active) {
+            const int col = S.col0 + k;
+            const bool fits = n <= A.cap_f;
+            if (fits) {
+                for (int p = n + q; p < ((n + 15) & ~15); p += 4) list[list_place(p)] = far16;
+                __builtin_amdgcn_wave_barrier();
+                ushort4 *out = reinterpret_cast<ushort4 *>(A.nbr16);
+                const ushort4 *rows = reinterpret_cast<const ushort4 *>(list);
+                const int nrow = list_rows(n);
+                for (int r = q; r < nrow; r += 4) out[(size_t)r * A.ls + col] = rows[r];
+            } else if (q == 0) {
+                S.bad = 1;
+            }
+            int nw = 0;
+            if (P.nw > 0 && A.wall_near[c0 + P.n[0] * (c1 + P.n[1] * c2)])
+                nw = wall_list_quad<ND>(P, F, Wv, s, col, A.ls, A.cap_w, q, A.wnbr);
+            if (q == 0) {
+                A.ord[col] = s;
+                A.cnt[col] = fits ? n : -1;
+                A.tbase[col] = S.ubase;
+                if (P.nw > 0) {
+                    A.wcnt[col] = nw;
+                    if (A.wtargets && nw != 0) A.wtargets[atomicAdd(&A.nne[2], 1)] = col;
+                }
+                A.thead[col] = make_int2(F.perm[s], self | n << kHeadCount | (nw != 0 ? kHeadWalls : 0));
+            }
+        }
+        __syncthreads();  // S.list is filled again
+    }
+}
+
+// Int lists of the targets of a brick that does not stage, one thread per target.
+// walls: also their wall lists and headers (not when brick_lists has written them).
+template <int ND>
+__device__ __forceinline__ void brick_int_lists(const DevParams &P, const FluidView &F,
+                                                const WallView &Wv, const ListsArgs &A,
+                                                const ListsSmem &S, int ntargets, int nrows,
+                                                bool walls)
+{
+    for (int k = threadIdx.x; k < ntargets; k += kListThreads) {
+        const int s = lists_target(S, nrows, k), col = S.col0 + k;
+        build_list<ND, false>(P, F, Wv, s, col, A.ls, A.cap_f, A.nbr, A.cnt);
+        // an overflowed list walks the cells, which need the SoA coordinates every kick
+        if (A.cnt[col] < 0) atomicAdd(&A.nne[3], 1);
+        A.tbase[col] = -1;
+        if (!walls) continue;
+        A.ord[col] = s;
+        if (P.nw > 0) {
+            const int c0 = cell_1d(F.x[s], P.lo[0], P.inv_cs[0], P.n[0]);
+            const int c1 = cell_1d(F.y[s], P.lo[1], P.inv_cs[1], P.n[1]);
+            const int c2 = (ND == 3) ? cell_1d(F.z[s], P.lo[2], P.inv_cs[2], P.n[2]) : 0;
+            if (A.wall_near[c0 + P.n[0] * (c1 + P.n[1] * c2)]) {
+                build_list<ND, true>(P, F, Wv, s, col, A.ls, A.cap_w, A.wnbr, A.wcnt);
+                if (A.wtargets && A.wcnt[col] != 0) A.wtargets[atomicAdd(&A.nne[2], 1)] = col;
+            } else {
+                A.wcnt[col] = 0;
+            }
+        }
+    }
+}
+
+// The rebuild after the cell-sorted gather, in one launch: the first nblocks blocks take the
+// bricks (columns of the targets, union, lists of the targets over the fluid and the walls),
+// the others build the Verlet lists of the wall particles (the Adami pass); both read only
+// the new cell-sorted order.
+//
+// The list build is bound by the candidates' tests and their reads.  From global memory, one
+// thread per target, unions, brick order and lists took 860 us and five launches at 1.02M
+// particles; here 720 us: the candidates come from the union's FP32 positions in LDS, four
+// lanes per target, and the int list of a staged target (4 bytes per entry) is not written
+// any more.  Two blocks of 512 threads share a compute unit (about 70 KB each).
+template <int ND>
+__global__ void __launch_bounds__(kListThreads, 4)
+    k_brick_lists(const int *flag, DevParams P, FluidView F, WallView Wv, ListsArgs A,
+                  WallListsArgs W, int nblocks)
+{
+    if (skip(flag)) return;
+    if ((int)blockIdx.x >= nblocks) {
+        wall_lists_body<ND>(blockIdx.x - nblocks, gridDim.x - nblocks, P, F, W.wpos, W.lw, W.cap, W.nbr,
+                            W.cnt, W.active, W.nactive, W.pw, W.rhow, W.wpv, W.wvel);
+        return;
+    }
+    __shared__ ListsSmem S;
+    const int tid = threadIdx.x;
+    const int ne = A.nne[0];
+    const int nuy = P.bc[1] + 2 * P.ur[1];
+    for (int turn = blockIdx.x;; ) {
+        if (turn >= ne) break;  // uniform over the block
+        const int b = A.nel[turn];
+        const int bx = b % P.nb[0], by = (b / P.nb[0]) % P.nb[1], bz = b / (P.nb[0] * P.nb[1]);
+        const int X0 = bx * P.bc[0], X1 = min(X0 + P.bc[0], P.n[0]) - 1;
+        const int Y0 = by * P.bc[1], Y1 = min(Y0 + P.bc[1], P.n[1]) - 1;
+        const int Z0 = (ND == 3) ? bz * P.bc[2] : 0;
+        const int Z1 = (ND == 3) ? min(Z0 + P.bc[2], P.n[2]) - 1 : 0;
+        // the targets: the brick's cell rows
+        const int nty = Y1 - Y0 + 1, nrows = nty * (Z1 - Z0 + 1);
+        int ts = 0, tn = 0;
+        if (tid < nrows) {
+            const int row = P.n[0] * (Y0 + tid % nty + P.n[1] * (Z0 + tid / nty));
+            ts = F.start[row + X0];
+            tn = F.start[row + X1 + 1] - ts;
+        }
+        int ntargets;
+        const int tt = lists_scan(tn, S.scan, ntargets);
+        if (tid < nrows) {
+            S.trow_s[tid] = ts;
+            S.trow_t[tid] = tt;
+        }
+        // the union: its rows, then (where it fits) its records
+        const int uy0 = Y0 - P.ur[1], uz0 = (ND == 3) ? Z0 - P.ur[2] : 0;
+        int tot = INT_MAX;
+        if (A.nbr16) {
+            const double m = P.hs_union;
+            const double bxlo = cell_lo(P, 0, X0, m), bxhi = cell_hi(P, 0, X1, m);
+            const double bylo = cell_lo(P, 1, Y0, m), byhi = cell_hi(P, 1, Y1, m);
+            const double bzlo = (ND == 3) ? cell_lo(P, 2, Z0, m) : 0.0;
+            const double bzhi = (ND == 3) ? cell_hi(P, 2, Z1, m) : 0.0;
+            int cntr = 0, gb = 0, x0 = 0, x1 = -1;
+            if (tid < P.maxr) {
+                const int cy = uy0 + tid % nuy;
+                const int cz = (ND == 3) ? uz0 + tid / nuy : 0;
+                if (cy >= 0 && cy < P.n[1] && cz >= 0 && cz < P.n[2]) {
+                    const double dy = fmax(0.0, fmax(cell_lo(P, 1, cy, m) - byhi, bylo - cell_hi(P, 1, cy, m)));
+                    double dz = 0.0;
+                    if constexpr (ND == 3)
+                        dz = fmax(0.0, fmax(cell_lo(P, 2, cz, m) - bzhi, bzlo - cell_hi(P, 2, cz, m)));
+                    const double r2 = P.rl_union2 - (dy * dy + dz * dz);
+                    if (r2 >= 0.0) {
+                        const double rx = sqrt(r2) * (1.0 + 1e-9) + m;
+                        x0 = cell_1d(bxlo - rx, P.lo[0], P.inv_cs[0], P.n[0]);
+                        x1 = min(cell_1d(bxhi + rx, P.lo[0], P.inv_cs[0], P.n[0]), x0 + P.ctab - 2);
+                        const int row = P.n[0] * (cy + P.n[1] * cz);
+                        gb = F.start[row + x0];
+                        cntr = F.start[row + x1 + 1] - gb;
+                    }
+                }
+            }
+            const int lds0 = lists_scan(cntr, S.scan, tot);
+            if (tid < P.maxr) {
+                S.row_gb[tid] = gb;
+                S.row_lds[tid] = lds0;
+                S.row_x0[tid] = (short)x0;
+                S.row_x1[tid] = (short)x1;
+            }
+            if (tid == 0) S.row_lds[P.maxr] = tot;
+            if (tot > P.brick_cap - 1) tot = INT_MAX;
+        }
+        if (tid == 0) {
+            A.bcount[b] = 0;  // clear for the next rebuild
+            S.col0 = atomicAdd(&A.nne[4], ntargets);
+            S.ubase = tot < INT_MAX ? atomicAdd(&A.nne[5], tot) : 0;
+            S.bad = 0;
+            S.item = atomicAdd(&A.nne[6], 1);
+        }
+        __syncthreads();
+        const int next = nblocks + S.item;
+        if (tot < INT_MAX && S.ubase > A.uidx_cap - tot) tot = INT_MAX;  // uniform
+        if (tot < INT_MAX) {
+            for (int i = tid; i < tot; i += kListThreads) {
+                const int r = bsearch_le(S.row_lds, P.maxr + 1, i);
+                const int s = S.row_gb[r] + (i - S.row_lds[r]);
+                A.uidx[S.ubase + i] = s;
+                const float4 c = F.xf[s];
+                S.x[i] = c.x;
+                S.y[i] = c.y;
+                if constexpr (ND == 3) S.z[i] = c.z;
+            }
+            for (int i = tid; i < P.maxr * P.ctab; i += kListThreads) {
+                const int r = i / P.ctab, c = S.row_x0[r] + (i - r * P.ctab);
+                if (S.row_x1[r] < S.row_x0[r] || c > S.row_x1[r] + 1) continue;
+                const int cy = uy0 + r % nuy, cz = (ND == 3) ? uz0 + r / nuy : 0;
+                S.ctab[i] = (unsigned short)(S.row_lds[r] + F.start[P.n[0] * (cy + P.n[1] * cz) + c] - S.row_gb[r]);
+            }
+            __syncthreads();
+            brick_lists<ND>(P, F, Wv, A, S, ntargets, nrows, uy0, uz0, nuy);  // ends with a barrier
+            if (S.bad) {  // some list overflowed
+                tot = INT_MAX;
+                brick_int_lists<ND>(P, F, Wv, A, S, ntargets, nrows, false);
+            }
+        } else {
+            brick_int_lists<ND>(P, F, Wv, A, S, ntargets, nrows, true);
+        }
+        if (tid == 0) A.bhead[turn] = make_int4(S.col0, S.col0 + ntargets, tot, tot < INT_MAX ? S.ubase : 0);
+        turn = next;
+        __syncthreads();  // S is written again
+    }
+}
 
 // Staged union: one record per particle as four 16-byte fields and one 8-byte field, each in
 // an array of its own, read with one ds_read_b128 (ds_read_b64) per field.  The 16-byte
@@ -1137,14 +1228,14 @@ struct BrickTables {
 template <int ND, bool ANT = false>
 struct BrickSmem {
     static constexpr int CAP = (ANT && ND == 3) ? kBrickCapGrad : kBrickCap;
-    static constexpr int ROWS = (ANT && ND == 3) ? kBrickMaxRowsGrad : kBrickMaxRows;
     // 3D: p0 {x, y}, p1 {z, rho}, p2 {vx, vy}, p3 {vz, p};  2D: p0 {x, y}, p1 {rho, vx},
     // p2 {vy, p} (p3 unused); vol: V = m / rho (SummationDensity: m)
-    double2 p0[CAP], p1[CAP], p2[CAP], p3[ND == 3 ? CAP : 1];
+    // (vol first: the other fields of a record lie at constant offsets from 16 times its number)
     double vol[CAP];
+    double2 p0[CAP], p1[CAP], p2[CAP], p3[ND == 3 ? CAP : 1];
     double2 g0[ANT ? CAP : 1];
     double g1[(ANT && ND == 3) ? CAP : 1];
-    BrickTables<ROWS> tab[2];  // this brick's and the next one's
+    int4 head[2];  // bhead of this brick and of the next one
 };
 
 // A staged record in registers.
@@ -1153,14 +1244,14 @@ struct BrickRec {
 };
 
 template <int ND, bool ANT>
-__device__ __forceinline__ BrickRec lds_rec(const BrickSmem<ND, ANT> &S, int e)
+__device__ __forceinline__ BrickRec lds_rec(const BrickSmem<ND, ANT> &S, int e16)
 {
     BrickRec n;
-    const double2 a = S.p0[e], b = S.p1[e], c = S.p2[e];
+    const double2 a = lds_at(S.p0, e16), b = lds_at(S.p1, e16), c = lds_at(S.p2, e16);
     n.x[0] = a.x;
     n.x[1] = a.y;
     if constexpr (ND == 3) {
-        const double2 d = S.p3[e];
+        const double2 d = lds_at(S.p3, e16);
         n.x[2] = b.x;
         n.rho = b.y;
         n.v[0] = c.x;
@@ -1175,18 +1266,18 @@ __device__ __forceinline__ BrickRec lds_rec(const BrickSmem<ND, ANT> &S, int e)
         n.v[2] = 0.0;
         n.p = c.y;
     }
-    n.V = S.vol[e];
+    n.V = lds_at(S.vol, e16);
     return n;
 }
 
 // The density gradient of staged record e (DensityDiffusionAntuono).
 template <int ND, bool ANT>
-__device__ __forceinline__ void lds_grad(const BrickSmem<ND, ANT> &S, int e, double *g)
+__device__ __forceinline__ void lds_grad(const BrickSmem<ND, ANT> &S, int e16, double *g)
 {
-    const double2 a = S.g0[e];
+    const double2 a = lds_at(S.g0, e16);
     g[0] = a.x;
     g[1] = a.y;
-    g[2] = (ND == 3) ? S.g1[e] : 0.0;
+    g[2] = (ND == 3) ? lds_at(S.g1, e16) : 0.0;
 }
 
 // The pair constants of the staged pair loop (scalar registers).
@@ -1290,20 +1381,19 @@ struct UnionShare {
     double4 a[2], c[2];
     double V[2], g[2][ANT ? ND : 1];
 
-    __device__ __forceinline__ void load(const DevParams &P, const FluidView &F,
-                                         const int *row_gb, const int *row_lds, int ntot)
+    // s: the sorted indices of the two records
+    __device__ __forceinline__ void load(const DevParams &P, const FluidView &F, int2 s)
     {
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-            const int i = (int)threadIdx.x + h * kBrickThreads;
-            const int r = bsearch_le(row_lds, P.maxr + 1, i);
-            const int s = i < ntot ? row_gb[r] + (i - row_lds[r]) : 0;
-            a[h] = F.rec[2 * (size_t)s];
-            c[h] = F.rec[2 * (size_t)s + 1];
-            V[h] = SUM ? F.vol[s].y : F.vol[s].x;
+            const uint32_t o = (uint32_t)(h ? s.y : s.x);
+            a[h] = ldo(F.rec, o * 64u);
+            c[h] = ldo(F.rec, o * 64u + 32u);
+            const double2 vm = ldo(F.vol, o * 16u);
+            V[h] = SUM ? vm.y : vm.x;
             if constexpr (ANT) {
 #pragma unroll
-                for (int d = 0; d < ND; d++) g[h][d] = P.ddgrad[(size_t)s * ND + d];
+                for (int d = 0; d < ND; d++) g[h][d] = P.ddgrad[(size_t)o * ND + d];
             }
         }
     }
@@ -1392,29 +1482,29 @@ __device__ __forceinline__ void brick_from_global(const DevParams &P, const Flui
     }
 }
 
-struct BrickArgs {
-    const int *ord, *bstart, *nel, *nne;
-    int *work;
-    const int *brow_gb, *brow_lds, *bntot;
-    const unsigned short *nbr16;
-    const int2 *thead;
-    const int *nbr, *cnt, *wcnt;
-    int ls;
-    double *dv;
-    const int *bfall;
-};
+// The sorted indices of this thread's two records of a union of n records from entry `first`
+// of uidx on (past n those of its last record, 0 of an empty union).
+__device__ __forceinline__ int2 union_share(const int *__restrict__ uidx, int first, int n)
+{
+    const int last = max(n - 1, 0);
+    const int a = uidx[first + min((int)threadIdx.x, last)];
+    const int b = uidx[first + min((int)threadIdx.x + kBrickThreads, last)];
+    return n > 0 ? make_int2(a, b) : make_int2(0, 0);
+}
 
 // Fluid-fluid kernel over the bricks, one block of kBrickThreads per compute unit.  Targets
 // with wall candidates are completed by k_fluid_walls.
 //
 // What bounds it: 1024 threads with one 147 KB union leave a compute unit one block, so
-// nothing hides a brick's chain of dependent loads (claim, brick header, row tables, records,
-// target headers: 24k of 57k cycles per brick at 1.02M particles) but the block itself.  So
-// the chain runs one brick ahead: while a brick's pair loop runs, wave 0 claims the brick
-// after the next one and reads its header and row tables; every wave that has finished its
-// targets loads its share of the next union into registers before it waits for the others;
-// and the targets' own records come from the staged union (thead).  Measured at 1.02M
-// particles, with the pair terms of BrickTarget: 299 -> 247 us per launch.
+// nothing hides a brick's chain of dependent loads (claim, brick header, record numbers,
+// records, target headers: 24k of 57k cycles per brick at 1.02M particles) but the block
+// itself.  So the chain runs one brick ahead: while a brick's pair loop runs, wave 0 claims
+// the brick after the next one and reads its header; every wave that has finished its targets
+// loads its share of the next union into registers before it waits for the others, and then
+// the headers and first list rows of its next targets; and the targets' own records come from
+// the staged union (thead).  Measured at 1.02M particles, with the pair terms of BrickTarget:
+// 299 -> 247 us per launch, and with uidx in place of searches of the union rows, the list
+// layout of list_place and the target headers read ahead 222 us.
 // Bricks: the first gridDim.x in the order of the blocks, then from the work counter (which
 // k_gather<0> and the stage kernel reset).
 // VISC: visc_mode(P), the viscosity form of the pair loop.  ANT: DensityDiffusionAntuono
@@ -1428,7 +1518,6 @@ __global__ void __launch_bounds__(kBrickThreads)
     using Smem = BrickSmem<ND, ANT>;
     __shared__ Smem S;
     const int tid = threadIdx.x;
-    const bool wave0 = tid < 64;
     if (blockIdx.x == 0 && tid == 0) *flag = 0;  // the rebuild (if any) is done
     const int ne = *A.nne;
     if ((int)blockIdx.x >= ne) return;  // uniform: a block without a brick
@@ -1448,66 +1537,66 @@ __global__ void __launch_bounds__(kBrickThreads)
         }
         S.vol[kFarSlot] = 0.0;
     }
-    auto read_tables = [&](int item, int k) {  // wave 0
-        S.tab[k].read(P, A.nel, A.bstart, A.bntot, A.brow_gb, A.brow_lds, item, ne, tid);
+    auto read_head = [&](int item, int k) {  // lane 0 of wave 0
+        S.head[k] = item < ne ? A.bhead[item] : make_int4(-1, -1, 0, 0);
     };
-    if (wave0) read_tables(blockIdx.x, 0);
-    __syncthreads();
-    int4 hd = S.tab[0].head;  // {brick or -1, first target, one past the last, union size}
+    int4 hd = A.bhead[blockIdx.x];  // {first target, one past the last, union size, first entry}
+    int nstage = hd.z <= kFarSlot ? hd.z : 0;
     {
         UnionShare<ND, ANT, SUM> share;
-        const int nstage = hd.w <= kFarSlot ? hd.w : 0;
-        share.load(P, F, S.tab[0].gb, S.tab[0].lds, nstage);
-        if (wave0) {
-            int item = ne;
-            if ((int)gridDim.x < ne) {
-                if (tid == 0) item = (int)gridDim.x + atomicAdd(A.work, 1);
-                item = __builtin_amdgcn_readfirstlane(item);
-            }
-            read_tables(item, 1);
-        }
+        share.load(P, F, union_share(A.uidx, hd.w, nstage));
+        if (tid == 0) read_head((int)gridDim.x < ne ? (int)gridDim.x + atomicAdd(A.work, 1) : ne, 1);
         share.store(S, nstage);
     }
-    __syncthreads();
-    // Four lanes per target: lane q of target i takes every fourth group of four list
-    // slots, starting at group q; the four partial sums are added across the lanes (a fixed
-    // butterfly) and lane 0 writes.  With four lanes a brick's targets (about 385) take two
-    // passes of 256 whose waves spread evenly over the four SIMDs; two lanes left a quarter
-    // of the waves idle and one SIMD with the most work (8% slower).
+    // Four lanes per target: lane q of target i takes the entries q, q + 4, ... of its list;
+    // the four partial sums are added across the lanes (a fixed butterfly) and lane 0 writes.
+    // With four lanes a brick's targets (about 385) take two passes of 256 whose waves spread
+    // evenly over the four SIMDs; two lanes left a quarter of the waves idle and one SIMD
+    // with the most work (8% slower).
     constexpr int kL = 4;
     const int q = tid & (kL - 1);
     const ushort4 *l4 = reinterpret_cast<const ushort4 *>(A.nbr16);
     const BrickConsts C(P);
+    // header and first list row of this thread's first target
+    auto column = [&](const int4 &head, int base) {
+        const int t = base + tid / kL;
+        return t < head.y ? t : head.x;
+    };
+    int2 th = A.thead[column(hd, hd.x)];
+    ushort4 cur4 = l4[(size_t)q * A.ls + column(hd, hd.x)];
+    __syncthreads();
     for (int cur = 0;; cur ^= 1) {
-        const int4 nx = S.tab[cur ^ 1].head;
+        const int4 nx = S.head[cur ^ 1];
+        const int nx_stage = nx.z <= kFarSlot ? nx.z : 0;
+        const int2 us = union_share(A.uidx, nx.w, nx_stage);
         int item = ne;  // the brick after the next one: its number arrives during the pair loop
         if (tid == 0 && nx.x >= 0) item = (int)gridDim.x + atomicAdd(A.work, 1);
-        if (hd.w <= kFarSlot) {
-            for (int base = hd.y; base < hd.z; base += kBrickThreads / kL) {
-                const int t = base + (tid / kL);
-                const bool active = t < hd.z;
-                const int col = active ? t : hd.y;
-                // the target: where its rates go, its record in the union, its list length
-                // and whether it has wall candidates
-                const int2 th = A.thead[col];
-                ushort4 cur4 = l4[(size_t)q * A.ls + col];
-                const BrickRec me = lds_rec<ND>(S, th.y & (kBrickCap - 1));
+        if (hd.z <= kFarSlot) {
+            for (int base = hd.x; base < hd.y; base += kBrickThreads / kL) {
+                const bool active = base + tid / kL < hd.y;
+                const int col = column(hd, base);
+                if (base > hd.x) {
+                    th = A.thead[col];
+                    cur4 = l4[(size_t)q * A.ls + col];
+                }
+                const int self = (th.y & (kBrickCap - 1)) * 16;
                 const int m = active ? (th.y >> kHeadCount) & kHeadCountMask : 0;
-                BrickTarget<ND, VISC, ANT, SUM> T(C, me);
-                if constexpr (ANT) lds_grad<ND>(S, th.y & (kBrickCap - 1), T.g);
+                BrickTarget<ND, VISC, ANT, SUM> T(C, lds_rec<ND>(S, self));
+                if constexpr (ANT) lds_grad<ND>(S, self, T.g);
                 double acc[3] = {0.0, 0.0, 0.0}, drho = 0.0;
-                // four LDS indices per 8-byte load, one group ahead of the pair terms
-                const int ng = (m + 3) >> 2;
-                for (int g = q; g < ng; g += kL) {
+                // four entries per 8-byte load, one row ahead of the pair terms
+                const int rows = list_rows(m);
+                for (int r = q; r < rows; r += kL) {
                     // rows clamped into the list rather than a select between a load and a
                     // register: the select made the compiler keep cur4 in scratch and issue
                     // a flat load, whose wait also held up every LDS read
-                    const ushort4 nxt4 = l4[(size_t)min(g + kL, ng - 1) * A.ls + col];
+                    const ushort4 nxt4 = l4[(size_t)min(r + kL, rows - 1) * A.ls + col];
                     // the candidates are independent chains without branches: two at a time
-                    // interleave within the register budget of four waves per SIMD
+                    // interleave within the register budget of four waves per SIMD; entries
+                    // past the end of the list are the far record's: exact zeros
+                    const int k = list_row_entries(m, r);
 #pragma unroll 1
-                    for (int h2 = 0; h2 < 2; h2++) {
-                        // slots past the end of the list read the far record: exact zeros
+                    for (int h2 = 0; h2 < k; h2 += 2) {
                         const int ea = h2 ? cur4.z : cur4.x, eb = h2 ? cur4.w : cur4.y;
                         const BrickRec na = lds_rec<ND>(S, ea);
                         const BrickRec nb = lds_rec<ND>(S, eb);
@@ -1530,29 +1619,30 @@ __global__ void __launch_bounds__(kBrickThreads)
                 }
                 if (active && q == 0) {
                     // with wall candidates k_fluid_walls adds the wall sum and then gravity
-                    constexpr int rows = SUM ? ND : ND + 1;
+                    constexpr int vrows = SUM ? ND : ND + 1;
                     const bool walls = (th.y & kHeadWalls) != 0;
-                    double *o = A.dv + (size_t)th.x * rows;
+                    double *o = A.dv + (size_t)th.x * vrows;
 #pragma unroll
                     for (int d = 0; d < ND; d++) o[d] = walls ? acc[d] : acc[d] + P.g[d];
                     if constexpr (!SUM) o[ND] = drho;
                 }
             }
         } else {
-            brick_from_global<ND, SUM>(P, F, A, hd.y, hd.z);
+            brick_from_global<ND, SUM>(P, F, A, hd.x, hd.y);
         }
         if (nx.x < 0) break;  // uniform: no brick after this one
-        // (of a brick that does not stage, some record of its first row: a load without a
-        // branch around it keeps the share in registers)
-        const int nstage = nx.w <= kFarSlot ? nx.w : 0;
+        // (a load without a branch around it keeps the share in registers; a brick that does
+        // not stage reads some valid record)
         UnionShare<ND, ANT, SUM> share;
-        share.load(P, F, S.tab[cur ^ 1].gb, S.tab[cur ^ 1].lds, nstage);
-        // wave 0 is the first to finish (the oldest wave wins the issue): the tables of this
-        // brick are no longer read, so it fills them with those of the brick after the next
-        if (wave0) read_tables(__builtin_amdgcn_readfirstlane(item), cur);
+        share.load(P, F, us);
+        th = A.thead[column(nx, nx.x)];
+        cur4 = l4[(size_t)q * A.ls + column(nx, nx.x)];
+        // wave 0 is the first to finish (the oldest wave wins the issue), and this brick's
+        // header is no longer read
+        if (tid == 0) read_head(item, cur);
         __syncthreads();  // every wave has finished with the staged union
         hd = nx;
-        share.store(S, nstage);
+        share.store(S, nx_stage);
         __syncthreads();
     }
 }
@@ -1566,8 +1656,8 @@ __global__ void __launch_bounds__(kBrickThreads)
     P = with_sound(P);
     const int ne = A.work[1];
     for (int k = blockIdx.x; k < ne; k += gridDim.x) {
-        const int b = A.bfall[k];
-        brick_from_global<ND, false>(P, F, A, A.bstart[b], A.bstart[b + 1]);
+        const int4 hd = A.bhead[A.bfall[k]];
+        brick_from_global<ND, false>(P, F, A, hd.x, hd.y);
     }
 }
 
@@ -1797,47 +1887,33 @@ template <int ND>
 struct GradSmem {
     double2 p0[kBrickCap], p1[kBrickCap];  // {x, y}, {z, rho} (2D: {0, rho})
     double vol[kBrickCap];
-    int row_gb[kBrickMaxRows], row_lds[kBrickMaxRows + 1];
     int item;
 };
 
 template <int ND>
 __global__ void __launch_bounds__(kBrickThreads)
-    k_antuono_gradient_brick(DevParams P, FluidView F, const int *__restrict__ ord,
-                             const int *__restrict__ bstart, const int *__restrict__ nel,
-                             const int *__restrict__ nne, int *__restrict__ work,
-                             const int *__restrict__ brow_gb, const int *__restrict__ brow_lds,
-                             const int *__restrict__ bntot,
-                             const unsigned short *__restrict__ nbr16,
-                             const int *__restrict__ nbr, const int *__restrict__ cnt, int ls)
+    k_antuono_gradient_brick(DevParams P, FluidView F, BrickArgs A)
 {
     __shared__ GradSmem<ND> S;
     const int tid = threadIdx.x;
-    const int ne = *nne;
+    const int ne = *A.nne, ls = A.ls;
     const int cap = P.brick_cap;
     while (true) {
-        if (tid == 0) S.item = atomicAdd(&work[2], 1);
+        if (tid == 0) S.item = atomicAdd(&A.work[2], 1);
         __syncthreads();
         const int item = S.item;
         if (item >= ne) break;
-        const int b = nel[item];
-        const int t0 = bstart[b], t1 = bstart[b + 1];
-        const int ntot = bntot[b];
+        const int4 hd = A.bhead[item];
+        const int t0 = hd.x, t1 = hd.y, ntot = hd.z;
         const bool staged = ntot <= cap - 1;
         if (staged) {
-            for (int r = tid; r <= P.maxr; r += kBrickThreads) {
-                if (r < P.maxr) S.row_gb[r] = brow_gb[(size_t)b * P.maxr + r];
-                S.row_lds[r] = brow_lds[(size_t)b * (P.maxr + 1) + r];
-            }
             if (tid == 0) {  // the far record: far away, zero volume
                 S.p0[cap - 1] = make_double2(kFar, kFar);
                 S.p1[cap - 1] = make_double2(kFar, 1.0);
                 S.vol[cap - 1] = 0.0;
             }
-            __syncthreads();
             for (int i = tid; i < ntot; i += kBrickThreads) {
-                const int r = bsearch_le(S.row_lds, P.maxr + 1, i);
-                const int g = S.row_gb[r] + (i - S.row_lds[r]);
+                const int g = A.uidx[hd.w + i];
                 const double4 a = F.rec[2 * (size_t)g];
                 S.p0[i] = make_double2(a.x, a.y);
                 S.p1[i] = make_double2(ND == 3 ? a.z : 0.0, a.w);
@@ -1850,14 +1926,14 @@ __global__ void __launch_bounds__(kBrickThreads)
             const int t = base + tid / 4;
             const bool active = t < t1;
             const int col = active ? t : t0;
-            const int s = ord[col];
+            const int s = A.ord[col];
             const double4 a = F.rec[2 * (size_t)s];
             const double xa[3] = {a.x, a.y, ND == 3 ? a.z : 0.0};
-            const int n = active ? cnt[col] : 0;
+            const int n = active ? A.cnt[col] : 0;
             GradSums gs;
             if (staged) {
-                const ushort4 *l4 = reinterpret_cast<const ushort4 *>(nbr16);
-                const int ng = (max(n, 0) + 3) >> 2;
+                const ushort4 *l4 = reinterpret_cast<const ushort4 *>(A.nbr16);
+                const int ng = list_rows(max(n, 0));
                 // rows clamped into the list rather than a select between a load and a
                 // register (which made the compiler issue flat loads)
                 ushort4 cur4 = l4[(size_t)min(q, max(ng - 1, 0)) * ls + col];
@@ -1867,16 +1943,16 @@ __global__ void __launch_bounds__(kBrickThreads)
 #pragma unroll
                     for (int k = 0; k < 4; k++) {
                         const int e = e4[k];
-                        const double2 b0 = S.p0[e], b1 = S.p1[e];
+                        const double2 b0 = lds_at(S.p0, e), b1 = lds_at(S.p1, e);
                         const double p0 = xa[0] - b0.x, p1 = xa[1] - b0.y;
                         const double p2 = (ND == 3) ? xa[2] - b1.x : 0.0;
                         const double d2 = dist2<ND>(p0, p1, p2);
-                        grad_add<ND>(gs, grad_vk(P, S.vol[e], d2), a.w - b1.y, p0, p1, p2);
+                        grad_add<ND>(gs, grad_vk(P, lds_at(S.vol, e), d2), a.w - b1.y, p0, p1, p2);
                     }
                     cur4 = nxt4;
                 }
             } else {
-                grad_sums_global<ND>(P, F, gs, xa, a.w, n, nbr, col, ls, q);
+                grad_sums_global<ND>(P, F, gs, xa, a.w, n, A.nbr, col, ls, q);
             }
             grad_finish<ND>(P, gs, active && q == 0, s);
         }
@@ -2150,8 +2226,7 @@ __global__ void k_nbr(DevParams P, int nrows, const double *__restrict__ rx,
 struct EvalPairsArgs {
     int pair;           // TPSPH_PAIR_*
     int lists, bricks;  // the kick's pair search
-    const int *ord, *bstart, *bntot, *brow_gb, *brow_lds;
-    int nbricks;
+    const int *ord, *tbase, *uidx;
     const unsigned short *nbr16;
     const int *nbr, *cnt, *wnbr, *wcnt;
     int ls;
@@ -2226,18 +2301,11 @@ __global__ void k_eval_pairs(DevParams P, FluidView F, WallView Wv, EvalPairsArg
             walk(Wv.start, P.hs_wall);
     } else {
         const int n = a.cnt[r];
-        int b = -1;
-        if (a.bricks) b = bsearch_le(a.bstart, a.nbricks, r);
-        if (b >= 0 && a.bntot[b] <= P.brick_cap - 1) {
-            // the brick list: four LDS indices per group, the far record pads the last group
-            const int *gb = a.brow_gb + (size_t)b * P.maxr;
-            const int *lds = a.brow_lds + (size_t)b * (P.maxr + 1);
-            const int ng = (max(n, 0) + 3) >> 2;
-            for (int g = 0; g < 4 * ng; g++) {
-                const int e = a.nbr16[((size_t)(g >> 2) * a.ls + r) * 4 + (g & 3)];
-                if (e == P.brick_cap - 1) continue;
-                const int row_e = bsearch_le(lds, P.maxr + 1, e);
-                consider(gb[row_e] + (e - lds[row_e]));
+        const int first = a.bricks ? a.tbase[r] : -1;
+        if (first >= 0) {  // the list of union records
+            for (int k = 0; k < n; k++) {
+                const int p = list_place(k);
+                consider(a.uidx[first + a.nbr16[((size_t)(p >> 2) * a.ls + r) * 4 + (p & 3)] / 16]);
             }
         } else if (n >= 0) {
             for (int k = 0; k < n; k++) consider(a.nbr[(size_t)k * a.ls + r]);
@@ -2323,20 +2391,25 @@ namespace {
 
 
 
-// Cell list of n points x (ND doubles per point, caller order) into start / perm.
+// Cell list of n points x (ND doubles per point, caller order) into start / perm, the members
+// of a cell by their index; without `ordered` in the order of the histogram's atomics (the
+// gather that follows orders them).
 template <int ND>
 int build_cells(tpsph_handle *h, const int *flag, int n, const double *x, int *cell, int *rank,
-                int *count, int *start, int *perm)
+                int *count, int *start, int *perm, bool ordered = true, int *zero = nullptr,
+                int nzero = 0)
 {
     // count is zero on entry (cleared at create, and again by k_scatter)
     const int nc = h->P.ncells;
-    if (n > 0)
-        hipLaunchKernelGGL((k_cells<ND>), dim3(gate_blocks(n)), dim3(kBlock), 0, h->stream, flag, h->P, n, x, cell, rank, count);
+    // (n = 0 too: it clears the scan's state)
+    hipLaunchKernelGGL((k_cells<ND>), dim3(gate_blocks(n)), dim3(kBlock), 0, h->stream, flag, h->P, n, x, cell, rank, count,
+                       h->scan_state, scan_words(nc + 1), zero, nzero);
     TRY(launch_check(h, "k_cells"));
     TRY(scan(h, flag, count, start, nc + 1));
     if (n > 0) {
         hipLaunchKernelGGL((k_scatter), dim3(gate_blocks(n)), dim3(kBlock), 0, h->stream, flag, n, cell, rank, start, perm, count);
-        hipLaunchKernelGGL((k_sort_cells), dim3(gate_blocks(nc)), dim3(kBlock), 0, h->stream, flag, nc, start, perm);
+        if (ordered)
+            hipLaunchKernelGGL((k_sort_cells), dim3(gate_blocks(nc)), dim3(kBlock), 0, h->stream, flag, nc, start, perm);
     }
     return launch_check(h, "k_scatter/k_sort_cells");
 }
@@ -2353,7 +2426,7 @@ int update_fluid(tpsph_handle *h, const double *v, const double *u, bool gathere
         hipLaunchKernelGGL((k_set_i32), dim3(1), dim3(1), 0, h->stream, h->flag, 0);
         hipLaunchKernelGGL((k_gather<ND, 0>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream,
             h->flag, h->bwork, h->P, h->f_perm, u, v, h->f_mass, h->xs, h->ys, h->zs, h->rec, h->vol,
-            h->snap, nullptr, nullptr, nullptr, nullptr, nullptr, 0,
+            h->snap, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
             h->search == TPSPH_SEARCH_LISTS ? h->counters + 3 : nullptr, nullptr, nullptr);
         return launch_check(h, "k_gather<0>");
     }
@@ -2361,48 +2434,43 @@ int update_fluid(tpsph_handle *h, const double *v, const double *u, bool gathere
         TimedScope t(h, TPSPH_TIME_GATHER);
         hipLaunchKernelGGL((k_gather<ND, 0>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream,
             h->flag, h->bwork, h->P, h->f_perm, u, v, h->f_mass, h->xs, h->ys, h->zs, h->rec, h->vol,
-            h->snap, nullptr, nullptr, nullptr, nullptr, nullptr, 0,
+            h->snap, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
             h->search == TPSPH_SEARCH_LISTS ? h->counters + 3 : nullptr, nullptr, nullptr);
         TRY(launch_check(h, "k_gather<0>"));
     }
     {
         TimedScope t(h, TPSPH_TIME_CELL_LIST);
-        TRY(build_cells<ND>(h, h->flag, nf, u, h->f_cell, h->f_rank, h->f_count, h->f_start,
-                            h->f_perm));
         const bool lists = h->search == TPSPH_SEARCH_LISTS;
-        // with lists the gather also counts the bricks (f_cell / f_rank are free again after
-        // the cell list build) and zeroes the list-build counters
+        TRY(build_cells<ND>(h, h->flag, nf, u, h->f_cell, h->f_rank, h->f_count, h->f_start,
+                            h->f_permu, false, lists ? h->counters : nullptr, kCounters));
+        // the gather orders the members of every cell and, with lists, finds the bricks
         hipLaunchKernelGGL((k_gather<ND, 1>), dim3(gate_blocks(nf)), dim3(kBlock), 0, h->stream,
-            h->flag, nullptr, h->P, h->f_perm, u, v, h->f_mass, h->xs, h->ys, h->zs, h->rec, h->vol,
-            h->snap, h->iperm, lists ? h->f_cell : nullptr, lists ? h->f_rank : nullptr,
-            lists ? h->bcount : nullptr, lists ? h->counters : nullptr, 4, nullptr, h->nrebuild,
-            lists ? h->xf : nullptr);
+            h->flag, nullptr, h->P, h->f_permu, u, v, h->f_mass, h->xs, h->ys, h->zs, h->rec, h->vol,
+            h->snap, h->iperm, h->f_cell, h->f_start, h->f_perm, lists ? h->bcount : nullptr,
+            h->nel, h->counters, nullptr, h->nrebuild, lists ? h->xf : nullptr);
         if (lists) {
-            TRY(scan(h, h->flag, h->bcount, h->bstart, h->nbricks + 1));
-            hipLaunchKernelGGL((k_brick_scatter), dim3(gate_blocks(nf)), dim3(kBlock), 0, h->stream,
-                h->flag, nf, h->f_cell, h->f_rank, h->bstart, h->ord, h->bcount);
-            const int gu = h->bricks ? std::max(1, std::min(h->nbricks, kGateBlocks)) : 0;
-            const int gw = h->nw > 0 ? nblocks(h->nw) : 0;
-            if (gu + gw > 0)
-                hipLaunchKernelGGL((k_brick_union_and_walls<ND>), dim3(gu + gw), dim3(kBlock), 0,
-                    h->stream, h->flag, h->P, h->fluid_view(),
-                    UnionArgs{h->f_start, h->bstart, h->nbricks, h->brow_gb, h->brow_lds, h->bntot,
-                              h->nel, h->counters},
-                    WallListsArgs{h->wpos, h->lw, h->cap_a, h->anbr, h->acnt, h->wactive,
-                                  h->counters + 1, h->pw, h->rhow, h->wpv, h->wvel},
-                    gu);
-            hipLaunchKernelGGL((k_lists<ND>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream,
+            const int gb = std::max(1, std::min(h->nbricks, 2 * h->n_cu));
+            const int gw = (h->nw + kListThreads - 1) / kListThreads;
+            hipLaunchKernelGGL((k_brick_lists<ND>), dim3(gb + gw), dim3(kListThreads), 0, h->stream,
                 h->flag, h->P, h->fluid_view(), h->wall_view(),
-                ListsArgs{h->ord, h->ls, h->cap_f, h->nbr, h->cnt, h->cap_w, h->wnbr, h->wcnt,
-                          h->wtargets, h->counters + 2, h->counters + 3, h->wall_near,
-                          h->brow_gb, h->brow_lds, h->bntot,
-                          h->bricks ? reinterpret_cast<unsigned long long *>(h->nbr16) : nullptr, h->thead});
-            TRY(launch_check(h, "k_lists"));
+                ListsArgs{h->nel, h->counters, h->bcount, h->ord, h->tbase, h->uidx, (int)h->uidx_cap,
+                          h->bhead, h->ls, h->cap_f, h->cap_w, h->nbr, h->cnt, h->wnbr, h->wcnt,
+                          h->wtargets, h->wall_near, h->nbr16, h->thead},
+                WallListsArgs{h->wpos, h->lw, h->cap_a, h->anbr, h->acnt, h->wactive,
+                              h->counters + 1, h->pw, h->rhow, h->wpv, h->wvel},
+                gb);
+            TRY(launch_check(h, "k_brick_lists"));
         }
         // the fluid kernel of this kick lowers the flag
         TRY(launch_check(h, "k_gather<1>"));
     }
     return TPSPH_OK;
+}
+
+BrickArgs brick_args(const tpsph_handle *h, double *dv)
+{
+    return {h->ord, h->counters, h->bwork, h->bhead, h->uidx, h->nbr16, h->thead, h->nbr, h->cnt,
+            h->wcnt, h->ls, dv, h->bfall};
 }
 
 // Everything a kick does before the fluid pass: the sound speed (adaptive), the cell-sorted
@@ -2431,9 +2499,8 @@ int prepare_impl(tpsph_handle *h, const double *v, const double *u, bool gathere
         if (h->search == TPSPH_SEARCH_LISTS && h->bricks)
             hipLaunchKernelGGL((k_sum_density_brick<ND>),
                 dim3(std::max(1, std::min(h->nbricks, h->n_cu))), dim3(kBrickThreads), 0,
-                h->stream, h->P, h->fluid_view(), h->wall_view(), h->ord, h->bstart, h->nel,
-                h->counters, h->bwork, h->brow_gb, h->brow_lds, h->bntot, h->nbr16, h->nbr,
-                h->cnt, h->wnbr, h->wcnt, h->ls, h->sum_rho);
+                h->stream, h->P, h->fluid_view(), h->wall_view(), brick_args(h, nullptr), h->wnbr,
+                h->sum_rho);
         else if (h->search == TPSPH_SEARCH_LISTS)
             hipLaunchKernelGGL((k_sum_density_lists<ND>), dim3(nblocks(4 * (int64_t)nf)), dim3(kBlock),
                                0, h->stream, h->P, h->fluid_view(), h->wall_view(), h->ord, h->nbr,
@@ -2460,12 +2527,6 @@ int prepare_impl(tpsph_handle *h, const double *v, const double *u, bool gathere
     return TPSPH_OK;
 }
 
-BrickArgs brick_args(const tpsph_handle *h, double *dv)
-{
-    return {h->ord, h->bstart, h->nel, h->counters, h->bwork, h->brow_gb, h->brow_lds, h->bntot,
-            h->nbr16, h->thead, h->nbr, h->cnt, h->wcnt, h->ls, dv, h->bfall};
-}
-
 template <int ND>
 int kick_impl(tpsph_handle *h, double *dv, const double *v, const double *u, bool gathered)
 {
@@ -2478,8 +2539,7 @@ int kick_impl(tpsph_handle *h, double *dv, const double *v, const double *u, boo
             if (lists && h->bricks)
                 hipLaunchKernelGGL((k_antuono_gradient_brick<ND>),
                     dim3(std::max(1, std::min(h->nbricks, h->n_cu))), dim3(kBrickThreads), 0,
-                    h->stream, h->P, h->fluid_view(), h->ord, h->bstart, h->nel, h->counters,
-                    h->bwork, h->brow_gb, h->brow_lds, h->bntot, h->nbr16, h->nbr, h->cnt, h->ls);
+                    h->stream, h->P, h->fluid_view(), brick_args(h, nullptr));
             else
                 hipLaunchKernelGGL((k_antuono_gradient<ND>), dim3(nblocks(4 * (int64_t)nf)), dim3(kBlock), 0,
                                    h->stream, h->P, h->fluid_view(), lists ? h->ord : nullptr,
@@ -2686,10 +2746,22 @@ int tpsph::derive_params(const tpsph_params *params, int nf, int nw, const doubl
             if (d >= 1 && d < nd) rows *= P.bc[d] + 2 * P.ur[d];
         }
         P.maxr = rows;
+        const double reach = R + P.hs_list_fluid;  // of a target's pencils
+        for (int d = 0; d < 3; d++)
+            P.lr[d] = (d >= 1 && d < nd) ? (int)std::ceil(reach / P.cs[d]) : 0;
+        P.ctab = P.bc[0] + 2 * ((int)std::floor((rl + 4.0 * margin) / P.cs[0]) + 1) + 2;
         P.rl_union2 = (rl + margin) * (rl + margin);
         P.hs_union = margin;
     }
     return TPSPH_OK;
+}
+
+// Whether the bricks stage: the union rows of a brick, their cell offsets and the rows of a
+// target's list fit the tables of the list build.
+static bool brick_rows_ok(const DevParams &P)
+{
+    const int rows = (2 * P.lr[1] + 1) * (P.nd == 3 ? 2 * P.lr[2] + 1 : 1);
+    return P.maxr <= kBrickMaxRows && P.maxr * P.ctab <= kCellTab && rows <= (P.nd == 3 ? 25 : 9);
 }
 
 int tpsph::validate(const tpsph_params *p, int64_t nf, int64_t nw, const double *fm, const double *wx,
@@ -2965,13 +3037,13 @@ int noalloc_kick(tpsph_handle *h, unsigned char *base, size_t *bytes, const doub
 {
     const int nf = h->nf, nw = h->nw;
     const int nc = h->P.ncells;
-    const int tiles = (nc + 1 + kScanTile - 1) / kScanTile;
     ScratchLayout L{base};
     h->flag = L.take<int>(1);
-    h->scan_tiles = L.take<int>((size_t)tiles + 1);
+    h->scan_state = L.take<unsigned long long>((size_t)scan_words(nc + 1));
     h->f_cell = L.take<int>(nf);
     h->f_rank = L.take<int>(nf);
     h->f_perm = L.take<int>(nf);
+    h->f_permu = L.take<int>(nf);
     h->iperm = L.take<int>(nf);
     h->f_count = L.take<int>((size_t)nc + 1);
     h->f_start = L.take<int>((size_t)nc + 1);
@@ -3092,7 +3164,7 @@ int tpsph_create(const tpsph_params *params, int64_t n_fluid, int64_t n_wall,
     h->search = params->pair_search;
     // SummationDensity on the Verlet lists needs the brick kernel (P.maxr within one scan
     // block); the automatic choice takes the cell walk otherwise
-    const bool sum_lists_ok = !P.summation || P.maxr <= kBrickMaxRows;
+    const bool sum_lists_ok = !P.summation || brick_rows_ok(P);
     if (h->search == TPSPH_SEARCH_AUTO)
         h->search = (P.half_skin > 0.0 && sum_lists_ok) ? TPSPH_SEARCH_LISTS : TPSPH_SEARCH_CELLS;
     if (h->search == TPSPH_SEARCH_LISTS && !sum_lists_ok) {
@@ -3148,9 +3220,8 @@ int tpsph_create(const tpsph_params *params, int64_t n_fluid, int64_t n_wall,
 #define CTRY(expr) \
     if ((rc = (expr)) != TPSPH_OK) return cleanup_fail(rc)
     const int nf = h->nf, nw = h->nw;
-    const int tiles = (int)((ncells + 1 + kScanTile - 1) / kScanTile);
     h->mixed = params->precision == TPSPH_PRECISION_MIXED;
-    if (h->mixed && !(h->search == TPSPH_SEARCH_LISTS && P.maxr <= kBrickMaxRows &&
+    if (h->mixed && !(h->search == TPSPH_SEARCH_LISTS && brick_rows_ok(P) &&
                       params->use_density_diffusion != TPSPH_DIFFUSION_ANTUONO)) {
         delete h;
         return fail(nullptr, TPSPH_ERR_ARGUMENT,
@@ -3181,10 +3252,11 @@ int tpsph_create(const tpsph_params *params, int64_t n_fluid, int64_t n_wall,
         }
         P.dyn = h->dyn;
     }
-    CTRY(dalloc(h, &h->scan_tiles, (size_t)tiles + 1));
+    CTRY(dalloc(h, &h->scan_state, (size_t)scan_words((int)ncells + 1)));
     CTRY(dalloc(h, &h->f_cell, nf));
     CTRY(dalloc(h, &h->f_rank, nf));
     CTRY(dalloc(h, &h->f_perm, nf));
+    CTRY(dalloc(h, &h->f_permu, nf));
     CTRY(dalloc(h, &h->f_count, (size_t)ncells + 1));
     CTRY(dalloc(h, &h->f_start, (size_t)ncells + 1));
     CTRY(dalloc(h, &h->f_mass, nf));
@@ -3207,27 +3279,33 @@ int tpsph_create(const tpsph_params *params, int64_t n_fluid, int64_t n_wall,
         CTRY(dalloc(h, &h->nbr, (size_t)h->cap_f * h->ls));
         CTRY(dalloc(h, &h->cnt, nf));
         CTRY(dalloc(h, &h->ord, nf));
-        CTRY(dalloc(h, &h->counters, 4));
+        CTRY(dalloc(h, &h->counters, kCounters));
         // the brick kernel (with DensityDiffusionAntuono its records also carry the density
         // gradients) whenever every brick's union rows fit one scan block
-        h->bricks = P.maxr <= (P.brick_cap == kBrickCapGrad ? kBrickMaxRowsGrad : kBrickMaxRows);
+        h->bricks = brick_rows_ok(P);
         if (h->bricks) {
-            CTRY(dalloc(h, &h->brow_gb, (size_t)h->nbricks * P.maxr));
-            CTRY(dalloc(h, &h->brow_lds, (size_t)h->nbricks * (P.maxr + 1)));
-            CTRY(dalloc(h, &h->bntot, h->nbricks));
-            CTRY(dalloc(h, &h->nel, h->nbricks));
+            // a cell lies in the unions of at most `times` bricks along an axis
+            int64_t times = 1;
+            for (int d = 0; d < nd; d++) {
+                const int beyond = (int)std::floor((std::sqrt(P.rl_union2) + 4.0 * P.hs_union) / P.cs[d]) + 1;
+                times *= (2 * beyond + P.bc[d] - 1) / P.bc[d] + 1;
+            }
+            h->uidx_cap = std::min<int64_t>(std::max<int64_t>(times * nf, 1), INT_MAX);
+            CTRY(dalloc(h, &h->uidx, (size_t)h->uidx_cap));
             // [0] the brick kernels' work counter, [1] the bricks the mixed-precision pass
             // leaves to the FP64 pass (listed in bfall), [2] the work counter of the brick
             // gradient pass (DensityDiffusionAntuono); all cleared by the kick's gather or
             // the stage kernel
             CTRY(dalloc(h, &h->bwork, 3));
             if (h->mixed) CTRY(dalloc(h, &h->bfall, (size_t)h->nbricks));
-            CTRY(dalloc(h, &h->nbr16, (size_t)h->cap_f * h->ls));
+            CTRY(dalloc(h, &h->nbr16, (size_t)((h->cap_f + 15) / 16 * 16) * h->ls));
             CTRY(dalloc(h, &h->thead, (size_t)h->ls));
         }
-        CTRY(dalloc(h, &h->bcount, (size_t)h->nbricks + 1));
-        CTRY(dalloc(h, &h->bstart, (size_t)h->nbricks + 1));
-        if (hipMemset(h->bcount, 0, ((size_t)h->nbricks + 1) * sizeof(int)) != hipSuccess) {
+        CTRY(dalloc(h, &h->bcount, (size_t)h->nbricks));
+        CTRY(dalloc(h, &h->nel, (size_t)std::min<int64_t>(h->nbricks, nf)));
+        CTRY(dalloc(h, &h->bhead, (size_t)std::min<int64_t>(h->nbricks, nf)));
+        CTRY(dalloc(h, &h->tbase, nf));
+        if (hipMemset(h->bcount, 0, (size_t)h->nbricks * sizeof(int)) != hipSuccess) {
             h->last_error = "clearing the brick counts failed";
             return cleanup_fail(TPSPH_ERR_HIP);
         }
@@ -3494,8 +3572,7 @@ int tpsph_kick_pairs_csr(tpsph_handle *h, int32_t pair, int64_t *offsets, int32_
     if (!offsets) return fail(h, TPSPH_ERR_ARGUMENT, "offsets must not be NULL");
     if (!h->have_kick) return fail(h, TPSPH_ERR_STATE, "no kick has been evaluated yet");
     const bool lists = h->search == TPSPH_SEARCH_LISTS;
-    const EvalPairsArgs a{pair, lists ? 1 : 0, h->bricks ? 1 : 0, h->ord, h->bstart, h->bntot,
-                          h->brow_gb, h->brow_lds, h->nbricks, h->nbr16, h->nbr, h->cnt,
+    const EvalPairsArgs a{pair, lists ? 1 : 0, h->bricks ? 1 : 0, h->ord, h->tbase, h->uidx, h->nbr16, h->nbr, h->cnt,
                           h->wnbr, h->wcnt, h->ls, h->anbr, h->acnt, h->lw, h->w_perm};
     const int nrows = pair == TPSPH_PAIR_WALL_FLUID ? h->nw : h->nf;
     if ((pair != TPSPH_PAIR_FLUID_FLUID && h->nw == 0) || h->nf == 0) {
@@ -3782,10 +3859,10 @@ void tpsph_destroy(tpsph_handle *h)
     if (!h) return;
     (void)hipStreamSynchronize(h->stream);
     void *ptrs[] = {h->flag, h->f_cell, h->f_rank, h->f_count, h->f_start, h->f_perm,
-                    h->scan_tiles, h->f_mass, h->xs, h->ys, h->zs, h->xf, h->wxf, h->snap, h->rec, h->vol,
+                    h->scan_state, h->f_permu, h->f_mass, h->xs, h->ys, h->zs, h->xf, h->wxf, h->snap, h->rec, h->vol,
                     h->w_start, h->w_perm, h->wx, h->wy, h->wz, h->wpos, h->wpv, h->wall_near,
-                    h->pw, h->nbr, h->cnt, h->wnbr, h->wcnt, h->anbr, h->acnt, h->ord, h->bcount, h->bstart,
-                    h->brow_gb, h->brow_lds, h->bntot, h->nel, h->counters, h->wactive, h->bwork, h->nbr16,
+                    h->pw, h->nbr, h->cnt, h->wnbr, h->wcnt, h->anbr, h->acnt, h->ord, h->bcount, h->tbase,
+                    h->uidx, h->bhead, h->nel, h->counters, h->wactive, h->bwork, h->nbr16,
                     h->wtargets, h->iperm, h->dyn, h->vmax_part, h->wvel, h->ddgrad,
                     h->rhow, h->st_v, h->st_u, h->st_dv, h->st_du, h->sol_dv, h->sol_tv,
                     h->sol_tu, h->integ, h->nrebuild, h->adj_kb, h->adj_coef, h->adj_th,

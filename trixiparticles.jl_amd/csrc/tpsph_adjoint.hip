@@ -293,7 +293,9 @@ template <int ND, bool ACC>
 __global__ void __launch_bounds__(kBlock)
     k_adj_fluid(int *flag, DevParams P, AdjConsts K, FluidView F, WallView Wv,
                 const int *__restrict__ ord, const int *__restrict__ nbr,
-                const int *__restrict__ cnt, const int *__restrict__ wnbr,
+                const int *__restrict__ cnt, const int *__restrict__ tbase,
+                const int *__restrict__ uidx, const unsigned short *__restrict__ nbr16,
+                const int *__restrict__ wnbr,
                 const int *__restrict__ wcnt, int ls, const double4 *__restrict__ kb,
                 const double2 *__restrict__ coef, double *__restrict__ vb,
                 double *__restrict__ ub, double *__restrict__ th)
@@ -315,8 +317,7 @@ __global__ void __launch_bounds__(kBlock)
     double xb[3] = {0.0, 0.0, 0.0}, vbr[3] = {0.0, 0.0, 0.0};
     double rhob = 0.0, pb = 0.0, alpha = 0.0, delta = 0.0;
     const int n = nbr ? cnt[t] : -1;
-    for_each_candidate<ND, kAdjLanes>(P, nbr, active ? n : 0, ls, t, F.start, P.hs_fluid, a.x, a.y,
-                                      a.z, active ? q : kAdjLanes, [&](int j) {
+    auto pair = [&](int j) {
         // every load of the candidate at once: one round trip instead of two
         const double4 na = F.rec[2 * (size_t)j];
         const double4 nb = F.rec[2 * (size_t)j + 1];
@@ -356,7 +357,28 @@ __global__ void __launch_bounds__(kBlock)
         }
         rhob += qa.rho_b;
         pb += qa.p;
-    });
+    };
+    const int first = tbase ? tbase[t] : -1;
+    if (first >= 0) {
+        // the list of union records of the target's brick (list_place), a row of four entries
+        // and their sorted indices one row ahead of the pair terms
+        const ushort4 *l4 = reinterpret_cast<const ushort4 *>(nbr16);
+        const int rows = active ? list_rows(n) : 0;
+        ushort4 e4 = l4[(size_t)min(q, max(rows - 1, 0)) * ls + t];
+        for (int r = q; r < rows; r += kAdjLanes) {
+            const ushort4 next = l4[(size_t)min(r + kAdjLanes, rows - 1) * ls + t];
+            const int k = list_row_entries(n, r);
+            const int j4[4] = {uidx[first + (e4.x >> 4)], k > 1 ? uidx[first + (e4.y >> 4)] : 0,
+                               k > 2 ? uidx[first + (e4.z >> 4)] : 0,
+                               k > 3 ? uidx[first + (e4.w >> 4)] : 0};
+#pragma unroll 1
+            for (int i = 0; i < k; i++) pair(i == 0 ? j4[0] : i == 1 ? j4[1] : i == 2 ? j4[2] : j4[3]);
+            e4 = next;
+        }
+    } else {
+        for_each_candidate<ND, kAdjLanes>(P, nbr, active ? n : 0, ls, t, F.start, P.hs_fluid, a.x,
+                                          a.y, a.z, active ? q : kAdjLanes, pair);
+    }
     if (P.nw > 0) {
         const int nw = wnbr ? wcnt[t] : -1;
         for_each_candidate<ND, kAdjLanes>(P, wnbr, active ? nw : 0, ls, t, Wv.start, P.hs_wall,
@@ -544,8 +566,8 @@ int adjoint_passes(tpsph_handle *h, double *vb, double *ub)
     hipLaunchKernelGGL((k_adj_fluid<ND, ACC>), dim3(nblocks(kAdjLanes * (int64_t)h->nf)), dim3(kBlock), 0, h->stream,
                        h->flag, h->P, K, h->fluid_view(), h->wall_view(),
                        lists ? h->ord : nullptr, lists ? h->nbr : nullptr,
-                       lists ? h->cnt : nullptr, lists ? h->wnbr : nullptr,
-                       lists ? h->wcnt : nullptr, h->ls, h->adj_kb, h->adj_coef, vb, ub,
+                       lists ? h->cnt : nullptr, h->bricks ? h->tbase : nullptr, h->uidx, h->nbr16,
+                       lists ? h->wnbr : nullptr, lists ? h->wcnt : nullptr, h->ls, h->adj_kb, h->adj_coef, vb, ub,
                        h->adj_th);
     return launch_check(h, "k_adj_fluid");
 }

@@ -75,8 +75,10 @@ __device__ __forceinline__ int local_cell(const DevParams &Q, const double *x)
 template <int ND>
 __global__ void k_bcells(DevParams P, const CaseDev *__restrict__ cases,
                          const int *__restrict__ pcase, int n, const double *__restrict__ x,
-                         int *__restrict__ cell, int *__restrict__ rank, int *__restrict__ count)
+                         int *__restrict__ cell, int *__restrict__ rank, int *__restrict__ count,
+                         unsigned long long *__restrict__ state, int words)
 {
+    clear_scan_state(state, words);
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const CaseDev &cs = cases[pcase[i]];
         DevParams Q = P;
@@ -302,7 +304,7 @@ int batch_kick(tpsph_batch *b, double *dv, const double *v, const double *u)
     hipStream_t st = h->stream;
     if (nf == 0) return TPSPH_OK;
     hipLaunchKernelGGL((k_bcells<ND>), dim3(gate_blocks(nf)), dim3(kBlock), 0, st, h->P, b->cases,
-                       b->fcase, nf, u, h->f_cell, h->f_rank, h->f_count);
+                       b->fcase, nf, u, h->f_cell, h->f_rank, h->f_count, h->scan_state, scan_words(nc + 1));
     TRY(launch_check(h, "k_bcells"));
     TRY(scan(h, nullptr, h->f_count, h->f_start, nc + 1));
     hipLaunchKernelGGL((k_scatter), dim3(gate_blocks(nf)), dim3(kBlock), 0, st, nullptr, nf, h->f_cell,
@@ -486,11 +488,10 @@ int tpsph_batch_create(const tpsph_params *params, int32_t n_cases, const tpsph_
     int rc;
 #define BTRY(expr) \
     if ((rc = (expr)) != TPSPH_OK) return cleanup(rc)
-    const int tiles = (nc + 1 + kScanTile - 1) / kScanTile;
     BTRY(dalloc(h, &b->cases, n_cases));
     BTRY(dalloc(h, &b->fcase, nf));
     BTRY(dalloc(h, &b->wcase, nw));
-    BTRY(dalloc(h, &h->scan_tiles, (size_t)tiles + 1));
+    BTRY(dalloc(h, &h->scan_state, (size_t)scan_words(nc + 1)));
     BTRY(dalloc(h, &h->f_cell, nf));
     BTRY(dalloc(h, &h->f_rank, nf));
     BTRY(dalloc(h, &h->f_perm, nf));
@@ -546,9 +547,9 @@ int tpsph_batch_create(const tpsph_params *params, int32_t n_cases, const tpsph_
             if (rc == TPSPH_OK) {
                 hipStream_t st = h->stream;
                 if (nd == 2)
-                    hipLaunchKernelGGL((k_bcells<2>), dim3(gate_blocks(nw)), dim3(kBlock), 0, st, h->P, b->cases, wc_d, (int)nw, wall_coordinates, wcell, wrank, wcount);
+                    hipLaunchKernelGGL((k_bcells<2>), dim3(gate_blocks(nw)), dim3(kBlock), 0, st, h->P, b->cases, wc_d, (int)nw, wall_coordinates, wcell, wrank, wcount, h->scan_state, scan_words(nc + 1));
                 else
-                    hipLaunchKernelGGL((k_bcells<3>), dim3(gate_blocks(nw)), dim3(kBlock), 0, st, h->P, b->cases, wc_d, (int)nw, wall_coordinates, wcell, wrank, wcount);
+                    hipLaunchKernelGGL((k_bcells<3>), dim3(gate_blocks(nw)), dim3(kBlock), 0, st, h->P, b->cases, wc_d, (int)nw, wall_coordinates, wcell, wrank, wcount, h->scan_state, scan_words(nc + 1));
                 rc = scan(h, nullptr, wcount, h->w_start, nc + 1);
                 if (rc == TPSPH_OK) {
                     hipLaunchKernelGGL((k_scatter), dim3(gate_blocks(nw)), dim3(kBlock), 0, st, nullptr, (int)nw, wcell, wrank, h->w_start, h->w_perm, wcount);
@@ -662,7 +663,7 @@ void tpsph_batch_destroy(tpsph_batch *b)
     tpsph_handle *h = &b->h;
     (void)hipStreamSynchronize(h->stream);
     drop_graph(b);
-    void *ptrs[] = {b->cases, b->fcase, b->wcase, h->scan_tiles, h->f_cell, h->f_rank, h->f_perm,
+    void *ptrs[] = {b->cases, b->fcase, b->wcase, h->scan_state, h->f_cell, h->f_rank, h->f_perm,
                     h->f_count, h->f_start, h->f_mass, h->xs, h->ys, h->zs, h->rec, h->vol,
                     h->w_start, h->w_perm, h->wx, h->wy, h->wz, h->wpos, h->wpv, h->pw,
                     h->rhow, h->wall_near, h->sol_dv, h->sol_tv, h->sol_tu};

@@ -21,7 +21,7 @@ namespace tpsph {
 
 constexpr int kBlock = 256;  // 4 wavefronts of 64
 constexpr int kCap = 32;     // neighbour-list entries per lane and phase
-constexpr int kScanItems = 8;
+constexpr int kScanItems = 16;
 constexpr int kScanTile = kBlock * kScanItems;
 constexpr int kBrickThreads = 1024;   // threads of the brick kernel (one block per CU), two
                                       // per target
@@ -30,13 +30,16 @@ constexpr int kBrickCapGrad = 1664;   // the same with DensityDiffusionAntuono's
                                       // gradients in the records (3D: 96 instead of 72 bytes)
 constexpr double kFar = 1e100;        // coordinate of the far record (never within R)
 constexpr int kBrickMaxRows = 256;    // union rows per brick (one scan block)
-constexpr int kBrickMaxRowsGrad = 144;  // the same beside the records of kBrickCapGrad
 // target header of the brick kernels (thead): {index in the caller's order, union record |
 // list length << kHeadCount | kHeadWalls with wall candidates}; a record needs 11 bits
 // (kBrickCap) and a length 13 (at most 4096)
 constexpr int kHeadCount = 11, kHeadCountMask = (1 << 13) - 1, kHeadWalls = 1 << 24;
+constexpr int kListThreads = 512;     // threads of the list build, four per target
+constexpr int kListArea = 16384;      // 16-bit list entries a block of it holds in LDS
+constexpr int kCellTab = 5120;        // cell offsets of a union in LDS (at most 121 rows x 40)
 constexpr int kGateBlocks = 1024;     // grid-stride kernels behind the rebuild flag: a small
                                       // grid keeps the launch cheap when the flag is down
+constexpr int kCounters = 7;          // tpsph_handle::counters
 constexpr int kPad = 4;               // NaN entries after the SoA coordinate arrays
 
 // message of the last failed tpsph_create (tpsph_last_error(NULL))
@@ -76,6 +79,8 @@ struct DevParams {
     // union rows of a brick: cells beyond the brick along y and z, rows per brick, and the
     // radius (list radius + margin) and cell growth (margin) of the union
     int ur[3], maxr;
+    int lr[3];  // cells within the list radius of a cell along y and z (rows of a target's list)
+    int ctab;   // cell offsets per union row (cells of its x-range and one more, at most)
     double rl_union2, hs_union;
     // LDS records of a brick (kBrickCap, or kBrickCapGrad with DensityDiffusionAntuono in
     // 3D): a union of up to brick_cap - 1 particles stages, the last record is the far record
@@ -642,6 +647,23 @@ __device__ __forceinline__ int bsearch_le(const int *pre, int n, int i)
     return lo;
 }
 
+// Layout of a target's list of union records (nbr16), four lanes to a target: entry n belongs to
+// lane n & 3, whose entries come in groups of four, one ushort4 each.  Row r holds group r >> 2
+// of lane r & 3, column col is the target, slot-major like the int lists: the lanes of a quad
+// read consecutive entries at a time, mostly consecutive records of the union (neighbouring
+// LDS banks: 26% fewer conflicts than with whole groups dealt in turn), and no lane has more
+// than one entry above the others.  An entry is the record's number times 16, its byte offset
+// in an LDS array of 16-byte fields.
+// list_rows: the rows with entries of a list of n; list_row_entries: those of row r;
+// list_place: the place of entry n among the 4 ushorts of each row.
+__host__ __device__ __forceinline__ int list_rows(int n) { return 4 * (n >> 4) + ((n & 15) < 4 ? (n & 15) : 4); }
+__host__ __device__ __forceinline__ int list_row_entries(int n, int r)
+{
+    const int k = (n - (16 * (r >> 2) + (r & 3)) + 3) >> 2;
+    return k < 4 ? k : 4;
+}
+__host__ __device__ __forceinline__ int list_place(int n) { return (n & ~15) + 4 * (n & 3) + ((n >> 2) & 3); }
+
 // bounds of cell c along axis d grown by hs; border cells reach to infinity outwards
 __device__ __forceinline__ double cell_lo(const DevParams &P, int d, int c, double hs)
 {
@@ -695,12 +717,13 @@ __device__ __forceinline__ int block_exclusive_scan(int value, int *s, int &tota
 // the items lie within n), zeros past n
 __device__ __forceinline__ void scan_load(const int *p, int base, int n, bool vec, int *v)
 {
-    static_assert(kScanItems == 8, "two int4 per thread");
+    static_assert(kScanItems % 4 == 0, "whole int4 per thread");
     if (vec && base + kScanItems <= n) {
-        const int4 a = *reinterpret_cast<const int4 *>(p + base);
-        const int4 b = *reinterpret_cast<const int4 *>(p + base + 4);
-        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-        v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+#pragma unroll
+        for (int k = 0; k < kScanItems; k += 4) {
+            const int4 a = *reinterpret_cast<const int4 *>(p + base + k);
+            v[k] = a.x; v[k + 1] = a.y; v[k + 2] = a.z; v[k + 3] = a.w;
+        }
     } else {
 #pragma unroll
         for (int k = 0; k < kScanItems; k++) v[k] = (base + k < n) ? p[base + k] : 0;
@@ -710,8 +733,9 @@ __device__ __forceinline__ void scan_load(const int *p, int base, int n, bool ve
 __device__ __forceinline__ void scan_store(int *p, int base, int n, bool vec, const int *r)
 {
     if (vec && base + kScanItems <= n) {
-        *reinterpret_cast<int4 *>(p + base) = make_int4(r[0], r[1], r[2], r[3]);
-        *reinterpret_cast<int4 *>(p + base + 4) = make_int4(r[4], r[5], r[6], r[7]);
+#pragma unroll
+        for (int k = 0; k < kScanItems; k += 4)
+            *reinterpret_cast<int4 *>(p + base + k) = make_int4(r[k], r[k + 1], r[k + 2], r[k + 3]);
     } else {
 #pragma unroll
         for (int k = 0; k < kScanItems; k++)
@@ -724,13 +748,27 @@ __device__ __forceinline__ bool aligned16(const void *p)
     return ((uintptr_t)p & 15u) == 0;
 }
 
+// Exclusive scan of n ints in one pass (decoupled look-back, Merrill and Garland 2016).  A
+// block takes the next tile from a ticket, publishes the tile's sum, adds up what the tiles
+// before it have published, 64 at a time, back to the first one whose prefix is known, and
+// publishes its own prefix.  Sum and state travel in one 64-bit word, so the words need no
+// fence beside them (on this part a device-scope release writes a whole L2 back); tickets are
+// taken in order, so every tile waited for is being worked on.  One launch and one pass over
+// the array in place of three launches and two passes: the launches cost 3 x 2.4 us on every
+// kick, also when nothing is rebuilt.
+// state[0]: the ticket, state[1 + tile]: {0 nothing, 1 sum, 2 prefix} << 32 | value, all zero on
+// entry (the histogram kernel before it clears them).
 [[maybe_unused]] __global__ void __launch_bounds__(kBlock)
-    k_scan_tiles(const int *flag, const int *in, int *out, int *tile_sums, int n)
+    k_scan(const int *flag, const int *in, int *out, unsigned long long *state, int n)
 {
     if (skip(flag)) return;
-    __shared__ int s[kBlock];
+    __shared__ int s[kBlock / 64];
+    __shared__ int s_tile, s_before;
+    if (threadIdx.x == 0) s_tile = (int)atomicAdd(&state[0], 1ull);
+    __syncthreads();
+    const int tile = s_tile;
     const bool vec = aligned16(in) && aligned16(out);
-    const int base = blockIdx.x * kScanTile + threadIdx.x * kScanItems;
+    const int base = tile * kScanTile + (int)threadIdx.x * kScanItems;
     int v[kScanItems];
     scan_load(in, base, n, vec, v);
     int sum = 0;
@@ -738,6 +776,37 @@ __device__ __forceinline__ bool aligned16(const void *p)
     for (int k = 0; k < kScanItems; k++) sum += v[k];
     int total;
     int run = block_exclusive_scan(sum, s, total);
+    if (threadIdx.x < 64) {
+        const int lane = threadIdx.x;
+        auto publish = [&](unsigned long long kind, int value) {
+            if (lane == 0)
+                __hip_atomic_store(&state[1 + tile], kind << 32 | (unsigned int)value,
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        };
+        int before = 0;
+        if (tile > 0) {
+            publish(1ull, total);
+            for (int last = tile - 1;; last -= 64) {
+                const int p = last - lane;
+                unsigned long long w = 2ull << 32;  // before the first tile: prefix 0
+                do {
+                    if (p >= 0 && (w >> 32 == 0 || w == 2ull << 32))
+                        w = __hip_atomic_load(&state[1 + p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                } while (__any(w >> 32 == 0));
+                const unsigned long long known = __ballot(w >> 32 == 2);
+                const int upto = known ? __ffsll((long long)known) - 1 : 63;
+                int add = lane <= upto ? (int)(unsigned int)w : 0;
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) add += __shfl_xor(add, o);
+                before += add;
+                if (known) break;
+            }
+        }
+        publish(2ull, before + total);
+        if (lane == 0) s_before = before;
+    }
+    __syncthreads();
+    run += s_before;
     int r[kScanItems];
 #pragma unroll
     for (int k = 0; k < kScanItems; k++) {
@@ -745,41 +814,16 @@ __device__ __forceinline__ bool aligned16(const void *p)
         run += v[k];
     }
     scan_store(out, base, n, vec, r);
-    if (threadIdx.x == 0) tile_sums[blockIdx.x] = total;
 }
 
-[[maybe_unused]] __global__ void __launch_bounds__(kBlock) k_scan_single(const int *flag, int *data, int n)
-{
-    if (skip(flag)) return;
-    __shared__ int s[kBlock];
-    int carry = 0;
-    for (int chunk = 0; chunk < n; chunk += kScanTile) {
-        int base = chunk + threadIdx.x * kScanItems;
-        int v[kScanItems];
-        int sum = 0;
-#pragma unroll
-        for (int k = 0; k < kScanItems; k++) {
-            v[k] = (base + k < n) ? data[base + k] : 0;
-            sum += v[k];
-        }
-        int total;
-        int run = carry + block_exclusive_scan(sum, s, total);
-#pragma unroll
-        for (int k = 0; k < kScanItems; k++) {
-            if (base + k < n) data[base + k] = run;
-            run += v[k];
-        }
-        carry += total;
-    }
-}
+// words of k_scan's state for n ints
+inline int scan_words(int n) { return 1 + (n + kScanTile - 1) / kScanTile; }
 
-[[maybe_unused]] __global__ void k_scan_add(const int *flag, int *out, const int *tile_sums, int n)
+// clears them (the histogram kernels call it)
+__device__ __forceinline__ void clear_scan_state(unsigned long long *state, int words)
 {
-    if (skip(flag)) return;
-    int i = blockIdx.x * kScanTile + threadIdx.x;
-    int add = tile_sums[blockIdx.x];
-    for (int k = 0; k < kScanItems; k++, i += kBlock)
-        if (i < n) out[i] += add;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x)
+        state[i] = 0ull;
 }
 
 // Also clears the histogram again: the counts are zero between builds, so the next build
@@ -836,8 +880,8 @@ struct tpsph_handle {
     int *flag = nullptr;  // rebuild of the fluid cell list pending
     // fluid cell list + cell-sorted state
     int *f_cell = nullptr, *f_rank = nullptr, *f_count = nullptr, *f_start = nullptr,
-        *f_perm = nullptr;
-    int *scan_tiles = nullptr;
+        *f_perm = nullptr, *f_permu = nullptr;  // f_permu: unordered inside a cell
+    unsigned long long *scan_state = nullptr;  // k_scan
     double *f_mass = nullptr;  // caller order
     double *xs = nullptr, *ys = nullptr, *zs = nullptr, *snap = nullptr;
     float4 *xf = nullptr;  // Verlet lists: FP32 positions at the last rebuild (+ kPad NaN)
@@ -856,10 +900,16 @@ struct tpsph_handle {
     int *nbr = nullptr, *cnt = nullptr, *wnbr = nullptr, *wcnt = nullptr;
     int ls = 0, cap_f = 0, cap_w = 0;
     // processing order of the list kernels (bricks of cells) and the bricks in LDS
-    int *ord = nullptr, *bcount = nullptr, *bstart = nullptr;
+    int *ord = nullptr, *bcount = nullptr;
     int nbricks = 0;
     bool bricks = false;
-    int *brow_gb = nullptr, *brow_lds = nullptr, *bntot = nullptr, *nel = nullptr, *bwork = nullptr;
+    // the non-empty bricks: number of the brick (nel), {first target, one past the last, union
+    // size (INT_MAX: does not stage), first entry in uidx} (bhead); per target, in the order
+    // of ord, its brick's first entry in uidx or -1 (tbase); uidx: sorted index of every
+    // union record
+    int *nel = nullptr, *tbase = nullptr, *uidx = nullptr, *bwork = nullptr;
+    int4 *bhead = nullptr;
+    int64_t uidx_cap = 0;
     int *bfall = nullptr;  // mixed precision: the bricks left to the FP64 pass
     unsigned short *nbr16 = nullptr;
     int2 *thead = nullptr;  // target headers of the brick kernels, in the order of ord
@@ -872,7 +922,8 @@ struct tpsph_handle {
     int *anbr = nullptr, *acnt = nullptr, *wactive = nullptr;
     int lw = 0, cap_a = 0;
     // counters rebuilt with the lists: [0] non-empty bricks, [1] active wall particles,
-    // [2] fluid particles with wall candidates (wtargets)
+    // [2] fluid particles with wall candidates (wtargets), [3] overflowed lists, [4] targets
+    // and [5] union records given to bricks so far, [6] work counter of the list build
     int *counters = nullptr, *wtargets = nullptr;
     int n_cu = 256;  // compute units of the device (grid of the brick kernel)
     // host-mode staging and solver scratch
@@ -995,14 +1046,11 @@ int derive_params(const tpsph_params *params, int nf, int nw, const double *lo,
 // the fluid-fluid pass of TPSPH_PRECISION_MIXED (tpsph_mixed.hip), in place of k_fluid_brick
 int launch_fluid_brick_mixed(tpsph_handle *h, double *dv);
 
-// Exclusive scan of n ints from in to out on the handle's stream (tile sums in h->scan_tiles).
+// Exclusive scan of n ints from in to out on the handle's stream (h->scan_state is clear).
 inline int scan(tpsph_handle *h, const int *flag, const int *in, int *out, int n)
 {
-    int tiles = (n + kScanTile - 1) / kScanTile;
-    hipLaunchKernelGGL((k_scan_tiles), dim3(tiles), dim3(kBlock), 0, h->stream, flag, in, out, h->scan_tiles, n);
-    hipLaunchKernelGGL((k_scan_single), dim3(1), dim3(kBlock), 0, h->stream, flag, h->scan_tiles, tiles);
-    hipLaunchKernelGGL((k_scan_add), dim3(tiles), dim3(kBlock), 0, h->stream, flag, out, h->scan_tiles, n);
-    return launch_check(h, "scan");
+    hipLaunchKernelGGL((k_scan), dim3(scan_words(n) - 1), dim3(kBlock), 0, h->stream, flag, in, out, h->scan_state, n);
+    return launch_check(h, "k_scan");
 }
 
 // gathered: the cell-sorted records already hold (v, u) (written by k_ck_stage_gather)

@@ -32,7 +32,6 @@ struct BrickSmem32 {
     float4 pa[kBrickCap];  // {x, y, z, rho - rho0} relative to the brick centre
     float4 pb[kBrickCap];  // {vx, vy, vz, p}
     float vol[kBrickCap];  // V = m / rho
-    int row_gb[kBrickMaxRows], row_lds[kBrickMaxRows + 1];
     int item;
     double org[3];         // the brick centre
 };
@@ -43,7 +42,7 @@ struct BrickSmem32 {
 // 2 delta h c}, written by k_sound_speed).
 struct Pair32 {
     float R2, az2, h_inv_half, kgrad_c, eps_h2, two_av_c, dd2, two_rho0, rho0;
-    int use_visc, maxr, nw;
+    int use_visc, nw;
     int nb0, nb1, bc[3];
     double lo[3], cs[3], g[3], rho0_64;
     const double *dyn;
@@ -62,7 +61,6 @@ Pair32 pair32(const DevParams &P)
     q.two_rho0 = (float)(2.0 * P.rho0);
     q.rho0 = (float)P.rho0;
     q.use_visc = P.use_visc;
-    q.maxr = P.maxr;
     q.nw = P.nw;
     q.nb0 = P.nb[0];
     q.nb1 = P.nb[1];
@@ -133,10 +131,9 @@ __device__ __forceinline__ void pair32_term(const Pair32 &q, const float4 &a, co
 template <int ND>
 __global__ void __launch_bounds__(kBrickThreads, 8)
     k_fluid_brick32(int *flag, Pair32 q, FluidView F, const int *__restrict__ ord,
-                    const int *__restrict__ bstart, const int *__restrict__ nel,
+                    const int *__restrict__ nel, const int4 *__restrict__ bhead,
                     const int *__restrict__ nne, int *__restrict__ work,
-                    const int *__restrict__ brow_gb, const int *__restrict__ brow_lds,
-                    const int *__restrict__ bntot, const unsigned short *__restrict__ nbr16,
+                    const int *__restrict__ uidx, const unsigned short *__restrict__ nbr16,
                     const int *__restrict__ cnt, int ls, const int *__restrict__ wcnt,
                     double *__restrict__ dv, int *__restrict__ bfall)
 {
@@ -154,15 +151,12 @@ __global__ void __launch_bounds__(kBrickThreads, 8)
         const int item = S.item;
         if (item >= ne) break;
         const int b = nel[item];
-        const int ntot = bntot[b];
+        const int4 hd = bhead[item];
+        const int ntot = hd.z;
         if (ntot > kBrickCap - 1) {  // left to the FP64 pass (uniform per block)
-            if (tid == 0) bfall[atomicAdd(&work[1], 1)] = b;
+            if (tid == 0) bfall[atomicAdd(&work[1], 1)] = item;
         } else {
-            const int t0 = bstart[b], t1 = bstart[b + 1];
-            for (int r = tid; r <= q.maxr; r += kBrickThreads) {
-                if (r < q.maxr) S.row_gb[r] = brow_gb[(size_t)b * q.maxr + r];
-                S.row_lds[r] = brow_lds[(size_t)b * (q.maxr + 1) + r];
-            }
+            const int t0 = hd.x, t1 = hd.y;
             if (tid == 0) {
                 const int bx = b % q.nb0, by = (b / q.nb0) % q.nb1, bz = b / (q.nb0 * q.nb1);
                 const int bc[3] = {bx, by, bz};
@@ -177,8 +171,7 @@ __global__ void __launch_bounds__(kBrickThreads, 8)
             __syncthreads();
             const double o0 = S.org[0], o1 = S.org[1], o2 = S.org[2];
             for (int i = tid; i < ntot; i += kBrickThreads) {
-                const int r = bsearch_le(S.row_lds, q.maxr + 1, i);
-                const int g = S.row_gb[r] + (i - S.row_lds[r]);
+                const int g = uidx[hd.w + i];
                 const double4 a = F.rec[2 * (size_t)g];
                 const double4 c = F.rec[2 * (size_t)g + 1];
                 S.pa[i] = make_float4((float)(a.x - o0), (float)(a.y - o1),
@@ -211,7 +204,7 @@ __global__ void __launch_bounds__(kBrickThreads, 8)
                 float acc[3] = {0.0f, 0.0f, 0.0f};
                 Kahan drho;
                 const ushort4 *l4 = reinterpret_cast<const ushort4 *>(nbr16);
-                const int ng = (max(n, 0) + 3) >> 2;
+                const int ng = list_rows(max(n, 0));
                 // list rows clamped into the list rather than selected (a select made the
                 // compiler issue flat loads, whose waits hold up the LDS reads)
                 ushort4 cur4 = l4[(size_t)min(half, max(ng - 1, 0)) * ls + col];
@@ -220,9 +213,10 @@ __global__ void __launch_bounds__(kBrickThreads, 8)
                     // one candidate at a time: eight waves per SIMD hide the LDS latency
                     const unsigned short e4[4] = {cur4.x, cur4.y, cur4.z, cur4.w};
                     float part = 0.0f;
+                    const int ke = list_row_entries(n, g);
 #pragma unroll 1
-                    for (int k = 0; k < 4; k++) {
-                        const int e = e4[k];
+                    for (int k = 0; k < ke; k++) {
+                        const int e = e4[k] >> 4;
                         pair32_term<ND>(q, S.pa[e], S.pb[e], S.vol[e], xa, va, drho_a, rho_a, p_a,
                                         inv_rho_a, acc, part);
                     }
@@ -254,15 +248,9 @@ __global__ void __launch_bounds__(kBrickThreads, 8)
 int tpsph::launch_fluid_brick_mixed(tpsph_handle *h, double *dv)
 {
     const int grid = std::max(1, std::min(h->nbricks, 2 * h->n_cu));
-    if (h->nd == 2)
-        hipLaunchKernelGGL((k_fluid_brick32<2>), dim3(grid), dim3(kBrickThreads), 0, h->stream,
-                           h->flag, pair32(h->P), h->fluid_view(), h->ord, h->bstart, h->nel,
-                           h->counters, h->bwork, h->brow_gb, h->brow_lds, h->bntot, h->nbr16,
-                           h->cnt, h->ls, h->wcnt, dv, h->bfall);
-    else
-        hipLaunchKernelGGL((k_fluid_brick32<3>), dim3(grid), dim3(kBrickThreads), 0, h->stream,
-                           h->flag, pair32(h->P), h->fluid_view(), h->ord, h->bstart, h->nel,
-                           h->counters, h->bwork, h->brow_gb, h->brow_lds, h->bntot, h->nbr16,
-                           h->cnt, h->ls, h->wcnt, dv, h->bfall);
+    const auto kernel = h->nd == 2 ? k_fluid_brick32<2> : k_fluid_brick32<3>;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBrickThreads), 0, h->stream, h->flag,
+                       pair32(h->P), h->fluid_view(), h->ord, h->nel, h->bhead, h->counters,
+                       h->bwork, h->uidx, h->nbr16, h->cnt, h->ls, h->wcnt, dv, h->bfall);
     return launch_check(h, "k_fluid_brick32");
 }
