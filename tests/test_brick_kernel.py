@@ -73,3 +73,40 @@ def test_bricks_match_oracle(tp, orc, nd, n, visc, kind):
             err = np.abs(got[:, col] - dv_ref[:, col]).max() / np.abs(dv_ref[:, col]).max()
             assert err <= RTOL, f"column {col}, kick {repeat}: {err:.3e}"
     semi.close()
+
+
+# cells per compact support along y and z / x, skin: short and long rows, one and four cells of
+# reach, lists of up to about 200 entries, and (3D, three cells) bricks that do not stage
+@pytest.mark.parametrize("nd,dx,div,xdiv,skin", [
+    (2, 0.02, 1, 1, 0.04), (2, 0.02, 4, 8, 0.04), (2, 0.02, 2, 3, 0.6),
+    (3, 0.04, 1, 1, 0.04), (3, 0.04, 1, 8, 0.04), (3, 0.04, 2, 8, 0.04), (3, 0.04, 2, 1, 0.04),
+    (3, 0.04, 2, 4, 0.45), (3, 0.04, 3, 4, 0.04),
+])
+def test_listed_pairs_match_bruteforce(tp, orc, nd, dx, div, xdiv, skin):
+    import torch
+    db = tp.dam_break(nd, dx)
+    semi = tp.Semidiscretization(db.fluid_system, db.boundary_system, cell_divisions=div,
+                                 x_cell_divisions=xdiv, skin=skin, pair_search="lists")
+    v0, u0 = semi.initial_state()
+    u = u0.cpu().numpy().copy()
+    rng = np.random.default_rng(4)
+    R = 2 * db.fluid_system.smoothing_length
+    u += rng.uniform(-0.3, 0.3, size=u.shape) * dx     # a disordered fluid
+    dv = torch.empty_like(v0)
+    move = rng.normal(size=u.shape)
+    move *= 0.45 * skin * R / np.linalg.norm(move, axis=1, keepdims=True)
+    xw = db.boundary_system.coordinates.T.copy()
+    for x in (u, u + move):                            # the build, then within half the skin
+        tp.kick(dv, v0, torch.from_numpy(x).cuda(), {"semi": semi}, 0.0)
+        for pair, xa, xb in ((tp.native.PAIR_FLUID_FLUID, x, x), (tp.native.PAIR_FLUID_WALL, x, xw),
+                             (tp.native.PAIR_WALL_FLUID, xw, x)):
+            off, idx = tp.kick_pairs(semi, pair)
+            roff, ridx = orc.neighbors(nd, R, xa, xb, brute=True)
+            if pair == tp.native.PAIR_FLUID_FLUID:     # the kick leaves the particle itself out
+                rows = np.repeat(np.arange(roff.size - 1), np.diff(roff))
+                keep = rows != ridx
+                roff = np.concatenate([[0], np.cumsum(np.bincount(rows[keep], minlength=roff.size - 1))])
+                ridx = ridx[keep]
+            assert np.array_equal(off, roff), f"pair {pair}: counts differ"
+            assert np.array_equal(idx.astype(np.int64), ridx), f"pair {pair}: sets differ"
+    semi.close()

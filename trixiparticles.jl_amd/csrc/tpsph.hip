@@ -81,8 +81,8 @@ __global__ void k_cells(const int *flag, DevParams P, int n, const double *__res
 // atomics were served in): a particle's place is the number of members with a smaller index.
 // With bcount it also counts the particles of every brick of cells and lists the bricks that
 // hold any (nel, nne of them; k_cells cleared it).
-// FP32 position for the pre-test of the list build: relative to the grid origin, NaN
-// outside the grid box (the list build then leaves the particle to the FP64 test)
+// FP32 position for the list builds: relative to the grid origin, NaN outside the grid box (the
+// list builds then take every candidate of the particle)
 template <int ND>
 __device__ __forceinline__ float4 list_f32(const DevParams &P, double x0, double x1, double x2)
 {
@@ -623,16 +623,10 @@ __device__ __forceinline__ void build_list(const DevParams &P, const FluidView &
 {
     const double xa = F.x[s], ya = F.y[s], za = (ND == 3) ? F.z[s] : 0.0;
     const int *start = WALL ? Wv.start : F.start;
-    const double *cx = WALL ? Wv.x : F.x;
-    const double *cy = WALL ? Wv.y : F.y;
-    const double *cz = WALL ? Wv.z : F.z;
-    const double rl2 = WALL ? P.rl2_wall : P.rl2_fluid;
-    // an FP32 test on the FP32 positions first; only a distance within a few FP32 ulps of
-    // the box size of the list radius (or a particle outside the grid box, NaN there) takes
-    // the FP64 test, so the lists are those of the FP64 test
+    // the FP32 test takes what is not surely beyond the list radius
     const float4 xaf = F.xf[s];
     const float4 *cf = WALL ? Wv.xf : F.xf;
-    const float in2 = WALL ? P.wlist_in2 : P.list_in2, out2 = WALL ? P.wlist_out2 : P.list_out2;
+    const float out2 = WALL ? P.wlist_out2 : P.list_out2;
     Pencils<ND> it;
     it.init(P, xa, ya, za, WALL ? P.hs_list_wall : P.hs_list_fluid);
     int n = 0, j, je;
@@ -650,10 +644,7 @@ __device__ __forceinline__ void build_list(const DevParams &P, const FluidView &
                 const float ex = xaf.x - q[k].x, ey = xaf.y - q[k].y;
                 const float ez = (ND == 3) ? xaf.z - q[k].z : 0.f;
                 const float d2f = ex * ex + ey * ey + ez * ez;
-                hit[k] = d2f <= in2;
-                if (!hit[k] && !(d2f > out2) && j + k < je)
-                    hit[k] = dist2<ND>(xa - cx[j + k], ya - cy[j + k],
-                                       (ND == 3) ? za - cz[j + k] : 0.0) <= rl2;
+                hit[k] = !(d2f > out2);
             }
 #pragma unroll
             for (int k = 0; k < 4; k++) {
@@ -685,14 +676,11 @@ __device__ __forceinline__ void
         int n = 0, j, je;
         while (it.next(P, F.start, j, je)) {
             for (; j < je; j++) {
-                // the FP32 pre-test of the list build, FP64 in its band (and for NaN)
+                // what is not surely beyond the list radius (see build_list)
                 const float4 q = F.xf[j];
                 const float ex = xwf.x - q.x, ey = xwf.y - q.y, ez = (ND == 3) ? xwf.z - q.z : 0.f;
                 const float d2f = ex * ex + ey * ey + ez * ez;
-                bool hit = d2f <= P.wlist_in2;
-                if (!hit && !(d2f > P.wlist_out2))
-                    hit = dist2<ND>(xw.x - F.x[j], xw.y - F.y[j], (ND == 3) ? xw.z - F.z[j] : 0.0) <= P.rl2_wall;
-                if (hit) {
+                if (!(d2f > P.wlist_out2)) {
                     if (n < cap) nbr[(size_t)n * lw + w] = j;
                     n++;
                 }
@@ -880,15 +868,18 @@ struct WallListsArgs {
 };
 
 struct ListsSmem {
+    // the last entries of every thread's list, slot-major: 64 lanes write 64 banks whatever
+    // slots they are at (aligned to a wave's ring: the slot is or-ed into the address)
+    alignas(kListRing * 128) unsigned short ring[kListThreads / 64][kListRing * 64];
     // FP32 positions of the union (relative to the grid origin) and their padding
     float x[kBrickCap + 4], y[kBrickCap + 4], z[kBrickCap + 4];
-    unsigned short list[kListArea];
     unsigned short ctab[kCellTab];
+    unsigned short near[kBrickCap];  // the targets with walls near their cell
     int row_gb[kBrickMaxRows], row_lds[kBrickMaxRows + 1];
     short row_x0[kBrickMaxRows], row_x1[kBrickMaxRows];
     int trow_s[kBrickMaxRows], trow_t[kBrickMaxRows + 1];
     int scan[kListThreads / 64];
-    int item, col0, ubase, bad;
+    int item, col0, ubase, bad, nnear;
 };
 
 // Exclusive scan over the kListThreads threads of a block.
@@ -922,142 +913,239 @@ __device__ __forceinline__ int lists_target(const ListsSmem &S, int nrows, int k
     return S.trow_s[r] + (k - S.trow_t[r]);
 }
 
-// Wall list of fluid particle s in column col, four lanes (q) to the particle: the pencils'
-// candidates four at a time, the hits placed by the quad's ballot.  Returns the count.
+// The FP32 positions and the cell offsets of the union whose rows are in S (n records of the
+// cell-sorted points with cell offsets `start`); uidx: also their sorted indices.
 template <int ND>
-__device__ __forceinline__ int wall_list_quad(const DevParams &P, const FluidView &F,
-                                              const WallView &Wv, int s, int col, int ls, int cap,
-                                              int q, int *__restrict__ nbr)
+__device__ __forceinline__ void stage_union(const DevParams &P, const int *__restrict__ start,
+                                            const float4 *__restrict__ xf, ListsSmem &S, int n,
+                                            int uy0, int uz0, int nuy, int *__restrict__ uidx)
 {
-    const double xa = F.x[s], ya = F.y[s], za = (ND == 3) ? F.z[s] : 0.0;
-    const float4 xaf = F.xf[s];
-    const int quad = (int)threadIdx.x & 60;
-    Pencils<ND> it;
-    it.init(P, xa, ya, za, P.hs_list_wall);
-    int n = 0, j, je;
-    while (it.next(P, Wv.start, j, je)) {  // uniform over the quad
-        for (; j < je; j += 4) {
-            const int k = j + q;  // kPad entries follow the arrays
-            const float4 c = Wv.xf[k];
-            const float ex = xaf.x - c.x, ey = xaf.y - c.y, ez = (ND == 3) ? xaf.z - c.z : 0.f;
-            const float d2f = ex * ex + ey * ey + ez * ez;
-            bool hit = d2f <= P.wlist_in2;
-            if (!hit && !(d2f > P.wlist_out2) && k < je)
-                hit = dist2<ND>(xa - Wv.x[k], ya - Wv.y[k], (ND == 3) ? za - Wv.z[k] : 0.0) <= P.rl2_wall;
-            hit = hit && k < je;
-            const int hits = (int)(__ballot(hit) >> quad) & 15;
-            const int place = n + __popc(hits & ((1 << q) - 1));
-            if (hit && place < cap) nbr[(size_t)place * ls + col] = k;
-            n += __popc(hits);
+    // four records per thread at a time: their row searches and loads overlap
+    static_assert(kBrickCap <= 4 * kListThreads && kBrickMaxRows == 256, "one pass of four, eight steps");
+    int r[4], s[4];
+    float4 c[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) r[k] = 0;
+#pragma unroll
+    for (int step = 128; step > 0; step >>= 1) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int to = r[k] + step;
+            if (to < P.maxr && S.row_lds[to] <= (int)threadIdx.x + k * kListThreads) r[k] = to;
         }
     }
-    return n <= cap ? n : -1;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int i = (int)threadIdx.x + k * kListThreads;
+        s[k] = i < n ? S.row_gb[r[k]] + (i - S.row_lds[r[k]]) : 0;
+        c[k] = xf[s[k]];
+    }
+    // (the division: exact for these sizes, i + 1/2 is at least 1 / 2 ctab off a multiple)
+    const float per_row = 1.0f / (float)P.ctab;
+    for (int i = threadIdx.x; i < P.maxr * P.ctab; i += kListThreads) {
+        const int u = (int)(((float)i + 0.5f) * per_row), x = S.row_x0[u] + (i - u * P.ctab);
+        if (S.row_x1[u] < S.row_x0[u] || x > S.row_x1[u] + 1) continue;
+        const int cy = uy0 + u % nuy, cz = (ND == 3) ? uz0 + u / nuy : 0;
+        S.ctab[i] = (unsigned short)(S.row_lds[u] + start[P.n[0] * (cy + P.n[1] * cz) + x] - S.row_gb[u]);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int i = (int)threadIdx.x + k * kListThreads;
+        if (i >= n) continue;
+        if (uidx) uidx[i] = s[k];
+        S.x[i] = c[k].x;
+        S.y[i] = c[k].y;
+        if constexpr (ND == 3) S.z[i] = c[k].z;
+    }
 }
 
-// The lists of one brick's targets by quads: four lanes share a target, lane q testing the
-// candidates q, q + 4, ... of each union row near it, from LDS.  Returns false through S.bad
-// when a list overflowed (the brick then does not stage).
+// 16 entries of a thread's ring, from list entry `first` (a multiple of 16) on, as the four rows
+// of list_place.
+__device__ __forceinline__ void ring_rows(const unsigned short *ring, int first,
+                                          ushort4 *__restrict__ out, int ls, int col)
+{
+    const unsigned short *r = ring + (first & (kListRing - 1)) * 64;
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+        out[(size_t)(first / 4 + q) * ls + col] = make_ushort4(r[64 * q], r[64 * (q + 4)], r[64 * (q + 8)], r[64 * (q + 12)]);
+}
+
+// The list of the target at sorted index s in column col, one thread per target: the candidates
+// of the staged union (of the fluid, WALL: of the walls) in the rows of cells near the target,
+// as Pencils enumerates them.  A row's candidates are tested four at a time without branches:
+// each is written behind the list (in the ring of the fluid list, whose 16 oldest entries go
+// to memory when it fills; a wall list is short and goes to memory as it is found), which
+// grows on a hit only.  Returns the number of entries (which may exceed the capacity: the
+// surplus is not written).
+template <int ND, bool WALL>
+__device__ __forceinline__ int union_list(const DevParams &P, const FluidView &F,
+                                          const ListsArgs &A, ListsSmem &S, int s, bool active,
+                                          int col, int self, double xa, double ya, double za,
+                                          int c1, int c2, int uy0, int uz0, int nuy)
+{
+    constexpr int kRows = ND == 3 ? 5 : 9;  // cell rows along y
+    const float4 xaf = F.xf[s];
+    const double hs = WALL ? P.hs_list_wall : P.hs_list_fluid;
+    const float out2 = WALL ? P.wlist_out2 : P.list_out2;
+    const int cap = WALL ? A.cap_w : A.cap_f;
+    ushort4 *out = reinterpret_cast<ushort4 *>(A.nbr16);
+    char *const ring = reinterpret_cast<char *>(S.ring);
+    const uint32_t lane_ring = (threadIdx.x >> 6) * (kListRing * 128u) + (threadIdx.x & 63) * 2u;
+    const double xc = (xa - P.lo[0]) * P.inv_cs[0];  // in cells
+    double y2[kRows];
+#pragma unroll
+    for (int j = 0; j < kRows; j++) {
+        const double y = transverse(P, 1, c1 + j - P.lr[1], ya, hs);
+        y2[j] = y * y;
+    }
+    uint32_t n = 0;  // 128 times the number of entries: the offset of the ring's next slot
+    uint32_t written = 0;
+    for (int dz = ND == 3 ? -P.lr[2] : 0; dz <= (ND == 3 ? P.lr[2] : 0); dz++) {
+        const int cz = ND == 3 ? c2 + dz : 0;
+        const double z = (ND == 3) ? transverse(P, 2, cz, za, hs) : 0.0;
+        const double rz2 = fma(-z, z, P.R2);
+        const bool okz = active && (ND == 2 || (cz >= 0 && cz < P.n[2]));
+        const int uz = (c1 - P.lr[1] - uy0) + nuy * (cz - uz0);
+#pragma unroll
+        for (int j = 0; j < kRows; j++) {
+            if (j > 2 * P.lr[1]) break;  // uniform
+            const int cy = c1 + j - P.lr[1], u = uz + j;
+            const double r2 = rz2 - y2[j];
+            int b = 0, e = 0;
+            if (okz && cy >= 0 && cy < P.n[1] && r2 >= 0.0) {
+                // conservative half-width: FP32 sqrt, enlarged well past its rounding error
+                const double rx = ((double)(__builtin_amdgcn_sqrtf((float)r2) * 1.000001f) + hs) * P.inv_cs[0];
+                const double last = (double)(P.n[0] - 1);  // cell_1d's clamping
+                const int x0 = max((int)fmin(fmax(xc - rx, 0.0), last), (int)S.row_x0[u]);
+                const int x1 = min((int)fmin(fmax(xc + rx, 0.0), last), (int)S.row_x1[u]);
+                const unsigned short *ct = S.ctab + u * P.ctab - S.row_x0[u];
+                if (x0 <= x1) {
+                    b = ct[x0];
+                    e = ct[x1 + 1];
+                }
+            }
+            // the target's own row in two parts, without the target
+            const bool own = !WALL && j == P.lr[1] && dz == 0;
+            const int e_last = e;
+            if (own) e = min(e, self);
+            for (int part = 0; part <= (own ? 1 : 0); part++) {
+                if (part == 1) {
+                    b = max(b, self + 1);
+                    e = e_last;
+                }
+                for (int k = b; k < e; k += 4) {
+                    bool hit[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const float ex = xaf.x - S.x[k + i], ey = xaf.y - S.y[k + i];
+                        const float ez = (ND == 3) ? xaf.z - S.z[k + i] : 0.f;
+                        // not surely beyond the list radius (NaN: outside the grid box)
+                        hit[i] = !(ex * ex + ey * ey + ez * ez > out2) & (k + i < e);
+                    }
+                    if constexpr (WALL) {
+                        const int w = S.row_gb[u] + (k - S.row_lds[u]);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            if (hit[i] && (int)n < cap) A.wnbr[(size_t)n * A.ls + col] = w + i;
+                            n += hit[i] ? 1u : 0u;
+                        }
+                    } else {
+                        const int k16 = k * 16;
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            *reinterpret_cast<unsigned short *>(ring + (lane_ring | (n & (kListRing * 128u - 1)))) =
+                                (unsigned short)(k16 + 16 * i);
+                            n += hit[i] ? 128u : 0u;
+                        }
+                        // (one slot stays free for the candidate that does not hit)
+                        if (__any(n - written > (kListRing - 5) * 128u) && n - written >= 16 * 128u) {
+                            if ((int)(written >> 7) < cap)
+                                ring_rows(S.ring[threadIdx.x >> 6] + (threadIdx.x & 63), (int)(written >> 7), out, A.ls, col);
+                            written += 16 * 128u;
+                        }
+                    }
+                }
+            }
+        }
+    }
+    if constexpr (WALL) return (int)n;
+    const int count = (int)(n >> 7);
+    if (active) {
+        for (int p = count; p < ((count + 15) & ~15); p++)
+            *reinterpret_cast<unsigned short *>(ring + (lane_ring | (((uint32_t)p * 128u) & (kListRing * 128u - 1)))) =
+                (unsigned short)((P.brick_cap - 1) * 16);
+        for (int w = (int)(written >> 7); w < min(count, cap); w += 16)
+            ring_rows(S.ring[threadIdx.x >> 6] + (threadIdx.x & 63), w, out, A.ls, col);
+    }
+    return count;
+}
+
+// The lists of one brick's targets over the fluid (its union is staged); lists the targets with
+// walls near their cell.  S.bad is set when a list overflowed (the brick then does not stage).
 template <int ND>
 __device__ __forceinline__ void brick_lists(const DevParams &P, const FluidView &F,
                                             const WallView &Wv, const ListsArgs &A, ListsSmem &S,
                                             int ntargets, int nrows, int uy0, int uz0, int nuy)
 {
-    const int tid = threadIdx.x, q = tid & 3, quad = tid & 60;
-    const int cap16 = (A.cap_f + 15) & ~15;
-    const int batch = max(1, min(kListThreads / 4, kListArea / cap16));
-    const int nry = 2 * P.lr[1] + 1, nr = nry * (ND == 3 ? 2 * P.lr[2] + 1 : 1);
-    constexpr int kRanges = (ND == 3 ? 25 : 9) / 4 + 1;  // rows per lane
-    const unsigned short far16 = (unsigned short)((P.brick_cap - 1) * 16);
-    for (int base = 0; base < ntargets; base += batch) {
-        const int tl = tid >> 2, k = base + tl;
-        const bool active = tl < batch && k < ntargets;
-        const int s = lists_target(S, nrows, active ? k : 0);
+    for (int base = 0; base < ntargets; base += kListThreads) {
+        const int k = base + (int)threadIdx.x;
+        const bool active = k < ntargets;
+        const int s = lists_target(S, nrows, active ? k : 0), col = S.col0 + k;
         const double xa = F.x[s], ya = F.y[s], za = (ND == 3) ? F.z[s] : 0.0;
-        const float4 xaf = F.xf[s];
         const int c0 = cell_1d(xa, P.lo[0], P.inv_cs[0], P.n[0]);
         const int c1 = cell_1d(ya, P.lo[1], P.inv_cs[1], P.n[1]);
         const int c2 = (ND == 3) ? cell_1d(za, P.lo[2], P.inv_cs[2], P.n[2]) : 0;
         const int own = (c1 - uy0) + nuy * (c2 - uz0);
         const int self = S.row_lds[own] + (s - S.row_gb[own]);
-        // the record ranges of the rows near the target (pencils): lane q has rows q, q + 4, ...
-        int range[kRanges];
-        const double hs = P.hs_list_fluid;
-#pragma unroll
-        for (int i = 0; i < kRanges; i++) {
-            const int r = 4 * i + q;
-            range[i] = 0;
-            const int cy = c1 + (ND == 3 ? r % nry : r) - P.lr[1];
-            const int cz = (ND == 3) ? c2 + r / nry - P.lr[2] : 0;
-            if (!active || r >= nr || cy < 0 || cy >= P.n[1] || cz < 0 || cz >= P.n[2]) continue;
-            const double dy = transverse(P, 1, cy, ya, hs);
-            const double dz = (ND == 3) ? transverse(P, 2, cz, za, hs) : 0.0;
-            const double r2 = P.R2 - fma(dy, dy, dz * dz);
-            if (r2 < 0.0) continue;
-            const double rx = (double)(__builtin_amdgcn_sqrtf((float)r2) * 1.000001f) + hs;
-            const int u = (cy - uy0) + nuy * (cz - uz0);
-            const int x0 = max(cell_1d(xa - rx, P.lo[0], P.inv_cs[0], P.n[0]), (int)S.row_x0[u]);
-            const int x1 = min(cell_1d(xa + rx, P.lo[0], P.inv_cs[0], P.n[0]), (int)S.row_x1[u]);
-            if (x0 > x1) continue;
-            const unsigned short *ct = S.ctab + u * P.ctab - S.row_x0[u];
-            range[i] = (int)ct[x0] | (int)ct[x1 + 1] << 16;
-        }
-        unsigned short *list = S.list + (active ? tl * cap16 : 0);
-        int n = 0;
-#pragma unroll
-        for (int r = 0; r < 4 * kRanges; r++) {
-            const int rg = r % 4 == 0   ? quad_bcast<0>(range[r / 4])
-                           : r % 4 == 1 ? quad_bcast<1>(range[r / 4])
-                           : r % 4 == 2 ? quad_bcast<2>(range[r / 4])
-                                        : quad_bcast<3>(range[r / 4]);
-            const int e = (int)((unsigned)rg >> 16);
-#pragma unroll 1
-            for (int b = rg & 0xffff; b < e; b += 4) {
-                const int k2 = b + q;
-                const float ex = xaf.x - S.x[k2], ey = xaf.y - S.y[k2];
-                const float ez = (ND == 3) ? xaf.z - S.z[k2] : 0.f;
-                const float d2f = ex * ex + ey * ey + ez * ez;
-                const bool valid = k2 < e && k2 != self;
-                bool hit = d2f <= P.list_in2;
-                if (!hit && !(d2f > P.list_out2) && valid) {  // the FP32 test's band (or NaN)
-                    const int u = bsearch_le(S.row_lds, P.maxr + 1, k2);
-                    const int j = S.row_gb[u] + (k2 - S.row_lds[u]);
-                    hit = dist2<ND>(xa - F.x[j], ya - F.y[j], (ND == 3) ? za - F.z[j] : 0.0) <= P.rl2_fluid;
-                }
-                hit = hit && valid;
-                const int hits = (int)(__ballot(hit) >> quad) & 15;
-                const int place = n + __popc(hits & ((1 << q) - 1));
-                if (hit && place < A.cap_f) list[list_place(place)] = (unsigned short)(k2 * 16);
-                n += __popc(hits);
-            }
-        }
+        const int n = union_list<ND, false>(P, F, A, S, s, active, col, self, xa, ya, za,
+                                            c1, c2, uy0, uz0, nuy);
         if (active) {
-            const int col = S.col0 + k;
-            const bool fits = n <= A.cap_f;
-            if (fits) {
-                for (int p = n + q; p < ((n + 15) & ~15); p += 4) list[list_place(p)] = far16;
-                __builtin_amdgcn_wave_barrier();
-                ushort4 *out = reinterpret_cast<ushort4 *>(A.nbr16);
-                const ushort4 *rows = reinterpret_cast<const ushort4 *>(list);
-                const int nrow = list_rows(n);
-                for (int r = q; r < nrow; r += 4) out[(size_t)r * A.ls + col] = rows[r];
-            } else if (q == 0) {
-                S.bad = 1;
-            }
-            int nw = 0;
-            if (P.nw > 0 && A.wall_near[c0 + P.n[0] * (c1 + P.n[1] * c2)])
-                nw = wall_list_quad<ND>(P, F, Wv, s, col, A.ls, A.cap_w, q, A.wnbr);
-            if (q == 0) {
-                A.ord[col] = s;
-                A.cnt[col] = fits ? n : -1;
-                A.tbase[col] = S.ubase;
-                if (P.nw > 0) {
-                    A.wcnt[col] = nw;
-                    if (A.wtargets && nw != 0) A.wtargets[atomicAdd(&A.nne[2], 1)] = col;
-                }
-                A.thead[col] = make_int2(F.perm[s], self | n << kHeadCount | (nw != 0 ? kHeadWalls : 0));
+            A.ord[col] = s;
+            A.cnt[col] = n <= A.cap_f ? n : -1;
+            A.tbase[col] = S.ubase;
+            A.thead[col] = make_int2(F.perm[s], self | n << kHeadCount);
+            if (n > A.cap_f) S.bad = 1;
+            if (P.nw > 0) {
+                if (A.wall_near[c0 + P.n[0] * (c1 + P.n[1] * c2)])
+                    S.near[atomicAdd(&S.nnear, 1)] = (unsigned short)k;
+                else
+                    A.wcnt[col] = 0;
             }
         }
-        __syncthreads();  // S.list is filled again
+    }
+}
+
+// The wall lists of the targets in S.near, the walls' union staged.
+template <int ND>
+__device__ __forceinline__ void brick_wall_lists(const DevParams &P, const FluidView &F,
+                                                 const WallView &Wv, const ListsArgs &A,
+                                                 ListsSmem &S, int nrows, int uy0, int uz0,
+                                                 int nuy, bool staged)
+{
+    for (int base = 0; base < S.nnear; base += kListThreads) {
+        const int i = base + (int)threadIdx.x;
+        const bool active = i < S.nnear;
+        const int k = S.near[active ? i : 0];
+        const int s = lists_target(S, nrows, k), col = S.col0 + k;
+        int n;
+        if (staged) {
+            const double xa = F.x[s], ya = F.y[s], za = (ND == 3) ? F.z[s] : 0.0;
+            const int c1 = cell_1d(ya, P.lo[1], P.inv_cs[1], P.n[1]);
+            const int c2 = (ND == 3) ? cell_1d(za, P.lo[2], P.inv_cs[2], P.n[2]) : 0;
+            n = union_list<ND, true>(P, F, A, S, s, active, col, 0, xa, ya, za, c1, c2,
+                                     uy0, uz0, nuy);
+            if (!active) continue;
+            n = n <= A.cap_w ? n : -1;
+            A.wcnt[col] = n;
+        } else {
+            if (!active) continue;
+            build_list<ND, true>(P, F, Wv, s, col, A.ls, A.cap_w, A.wnbr, A.wcnt);
+            n = A.wcnt[col];
+        }
+        if (n != 0) {
+            A.thead[col].y |= kHeadWalls;
+            if (A.wtargets) A.wtargets[atomicAdd(&A.nne[2], 1)] = col;
+        }
     }
 }
 
@@ -1096,11 +1184,16 @@ __device__ __forceinline__ void brick_int_lists(const DevParams &P, const FluidV
 // the others build the Verlet lists of the wall particles (the Adami pass); both read only
 // the new cell-sorted order.
 //
-// The list build is bound by the candidates' tests and their reads.  From global memory, one
-// thread per target, unions, brick order and lists took 860 us and five launches at 1.02M
-// particles; here 720 us: the candidates come from the union's FP32 positions in LDS, four
-// lanes per target, and the int list of a staged target (4 bytes per entry) is not written
-// any more.  Two blocks of 512 threads share a compute unit (about 70 KB each).
+// The list build is bound by the VALU work of the candidates' tests (1.02M particles: 88k of
+// 146k cycles per brick).  The candidates' FP32 positions come from the staged union (from
+// global memory the address units were busy for 470 of 680 us); one thread per target tests
+// four candidates per step (four lanes per target: a row of cells holds about five
+// candidates, so the lanes idle, and what a row costs besides its tests is paid by four times
+// as many waves); the test is the FP32 one alone; the int list of a staged target (4 bytes per
+// entry) is not written any more; the walls of a brick are staged the same way, for the
+// targets near one only (four lanes per target on global memory: 157 us, here 40).  Bricks,
+// unions and lists took 860 us and five launches, four lanes per target 720, this form 495.
+// Two blocks of 512 threads share a compute unit (76 KB each).
 template <int ND>
 __global__ void __launch_bounds__(kListThreads, 4)
     k_brick_lists(const int *flag, DevParams P, FluidView F, WallView Wv, ListsArgs A,
@@ -1182,32 +1275,45 @@ __global__ void __launch_bounds__(kListThreads, 4)
             S.col0 = atomicAdd(&A.nne[4], ntargets);
             S.ubase = tot < INT_MAX ? atomicAdd(&A.nne[5], tot) : 0;
             S.bad = 0;
+            S.nnear = 0;
             S.item = atomicAdd(&A.nne[6], 1);
         }
         __syncthreads();
         const int next = nblocks + S.item;
         if (tot < INT_MAX && S.ubase > A.uidx_cap - tot) tot = INT_MAX;  // uniform
         if (tot < INT_MAX) {
-            for (int i = tid; i < tot; i += kListThreads) {
-                const int r = bsearch_le(S.row_lds, P.maxr + 1, i);
-                const int s = S.row_gb[r] + (i - S.row_lds[r]);
-                A.uidx[S.ubase + i] = s;
-                const float4 c = F.xf[s];
-                S.x[i] = c.x;
-                S.y[i] = c.y;
-                if constexpr (ND == 3) S.z[i] = c.z;
-            }
-            for (int i = tid; i < P.maxr * P.ctab; i += kListThreads) {
-                const int r = i / P.ctab, c = S.row_x0[r] + (i - r * P.ctab);
-                if (S.row_x1[r] < S.row_x0[r] || c > S.row_x1[r] + 1) continue;
-                const int cy = uy0 + r % nuy, cz = (ND == 3) ? uz0 + r / nuy : 0;
-                S.ctab[i] = (unsigned short)(S.row_lds[r] + F.start[P.n[0] * (cy + P.n[1] * cz) + c] - S.row_gb[r]);
-            }
+            stage_union<ND>(P, F.start, F.xf, S, tot, uy0, uz0, nuy, A.uidx + S.ubase);
             __syncthreads();
-            brick_lists<ND>(P, F, Wv, A, S, ntargets, nrows, uy0, uz0, nuy);  // ends with a barrier
+            brick_lists<ND>(P, F, Wv, A, S, ntargets, nrows, uy0, uz0, nuy);
+            __syncthreads();
             if (S.bad) {  // some list overflowed
                 tot = INT_MAX;
                 brick_int_lists<ND>(P, F, Wv, A, S, ntargets, nrows, false);
+            }
+            if (S.nnear > 0) {
+                // the union of the walls: the same cell rows (the fluid's list radius reaches
+                // further than the walls')
+                int gb = 0, cntr = 0;
+                if (tid < P.maxr && S.row_x0[tid] <= S.row_x1[tid]) {
+                    const int cy = uy0 + tid % nuy, cz = (ND == 3) ? uz0 + tid / nuy : 0;
+                    const int row = P.n[0] * (cy + P.n[1] * cz);
+                    gb = Wv.start[row + S.row_x0[tid]];
+                    cntr = Wv.start[row + S.row_x1[tid] + 1] - gb;
+                }
+                int wtot;
+                const int lds0 = lists_scan(cntr, S.scan, wtot);
+                const bool staged = wtot <= kBrickCap - 1;
+                if (tid < P.maxr) {
+                    S.row_gb[tid] = gb;
+                    S.row_lds[tid] = lds0;
+                }
+                if (tid == 0) S.row_lds[P.maxr] = wtot;
+                __syncthreads();
+                if (staged) {
+                    stage_union<ND>(P, Wv.start, Wv.xf, S, wtot, uy0, uz0, nuy, nullptr);
+                    __syncthreads();
+                }
+                brick_wall_lists<ND>(P, F, Wv, A, S, nrows, uy0, uz0, nuy, staged);
             }
         } else {
             brick_int_lists<ND>(P, F, Wv, A, S, ntargets, nrows, true);
@@ -2693,11 +2799,13 @@ int tpsph::derive_params(const tpsph_params *params, int nf, int nw, const doubl
     if (ncells > (int64_t)INT32_MAX / 4)
         return fail(nullptr, TPSPH_ERR_ARGUMENT, "cell grid too large (domain / smoothing_length)");
     P.ncells = (int)ncells;
-    // FP32 pre-test of the fluid list build.  A position inside the grid box is stored as
+    // FP32 test of the list builds.  A position inside the grid box is stored as
     // fl32(x - lo), off by at most 2^-24 L (L the box's longest side), so an FP32 distance d'
     // is off by at most 3.5 * 2^-24 L + 2^-24 d from the FP64 one d, and its square by a
-    // further 3.1 * 2^-24 relative: with e = 4 * 2^-24 (L + rl) the bounds leave a margin of
-    // at least 2^-24 rl on either side of the list radius rl
+    // further 3.1 * 2^-24 relative: with e = 4 * 2^-24 (L + rl) the bound leaves a margin of
+    // at least 2^-24 rl beyond the list radius rl.  The lists take whatever is within it: a
+    // few candidates more than the list radius holds (every kick applies the exact radius
+    // test), in exchange for no FP64 test in the build
     {
         const double u = 0x1p-24;
         double L = 0.0;
@@ -2705,17 +2813,14 @@ int tpsph::derive_params(const tpsph_params *params, int nf, int nw, const doubl
             P.box[d] = d < nd ? P.n[d] * P.cs[d] : 0.0;
             L = std::fmax(L, P.box[d]);
         }
-        auto bounds = [&](double rl2, float &fi, float &fo) {
+        auto bound = [&](double rl2) {
             const double rl = std::sqrt(rl2), e = 4.0 * u * (L + rl);
-            const double in2 = rl > e ? (rl - e) * (rl - e) * (1.0 - 4.0 * u) : -1.0;
             const double out2 = (rl + e) * (rl + e) * (1.0 + 4.0 * u);
-            fi = (float)in2;
-            fo = (float)out2;
-            if ((double)fi > in2) fi = std::nextafter(fi, -INFINITY);
-            if ((double)fo < out2) fo = std::nextafter(fo, INFINITY);
+            const float fo = (float)out2;
+            return (double)fo < out2 ? std::nextafter(fo, INFINITY) : fo;
         };
-        bounds(P.rl2_fluid, P.list_in2, P.list_out2);
-        bounds(P.rl2_wall, P.wlist_in2, P.wlist_out2);
+        P.list_out2 = bound(P.rl2_fluid);
+        P.wlist_out2 = bound(P.rl2_wall);
     }
     {
         // bricks of 3 (3D) or 8 (2D) cell spans per side, about 3.1 R (8.3 R) wide, in 3D

@@ -34,8 +34,8 @@ constexpr int kBrickMaxRows = 256;    // union rows per brick (one scan block)
 // list length << kHeadCount | kHeadWalls with wall candidates}; a record needs 11 bits
 // (kBrickCap) and a length 13 (at most 4096)
 constexpr int kHeadCount = 11, kHeadCountMask = (1 << 13) - 1, kHeadWalls = 1 << 24;
-constexpr int kListThreads = 512;     // threads of the list build, four per target
-constexpr int kListArea = 16384;      // 16-bit list entries a block of it holds in LDS
+constexpr int kListThreads = 512;     // threads of the list build, one per target
+constexpr int kListRing = 32;         // entries a thread of it holds before it writes 16 of them
 constexpr int kCellTab = 5120;        // cell offsets of a union in LDS (at most 121 rows x 40)
 constexpr int kGateBlocks = 1024;     // grid-stride kernels behind the rebuild flag: a small
                                       // grid keeps the launch cheap when the flag is down
@@ -68,12 +68,10 @@ struct DevParams {
     double half_skin, half_skin2;
     // Verlet lists: squared list radii and the cell growth that makes the pencils reach them
     double rl2_fluid, rl2_wall, hs_list_fluid, hs_list_wall;
-    // FP32 pre-test of the fluid list build (positions relative to lo inside the grid box
-    // box[d]): a squared FP32 distance at most list_in2 is surely within the list radius,
-    // one above list_out2 surely beyond it
+    // FP32 test of the list builds (positions relative to lo inside the grid box box[d]): a
+    // squared FP32 distance above list_out2 (walls: wlist_out2) is surely beyond the list radius
     double box[3];
-    float list_in2, list_out2;
-    float wlist_in2, wlist_out2;  // the same bounds for the wall list radius
+    float list_out2, wlist_out2;
     // bricks of cells (processing order of the list kernels): cells per brick, bricks per axis
     int bc[3], nb[3];
     // union rows of a brick: cells beyond the brick along y and z, rows per brick, and the
