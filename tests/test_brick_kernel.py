@@ -31,7 +31,8 @@ def fluid_block(tp, nd, n_per_dim, viscosity, summation=False, diffusion=None, d
 VISCOSITY = {"none": None, "alpha": dict(alpha=0.02, beta=0.0), "beta": dict(alpha=0.02, beta=1.5)}
 
 
-# bricks of about 6.9 x 7.5 x 7.5 (3D) or 20 x 20 (2D) spacings; 256 blocks
+# bricks of about 6.9 x 7.5 x 7.5 (3D) or 20 x 20 (2D) spacings, smaller ones for fluids that
+# would not fill 256 blocks with these (below about 74,000 or 77,000 particles)
 @pytest.mark.parametrize("nd,n,visc,kind", [
     (3, (5, 4, 3), "alpha", "continuity"),
     (3, (30, 23, 16), "none", "continuity"),
@@ -40,11 +41,14 @@ VISCOSITY = {"none": None, "alpha": dict(alpha=0.02, beta=0.0), "beta": dict(alp
     (3, (70, 60, 60), "alpha", "continuity"),      # three and more per block
     (3, (48, 48, 48), "beta", "summation"),
     (3, (30, 23, 16), "none", "summation"),
+    (3, (44, 42, 39), "alpha", "continuity"),      # just below and above full bricks
+    (3, (44, 42, 41), "alpha", "continuity"),
     (3, (48, 48, 48), "alpha", "antuono"),
     (2, (37, 21), "beta", "continuity"),
     (2, (420, 380), "alpha", "continuity"),        # 399 bricks and more
     (2, (420, 380), "none", "summation"),
     (2, (120, 90), "beta", "antuono"),
+    (2, (300, 250), "alpha", "continuity"),
 ])
 def test_bricks_match_oracle(tp, orc, nd, n, visc, kind):
     import torch

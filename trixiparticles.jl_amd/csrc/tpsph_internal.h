@@ -1038,8 +1038,11 @@ int validate(const tpsph_params *p, int64_t nf, int64_t nw, const double *fm, co
 
 // The device parameters of params for nf fluid and nw wall particles on the grid of the box
 // [lo, hi]: kernel and state-equation constants, cells, skin radii and bricks.
+// volume: mean volume of a fluid particle, slots: bricks the device takes at a time (0: bricks
+// of the full size).
 int derive_params(const tpsph_params *params, int nf, int nw, const double *lo,
-                  const double *hi, DevParams &P, int &nbricks);
+                  const double *hi, DevParams &P, int &nbricks, double volume = 0.0,
+                  int slots = 0);
 
 // the fluid-fluid pass of TPSPH_PRECISION_MIXED (tpsph_mixed.hip), in place of k_fluid_brick
 int launch_fluid_brick_mixed(tpsph_handle *h, double *dv);
