@@ -49,15 +49,17 @@ namespace {
 // cell list (counting sort), every kernel gated by the rebuild flag (nullptr = always)
 // ------------------------------------------------------------------------------------------
 
+// counters: zeroed (nullptr: none).
 template <int ND>
-__global__ void k_cells(const int *flag, DevParams P, int n, const double *__restrict__ x,
-                        int *__restrict__ cell, int *__restrict__ rank, int *__restrict__ count,
-                        unsigned long long *__restrict__ state, int words,
-                        int *__restrict__ zero, int nzero)
+__global__ void k_cells(const DevHandle *__restrict__ H, const int *flag, int n,
+                        const double *__restrict__ x, int *__restrict__ cell,
+                        int *__restrict__ rank, int *__restrict__ count,
+                        int *__restrict__ counters)
 {
     if (skip(flag)) return;
-    clear_scan_state(state, words);
-    if (zero && blockIdx.x == 0 && (int)threadIdx.x < nzero) zero[threadIdx.x] = 0;
+    const DevParams P = H->params();
+    clear_scan_state(H->scan_state, H->scan_words);
+    if (counters && blockIdx.x == 0 && (int)threadIdx.x < kCounters) counters[threadIdx.x] = 0;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const double *xi = x + (size_t)i * ND;
         int c0 = cell_1d(xi[0], P.lo[0], P.inv_cs[0], P.n[0]);
@@ -110,18 +112,19 @@ __global__ void k_wall_f32(DevParams P, int nw, const double4 *__restrict__ wpos
 }
 
 template <int ND, int MODE>
-__global__ void k_gather(int *flag, int *work, DevParams P, const int *__restrict__ perm,
-                         const double *__restrict__ u, const double *__restrict__ v,
-                         const double *__restrict__ m, double *__restrict__ xs,
-                         double *__restrict__ ys, double *__restrict__ zs,
-                         double4 *__restrict__ rec, double2 *__restrict__ vol,
-                         double *__restrict__ snap, int *__restrict__ iperm,
-                         const int *__restrict__ cell, const int *__restrict__ start,
-                         int *__restrict__ perm_out, int *__restrict__ bcount,
-                         int *__restrict__ nel, int *__restrict__ nne,
-                         const int *__restrict__ noverflow, int *__restrict__ nrebuild,
-                         float4 *__restrict__ xf)
+__global__ void k_gather(const DevHandle *__restrict__ H, const double *__restrict__ u,
+                         const double *__restrict__ v)
 {
+    DevParams P = H->params();
+    int *flag = H->flag, *work = H->bwork, *iperm = H->iperm, *perm_out = H->f_perm;
+    const int *perm = MODE == 0 ? H->f_perm : H->f_permu;
+    const double *m = H->mass;
+    double *xs = H->xs, *ys = H->ys, *zs = H->zs, *snap = H->snap;
+    double4 *rec = H->rec;
+    double2 *vol = H->vol;
+    const int *cell = H->f_cell, *start = H->f_start, *noverflow = H->noverflow;
+    int *bcount = H->bcount, *nel = H->nel, *nne = H->counters;
+    float4 *xf = H->xf;
     P = with_sound(P);
     const int f = *flag;
     // MODE 0 runs first in every kick: it resets the work counter of the brick kernel
@@ -203,7 +206,7 @@ __global__ void k_gather(int *flag, int *work, DevParams P, const int *__restric
                 nel[atomicAdd(nne, 1)] = b;
         }
     }
-    if (MODE == 1 && nrebuild && blockIdx.x == 0 && threadIdx.x == 0) *nrebuild += 1;
+    if (MODE == 1 && H->nrebuild && blockIdx.x == 0 && threadIdx.x == 0) *H->nrebuild += 1;
 }
 
 
@@ -215,11 +218,15 @@ __global__ void k_gather(int *flag, int *work, DevParams P, const int *__restric
 // end).  A count of -1 (overflow) walks the cells on the first lane.
 template <int ND, int LANES>
 __global__ void __launch_bounds__(kBlock)
-    k_wall(DevParams P, FluidView F, const double4 *__restrict__ wpos, double *__restrict__ pw,
-           double *__restrict__ rhow, double2 *__restrict__ wpv, const int *__restrict__ alist,
-           const int *__restrict__ acnt, int lw, const int *__restrict__ active,
-           const int *__restrict__ nactive, double *__restrict__ wvel)
+    k_wall(const DevHandle *__restrict__ H)
 {
+    DevParams P = H->params();
+    const FluidView F = H->fluid();
+    const double4 *wpos = H->wpos;
+    double *pw = H->pw, *rhow = H->rhow, *wvel = H->wvel;
+    double2 *wpv = H->wpv;
+    const int *alist = H->anbr, *acnt = H->acnt, *active = H->wactive, *nactive = H->counters + 1;
+    const int lw = H->lw;
     P = with_sound(P);
     const int na = alist ? *nactive : P.nw;
     const int q = threadIdx.x % LANES;
@@ -263,11 +270,13 @@ __global__ void __launch_bounds__(kBlock)
 // of dv only).
 template <int ND, bool SUM = false>
 __global__ void __launch_bounds__(kBlock)
-    k_fluid(int *flag, DevParams P, FluidView F, WallView Wv,
-            const unsigned char *__restrict__ wall_near, double *__restrict__ dv)
+    k_fluid(const DevHandle *__restrict__ H, double *__restrict__ dv)
 {
-    P = with_sound(P);
-    if (blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;  // the rebuild (if any) is done
+    const DevParams P = with_sound(H->params());
+    const FluidView F = H->fluid();
+    const WallView Wv = H->walls();
+    const unsigned char *wall_near = H->wall_near;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *H->flag = 0;  // the rebuild (if any) is done
     __shared__ int lists[kCap * kBlock];
     int *lst = lists + threadIdx.x;
     const int s = xcd_tile(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
@@ -330,9 +339,13 @@ __global__ void __launch_bounds__(kBlock)
 // then sets the records, so that no lane reads a record another lane writes.
 template <int ND>
 __global__ void __launch_bounds__(kBlock)
-    k_sum_density(DevParams P, FluidView F, WallView Wv,
-                  const unsigned char *__restrict__ wall_near, double *__restrict__ rho)
+    k_sum_density(const DevHandle *__restrict__ H)
 {
+    const DevParams P = H->params();
+    const FluidView F = H->fluid();
+    const WallView Wv = H->walls();
+    const unsigned char *wall_near = H->wall_near;
+    double *rho = H->sum_rho;
     const int s = xcd_tile(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
     if (s >= P.nf) return;
     const double x0 = F.x[s], x1 = F.y[s], x2 = (ND == 3) ? F.z[s] : 0.0;
@@ -370,11 +383,14 @@ __global__ void __launch_bounds__(kBlock)
 // in a fixed order.
 template <int ND>
 __global__ void __launch_bounds__(kBlock)
-    k_sum_density_lists(DevParams P, FluidView F, WallView Wv, const int *__restrict__ ord,
-                        const int *__restrict__ nbr, const int *__restrict__ cnt,
-                        const int *__restrict__ wnbr, const int *__restrict__ wcnt, int ls,
-                        double *__restrict__ rho)
+    k_sum_density_lists(const DevHandle *__restrict__ H)
 {
+    const DevParams P = H->params();
+    const FluidView F = H->fluid();
+    const WallView Wv = H->walls();
+    const int *ord = H->ord, *nbr = H->nbr, *cnt = H->cnt, *wnbr = H->wnbr, *wcnt = H->wcnt;
+    const int ls = H->ls;
+    double *rho = H->sum_rho;
     const int q = threadIdx.x % 4;
     const int t = (blockIdx.x * blockDim.x + threadIdx.x) / 4;
     const bool active = t < P.nf;
@@ -424,7 +440,7 @@ __global__ void __launch_bounds__(kBlock)
     if (active && q == 0) rho[s] = sum;
 }
 
-// Arguments of the brick kernels (see tpsph_handle).
+// The brick kernels' part of the handle (see tpsph_handle).
 struct BrickArgs {
     const int *ord, *nne;
     int *work;
@@ -436,6 +452,13 @@ struct BrickArgs {
     int ls;
     double *dv;
     const int *bfall;
+
+    __device__ __forceinline__ explicit BrickArgs(const DevHandle &H, double *rates = nullptr)
+        : ord(H.ord), nne(H.counters), work(H.bwork), bhead(H.bhead), uidx(H.uidx),
+          nbr16(H.nbr16), thead(H.thead), nbr(H.nbr), cnt(H.cnt), wcnt(H.wcnt), ls(H.ls),
+          dv(rates), bfall(H.bfall)
+    {
+    }
 };
 
 // The 16-byte (8-byte) field of the record at byte offset e16 (16 times its number).
@@ -461,9 +484,14 @@ struct SumSmem {
 
 template <int ND>
 __global__ void __launch_bounds__(kBrickThreads)
-    k_sum_density_brick(DevParams P, FluidView F, WallView Wv, BrickArgs A,
-                        const int *__restrict__ wnbr, double *__restrict__ rho)
+    k_sum_density_brick(const DevHandle *__restrict__ H)
 {
+    const DevParams P = H->params();
+    const FluidView F = H->fluid();
+    const WallView Wv = H->walls();
+    const BrickArgs A(*H);
+    const int *wnbr = H->wnbr;
+    double *rho = H->sum_rho;
     __shared__ SumSmem<ND> S;
     const int tid = threadIdx.x;
     const int ne = *A.nne, ls = A.ls;
@@ -562,10 +590,13 @@ __global__ void __launch_bounds__(kBrickThreads)
 
 // The records of the summed densities: rho, the state equation's pressure and V = m / rho.
 __global__ void __launch_bounds__(kBlock)
-    k_sum_finish(DevParams P, int nf, const double *__restrict__ rho, double4 *__restrict__ rec,
-                 double2 *__restrict__ vol)
+    k_sum_finish(const DevHandle *__restrict__ H)
 {
-    P = with_sound(P);
+    const DevParams P = with_sound(H->params());
+    const int nf = P.nf;
+    const double *rho = H->sum_rho;
+    double4 *rec = H->rec;
+    double2 *vol = H->vol;
     const int s = blockIdx.x * kBlock + threadIdx.x;
     if (s >= nf) return;
     const double r = rho[s];
@@ -708,13 +739,14 @@ __device__ __forceinline__ void
 // radius test (and the zero-distance skip) selects the pairs.
 template <int ND>
 __global__ void __launch_bounds__(kBlock)
-    k_fluid_list(int *flag, DevParams P, FluidView F, WallView Wv, const int *__restrict__ ord,
-                 const int *__restrict__ nbr, const int *__restrict__ cnt,
-                 const int *__restrict__ wnbr, const int *__restrict__ wcnt, int ls,
-                 double *__restrict__ dv)
+    k_fluid_list(const DevHandle *__restrict__ H, double *__restrict__ dv)
 {
-    P = with_sound(P);
-    if (blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;  // the rebuild (if any) is done
+    const DevParams P = with_sound(H->params());
+    const FluidView F = H->fluid();
+    const WallView Wv = H->walls();
+    const int *ord = H->ord, *nbr = H->nbr, *cnt = H->cnt, *wnbr = H->wnbr, *wcnt = H->wcnt;
+    const int ls = H->ls;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *H->flag = 0;  // the rebuild (if any) is done
     // 8 KiB per wavefront: the staging area (64 records x 80 bytes) while the lists are
     // streamed, then the int lists (kCap x 64 lanes) of the cell-walk fallback
     constexpr int kWaveUnits = 64 * kCap / 4;  // 16-byte units
@@ -846,9 +878,10 @@ __global__ void __launch_bounds__(kBlock)
 // Without staging (h->bricks false: the union rows of a brick exceed kBrickMaxRows) every brick
 // takes the int lists.
 // ------------------------------------------------------------------------------------------
+// The list build's part of the handle (see tpsph_handle).
 struct ListsArgs {
     const int *nel;
-    int *nne;  // counters (see tpsph_handle): [0] bricks ... [6] work counter
+    int *nne;  // counters: [0] bricks ... [6] work counter
     int *bcount, *ord, *tbase, *uidx;
     int uidx_cap;
     int4 *bhead;
@@ -857,14 +890,14 @@ struct ListsArgs {
     const unsigned char *wall_near;
     unsigned short *nbr16;  // nullptr: no brick stages
     int2 *thead;
-};
-struct WallListsArgs {
-    const double4 *wpos;
-    int lw, cap;
-    int *nbr, *cnt, *active, *nactive;
-    double *pw, *rhow;
-    double2 *wpv;
-    double *wvel;
+
+    __device__ __forceinline__ explicit ListsArgs(const DevHandle &H)
+        : nel(H.nel), nne(H.counters), bcount(H.bcount), ord(H.ord), tbase(H.tbase), uidx(H.uidx),
+          uidx_cap(H.uidx_cap), bhead(H.bhead), ls(H.ls), cap_f(H.cap_f), cap_w(H.cap_w),
+          nbr(H.nbr), cnt(H.cnt), wnbr(H.wnbr), wcnt(H.wcnt), wtargets(H.wtargets),
+          wall_near(H.wall_near), nbr16(H.nbr16), thead(H.thead)
+    {
+    }
 };
 
 struct ListsSmem {
@@ -1196,15 +1229,19 @@ __device__ __forceinline__ void brick_int_lists(const DevParams &P, const FluidV
 // Two blocks of 512 threads share a compute unit (76 KB each).
 template <int ND>
 __global__ void __launch_bounds__(kListThreads, 4)
-    k_brick_lists(const int *flag, DevParams P, FluidView F, WallView Wv, ListsArgs A,
-                  WallListsArgs W, int nblocks)
+    k_brick_lists(const DevHandle *__restrict__ H, int nblocks)
 {
-    if (skip(flag)) return;
+    if (skip(H->flag)) return;
+    const DevParams P = H->params();
+    const FluidView F = H->fluid();
     if ((int)blockIdx.x >= nblocks) {
-        wall_lists_body<ND>(blockIdx.x - nblocks, gridDim.x - nblocks, P, F, W.wpos, W.lw, W.cap, W.nbr,
-                            W.cnt, W.active, W.nactive, W.pw, W.rhow, W.wpv, W.wvel);
+        wall_lists_body<ND>(blockIdx.x - nblocks, gridDim.x - nblocks, P, F, H->wpos, H->lw, H->cap_a,
+                            H->anbr, H->acnt, H->wactive, H->counters + 1, H->pw, H->rhow, H->wpv,
+                            H->wvel);
         return;
     }
+    const WallView Wv = H->walls();
+    const ListsArgs A(*H);
     __shared__ ListsSmem S;
     const int tid = threadIdx.x;
     const int ne = A.nne[0];
@@ -1618,13 +1655,15 @@ __device__ __forceinline__ int2 union_share(const int *__restrict__ uidx, int fi
 // (pressure slot staged as p / rho^2, no density rate, dv of ND rows).
 template <int ND, int VISC = kViscAlpha, bool ANT = false, bool SUM = false>
 __global__ void __launch_bounds__(kBrickThreads)
-    k_fluid_brick(int *flag, DevParams P, FluidView F, BrickArgs A)
+    k_fluid_brick(const DevHandle *__restrict__ H, double *__restrict__ dv)
 {
-    P = with_sound(P);
+    const DevParams P = with_sound(H->params());
+    const FluidView F = H->fluid();
+    const BrickArgs A(*H, dv);
     using Smem = BrickSmem<ND, ANT>;
     __shared__ Smem S;
     const int tid = threadIdx.x;
-    if (blockIdx.x == 0 && tid == 0) *flag = 0;  // the rebuild (if any) is done
+    if (blockIdx.x == 0 && tid == 0) *H->flag = 0;  // the rebuild (if any) is done
     const int ne = *A.nne;
     if ((int)blockIdx.x >= ne) return;  // uniform: a block without a brick
     constexpr int kFarSlot = Smem::CAP - 1;
@@ -1757,9 +1796,11 @@ __global__ void __launch_bounds__(kBrickThreads)
 // FP64: the work[1] bricks it listed in bfall, taken by blocks in turn.
 template <int ND>
 __global__ void __launch_bounds__(kBrickThreads)
-    k_fluid_brick_global(DevParams P, FluidView F, BrickArgs A)
+    k_fluid_brick_global(const DevHandle *__restrict__ H, double *__restrict__ dv)
 {
-    P = with_sound(P);
+    const DevParams P = with_sound(H->params());
+    const FluidView F = H->fluid();
+    const BrickArgs A(*H, dv);
     const int ne = A.work[1];
     for (int k = blockIdx.x; k < ne; k += gridDim.x) {
         const int4 hd = A.bhead[A.bfall[k]];
@@ -1774,12 +1815,14 @@ __global__ void __launch_bounds__(kBrickThreads)
 // SUM: SummationDensity (the target's p / rho^2 in the pressure slot, dv of ND rows).
 template <int ND, bool SUM = false>
 __global__ void __launch_bounds__(kBlock)
-    k_fluid_walls(DevParams P, FluidView F, WallView Wv, const int *__restrict__ ord,
-                  const int *__restrict__ wtargets, const int *__restrict__ nwtargets,
-                  const int *__restrict__ wnbr, const int *__restrict__ wcnt, int ls,
-                  double *__restrict__ dv)
+    k_fluid_walls(const DevHandle *__restrict__ H, double *__restrict__ dv)
 {
-    P = with_sound(P);
+    const DevParams P = with_sound(H->params());
+    const FluidView F = H->fluid();
+    const WallView Wv = H->walls();
+    const int *ord = H->ord, *wtargets = H->wtargets, *nwtargets = H->counters + 2;
+    const int *wnbr = H->wnbr, *wcnt = H->wcnt;
+    const int ls = H->ls;
     constexpr int kLanes = 4;
     __shared__ int lists[kCap * kBlock];  // only for particles whose wall list overflowed
     int *lst = lists + threadIdx.x;
@@ -1969,9 +2012,12 @@ __device__ __forceinline__ void grad_sums_global(const DevParams &P, const Fluid
 // without lists (nbr == nullptr), the cell walk of every particle.
 template <int ND>
 __global__ void __launch_bounds__(kBlock)
-    k_antuono_gradient(DevParams P, FluidView F, const int *__restrict__ ord,
-                       const int *__restrict__ nbr, const int *__restrict__ cnt, int ls)
+    k_antuono_gradient(const DevHandle *__restrict__ H, bool lists)
 {
+    const DevParams P = H->params();
+    const FluidView F = H->fluid();
+    const int *ord = H->ord, *nbr = lists ? (const int *)H->nbr : nullptr, *cnt = H->cnt;
+    const int ls = H->ls;
     const int q = threadIdx.x % 4;
     const int t = (blockIdx.x * blockDim.x + threadIdx.x) / 4;
     const bool active = t < P.nf;
@@ -1998,8 +2044,11 @@ struct GradSmem {
 
 template <int ND>
 __global__ void __launch_bounds__(kBrickThreads)
-    k_antuono_gradient_brick(DevParams P, FluidView F, BrickArgs A)
+    k_antuono_gradient_brick(const DevHandle *__restrict__ H)
 {
+    const DevParams P = H->params();
+    const FluidView F = H->fluid();
+    const BrickArgs A(*H);
     __shared__ GradSmem<ND> S;
     const int tid = threadIdx.x;
     const int ne = *A.nne, ls = A.ls;
@@ -2087,14 +2136,18 @@ __global__ void k_drift(int nf, int vrows, const double *__restrict__ v, double 
 // the last rebuild.
 template <int ND>
 __global__ void __launch_bounds__(kBlock)
-    k_ck_stage_gather(int *flag, int *work, DevParams P, int nf, double *__restrict__ v,
+    k_ck_stage_gather(const DevHandle *__restrict__ H, double *__restrict__ v,
                       double *__restrict__ u, double *__restrict__ tv, double *__restrict__ tu,
-                      const double *__restrict__ dv, double a, double b, double dt, int first,
-                      const int *__restrict__ iperm, const double *__restrict__ m,
-                      double *__restrict__ xs, double *__restrict__ ys, double *__restrict__ zs,
-                      double4 *__restrict__ rec, double2 *__restrict__ vol,
-                      const double *__restrict__ snap, const int *__restrict__ noverflow)
+                      const double *__restrict__ dv, double a, double b, double dt, int first)
 {
+    DevParams P = H->params();
+    int *flag = H->flag, *work = H->bwork;
+    const int *iperm = H->iperm, *noverflow = H->noverflow;
+    const double *m = H->mass, *snap = H->snap;
+    double *xs = H->xs, *ys = H->ys, *zs = H->zs;
+    double4 *rec = H->rec;
+    double2 *vol = H->vol;
+    const int nf = P.nf;
     P = with_sound(P);
     const int i0 = blockIdx.x * kBlock;
     const int np = min(kBlock, nf - i0);
@@ -2176,9 +2229,12 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 __global__ void __launch_bounds__(kBlock)
-    k_sound_speed(DevParams P, int nparts, const double *__restrict__ part, double *__restrict__ dyn,
-                  double alpha, double delta)
+    k_sound_speed(const DevHandle *__restrict__ H, int nparts)
 {
+    const DevParams P = H->params();
+    const double *part = H->vmax_part;
+    double *dyn = H->dyn;
+    const double alpha = H->alpha, delta = H->delta;
     __shared__ double s[kBlock];
     double m = 0.0;
     for (int i = threadIdx.x; i < nparts; i += kBlock) m = fmax(m, part[i]);
@@ -2502,14 +2558,13 @@ namespace {
 // gather that follows orders them).
 template <int ND>
 int build_cells(tpsph_handle *h, const int *flag, int n, const double *x, int *cell, int *rank,
-                int *count, int *start, int *perm, bool ordered = true, int *zero = nullptr,
-                int nzero = 0)
+                int *count, int *start, int *perm, bool ordered = true, int *counters = nullptr)
 {
     // count is zero on entry (cleared at create, and again by k_scatter)
     const int nc = h->P.ncells;
     // (n = 0 too: it clears the scan's state)
-    hipLaunchKernelGGL((k_cells<ND>), dim3(gate_blocks(n)), dim3(kBlock), 0, h->stream, flag, h->P, n, x, cell, rank, count,
-                       h->scan_state, scan_words(nc + 1), zero, nzero);
+    hipLaunchKernelGGL((k_cells<ND>), dim3(gate_blocks(n)), dim3(kBlock), 0, h->stream, h->dev, flag, n, x,
+                       cell, rank, count, counters);
     TRY(launch_check(h, "k_cells"));
     TRY(scan(h, flag, count, start, nc + 1));
     if (n > 0) {
@@ -2530,53 +2585,32 @@ int update_fluid(tpsph_handle *h, const double *v, const double *u, bool gathere
     if (keep_order) {
         // the order and the lists stand: only the records of (v, u)
         hipLaunchKernelGGL((k_set_i32), dim3(1), dim3(1), 0, h->stream, h->flag, 0);
-        hipLaunchKernelGGL((k_gather<ND, 0>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream,
-            h->flag, h->bwork, h->P, h->f_perm, u, v, h->f_mass, h->xs, h->ys, h->zs, h->rec, h->vol,
-            h->snap, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
-            h->search == TPSPH_SEARCH_LISTS ? h->counters + 3 : nullptr, nullptr, nullptr);
+        hipLaunchKernelGGL((k_gather<ND, 0>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream, h->dev, u, v);
         return launch_check(h, "k_gather<0>");
     }
     if (!gathered) {  // else the stage kernel wrote the records of (v, u)
         TimedScope t(h, TPSPH_TIME_GATHER);
-        hipLaunchKernelGGL((k_gather<ND, 0>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream,
-            h->flag, h->bwork, h->P, h->f_perm, u, v, h->f_mass, h->xs, h->ys, h->zs, h->rec, h->vol,
-            h->snap, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
-            h->search == TPSPH_SEARCH_LISTS ? h->counters + 3 : nullptr, nullptr, nullptr);
+        hipLaunchKernelGGL((k_gather<ND, 0>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream, h->dev, u, v);
         TRY(launch_check(h, "k_gather<0>"));
     }
     {
         TimedScope t(h, TPSPH_TIME_CELL_LIST);
         const bool lists = h->search == TPSPH_SEARCH_LISTS;
         TRY(build_cells<ND>(h, h->flag, nf, u, h->f_cell, h->f_rank, h->f_count, h->f_start,
-                            h->f_permu, false, lists ? h->counters : nullptr, kCounters));
-        // the gather orders the members of every cell and, with lists, finds the bricks
-        hipLaunchKernelGGL((k_gather<ND, 1>), dim3(gate_blocks(nf)), dim3(kBlock), 0, h->stream,
-            h->flag, nullptr, h->P, h->f_permu, u, v, h->f_mass, h->xs, h->ys, h->zs, h->rec, h->vol,
-            h->snap, h->iperm, h->f_cell, h->f_start, h->f_perm, lists ? h->bcount : nullptr,
-            h->nel, h->counters, nullptr, h->nrebuild, lists ? h->xf : nullptr);
+                            h->f_permu, h->f_permu == h->f_perm, lists ? h->counters : nullptr));
+        // the gather orders the members of every cell (where the scatter had an array of its
+        // own; in place k_sort_cells has done it) and, with lists, finds the bricks
+        hipLaunchKernelGGL((k_gather<ND, 1>), dim3(gate_blocks(nf)), dim3(kBlock), 0, h->stream, h->dev, u, v);
         if (lists) {
             const int gb = std::max(1, std::min(h->nbricks, 2 * h->n_cu));
             const int gw = (h->nw + kListThreads - 1) / kListThreads;
-            hipLaunchKernelGGL((k_brick_lists<ND>), dim3(gb + gw), dim3(kListThreads), 0, h->stream,
-                h->flag, h->P, h->fluid_view(), h->wall_view(),
-                ListsArgs{h->nel, h->counters, h->bcount, h->ord, h->tbase, h->uidx, (int)h->uidx_cap,
-                          h->bhead, h->ls, h->cap_f, h->cap_w, h->nbr, h->cnt, h->wnbr, h->wcnt,
-                          h->wtargets, h->wall_near, h->nbr16, h->thead},
-                WallListsArgs{h->wpos, h->lw, h->cap_a, h->anbr, h->acnt, h->wactive,
-                              h->counters + 1, h->pw, h->rhow, h->wpv, h->wvel},
-                gb);
+            hipLaunchKernelGGL((k_brick_lists<ND>), dim3(gb + gw), dim3(kListThreads), 0, h->stream, h->dev, gb);
             TRY(launch_check(h, "k_brick_lists"));
         }
         // the fluid kernel of this kick lowers the flag
         TRY(launch_check(h, "k_gather<1>"));
     }
     return TPSPH_OK;
-}
-
-BrickArgs brick_args(const tpsph_handle *h, double *dv)
-{
-    return {h->ord, h->counters, h->bwork, h->bhead, h->uidx, h->nbr16, h->thead, h->nbr, h->cnt,
-            h->wcnt, h->ls, dv, h->bfall};
 }
 
 // Everything a kick does before the fluid pass: the sound speed (adaptive), the cell-sorted
@@ -2593,8 +2627,7 @@ int prepare_impl(tpsph_handle *h, const double *v, const double *u, bool gathere
         TimedScope t(h, TPSPH_TIME_GATHER);
         const int nb = gate_blocks(nf);
         hipLaunchKernelGGL((k_vmax<ND>), dim3(nb), dim3(kBlock), 0, h->stream, nf, h->P.vrows, v, h->vmax_part);
-        hipLaunchKernelGGL((k_sound_speed), dim3(1), dim3(kBlock), 0, h->stream, h->P, nb,
-                           h->vmax_part, h->dyn, h->params.alpha, h->params.delta);
+        hipLaunchKernelGGL((k_sound_speed), dim3(1), dim3(kBlock), 0, h->stream, h->dev, nb);
         TRY(launch_check(h, "k_vmax/k_sound_speed"));
         gathered = false;
     }
@@ -2603,31 +2636,21 @@ int prepare_impl(tpsph_handle *h, const double *v, const double *u, bool gathere
         // compute_density! before the state equation (wcsph/system.jl:291-301, 323-326)
         TimedScope t(h, TPSPH_TIME_GATHER);
         if (h->search == TPSPH_SEARCH_LISTS && h->bricks)
-            hipLaunchKernelGGL((k_sum_density_brick<ND>),
-                dim3(std::max(1, std::min(h->nbricks, h->n_cu))), dim3(kBrickThreads), 0,
-                h->stream, h->P, h->fluid_view(), h->wall_view(), brick_args(h, nullptr), h->wnbr,
-                h->sum_rho);
+            hipLaunchKernelGGL((k_sum_density_brick<ND>), dim3(std::max(1, std::min(h->nbricks, h->n_cu))),
+                               dim3(kBrickThreads), 0, h->stream, h->dev);
         else if (h->search == TPSPH_SEARCH_LISTS)
-            hipLaunchKernelGGL((k_sum_density_lists<ND>), dim3(nblocks(4 * (int64_t)nf)), dim3(kBlock),
-                               0, h->stream, h->P, h->fluid_view(), h->wall_view(), h->ord, h->nbr,
-                               h->cnt, h->wnbr, h->wcnt, h->ls, h->sum_rho);
+            hipLaunchKernelGGL((k_sum_density_lists<ND>), dim3(nblocks(4 * (int64_t)nf)), dim3(kBlock), 0, h->stream, h->dev);
         else
-            hipLaunchKernelGGL((k_sum_density<ND>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream,
-                               h->P, h->fluid_view(), h->wall_view(), h->wall_near, h->sum_rho);
-        hipLaunchKernelGGL((k_sum_finish), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream, h->P,
-                           nf, h->sum_rho, h->rec, h->vol);
+            hipLaunchKernelGGL((k_sum_density<ND>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream, h->dev);
+        hipLaunchKernelGGL((k_sum_finish), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream, h->dev);
         TRY(launch_check(h, "k_sum_density"));
     }
     if (nw > 0) {
         TimedScope t(h, TPSPH_TIME_WALL);
         if (h->anbr)
-            hipLaunchKernelGGL((k_wall<ND, 4>), dim3(gate_blocks(4 * (int64_t)nw)), dim3(kBlock), 0,
-                h->stream, h->P, h->fluid_view(), h->wpos, h->pw, h->rhow, h->wpv, h->anbr, h->acnt,
-                h->lw, h->wactive, h->counters + 1, h->wvel);
+            hipLaunchKernelGGL((k_wall<ND, 4>), dim3(gate_blocks(4 * (int64_t)nw)), dim3(kBlock), 0, h->stream, h->dev);
         else
-            hipLaunchKernelGGL((k_wall<ND, 1>), dim3(nblocks(nw)), dim3(kBlock), 0, h->stream, h->P,
-                h->fluid_view(), h->wpos, h->pw, h->rhow, h->wpv, nullptr, nullptr, h->lw, nullptr,
-                nullptr, h->wvel);
+            hipLaunchKernelGGL((k_wall<ND, 1>), dim3(nblocks(nw)), dim3(kBlock), 0, h->stream, h->dev);
         TRY(launch_check(h, "k_wall"));
     }
     return TPSPH_OK;
@@ -2644,22 +2667,18 @@ int kick_impl(tpsph_handle *h, double *dv, const double *v, const double *u, boo
             const bool lists = h->search == TPSPH_SEARCH_LISTS;
             if (lists && h->bricks)
                 hipLaunchKernelGGL((k_antuono_gradient_brick<ND>),
-                    dim3(std::max(1, std::min(h->nbricks, h->n_cu))), dim3(kBrickThreads), 0,
-                    h->stream, h->P, h->fluid_view(), brick_args(h, nullptr));
+                    dim3(std::max(1, std::min(h->nbricks, h->n_cu))), dim3(kBrickThreads), 0, h->stream, h->dev);
             else
                 hipLaunchKernelGGL((k_antuono_gradient<ND>), dim3(nblocks(4 * (int64_t)nf)), dim3(kBlock), 0,
-                                   h->stream, h->P, h->fluid_view(), lists ? h->ord : nullptr,
-                                   lists ? h->nbr : nullptr, lists ? h->cnt : nullptr, h->ls);
+                                   h->stream, h->dev, lists);
             TRY(launch_check(h, "k_antuono_gradient"));
         }
         if (h->search == TPSPH_SEARCH_LISTS && h->bricks && h->mixed) {
             TRY(launch_fluid_brick_mixed(h, dv));
             hipLaunchKernelGGL((k_fluid_brick_global<ND>), dim3(std::max(1, std::min(h->nbricks, h->n_cu))),
-                dim3(kBrickThreads), 0, h->stream, h->P, h->fluid_view(), brick_args(h, dv));
+                dim3(kBrickThreads), 0, h->stream, h->dev, dv);
             if (nw > 0)
-                hipLaunchKernelGGL((k_fluid_walls<ND>), dim3(gate_blocks(4 * (int64_t)nf)), dim3(kBlock), 0, h->stream,
-                    h->P, h->fluid_view(), h->wall_view(), h->ord, h->wtargets, h->counters + 2,
-                    h->wnbr, h->wcnt, h->ls, dv);
+                hipLaunchKernelGGL((k_fluid_walls<ND>), dim3(gate_blocks(4 * (int64_t)nf)), dim3(kBlock), 0, h->stream, h->dev, dv);
         } else if (h->search == TPSPH_SEARCH_LISTS && h->bricks) {
             const int vm = visc_mode(h->P);
             const bool ant = h->P.ddgrad != nullptr, sum = h->P.summation != 0;
@@ -2673,22 +2692,17 @@ int kick_impl(tpsph_handle *h, double *dv, const double *v, const double *u, boo
                       : (vm == kViscNone    ? k_fluid_brick<ND, kViscNone>
                          : vm == kViscAlpha ? k_fluid_brick<ND, kViscAlpha>
                                             : k_fluid_brick<ND, kViscAlphaBeta>);
-            hipLaunchKernelGGL(brick, dim3(std::max(1, std::min(h->nbricks, h->n_cu))),
-                dim3(kBrickThreads), 0, h->stream, h->flag, h->P, h->fluid_view(), brick_args(h, dv));
+            hipLaunchKernelGGL(brick, dim3(std::max(1, std::min(h->nbricks, h->n_cu))), dim3(kBrickThreads), 0,
+                h->stream, h->dev, dv);
             const auto walls = sum ? k_fluid_walls<ND, true> : k_fluid_walls<ND, false>;
             if (nw > 0)
-                hipLaunchKernelGGL(walls, dim3(gate_blocks(4 * (int64_t)nf)), dim3(kBlock), 0, h->stream,
-                    h->P, h->fluid_view(), h->wall_view(), h->ord, h->wtargets, h->counters + 2,
-                    h->wnbr, h->wcnt, h->ls, dv);
+                hipLaunchKernelGGL(walls, dim3(gate_blocks(4 * (int64_t)nf)), dim3(kBlock), 0, h->stream, h->dev, dv);
         } else if (h->search == TPSPH_SEARCH_LISTS) {
-            hipLaunchKernelGGL((k_fluid_list<ND>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream,
-                h->flag, h->P, h->fluid_view(), h->wall_view(), h->ord, h->nbr, h->cnt, h->wnbr, h->wcnt, h->ls, dv);
+            hipLaunchKernelGGL((k_fluid_list<ND>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream, h->dev, dv);
         } else if (h->P.summation) {
-            hipLaunchKernelGGL((k_fluid<ND, true>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream,
-                h->flag, h->P, h->fluid_view(), h->wall_view(), h->wall_near, dv);
+            hipLaunchKernelGGL((k_fluid<ND, true>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream, h->dev, dv);
         } else {
-            hipLaunchKernelGGL((k_fluid<ND>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream, h->flag,
-                h->P, h->fluid_view(), h->wall_view(), h->wall_near, dv);
+            hipLaunchKernelGGL((k_fluid<ND>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream, h->dev, dv);
         }
         TRY(launch_check(h, "k_fluid"));
     }
@@ -3013,16 +3027,9 @@ int tpsph::run_ck2n54(tpsph_handle *h, double *v, double *u, double dt, int64_t 
             }
             TRY(kick_dispatch(h, h->sol_dv, v, u, gathered));
             TimedScope ts(h, TPSPH_TIME_STAGE);
-            if (h->nd == 2)
-                hipLaunchKernelGGL((k_ck_stage_gather<2>), dim3(nblocks(h->nf)), dim3(kBlock), 0, h->stream,
-                    h->flag, h->bwork, h->P, h->nf, v, u, h->sol_tv, h->sol_tu, h->sol_dv, kCkA[i], kCkB[i], dt,
-                    i == 0, h->iperm, h->f_mass, h->xs, h->ys, h->zs, h->rec, h->vol, h->snap,
-                    h->search == TPSPH_SEARCH_LISTS ? h->counters + 3 : nullptr);
-            else
-                hipLaunchKernelGGL((k_ck_stage_gather<3>), dim3(nblocks(h->nf)), dim3(kBlock), 0, h->stream,
-                    h->flag, h->bwork, h->P, h->nf, v, u, h->sol_tv, h->sol_tu, h->sol_dv, kCkA[i], kCkB[i], dt,
-                    i == 0, h->iperm, h->f_mass, h->xs, h->ys, h->zs, h->rec, h->vol, h->snap,
-                    h->search == TPSPH_SEARCH_LISTS ? h->counters + 3 : nullptr);
+            hipLaunchKernelGGL(h->nd == 2 ? k_ck_stage_gather<2> : k_ck_stage_gather<3>, dim3(nblocks(h->nf)),
+                               dim3(kBlock), 0, h->stream, h->dev, v, u, h->sol_tv, h->sol_tu, h->sol_dv,
+                               kCkA[i], kCkB[i], dt, (int)(i == 0));
             TRY(launch_check(h, "k_ck_stage_gather"));
             gathered = true;
         }
@@ -3034,6 +3041,34 @@ int tpsph::run_ck2n54(tpsph_handle *h, double *v, double *u, double dt, int64_t 
 
 namespace {
 
+
+__global__ void k_put_handle(DevHandle image, DevHandle *dev) { *dev = image; }
+
+// Writes what the kernels read of the handle to h->dev (by a kernel: no host memory is read
+// later, so the write can be captured in a graph).
+int put_handle(tpsph_handle *h)
+{
+    DevHandle d;
+    d.P = h->P;
+    d.f_start = h->f_start; d.f_perm = h->f_perm; d.xs = h->xs; d.ys = h->ys; d.zs = h->zs;
+    d.rec = h->rec; d.vol = h->vol; d.xf = h->xf;
+    d.w_start = h->w_start; d.wx = h->wx; d.wy = h->wy; d.wz = h->wz; d.wpos = h->wpos;
+    d.wpv = h->wpv; d.wvel = h->wvel; d.wxf = h->wxf; d.pw = h->pw; d.rhow = h->rhow;
+    d.flag = h->flag; d.f_cell = h->f_cell; d.f_permu = h->f_permu; d.iperm = h->iperm;
+    d.nrebuild = h->nrebuild; d.counters = h->counters; d.scan_state = h->scan_state;
+    d.scan_words = scan_words(h->P.ncells + 1);
+    d.snap = h->snap; d.mass = h->f_mass; d.wall_near = h->wall_near;
+    d.bcount = h->bcount; d.nel = h->nel; d.ord = h->ord; d.tbase = h->tbase; d.uidx = h->uidx;
+    d.nbr = h->nbr; d.cnt = h->cnt; d.wnbr = h->wnbr; d.wcnt = h->wcnt; d.wtargets = h->wtargets;
+    d.noverflow = h->search == TPSPH_SEARCH_LISTS ? h->counters + 3 : nullptr;
+    d.bwork = h->bwork; d.bfall = h->bfall; d.bhead = h->bhead; d.nbr16 = h->nbr16; d.thead = h->thead;
+    d.uidx_cap = (int)h->uidx_cap; d.ls = h->ls; d.cap_f = h->cap_f; d.cap_w = h->cap_w;
+    d.anbr = h->anbr; d.acnt = h->acnt; d.wactive = h->wactive; d.lw = h->lw; d.cap_a = h->cap_a;
+    d.dyn = h->dyn; d.ddgrad = h->ddgrad; d.vmax_part = h->vmax_part; d.sum_rho = h->sum_rho;
+    d.alpha = h->params.alpha; d.delta = h->params.delta;
+    hipLaunchKernelGGL((k_put_handle), dim3(1), dim3(1), 0, h->stream, d, h->dev);
+    return launch_check(h, "k_put_handle");
+}
 
 // CSR of nrows rows in the caller's order from a count launch and a fill launch of the same
 // kernel: launch(fill, counts, offsets, idx).  offsets / idx may be host or device memory.
@@ -3096,9 +3131,15 @@ int emit_csr(tpsph_handle *h, int nrows, Launch launch, int64_t *offsets, int32_
 // by kernels, so the call records no memset (it can be captured in a HIP graph).
 // ------------------------------------------------------------------------------------------
 constexpr size_t kScratchBytes = size_t(64) << 20;  // 64 MiB per device
+// behind them what depends on no particle: the kernels' copy of the handle and the scan's state
+// (at most one word per kScanTile of the cells that fit, 17 bytes each)
+constexpr size_t kScratchHandle = 2048, kScratchTail = size_t(16) << 10;
+static_assert(sizeof(DevHandle) <= kScratchHandle &&
+                  kScratchHandle + 8 * (kScratchBytes / 17 / kScanTile + 2) <= kScratchTail,
+              "the tail holds the handle and the scan's state");
 constexpr int kMaxDevices = 64;
 
-__device__ __align__(256) unsigned char scratch[kScratchBytes];
+__device__ __align__(256) unsigned char scratch[kScratchBytes + kScratchTail];
 
 __global__ void k_fill_i32(int *p, int value, int n)
 {
@@ -3165,11 +3206,10 @@ int noalloc_kick(tpsph_handle *h, unsigned char *base, size_t *bytes, const doub
     const int nc = h->P.ncells;
     ScratchLayout L{base};
     h->flag = L.take<int>(1);
-    h->scan_state = L.take<unsigned long long>((size_t)scan_words(nc + 1));
     h->f_cell = L.take<int>(nf);
     h->f_rank = L.take<int>(nf);
     h->f_perm = L.take<int>(nf);
-    h->f_permu = L.take<int>(nf);
+    h->f_permu = h->f_perm;  // ordered in place (k_sort_cells)
     h->iperm = L.take<int>(nf);
     h->f_count = L.take<int>((size_t)nc + 1);
     h->f_start = L.take<int>((size_t)nc + 1);
@@ -3192,6 +3232,8 @@ int noalloc_kick(tpsph_handle *h, unsigned char *base, size_t *bytes, const doub
     h->wall_near = L.take<unsigned char>(nc);
     *bytes = L.used;
     if (!base) return TPSPH_OK;
+    h->dev = reinterpret_cast<DevHandle *>(base + kScratchBytes);
+    h->scan_state = reinterpret_cast<unsigned long long *>(base + kScratchBytes + kScratchHandle);
     hipStream_t st = h->stream;
     const double nan = __builtin_nan("");
     // what must start at zero (or NaN): histograms, the wall-near flags, the SoA padding
@@ -3204,6 +3246,8 @@ int noalloc_kick(tpsph_handle *h, unsigned char *base, size_t *bytes, const doub
         hipLaunchKernelGGL((k_fill_f64), dim3(gate_blocks(nw + kPad)), dim3(kBlock), 0, st, a, nan, nw + kPad);
     hipLaunchKernelGGL((k_set_i32), dim3(1), dim3(1), 0, st, h->flag, 1);
     TRY(launch_check(h, "tpsph_kick_noalloc clearing"));
+    h->f_mass = const_cast<double *>(fluid_mass);
+    TRY(put_handle(h));
     // static walls: cell list, sorted positions and masses, cells near walls
     if (nw > 0) {
         TRY(build_cells<ND>(h, nullptr, nw, wall_x, w_cell, w_rank, w_count, h->w_start, h->w_perm));
@@ -3212,7 +3256,6 @@ int noalloc_kick(tpsph_handle *h, unsigned char *base, size_t *bytes, const doub
         hipLaunchKernelGGL((k_wall_near<ND>), dim3(nblocks(nw)), dim3(kBlock), 0, st, h->P, nw, h->wpos, h->wall_near);
         TRY(launch_check(h, "tpsph_kick_noalloc walls"));
     }
-    h->f_mass = const_cast<double *>(fluid_mass);
     return kick_impl<ND>(h, dv, v, u, false);
 }
 
@@ -3482,6 +3525,8 @@ int tpsph_create(const tpsph_params *params, int64_t n_fluid, int64_t n_wall,
             return cleanup_fail(TPSPH_ERR_HIP);
         }
     }
+    CTRY(dalloc(h, &h->dev, 1));
+    CTRY(put_handle(h));
     // static wall cell list
     if (nw > 0) {
         double *wx_d = nullptr, *wm_d = nullptr;
@@ -3999,7 +4044,7 @@ void tpsph_destroy(tpsph_handle *h)
                     h->rhow, h->st_v, h->st_u, h->st_dv, h->st_du, h->sol_dv, h->sol_tv,
                     h->sol_tu, h->integ, h->nrebuild, h->adj_kb, h->adj_coef, h->adj_th,
                     h->adj_gw, h->adj_red, h->adj_vb, h->adj_ub, h->adj_tvb, h->adj_tub,
-                    h->adj_ck, h->adj_st, h->sum_rho, h->bfall, h->thead};
+                    h->adj_ck, h->adj_st, h->sum_rho, h->bfall, h->thead, h->dev};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     for (hipEvent_t e : h->event_pool) (void)hipEventDestroy(e);

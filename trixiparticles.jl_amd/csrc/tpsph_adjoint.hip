@@ -218,12 +218,16 @@ __global__ void __launch_bounds__(kBlock)
 // partial along g: cN sum_f rho_f ghat.(x_w - x_f) W_wf.
 template <int ND>
 __global__ void __launch_bounds__(kBlock)
-    k_adj_wall(DevParams P, AdjConsts K, FluidView F, const double4 *__restrict__ wpos,
-               const double *__restrict__ pw, const double *__restrict__ rhow,
-               const double2 *__restrict__ wpv, const int *__restrict__ alist,
-               const int *__restrict__ acnt, int lw, const double4 *__restrict__ kb,
+    k_adj_wall(const DevHandle *__restrict__ H, AdjConsts K, const double4 *__restrict__ kb,
                double2 *__restrict__ coef, double *__restrict__ gw)
 {
+    const DevParams P = H->params();
+    const FluidView F = H->fluid();
+    const double4 *wpos = H->wpos;
+    const double *pw = H->pw, *rhow = H->rhow;
+    const double2 *wpv = H->wpv;
+    const int *alist = H->anbr, *acnt = H->acnt;
+    const int lw = H->lw;
     // four lanes per wall particle (the loop bound is uniform per group of lanes, so the
     // partners shuffle together); lane q takes the list entries q, q + 4, ...
     const int q = threadIdx.x % kAdjLanes;
@@ -291,15 +295,18 @@ __global__ void __launch_bounds__(kBlock)
 // the partials along alpha, delta and g into th[3 i ..].
 template <int ND, bool ACC>
 __global__ void __launch_bounds__(kBlock)
-    k_adj_fluid(int *flag, DevParams P, AdjConsts K, FluidView F, WallView Wv,
-                const int *__restrict__ ord, const int *__restrict__ nbr,
-                const int *__restrict__ cnt, const int *__restrict__ tbase,
-                const int *__restrict__ uidx, const unsigned short *__restrict__ nbr16,
-                const int *__restrict__ wnbr,
-                const int *__restrict__ wcnt, int ls, const double4 *__restrict__ kb,
-                const double2 *__restrict__ coef, double *__restrict__ vb,
-                double *__restrict__ ub, double *__restrict__ th)
+    k_adj_fluid(const DevHandle *__restrict__ H, AdjConsts K,
+                const double4 *__restrict__ kb, const double2 *__restrict__ coef,
+                double *__restrict__ vb, double *__restrict__ ub, double *__restrict__ th)
 {
+    const DevParams P = H->params();
+    const FluidView F = H->fluid();
+    const WallView Wv = H->walls();
+    const int *ord = H->ord, *nbr = H->nbr, *cnt = H->cnt, *uidx = H->uidx, *wnbr = H->wnbr;
+    const int *wcnt = H->wcnt, *tbase = uidx ? (const int *)H->tbase : nullptr;
+    const unsigned short *nbr16 = H->nbr16;
+    const int ls = H->ls;
+    int *flag = H->flag;
     if (blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;  // the rebuild (if any) is done
     const int q = threadIdx.x % kAdjLanes;
     const int tt = (xcd_tile(blockIdx.x, gridDim.x) * kBlock + (int)threadIdx.x) / kAdjLanes;
@@ -555,20 +562,13 @@ int adjoint_passes(tpsph_handle *h, double *vb, double *ub)
 {
     TimedScope ts(h, TPSPH_TIME_ADJOINT);
     const AdjConsts K = adj_consts(h);
-    const bool lists = h->search == TPSPH_SEARCH_LISTS;
     if (h->nw > 0) {
         hipLaunchKernelGGL((k_adj_wall<ND>), dim3(nblocks(kAdjLanes * (int64_t)h->nw)), dim3(kBlock), 0, h->stream,
-                           h->P, K, h->fluid_view(), h->wpos, h->pw, h->rhow, h->wpv,
-                           lists ? h->anbr : nullptr, lists ? h->acnt : nullptr, h->lw,
-                           h->adj_kb, h->adj_coef, h->adj_gw);
+                           h->dev, K, h->adj_kb, h->adj_coef, h->adj_gw);
         TRY(launch_check(h, "k_adj_wall"));
     }
     hipLaunchKernelGGL((k_adj_fluid<ND, ACC>), dim3(nblocks(kAdjLanes * (int64_t)h->nf)), dim3(kBlock), 0, h->stream,
-                       h->flag, h->P, K, h->fluid_view(), h->wall_view(),
-                       lists ? h->ord : nullptr, lists ? h->nbr : nullptr,
-                       lists ? h->cnt : nullptr, h->bricks ? h->tbase : nullptr, h->uidx, h->nbr16,
-                       lists ? h->wnbr : nullptr, lists ? h->wcnt : nullptr, h->ls, h->adj_kb, h->adj_coef, vb, ub,
-                       h->adj_th);
+                       h->dev, K, h->adj_kb, h->adj_coef, vb, ub, h->adj_th);
     return launch_check(h, "k_adj_fluid");
 }
 

@@ -139,6 +139,68 @@ struct WallView {
     const double *vel;   // wall velocity for the viscosity (3 per particle), or nullptr
     const float4 *xf = nullptr;  // the FP32 positions of the list build (Verlet lists only)
 };
+// Pointer to global memory inside a struct that lives in device memory: loaded as such, so that
+// accesses through it are global ones (a generic pointer loaded from memory gives flat
+// accesses, which also hold up the LDS counter).
+template <typename T>
+struct GlobalPtr {
+    typedef __attribute__((address_space(1))) T *Address;
+    Address p;
+    __host__ __device__ GlobalPtr(T *x = nullptr) : p((Address)(uintptr_t)x) {}
+    __device__ __forceinline__ operator T *() const { return (T *)p; }
+};
+
+// What the kernels of a kick read of a handle, in device memory: the kernels take its address
+// and the caller's arrays.  A launch costs the host 2.8 us with 16 bytes of arguments and 4.1 us
+// with the kilobyte that the parameters and arrays are by value (measured), and a kick of a
+// small fluid is as long as its launches take.  Written once, at create.
+struct DevHandle {
+    DevParams P;
+    // FluidView and WallView
+    GlobalPtr<int> f_start, f_perm;
+    GlobalPtr<double> xs, ys, zs;
+    GlobalPtr<double4> rec;
+    GlobalPtr<double2> vol;
+    GlobalPtr<float4> xf;
+    GlobalPtr<const int> w_start;
+    GlobalPtr<const double> wx, wy, wz;
+    GlobalPtr<const double4> wpos;
+    GlobalPtr<double2> wpv;
+    GlobalPtr<double> wvel;
+    GlobalPtr<const float4> wxf;
+    GlobalPtr<double> pw, rhow;
+    // cell list
+    GlobalPtr<int> flag, f_cell, f_permu, iperm, nrebuild, counters;
+    GlobalPtr<unsigned long long> scan_state;
+    int scan_words;
+    GlobalPtr<double> snap;
+    GlobalPtr<const double> mass;
+    GlobalPtr<const unsigned char> wall_near;
+    // Verlet lists and bricks (null without)
+    GlobalPtr<int> bcount, nel, ord, tbase, uidx, nbr, cnt, wnbr, wcnt, wtargets, noverflow, bwork,
+        bfall;
+    GlobalPtr<int4> bhead;
+    GlobalPtr<unsigned short> nbr16;
+    GlobalPtr<int2> thead;
+    int uidx_cap, ls, cap_f, cap_w;
+    // Adami lists
+    GlobalPtr<int> anbr, acnt, wactive;
+    int lw, cap_a;
+    // adaptive sound speed, summed densities
+    GlobalPtr<double> dyn, ddgrad, vmax_part, sum_rho;
+    double alpha, delta;
+
+    __device__ __forceinline__ DevParams params() const
+    {
+        DevParams Q = P;
+        Q.dyn = dyn;
+        Q.ddgrad = ddgrad;
+        return Q;
+    }
+    __device__ __forceinline__ FluidView fluid() const { return {f_start, f_perm, xs, ys, zs, rec, vol, xf}; }
+    __device__ __forceinline__ WallView walls() const { return {w_start, wx, wy, wz, wpos, wpv, wvel, wxf}; }
+};
+
 // ------------------------------------------------------------------------------------------
 // device helpers
 // ------------------------------------------------------------------------------------------
@@ -953,6 +1015,8 @@ struct tpsph_handle {
     std::vector<hipEvent_t> event_pool;
     size_t events_used = 0;
     std::vector<Rec> records;
+
+    tpsph::DevHandle *dev = nullptr;  // what the kernels read (device memory)
 
     tpsph::FluidView fluid_view() const { return {f_start, f_perm, xs, ys, zs, rec, vol, xf}; }
     tpsph::WallView wall_view() const { return {w_start, wx, wy, wz, wpos, wpv, wvel, wxf}; }

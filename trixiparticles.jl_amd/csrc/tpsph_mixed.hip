@@ -130,20 +130,22 @@ __device__ __forceinline__ void pair32_term(const Pair32 &q, const float4 &a, co
 // kernel.
 template <int ND>
 __global__ void __launch_bounds__(kBrickThreads, 8)
-    k_fluid_brick32(int *flag, Pair32 q, FluidView F, const int *__restrict__ ord,
-                    const int *__restrict__ nel, const int4 *__restrict__ bhead,
-                    const int *__restrict__ nne, int *__restrict__ work,
-                    const int *__restrict__ uidx, const unsigned short *__restrict__ nbr16,
-                    const int *__restrict__ cnt, int ls, const int *__restrict__ wcnt,
-                    double *__restrict__ dv, int *__restrict__ bfall)
+    k_fluid_brick32(const DevHandle *__restrict__ H, Pair32 q, double *__restrict__ dv)
 {
+    const FluidView F = H->fluid();
+    const int *ord = H->ord, *nel = H->nel, *uidx = H->uidx, *cnt = H->cnt, *wcnt = H->wcnt;
+    const int4 *bhead = H->bhead;
+    const unsigned short *nbr16 = H->nbr16;
+    const int *nne = H->counters;
+    int *work = H->bwork, *bfall = H->bfall;
+    const int ls = H->ls;
     if (q.dyn) {  // the sound speed of this kick
         q.two_av_c = (float)(2.0 * q.dyn[2]);
         q.dd2 = (float)q.dyn[3];
     }
     __shared__ BrickSmem32<ND> S;
     const int tid = threadIdx.x;
-    if (blockIdx.x == 0 && tid == 0) *flag = 0;  // the rebuild (if any) is done
+    if (blockIdx.x == 0 && tid == 0) *H->flag = 0;  // the rebuild (if any) is done
     const int ne = *nne;
     while (true) {
         if (tid == 0) S.item = atomicAdd(work, 1);
@@ -249,8 +251,6 @@ int tpsph::launch_fluid_brick_mixed(tpsph_handle *h, double *dv)
 {
     const int grid = std::max(1, std::min(h->nbricks, 2 * h->n_cu));
     const auto kernel = h->nd == 2 ? k_fluid_brick32<2> : k_fluid_brick32<3>;
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBrickThreads), 0, h->stream, h->flag,
-                       pair32(h->P), h->fluid_view(), h->ord, h->nel, h->bhead, h->counters,
-                       h->bwork, h->uidx, h->nbr16, h->cnt, h->ls, h->wcnt, dv, h->bfall);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBrickThreads), 0, h->stream, h->dev, pair32(h->P), dv);
     return launch_check(h, "k_fluid_brick32");
 }
