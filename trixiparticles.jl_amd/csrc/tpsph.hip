@@ -2582,12 +2582,7 @@ int update_fluid(tpsph_handle *h, const double *v, const double *u, bool gathere
 {
     const int nf = h->nf;
     if (nf == 0) return TPSPH_OK;
-    if (keep_order) {
-        // the order and the lists stand: only the records of (v, u)
-        hipLaunchKernelGGL((k_set_i32), dim3(1), dim3(1), 0, h->stream, h->flag, 0);
-        hipLaunchKernelGGL((k_gather<ND, 0>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream, h->dev, u, v);
-        return launch_check(h, "k_gather<0>");
-    }
+    if (keep_order) return TPSPH_OK;  // the order and the lists stand, the caller wrote the records
     if (!gathered) {  // else the stage kernel wrote the records of (v, u)
         TimedScope t(h, TPSPH_TIME_GATHER);
         hipLaunchKernelGGL((k_gather<ND, 0>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream, h->dev, u, v);

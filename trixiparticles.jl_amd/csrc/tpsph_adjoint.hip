@@ -42,92 +42,166 @@ namespace {
 constexpr int kRedBlocks = 256;  // blocks of the deterministic parameter reduction
 constexpr int kAdjLanes = 4;     // lanes per particle of the adjoint passes
 
-// Constants of the parameter derivatives: d dd2 / d delta and the unit gravity direction.
+// Constants of the parameter derivatives (d dd2 / d delta and the unit gravity direction) and of
+// the fluid pairs: alpha c and beta of the viscosity (zero without) and -1/(2 h), -3/(2 h).
 struct AdjConsts {
     double dd2_per_delta;
     double ghat[3];
+    double visc, beta, minus_half_h_inv, minus_3half_h_inv;
 };
 
-// The geometry of one pair at squared distance d2 (shared by the pair's two terms):
-// distance d and 1/d, the kernel factor kdr (grad W = kdr r_ab), (d kdr / d distance) / d
-// (d kdr / d r_ab = dkdr r_ab) and 1 / (d2 + eps h^2) of the viscosity.  sqrt and the
+// d phi_ab / d(inputs) of the term of fluid particle a with wall partner b (at rest, without
+// viscosity and density diffusion): r_ab (r), its square d2, v_a (va), the density and pressure
+// of a, rho_b and V_b = m_b / rho_b of the wall and its pressure, and the adjoint weights G (of
+// dv_a) and gr (of drho_a).
+// Outputs: d phi / d r_ab, d phi / d vr (d phi / d v_a = vr r_ab), d phi / d rho_a,
+// d phi / d rho_b (total: also through V_b) and d phi / d p_a = d phi / d p_b.  sqrt and the
 // reciprocals are the refined hardware approximations of the forward pass (within a few ulp).
-struct PairGeom {
-    double d, inv_d, kdr, dkdr, inv_q;
-};
-
-__device__ __forceinline__ PairGeom pair_geom(const DevParams &P, double d2)
-{
-    PairGeom g;
-    g.d = sqrt_pos(d2);
-    g.inv_d = rcp_pos(g.d);
-    const double w = 1.0 - 0.5 * P.h_inv * g.d;
-    g.kdr = P.kgrad_c * (w * w * w);
-    g.dkdr = P.kgrad_c * (-1.5 * P.h_inv) * (w * w) * g.inv_d;
-    g.inv_q = rcp_pos(d2 + P.eps_h2);
-    return g;
-}
-
-// d phi_ab / d(inputs) of one pair term in the equation of particle a with partner b:
-//   r_ab = x_a - x_b (r), the pair geometry pg, v_ab (vab, zero for a wall partner),
-//   vr = v_ab . r_ab, the densities with their reciprocals, the pressures, V_b = m_b / rho_b
-//   and m_b of the pair, 1 / (rho_a + rho_b), and the adjoint weights G (of dv_a) and gr (of
-//   drho_a).
-// Outputs: d phi / d r_ab, d phi / d vr (d phi / d v_a = vr r_ab, d phi / d v_b = -vr r_ab),
-// d phi / d rho_a, d phi / d rho_b (total: also through V_b), d phi / d p_a = d phi / d p_b,
-// and the derivatives along alpha and delta.  FLUID: fluid partner (viscosity and density
-// diffusion); a wall partner has neither (the wall model's viscosity is `nothing`).
-struct PairAdj {
+struct WallAdj {
     double r[3];
     double vr;
     double rho_a, rho_b, p;
-    double alpha, delta;
 };
 
-template <int ND, bool FLUID>
-__device__ __forceinline__ PairAdj pair_adj(const DevParams &P, const AdjConsts &K,
-                                            const double *r, const PairGeom &pg,
-                                            const double *vab, double vr, double rho_a,
-                                            double inv_rho_a, double rho_b, double inv_rho_b,
-                                            double inv_sum, double p_a, double p_b,
-                                            double V_b, double m_b, const double *G, double gr)
+template <int ND>
+__device__ __forceinline__ WallAdj wall_adj(const DevParams &P, const double *r, double d2,
+                                            const double *va, double rho_a, double inv_rho_a,
+                                            double inv_rho_b, double p_a, double p_b, double V_b,
+                                            const double *G, double gr)
 {
-    PairAdj o;
-    const double kdr = pg.kdr, dkdr = pg.dkdr;
-    double A = G[0] * r[0] + G[1] * r[1];
-    if constexpr (ND == 3) A += G[2] * r[2];
-    double fac = -V_b * (p_a + p_b) * inv_rho_a;
-    double visc = 0.0, dvisc_dvr = 0.0, dvisc_dq = 0.0, dvisc_dalpha = 0.0;
-    if (FLUID && P.use_visc && vr < 0.0) {
-        // (m_b alpha c mu + m_b beta mu^2) / rho_mean, mu = h vr / q, q = d2 + eps h^2
-        const double mu = P.h * vr * pg.inv_q;
-        const double two_m = 2.0 * m_b * inv_sum;
-        visc = two_m * (P.alpha * P.c * mu + P.beta * (mu * mu));
-        const double dmu = two_m * (P.alpha * P.c + 2.0 * P.beta * mu);
-        dvisc_dvr = dmu * P.h * pg.inv_q;
-        dvisc_dq = -dmu * mu * pg.inv_q;
-        dvisc_dalpha = two_m * P.c * mu;
-    }
-    fac += visc;
-    const double dd2 = FLUID ? P.dd2 : 0.0;
-    const double E = dd2 * (rho_a - rho_b) + rho_a * vr;  // drho_ab = V_b kdr E
-    const double kA = kdr * A;                            // dv_ab = fac kdr r_ab
-    const double dphi_dkdr = fac * A + gr * V_b * E;
-    o.vr = kA * dvisc_dvr + gr * V_b * kdr * rho_a;
-    const double radial = dphi_dkdr * dkdr + 2.0 * kA * dvisc_dq;
+    WallAdj o;
+    const double d = sqrt_pos(d2);
+    const double w = 1.0 - 0.5 * P.h_inv * d;
+    const double kdr = P.kgrad_c * (w * w * w);  // grad W = kdr r_ab
+    const double dkdr = P.kgrad_c * (-1.5 * P.h_inv) * (w * w) * rcp_pos(d);  // d kdr / d r_ab = dkdr r_ab
+    double A = G[0] * r[0] + G[1] * r[1], vr = va[0] * r[0] + va[1] * r[1];
+    if constexpr (ND == 3) A += G[2] * r[2], vr += va[2] * r[2];
+    const double fac = -V_b * (p_a + p_b) * inv_rho_a;
+    const double E = rho_a * vr;  // drho_ab = V_b kdr E
+    const double kA = kdr * A;    // dv_ab = fac kdr r_ab
+    const double radial = (fac * A + gr * V_b * E) * dkdr;
+    o.vr = gr * V_b * kdr * rho_a;
 #pragma unroll
     for (int k = 0; k < 3; k++) o.r[k] = 0.0;
 #pragma unroll
-    for (int k = 0; k < ND; k++) o.r[k] = kdr * fac * G[k] + o.vr * vab[k] + radial * r[k];
+    for (int k = 0; k < ND; k++) o.r[k] = kdr * fac * G[k] + o.vr * va[k] + radial * r[k];
     o.p = -kA * V_b * inv_rho_a;
-    o.rho_a = kA * (V_b * (p_a + p_b) * (inv_rho_a * inv_rho_a) - visc * inv_sum) +
-              gr * V_b * kdr * (dd2 + vr);
-    const double dphi_dVb = -kA * (p_a + p_b) * inv_rho_a + gr * kdr * E;
-    o.rho_b = -kA * visc * inv_sum - gr * V_b * kdr * dd2 - dphi_dVb * V_b * inv_rho_b;
-    o.alpha = kA * dvisc_dalpha;
-    o.delta = FLUID ? gr * V_b * kdr * K.dd2_per_delta * (rho_a - rho_b) : 0.0;
+    o.rho_a = kA * (V_b * (p_a + p_b) * (inv_rho_a * inv_rho_a)) + gr * V_b * kdr * vr;
+    o.rho_b = (kA * (p_a + p_b) * inv_rho_a - gr * kdr * E) * V_b * inv_rho_b;
     return o;
 }
+
+// A fluid particle of the fluid-fluid pullback: its state and the adjoint weights of its rates.
+struct AdjRec {
+    double x[3], rho, v[3], p, V, G[3], gr;
+};
+
+// What the fluid-fluid pairs of one particle c (the target) add to d L / d state_c, and their
+// parts of the alpha and delta derivatives.
+//
+// Both terms of a pair at once, phi_cj + phi_jc.  With K the kernel factor (grad W = K r),
+// r = x_c - x_j, v = v_c - v_j, w = 1 / (rho_c rho_j), D = m_j G_c - m_c G_j, T = D.r,
+// B = Pi - (p_c + p_j) w and Pi the viscosity per partner mass,
+//   phi_cj + phi_jc = K (T B + dd2 (rho_c - rho_j) X + v.r Z),
+//   X = g_c V_j - g_j V_c,   Z = g_c V_j rho_c + g_j V_c rho_j   (g: the weight of drho)
+// so the sums share all but a few of their operations (two terms one after the other: about 190
+// instructions for a pair, this form 120).  Every unordered pair meets both its particles, so
+// alpha and delta take half of its two terms from each.
+template <int ND>
+struct AdjTarget {
+    AdjRec c;
+    double m, inv_rho;
+    double xb[3] = {0.0, 0.0, 0.0}, vb[3] = {0.0, 0.0, 0.0};
+    double rhob = 0.0, pb = 0.0, alpha = 0.0, delta = 0.0;
+
+    __device__ __forceinline__ void set(const AdjRec &target)
+    {
+        c = target;
+        m = c.rho * c.V;
+        inv_rho = rcp_pos(c.rho);
+    }
+
+    __device__ __forceinline__ void pair(const DevParams &P, const AdjConsts &C, const AdjRec &j)
+    {
+        const double r0 = c.x[0] - j.x[0], r1 = c.x[1] - j.x[1];
+        const double r2 = (ND == 3) ? c.x[2] - j.x[2] : 0.0;
+        const double d2 = dist2<ND>(r0, r1, r2);
+        if (!(d2 <= P.R2 && d2 >= P.az2)) return;
+        // sqrt_pos and the reciprocal of its result
+        const double y = __builtin_amdgcn_rsq(d2);
+        const double g = d2 * y;
+        const double d = fma(g, fma(-0.5 * y, g, 0.5), g);
+        const double inv_d = fma(y, fma(-d, y, 1.0), y);
+        const double w1 = fma(C.minus_half_h_inv, d, 1.0);
+        const double w2 = w1 * w1;
+        const double K = w2 * w1;  // without its constant (scale)
+        const double dK = C.minus_3half_h_inv * w2 * inv_d;
+        // one reciprocal for 1 / (d^2 + eps h^2), 1 / (rho_c + rho_j) and 1 / (rho_c rho_j)
+        const double q = d2 + P.eps_h2, sum = c.rho + j.rho, prod = c.rho * j.rho;
+        const double ps = prod * sum;
+        const double qps = q * ps, R1 = rcp_pos(qps);
+        const double R = fma(R1, fma(-qps, R1, 1.0), R1);  // (three results share its error)
+        const double inv_q = R * ps, Rq = R * q;
+        const double w = Rq * sum, inv_sum = Rq * prod;
+
+        const double v0 = c.v[0] - j.v[0], v1 = c.v[1] - j.v[1];
+        const double v2 = (ND == 3) ? c.v[2] - j.v[2] : 0.0;
+        double vr = v0 * r0 + v1 * r1;
+        const double mj = j.rho * j.V;
+        const double D0 = mj * c.G[0] - m * j.G[0], D1 = mj * c.G[1] - m * j.G[1];
+        const double D2 = (ND == 3) ? mj * c.G[2] - m * j.G[2] : 0.0;
+        double T = D0 * r0 + D1 * r1;
+        if constexpr (ND == 3) {
+            vr += v2 * r2;
+            T += D2 * r2;
+        }
+        // Pi = 2 (alpha c mu + beta mu^2) / (rho_c + rho_j), mu = h min(vr, 0) / q
+        const double mu = P.h * (fmin(vr, 0.0) * inv_q);
+        const double two_inv = 2.0 * inv_sum;
+        const double t1 = fma(C.beta, mu, C.visc), t2 = fma(C.beta, mu, t1);
+        const double Pi = two_inv * (mu * t1);
+        const double dmu = two_inv * t2;  // d Pi / d mu
+        const double Pi_vr = vr < 0.0 ? dmu * (P.h * inv_q) : 0.0;
+
+        const double Sw = (c.p + j.p) * w, B = Pi - Sw;
+        const double gV = c.gr * j.V, gj = j.gr * c.V;
+        const double X = gV - gj, Z = fma(gV, c.rho, gj * j.rho);
+        const double diff = c.rho - j.rho, dd = P.dd2 * diff;
+        const double all = fma(T, B, fma(dd, X, vr * Z));
+        const double KT = K * T;
+        const double Kv = fma(KT, Pi_vr, K * Z);                       // along v (x) and r (v)
+        const double rad = fma(dK, all, -2.0 * KT * (dmu * mu) * inv_q);  // along r (x)
+        const double KB = K * B;
+        xb[0] += fma(KB, D0, fma(Kv, v0, rad * r0));
+        xb[1] += fma(KB, D1, fma(Kv, v1, rad * r1));
+        vb[0] = fma(Kv, r0, vb[0]);
+        vb[1] = fma(Kv, r1, vb[1]);
+        if constexpr (ND == 3) {
+            xb[2] += fma(KB, D2, fma(Kv, v2, rad * r2));
+            vb[2] = fma(Kv, r2, vb[2]);
+        }
+        pb = fma(-KT, w, pb);
+        const double dens = fma(P.dd2, X, fma(vr, gV, (dd - vr * j.rho) * (gj * inv_rho)));
+        rhob = fma(KT, Sw * inv_rho - Pi * inv_sum, fma(K, dens, rhob));
+        alpha = fma(KT, two_inv * mu, alpha);
+        delta = fma(K, diff * X, delta);
+    }
+
+    // the kernel's constant, common to all pairs
+    __device__ __forceinline__ void scale(const DevParams &P)
+    {
+        const double f = P.kgrad_c;
+#pragma unroll
+        for (int k = 0; k < ND; k++) {
+            xb[k] *= f;
+            vb[k] *= f;
+        }
+        rhob *= f;
+        pb *= f;
+        alpha *= f;
+        delta *= f;
+    }
+};
 
 // d p / d rho of StateEquationCole (state_equations.jl:100-129), zero where it clips
 __host__ __device__ __forceinline__ double dpressure_drho(const DevParams &P, double rho)
@@ -178,15 +252,40 @@ __device__ __forceinline__ double group_sum(double v)
 //   STAGE = false: from a caller's dv_bar (the pullback of one kick);
 //   STAGE = true: the reversed stage map, tbar += B ybar, kbar = dt tbar, the drift's
 //   vbar += kbar_u, tbar *= A (register adjoints tvb / tub, state adjoints vb / ub).
-template <int ND, bool STAGE>
+// GATHER: also the cell-sorted records of the stage's state (v, u) in the order of the last
+// rebuild, which stands (the segment is 2D and small more often than not, and then as long as
+// its launches take).
+template <int ND, bool STAGE, bool GATHER>
 __global__ void __launch_bounds__(kBlock)
-    k_adj_weights(int nf, const int *__restrict__ iperm, const double *__restrict__ dv_bar,
+    k_adj_weights(const DevHandle *__restrict__ H, const double *__restrict__ v,
+                  const double *__restrict__ u, const double *__restrict__ dv_bar,
                   double *__restrict__ vb, double *__restrict__ ub, double *__restrict__ tvb,
                   double *__restrict__ tub, double a, double b, double dt,
                   double4 *__restrict__ kb)
 {
     const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= nf) return;
+    if (i >= H->P.nf) return;
+    const int s = H->iperm[i];
+    if constexpr (GATHER) {
+        const DevParams P = H->params();
+        double x[3] = {0.0, 0.0, 0.0}, vv[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+        for (int d = 0; d < ND; d++) {
+            x[d] = u[(size_t)i * ND + d];
+            vv[d] = v[(size_t)i * (ND + 1) + d];
+        }
+        const double rho = v[(size_t)i * (ND + 1) + ND], m = H->mass[i];
+        H->rec[2 * (size_t)s] = make_double4(x[0], x[1], x[2], rho);
+        H->rec[2 * (size_t)s + 1] = make_double4(vv[0], vv[1], vv[2], state_equation(P, rho));
+        H->vol[s] = make_double2(m / rho, m);
+        // for the cell walks (see k_gather)
+        const int *noverflow = H->noverflow;
+        if (!noverflow || *noverflow != 0) {
+            H->xs[s] = x[0];
+            H->ys[s] = x[1];
+            if constexpr (ND == 3) H->zs[s] = x[2];
+        }
+    }
     double k[ND + 1];
     if constexpr (STAGE) {
 #pragma unroll
@@ -207,16 +306,16 @@ __global__ void __launch_bounds__(kBlock)
 #pragma unroll
         for (int c = 0; c <= ND; c++) k[c] = dv_bar[(size_t)i * (ND + 1) + c];
     }
-    kb[iperm[i]] = make_double4(k[0], k[1], ND == 3 ? k[2] : 0.0, k[ND]);
+    kb[s] = make_double4(k[0], k[1], ND == 3 ? k[2] : 0.0, k[ND]);
 }
 
 // Adjoint of the Adami pass, four lanes per wall particle (wall-sorted order w): the adjoints
 // of p_w and rho_w from the fluid-wall terms of the fluid near w, through the inverse state
 // equation and the clipping to the adjoint of the unclipped p_w = N_w / V_w with
 //   N_w = sum_f (p_offset + p_f + rho_f g.(x_w - x_f)) W_wf,   V_w = sum_f W_wf,
-// stored as coef[w] = {cN, cV}: d L / d N_w = cN, d L / d V_w = cV.  gw[w] accumulates the
-// partial along g: cN sum_f rho_f ghat.(x_w - x_f) W_wf.
-template <int ND>
+// stored as coef[w] = {cN, cV}: d L / d N_w = cN, d L / d V_w = cV.  gw[w] accumulates (ACC) or
+// takes the partial along g: cN sum_f rho_f ghat.(x_w - x_f) W_wf.
+template <int ND, bool ACC>
 __global__ void __launch_bounds__(kBlock)
     k_adj_wall(const DevHandle *__restrict__ H, AdjConsts K, const double4 *__restrict__ kb,
                double2 *__restrict__ coef, double *__restrict__ gw)
@@ -236,10 +335,11 @@ __global__ void __launch_bounds__(kBlock)
     const int n = alist ? acnt[w] : -1;
     if (n == 0) {  // no fluid within reach: p_w and rho_w are constants
         if (q == 0) coef[w] = make_double2(0.0, 0.0);
+        if (!ACC && q == 0) gw[w] = 0.0;
         return;
     }
     const double4 xw = wpos[w];
-    const double p_w = pw[w], rho_w = rhow[w], V_w = wpv[w].y, m_w = xw.w;
+    const double p_w = pw[w], rho_w = rhow[w], V_w = wpv[w].y;
     const double inv_rho_w = rcp_pos(rho_w);
     double pbar = 0.0, rbar = 0.0, vol = 0.0, gsum = 0.0;
     for_each_candidate<ND, kAdjLanes>(P, alist, n, lw, w, F.start, P.hs_fluid, xw.x, xw.y, xw.z, q, [&](int j) {
@@ -258,12 +358,8 @@ __global__ void __launch_bounds__(kBlock)
         const double4 g = kb[j];
         const double r[3] = {-p0, -p1, -p2};  // r_ab = x_f - x_w
         const double va[3] = {b.x, b.y, b.z};
-        double vr = va[0] * r[0] + va[1] * r[1];
-        if constexpr (ND == 3) vr += va[2] * r[2];
         const double G[3] = {g.x, g.y, g.z};
-        const PairGeom pg = pair_geom(P, d2);
-        const PairAdj o = pair_adj<ND, false>(P, K, r, pg, va, vr, a.w, rcp_pos(a.w), rho_w,
-                                              inv_rho_w, 0.0, b.w, p_w, V_w, m_w, G, g.w);
+        const WallAdj o = wall_adj<ND>(P, r, d2, va, a.w, rcp_pos(a.w), inv_rho_w, b.w, p_w, V_w, G, g.w);
         pbar += o.p;
         rbar += o.rho_b;
     });
@@ -284,15 +380,108 @@ __global__ void __launch_bounds__(kBlock)
         }
     }
     coef[w] = make_double2(cN, cV);
-    gw[w] += cN * gsum;
+    gw[w] = ACC ? gw[w] + cN * gsum : cN * gsum;
+}
+
+// The record of sorted particle s from global memory.
+template <int ND>
+__device__ __forceinline__ AdjRec adj_load(const FluidView &F, const double4 *__restrict__ kb, int s)
+{
+    const double4 a = F.rec[2 * (size_t)s], b = F.rec[2 * (size_t)s + 1], g = kb[s];
+    return {{a.x, a.y, a.z}, a.w, {b.x, b.y, b.z}, b.w, F.vol[s].x, {g.x, g.y, g.z}, g.w};
+}
+
+// The wall part of d L / d state_c (list column t, lane q of LANES): c's own fluid-wall terms and
+// its part in the Adami sums of the wall particles near it.  The parameters are read again:
+// held through the fluid pairs' loop they do not fit the scalar registers.
+template <int ND, int LANES>
+__device__ __forceinline__ void adj_walls(const DevHandle *handle, const double2 *__restrict__ coef,
+                                          int t, int q, AdjTarget<ND> &T)
+{
+    const DevHandle *H = read_again(handle);
+    const DevParams P = H->params();
+    const WallView Wv = H->walls();
+    const int *wnbr = H->wnbr;
+    const int nw = wnbr ? (int)H->wcnt[t] : -1;
+    const double *xc = T.c.x, *v_c = T.c.v;
+    for_each_candidate<ND, LANES>(P, wnbr, nw, H->ls, t, Wv.start, P.hs_wall, xc[0], xc[1], xc[2], q, [&](int w) {
+        const double4 xw = Wv.pos[w];
+        double r[3] = {xc[0] - xw.x, xc[1] - xw.y, (ND == 3) ? xc[2] - xw.z : 0.0};
+        const double d2 = dist2<ND>(r[0], r[1], r[2]);
+        if (d2 > P.R2) return;
+        const double2 pv = Wv.pv[w];
+        const double2 cf = coef[w];
+        // the Adami sums of w: N_w and V_w depend on p_c, rho_c and x_c
+        const double dist = sqrt(d2);  // d2 may be 0 here
+        const double W = wendland_c2(P, dist);
+        const double ww = 1.0 - 0.5 * P.h_inv * dist;
+        const double kdrW = dist < P.two_h ? P.kgrad_c * (ww * ww * ww) : 0.0;
+        double gx = -(P.g[0] * r[0] + P.g[1] * r[1]);  // g.(x_w - x_c)
+        if constexpr (ND == 3) gx -= P.g[2] * r[2];
+        T.pb += cf.x * W;
+        T.rhob += cf.x * gx * W;
+        const double radial = cf.x * ((P.p_offset + T.c.p) + T.c.rho * gx) + cf.y;
+#pragma unroll
+        for (int k = 0; k < ND; k++) T.xb[k] += -cf.x * T.c.rho * P.g[k] * W + radial * kdrW * r[k];
+        if (d2 < P.az2) return;
+        // own fluid-wall term (v_w = 0)
+        const WallAdj o = wall_adj<ND>(P, r, d2, v_c, T.c.rho, T.inv_rho, pv.y / xw.w, T.c.p, pv.x, pv.y, T.c.G, T.c.gr);
+#pragma unroll
+        for (int k = 0; k < ND; k++) {
+            T.xb[k] += o.r[k];
+            T.vb[k] += o.vr * r[k];
+        }
+        T.rhob += o.rho_a;
+        T.pb += o.p;
+    });
+}
+
+// Sums over the LANES lanes of a target, then the state equation and gravity; lane 0 of an active
+// target adds (ACC) or writes d L / d state_c into vb (v, rho) and ub (x) at row i of the
+// caller's order, and the partials along alpha, delta and g into th[3 i ..].
+template <int ND, int LANES, bool ACC>
+__device__ __forceinline__ void adj_finish(const DevHandle *handle, const AdjConsts &K, AdjTarget<ND> &T,
+                                           bool write, int i, double *__restrict__ vb,
+                                           double *__restrict__ ub, double *__restrict__ th)
+{
+#pragma unroll
+    for (int k = 0; k < ND; k++) {
+        T.xb[k] = group_sum<LANES>(T.xb[k]);
+        T.vb[k] = group_sum<LANES>(T.vb[k]);
+    }
+    T.rhob = group_sum<LANES>(T.rhob);
+    T.pb = group_sum<LANES>(T.pb);
+    T.alpha = group_sum<LANES>(T.alpha);
+    T.delta = group_sum<LANES>(T.delta);
+    if (!write) return;
+    const DevParams P = read_again(handle)->params();
+    T.rhob += T.pb * dpressure_drho(P, T.c.rho);
+    double gpart = T.c.G[0] * K.ghat[0] + T.c.G[1] * K.ghat[1];  // gravity: dv += g ghat
+    if constexpr (ND == 3) gpart += T.c.G[2] * K.ghat[2];
+    double *vi = vb + (size_t)i * (ND + 1), *ui = ub + (size_t)i * ND, *ti = th + 3 * (size_t)i;
+#pragma unroll
+    for (int k = 0; k < ND; k++) {
+        vi[k] = ACC ? vi[k] + T.vb[k] : T.vb[k];
+        ui[k] = ACC ? ui[k] + T.xb[k] : T.xb[k];
+    }
+    vi[ND] = ACC ? vi[ND] + T.rhob : T.rhob;
+    // half of both terms of every pair (see AdjTarget)
+    const double alpha = 0.5 * P.c * T.alpha, delta = 0.5 * K.dd2_per_delta * T.delta;
+    ti[0] = ACC ? ti[0] + alpha : alpha;
+    ti[1] = ACC ? ti[1] + delta : delta;
+    ti[2] = ACC ? ti[2] + gpart : gpart;
 }
 
 // Adjoint of the fluid terms of fluid particle c, four lanes per particle (lane q takes the
 // list entries q, q + 4, ...; the partial sums are added across the four lanes in a fixed
-// order): its own fluid-fluid and fluid-wall terms, its partners' fluid-fluid terms, its part
-// in the Adami sums of the wall particles near it, the state equation and gravity.  Adds
-// (ACC) or writes d L / d state_c into vb (v, rho) and ub (x) in the caller's order, and adds
-// the partials along alpha, delta and g into th[3 i ..].
+// order): its fluid-fluid pairs, its fluid-wall terms and its part in the Adami sums of the
+// wall particles near it, the state equation and gravity.
+// What bounds it: the gathers of the candidates through the L1 (116 bytes of a record, its volume,
+// its weights and its index) at three waves per SIMD.  250k particles in 3D, pullback of one
+// kick: 203 us with the two terms of a pair one after the other, 168 with AdjTarget's; held to
+// 128 registers (four waves) 48 bytes spill and it takes 184.  Candidates from unions staged in
+// LDS brick by brick took 239 us (a block of 512 threads, the FP64 chains of two waves per SIMD
+// exposed) and 264 (1,024 threads, which spill). 
 template <int ND, bool ACC>
 __global__ void __launch_bounds__(kBlock)
     k_adj_fluid(const DevHandle *__restrict__ H, AdjConsts K,
@@ -301,75 +490,25 @@ __global__ void __launch_bounds__(kBlock)
 {
     const DevParams P = H->params();
     const FluidView F = H->fluid();
-    const WallView Wv = H->walls();
-    const int *ord = H->ord, *nbr = H->nbr, *cnt = H->cnt, *uidx = H->uidx, *wnbr = H->wnbr;
-    const int *wcnt = H->wcnt, *tbase = uidx ? (const int *)H->tbase : nullptr;
-    const unsigned short *nbr16 = H->nbr16;
-    const int ls = H->ls;
-    int *flag = H->flag;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;  // the rebuild (if any) is done
+    const int *ord = H->ord, *nbr = H->nbr, *cnt = H->cnt;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *H->flag = 0;  // the rebuild (if any) is done
     const int q = threadIdx.x % kAdjLanes;
     const int tt = (xcd_tile(blockIdx.x, gridDim.x) * kBlock + (int)threadIdx.x) / kAdjLanes;
     // the loop bound is uniform per group of lanes, so the partners shuffle together
     const bool active = tt < P.nf;
     const int t = active ? tt : P.nf - 1;
     const int s = ord ? ord[t] : t;
-    const double4 a = F.rec[2 * (size_t)s], b = F.rec[2 * (size_t)s + 1];
-    const double2 vc = F.vol[s];
-    const double4 g = kb[s];
-    const double xc[3] = {a.x, a.y, a.z}, v_c[3] = {b.x, b.y, b.z};
-    const double rho_c = a.w, p_c = b.w, V_c = vc.x, m_c = vc.y, inv_rho_c = rcp_pos(rho_c);
-    const double G[3] = {g.x, g.y, g.z};
-    const double gr = g.w;
-    double xb[3] = {0.0, 0.0, 0.0}, vbr[3] = {0.0, 0.0, 0.0};
-    double rhob = 0.0, pb = 0.0, alpha = 0.0, delta = 0.0;
+    AdjTarget<ND> T;
+    T.set(adj_load<ND>(F, kb, s));
     const int n = nbr ? cnt[t] : -1;
-    auto pair = [&](int j) {
-        // every load of the candidate at once: one round trip instead of two
-        const double4 na = F.rec[2 * (size_t)j];
-        const double4 nb = F.rec[2 * (size_t)j + 1];
-        const double2 nv = F.vol[j];
-        const double4 gn = kb[j];
-        double r[3] = {xc[0] - na.x, xc[1] - na.y, (ND == 3) ? xc[2] - na.z : 0.0};
-        const double d2 = dist2<ND>(r[0], r[1], r[2]);
-        if (!(d2 <= P.R2 && d2 >= P.az2)) return;
-        double vab[3] = {v_c[0] - nb.x, v_c[1] - nb.y, (ND == 3) ? v_c[2] - nb.z : 0.0};
-        double vr = vab[0] * r[0] + vab[1] * r[1];
-        if constexpr (ND == 3) vr += vab[2] * r[2];
-        // the geometry and the density reciprocals of the pair serve both of its terms
-        const PairGeom pg = pair_geom(P, d2);
-        const double inv_rho_j = rcp_pos(na.w), inv_sum = rcp_pos(rho_c + na.w);
-        // own term: c's rates with partner j
-        const PairAdj o = pair_adj<ND, true>(P, K, r, pg, vab, vr, rho_c, inv_rho_c, na.w,
-                                             inv_rho_j, inv_sum, p_c, nb.w, nv.x, nv.y, G, gr);
-#pragma unroll
-        for (int k = 0; k < ND; k++) {
-            xb[k] += o.r[k];
-            vbr[k] += o.vr * r[k];
-        }
-        rhob += o.rho_a;
-        pb += o.p;
-        alpha += o.alpha;
-        delta += o.delta;
-        // partner term: j's rates with partner c (r_jc = -r, v_jc = -v_ab, same vr)
-        const double rn[3] = {-r[0], -r[1], -r[2]};
-        const double vn[3] = {-vab[0], -vab[1], -vab[2]};
-        const double Gn[3] = {gn.x, gn.y, gn.z};
-        const PairAdj qa = pair_adj<ND, true>(P, K, rn, pg, vn, vr, na.w, inv_rho_j, rho_c,
-                                              inv_rho_c, inv_sum, nb.w, p_c, V_c, m_c, Gn, gn.w);
-#pragma unroll
-        for (int k = 0; k < ND; k++) {
-            xb[k] -= qa.r[k];
-            vbr[k] += qa.vr * r[k];
-        }
-        rhob += qa.rho_b;
-        pb += qa.p;
-    };
-    const int first = tbase ? tbase[t] : -1;
+    auto pair = [&](int j) { T.pair(P, K, adj_load<ND>(F, kb, j)); };
+    const int *uidx = H->uidx;
+    const int first = uidx ? (int)H->tbase[t] : -1;
     if (first >= 0) {
         // the list of union records of the target's brick (list_place), a row of four entries
         // and their sorted indices one row ahead of the pair terms
-        const ushort4 *l4 = reinterpret_cast<const ushort4 *>(nbr16);
+        const ushort4 *l4 = reinterpret_cast<const ushort4 *>((const unsigned short *)H->nbr16);
+        const int ls = H->ls;
         const int rows = active ? list_rows(n) : 0;
         ushort4 e4 = l4[(size_t)min(q, max(rows - 1, 0)) * ls + t];
         for (int r = q; r < rows; r += kAdjLanes) {
@@ -383,73 +522,12 @@ __global__ void __launch_bounds__(kBlock)
             e4 = next;
         }
     } else {
-        for_each_candidate<ND, kAdjLanes>(P, nbr, active ? n : 0, ls, t, F.start, P.hs_fluid, a.x,
-                                          a.y, a.z, active ? q : kAdjLanes, pair);
+        for_each_candidate<ND, kAdjLanes>(P, nbr, active ? n : 0, H->ls, t, F.start, P.hs_fluid, T.c.x[0],
+                                          T.c.x[1], T.c.x[2], active ? q : kAdjLanes, pair);
     }
-    if (P.nw > 0) {
-        const int nw = wnbr ? wcnt[t] : -1;
-        for_each_candidate<ND, kAdjLanes>(P, wnbr, active ? nw : 0, ls, t, Wv.start, P.hs_wall,
-                                          a.x, a.y, a.z, active ? q : kAdjLanes, [&](int w) {
-            const double4 xw = Wv.pos[w];
-            double r[3] = {xc[0] - xw.x, xc[1] - xw.y, (ND == 3) ? xc[2] - xw.z : 0.0};
-            const double d2 = dist2<ND>(r[0], r[1], r[2]);
-            if (d2 > P.R2) return;
-            const double2 pv = Wv.pv[w];
-            const double2 cf = coef[w];
-            // the Adami sums of w: N_w and V_w depend on p_c, rho_c and x_c
-            const double dist = sqrt(d2);  // d2 may be 0 here
-            const double W = wendland_c2(P, dist);
-            const double ww = 1.0 - 0.5 * P.h_inv * dist;
-            const double kdrW = dist < P.two_h ? P.kgrad_c * (ww * ww * ww) : 0.0;
-            double gx = -(P.g[0] * r[0] + P.g[1] * r[1]);  // g.(x_w - x_c)
-            if constexpr (ND == 3) gx -= P.g[2] * r[2];
-            pb += cf.x * W;
-            rhob += cf.x * gx * W;
-            const double radial = cf.x * ((P.p_offset + p_c) + rho_c * gx) + cf.y;
-#pragma unroll
-            for (int k = 0; k < ND; k++) xb[k] += -cf.x * rho_c * P.g[k] * W + radial * kdrW * r[k];
-            if (d2 < P.az2) return;
-            // own fluid-wall term (v_w = 0)
-            double vr = v_c[0] * r[0] + v_c[1] * r[1];
-            if constexpr (ND == 3) vr += v_c[2] * r[2];
-            const double inv_rho_w = pv.y / xw.w, rho_w = xw.w / pv.y;
-            const PairGeom pg = pair_geom(P, d2);
-            const PairAdj o = pair_adj<ND, false>(P, K, r, pg, v_c, vr, rho_c, inv_rho_c, rho_w,
-                                                  inv_rho_w, 0.0, p_c, pv.x, pv.y, xw.w, G, gr);
-#pragma unroll
-            for (int k = 0; k < ND; k++) {
-                xb[k] += o.r[k];
-                vbr[k] += o.vr * r[k];
-            }
-            rhob += o.rho_a;
-            pb += o.p;
-        });
-    }
-#pragma unroll
-    for (int k = 0; k < ND; k++) {
-        xb[k] = group_sum<kAdjLanes>(xb[k]);
-        vbr[k] = group_sum<kAdjLanes>(vbr[k]);
-    }
-    rhob = group_sum<kAdjLanes>(rhob);
-    pb = group_sum<kAdjLanes>(pb);
-    alpha = group_sum<kAdjLanes>(alpha);
-    delta = group_sum<kAdjLanes>(delta);
-    if (!active || q != 0) return;
-    rhob += pb * dpressure_drho(P, rho_c);
-    double gpart = G[0] * K.ghat[0] + G[1] * K.ghat[1];  // gravity: dv += g ghat
-    if constexpr (ND == 3) gpart += G[2] * K.ghat[2];
-    const int i = F.perm[s];
-    double *vi = vb + (size_t)i * (ND + 1);
-    double *ui = ub + (size_t)i * ND;
-#pragma unroll
-    for (int k = 0; k < ND; k++) {
-        vi[k] = ACC ? vi[k] + vbr[k] : vbr[k];
-        ui[k] = ACC ? ui[k] + xb[k] : xb[k];
-    }
-    vi[ND] = ACC ? vi[ND] + rhob : rhob;
-    th[3 * (size_t)i] += alpha;
-    th[3 * (size_t)i + 1] += delta;
-    th[3 * (size_t)i + 2] += gpart;
+    T.scale(P);
+    if (P.nw > 0 && active) adj_walls<ND, kAdjLanes>(H, coef, t, q, T);
+    adj_finish<ND, kAdjLanes, ACC>(H, K, T, active && q == 0, F.perm[s], vb, ub, th);
 }
 
 __global__ void __launch_bounds__(kBlock) k_adj_fill(double *p, size_t n, double value)
@@ -460,7 +538,8 @@ __global__ void __launch_bounds__(kBlock) k_adj_fill(double *p, size_t n, double
 
 // Deterministic sums of the parameter partials: block k sums a fixed strided share of the
 // fluid partials th (3 per particle) and of the wall partials gw (added to g) with a fixed
-// tree; k_adj_sum_final adds the block results in block order.
+// tree; k_adj_sum_final adds the block results with another (one thread after the other took
+// 28 us).
 __global__ void __launch_bounds__(kBlock)
     k_adj_sum(int nf, const double *__restrict__ th, int nw, const double *__restrict__ gw,
               double *__restrict__ part)
@@ -485,12 +564,22 @@ __global__ void __launch_bounds__(kBlock)
     if ((int)threadIdx.x < 3) part[(size_t)blockIdx.x * 3 + threadIdx.x] = s[threadIdx.x][0];
 }
 
-__global__ void k_adj_sum_final(int nparts, const double *__restrict__ part, double *__restrict__ out)
+__global__ void __launch_bounds__(kRedBlocks)
+    k_adj_sum_final(int nparts, const double *__restrict__ part, double *__restrict__ out)
 {
-    if ((int)threadIdx.x >= 3) return;
-    double acc = 0.0;
-    for (int b = 0; b < nparts; b++) acc += part[(size_t)b * 3 + threadIdx.x];
-    out[threadIdx.x] = acc;
+    __shared__ double s[3][kRedBlocks];
+    const int b = threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < 3; k++) s[k][b] = b < nparts ? part[(size_t)b * 3 + k] : 0.0;
+    __syncthreads();
+    for (int o = kRedBlocks / 2; o > 0; o >>= 1) {
+        if (b < o) {
+#pragma unroll
+            for (int k = 0; k < 3; k++) s[k][b] += s[k][b + o];
+        }
+        __syncthreads();
+    }
+    if (b < 3) out[b] = s[b][0];
 }
 
 int check_supported(tpsph_handle *h)
@@ -517,6 +606,10 @@ AdjConsts adj_consts(const tpsph_handle *h)
     for (int d = 0; d < 3; d++) g2 += P.g[d] * P.g[d];
     const double g = std::sqrt(g2);
     for (int d = 0; d < 3; d++) K.ghat[d] = g > 0.0 ? P.g[d] / g : 0.0;
+    K.visc = P.use_visc ? P.alpha * P.c : 0.0;
+    K.beta = P.use_visc ? P.beta : 0.0;
+    K.minus_half_h_inv = -0.5 * P.h_inv;
+    K.minus_3half_h_inv = -1.5 * P.h_inv;
     return K;
 }
 
@@ -563,7 +656,7 @@ int adjoint_passes(tpsph_handle *h, double *vb, double *ub)
     TimedScope ts(h, TPSPH_TIME_ADJOINT);
     const AdjConsts K = adj_consts(h);
     if (h->nw > 0) {
-        hipLaunchKernelGGL((k_adj_wall<ND>), dim3(nblocks(kAdjLanes * (int64_t)h->nw)), dim3(kBlock), 0, h->stream,
+        hipLaunchKernelGGL((k_adj_wall<ND, ACC>), dim3(nblocks(kAdjLanes * (int64_t)h->nw)), dim3(kBlock), 0, h->stream,
                            h->dev, K, h->adj_kb, h->adj_coef, h->adj_gw);
         TRY(launch_check(h, "k_adj_wall"));
     }
@@ -578,7 +671,7 @@ int reduce_params(tpsph_handle *h, double *param_bar)
     hipLaunchKernelGGL(k_adj_sum, dim3(grid), dim3(kBlock), 0, h->stream, h->nf, h->adj_th, h->nw,
                        h->adj_gw, h->adj_red);
     double *res = h->adj_red + 3 * (size_t)kRedBlocks;
-    hipLaunchKernelGGL(k_adj_sum_final, dim3(1), dim3(64), 0, h->stream, grid, h->adj_red, res);
+    hipLaunchKernelGGL(k_adj_sum_final, dim3(1), dim3(kRedBlocks), 0, h->stream, grid, h->adj_red, res);
     TRY(launch_check(h, "k_adj_sum"));
     if (param_bar) {
         HIP_TRY(h, hipMemcpyAsync(param_bar, res, 3 * sizeof(double), hipMemcpyDefault, h->stream));
@@ -592,10 +685,8 @@ int kick_vjp_impl(tpsph_handle *h, const double *dv_bar, const double *v, const 
                   double *v_bar, double *u_bar, double *param_bar)
 {
     TRY(prepare_dispatch(h, v, u));
-    TRY(fill(h, h->adj_th, 3 * (size_t)h->nf, 0.0));
-    TRY(fill(h, h->adj_gw, (size_t)h->nw, 0.0));
-    hipLaunchKernelGGL((k_adj_weights<ND, false>), dim3(nblocks(h->nf)), dim3(kBlock), 0,
-                       h->stream, h->nf, h->iperm, dv_bar, nullptr, nullptr, nullptr, nullptr,
+    hipLaunchKernelGGL((k_adj_weights<ND, false, false>), dim3(nblocks(h->nf)), dim3(kBlock), 0,
+                       h->stream, h->dev, nullptr, nullptr, dv_bar, nullptr, nullptr, nullptr, nullptr,
                        0.0, 0.0, 0.0, h->adj_kb);
     TRY(launch_check(h, "k_adj_weights"));
     TRY((adjoint_passes<ND, false>(h, v_bar, u_bar)));
@@ -640,11 +731,14 @@ int reverse_impl(tpsph_handle *h, const double *vT_bar, const double *uT_bar, do
             for (int i = 4; i >= 0; i--) {
                 const size_t e = (size_t)(5 * s + i);
                 const double *yv = st_v + e * nv, *yu = st_u + e * nu;
-                TRY(prepare_dispatch(h, yv, yu, keep_order));
-                hipLaunchKernelGGL((k_adj_weights<ND, true>), dim3(nblocks(h->nf)), dim3(kBlock), 0,
-                                   h->stream, h->nf, h->iperm, nullptr, h->adj_vb, h->adj_ub,
+                // (with a rebuild the weights follow it: they go to the new order)
+                if (!keep_order) TRY(prepare_dispatch(h, yv, yu));
+                const auto weights = keep_order ? k_adj_weights<ND, true, true> : k_adj_weights<ND, true, false>;
+                hipLaunchKernelGGL(weights, dim3(nblocks(h->nf)), dim3(kBlock), 0,
+                                   h->stream, h->dev, yv, yu, nullptr, h->adj_vb, h->adj_ub,
                                    h->adj_tvb, h->adj_tub, kCkA[i], kCkB[i], h->adj_dt, h->adj_kb);
                 TRY(launch_check(h, "k_adj_weights"));
+                if (keep_order) TRY(prepare_dispatch(h, yv, yu, true));
                 TRY((adjoint_passes<ND, true>(h, h->adj_vb, h->adj_ub)));
             }
         }

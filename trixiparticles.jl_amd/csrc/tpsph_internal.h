@@ -204,6 +204,15 @@ struct DevHandle {
 // ------------------------------------------------------------------------------------------
 // device helpers
 // ------------------------------------------------------------------------------------------
+// The handle as a pointer of its own: what is read through it is loaded where it is used (as
+// scalars, the handle is constant), not held in registers from the start of the kernel.
+__device__ __forceinline__ const DevHandle *read_again(const DevHandle *H)
+{
+    uintptr_t a = (uintptr_t)H;
+    asm volatile("" : "+s"(a));
+    return (const DevHandle *)(const __attribute__((address_space(4))) DevHandle *)a;
+}
+
 // Julia's max(x, 0) for Float64: NaN propagates, -0.0 becomes +0.0.
 __device__ __forceinline__ double julia_max0(double x) { return (x != x) ? x : (x > 0.0 ? x : 0.0); }
 
