@@ -5,9 +5,9 @@
 //                    permutation, fluid state equation, and flag a rebuild if any particle
 //                    moved by more than half the skin since the last cell-list build;
 //   2. rebuild, only when flagged (every kernel reads the flag and returns otherwise; the
-//      fluid kernel of step 4 lowers the flag again): k_cells + k_scan + k_scatter (a counting
-//      sort on the linear cell index), k_gather<1> (makes the sort stable, gathers again,
-//      snapshot of the build positions) and, with Verlet lists, k_brick_lists (bricks, unions,
+//      fluid kernel of step 4 lowers the flag again): k_links + k_scan + k_gather<1> (a stable
+//      counting sort on the linear cell index that gathers again, with a snapshot of the build
+//      positions; one kernel, k_sort, for small fluids) and, with Verlet lists, k_brick_lists (bricks, unions,
 //      fluid and wall candidates within R + skin);
 //   3. k_wall        Adami pressure extrapolation + inverse state equation per wall particle;
 //   4. the fused fluid-fluid + fluid-wall interaction + gravity, results scattered back to
@@ -49,26 +49,56 @@ namespace {
 // cell list (counting sort), every kernel gated by the rebuild flag (nullptr = always)
 // ------------------------------------------------------------------------------------------
 
-// counters: zeroed (nullptr: none).
+template <int ND>
+__device__ __forceinline__ int cell_of(const DevParams &P, double x0, double x1, double x2)
+{
+    const int c0 = cell_1d(x0, P.lo[0], P.inv_cs[0], P.n[0]);
+    const int c1 = cell_1d(x1, P.lo[1], P.inv_cs[1], P.n[1]);
+    const int c2 = (ND == 3) ? cell_1d(x2, P.lo[2], P.inv_cs[2], P.n[2]) : 0;
+    return c0 + P.n[0] * (c1 + P.n[1] * c2);
+}
+
 template <int ND>
 __global__ void k_cells(const DevHandle *__restrict__ H, const int *flag, int n,
                         const double *__restrict__ x, int *__restrict__ cell,
-                        int *__restrict__ rank, int *__restrict__ count,
-                        int *__restrict__ counters)
+                        int *__restrict__ rank, int *__restrict__ count)
 {
     if (skip(flag)) return;
     const DevParams P = H->params();
-    clear_scan_state(H->scan_state, H->scan_words);
-    if (counters && blockIdx.x == 0 && (int)threadIdx.x < kCounters) counters[threadIdx.x] = 0;
+    clear_scan_state(H->scan_state, H->scan_words, blockIdx.x, gridDim.x);
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const double *xi = x + (size_t)i * ND;
-        int c0 = cell_1d(xi[0], P.lo[0], P.inv_cs[0], P.n[0]);
-        int c1 = cell_1d(xi[1], P.lo[1], P.inv_cs[1], P.n[1]);
-        int c2 = (ND == 3) ? cell_1d(xi[2], P.lo[2], P.inv_cs[2], P.n[2]) : 0;
-        int lin = c0 + P.n[0] * (c1 + P.n[1] * c2);
-        cell[i] = lin;
-        rank[i] = atomicAdd(&count[lin], 1);
+        const int c = cell_of<ND>(P, xi[0], xi[1], ND == 3 ? xi[2] : 0.0);
+        cell[i] = c;
+        rank[i] = atomicAdd(&count[c], 1);
     }
+}
+
+// The fluid's cells as chains: head[c] is the member of cell c that came last, next[i] the one
+// before i; count[c] of them belong to the cell, whatever head and the first member's next held
+// before (so neither is ever cleared).  k_gather<1> finds a particle's place by the chain and
+// the scanned counts, without the two passes that write and order the members of every cell.
+// Also clears the scan's state and the list build's counters.  Block bx of nb.
+template <int ND>
+__device__ __forceinline__ void links_body(const DevHandle *H, int bx, int nb, const double *__restrict__ x)
+{
+    const DevParams P = H->params();
+    int *head = H->f_head, *next = H->f_next, *count = H->f_count, *counters = H->counters;
+    clear_scan_state(H->scan_state, H->scan_words, bx, nb);
+    if (counters && bx == 0 && (int)threadIdx.x < kCounters) counters[threadIdx.x] = 0;
+    for (int i = bx * (int)blockDim.x + (int)threadIdx.x; i < P.nf; i += nb * (int)blockDim.x) {
+        const double *xi = x + (size_t)i * ND;
+        const int c = cell_of<ND>(P, xi[0], xi[1], ND == 3 ? xi[2] : 0.0);
+        atomicAdd(&count[c], 1);
+        next[i] = atomicExch(&head[c], i);
+    }
+}
+
+template <int ND>
+__global__ void k_links(const DevHandle *__restrict__ H, const double *__restrict__ x)
+{
+    if (skip(H->flag)) return;
+    links_body<ND>(H, blockIdx.x, gridDim.x, x);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -76,13 +106,20 @@ __global__ void k_cells(const DevHandle *__restrict__ H, const int *flag, int n,
 //   MODE 0: runs when no rebuild is pending; flags one if a particle left its skin.  A block
 //           that starts after another block raised the flag returns early: the rebuild that
 //           follows gathers everything again.
-//   MODE 1: runs after a rebuild; stores the build positions.
+//   MODE 1: runs at a rebuild; stores the build positions.
+//   MODE 2: the same with a finished permutation (tpsph_kick_noalloc).
 // ------------------------------------------------------------------------------------------
-// MODE 1 takes the members of every cell in the order the histogram's atomics gave (permu) and
-// orders them by particle index on the way (the stable counting sort, whatever order the
-// atomics were served in): a particle's place is the number of members with a smaller index.
-// With bcount it also counts the particles of every brick of cells and lists the bricks that
-// hold any (nel, nne of them; k_cells cleared it).
+// MODE 1 puts particle i behind the members of its cell with a smaller index (the stable counting
+// sort, whatever order the atomics of k_links were served in), which it counts along the cell's
+// chain.  With bcount it also counts the particles of every brick of cells and lists the bricks
+// that hold any (nel, nne of them; k_links cleared it).
+// The counters of the brick kernels (work) and of k_sort, cleared by the first kernel of every kick
+__device__ __forceinline__ void reset_counters(int *work, int *sort_ctl)
+{
+    if (work && threadIdx.x < 3) work[threadIdx.x] = 0;
+    if (sort_ctl && threadIdx.x < kSortCtl) sort_ctl[threadIdx.x] = 0;
+}
+
 // FP32 position for the list builds: relative to the grid origin, NaN outside the grid box (the
 // list builds then take every candidate of the particle)
 template <int ND>
@@ -112,23 +149,23 @@ __global__ void k_wall_f32(DevParams P, int nw, const double4 *__restrict__ wpos
 }
 
 template <int ND, int MODE>
-__global__ void k_gather(const DevHandle *__restrict__ H, const double *__restrict__ u,
-                         const double *__restrict__ v)
+__device__ __forceinline__ void gather_body(const DevHandle *H, int bx, int nb,
+                                            const double *__restrict__ u,
+                                            const double *__restrict__ v)
 {
     DevParams P = H->params();
-    int *flag = H->flag, *work = H->bwork, *iperm = H->iperm, *perm_out = H->f_perm;
-    const int *perm = MODE == 0 ? H->f_perm : H->f_permu;
+    int *flag = H->flag, *work = H->bwork, *iperm = H->iperm, *perm = H->f_perm;
     const double *m = H->mass;
     double *xs = H->xs, *ys = H->ys, *zs = H->zs, *snap = H->snap;
     double4 *rec = H->rec;
     double2 *vol = H->vol;
-    const int *cell = H->f_cell, *start = H->f_start, *noverflow = H->noverflow;
+    const int *start = H->f_start, *head = H->f_head, *next = H->f_next, *noverflow = H->noverflow;
     int *bcount = H->bcount, *nel = H->nel, *nne = H->counters;
     float4 *xf = H->xf;
     P = with_sound(P);
     const int f = *flag;
-    // MODE 0 runs first in every kick: it resets the work counter of the brick kernel
-    if (MODE == 0 && work && blockIdx.x == 0 && threadIdx.x == 0) work[0] = work[1] = work[2] = 0;
+    // MODE 0 runs first in every kick: it resets the counters of the kernels that follow
+    if (MODE == 0 && bx == 0) reset_counters(work, H->sort_ctl);
     if ((MODE == 0) == (f != 0)) return;
     const size_t nf = (size_t)P.nf;
     // with Verlet lists the SoA coordinates are read between rebuilds only by the cell walk
@@ -136,31 +173,33 @@ __global__ void k_gather(const DevHandle *__restrict__ H, const double *__restri
     const bool soa = !noverflow || *noverflow != 0;
     // the loop bound is uniform per wavefront (blockDim is a multiple of 64): the brick
     // counting below works on whole wavefronts
-    for (int s0 = blockIdx.x * blockDim.x; s0 < P.nf; s0 += gridDim.x * blockDim.x) {
+    for (int s0 = bx * (int)blockDim.x; s0 < P.nf; s0 += nb * (int)blockDim.x) {
         int s = s0 + (int)threadIdx.x;
         const bool in = s < P.nf;
-        int b = -1;          // brick of the particle (MODE 1 with bcount)
+        int b = -1;          // brick of the particle (at a rebuild with bcount)
         bool moved = false;  // left its skin (MODE 0)
         if (in) {
-            const int i = perm[s];
-            if constexpr (MODE == 1) {
-                const int c = cell[i];
-                const int c_end = start[c + 1];
-                int k = start[c];
-                s = k;
-                for (; k < c_end; k++) s += perm[k] < i ? 1 : 0;
-                perm_out[s] = i;
-            }
+            const int i = MODE == 1 ? s : perm[s];
             double x[3] = {0.0, 0.0, 0.0}, vv[3] = {0.0, 0.0, 0.0};
 #pragma unroll
             for (int d = 0; d < ND; d++) {
                 x[d] = u[(size_t)i * ND + d];
                 vv[d] = v[(size_t)i * P.vrows + d];
             }
+            if constexpr (MODE == 1) {
+                const int c = cell_of<ND>(P, x[0], x[1], x[2]);
+                const int b0 = start[c], members = start[c + 1] - b0;
+                s = b0;
+                for (int k = 0, j = head[c]; k < members; k++) {
+                    s += j < i ? 1 : 0;
+                    if (k + 1 < members) j = next[j];
+                }
+                perm[s] = i;
+            }
             // SummationDensity: density and pressure are written by k_sum_finish
             const double rho = P.summation ? 1.0 : v[(size_t)i * (ND + 1) + ND];
             const double mass = m[i];
-            if (MODE == 1 || soa) {
+            if (MODE != 0 || soa) {
                 xs[s] = x[0];
                 ys[s] = x[1];
                 if constexpr (ND == 3) zs[s] = x[2];
@@ -192,9 +231,8 @@ __global__ void k_gather(const DevHandle *__restrict__ H, const double *__restri
             }
         }
         if constexpr (MODE == 0) raise_rebuild_flag(flag, moved);
-        if (MODE == 1 && bcount) {
-            // a wavefront holds consecutive cell-sorted particles, so equal bricks come in
-            // runs: the first lane of a run adds the run with one atomic, and whoever finds a
+        if (MODE != 0 && bcount) {
+            // neighbouring particles mostly share a brick, so equal bricks come in runs: the first lane of a run adds the run with one atomic, and whoever finds a
             // brick empty lists it
             const int lane = (int)threadIdx.x & 63;
             const int prev = __shfl_up(b, 1);
@@ -206,7 +244,75 @@ __global__ void k_gather(const DevHandle *__restrict__ H, const double *__restri
                 nel[atomicAdd(nne, 1)] = b;
         }
     }
-    if (MODE == 1 && H->nrebuild && blockIdx.x == 0 && threadIdx.x == 0) *H->nrebuild += 1;
+    if (MODE != 0 && H->nrebuild && bx == 0 && threadIdx.x == 0) *H->nrebuild += 1;
+}
+
+template <int ND, int MODE>
+__global__ void k_gather(const DevHandle *__restrict__ H, const double *__restrict__ u,
+                         const double *__restrict__ v)
+{
+    gather_body<ND, MODE>(H, blockIdx.x, gridDim.x, u, v);
+}
+
+// k_links, k_scan and k_gather<1> in one launch, which like theirs returns at once while the flag
+// is down: a launch costs a kick of a small fluid 2.5 us, whether it does anything or not.
+//
+// Items are handed out by a ticket in the order of the phases (`items` of the particles, `tiles`
+// of the scan, `items` of the gather), and an item waits until every item of the phase before
+// is done.  Those are in the hands of blocks that run already and that wait for still earlier
+// phases only, so the waits end whatever number of blocks the device holds at a time.  What a
+// phase wrote is released by its block at device scope and acquired by the waiting one.
+//
+// A kick without a rebuild saves two launches, a rebuild costs more than by three launches (45k
+// particles in 2D: 29 us against 21, each phase waits for tickets, counts and cold caches).
+// us per pass, three kernels -> this one: kick of 2k in 2D 29.9 -> 24.0, of 48k in 3D 56.9 ->
+// 53.6, two steps of 128k with SummationDensity 1290 -> 1248; two steps of 45k in 2D with a
+// rebuild at four of ten kicks 557 -> 581.  Larger fluids (kSortMax) take the three kernels:
+// their rebuild needs the whole device (1.02M particles: 350 us more with 128 blocks).
+template <int ND>
+__global__ void __launch_bounds__(kSortThreads)
+    k_sort(const DevHandle *__restrict__ H, const double *__restrict__ u,
+           const double *__restrict__ v, int items, int tiles)
+{
+    if (skip(H->flag)) return;
+    __shared__ int s[kSortThreads / 64];
+    __shared__ int s_ticket, s_before;
+    int *ctl = H->sort_ctl;  // lines of kSortLine ints: the ticket, then the items done of every phase
+    const int ncells = H->P.ncells;
+    if (threadIdx.x == 0) s_ticket = atomicAdd(&ctl[0], 1);
+    __syncthreads();
+    while (true) {
+        int item = s_ticket, phase = 0, before = 0;
+        for (int n = items; phase < 3 && item >= n; n = phase == 1 ? tiles : items) {
+            item -= n;
+            before = n;
+            phase++;
+        }
+        if (phase == 3) return;  // uniform: every item is taken
+        if (phase > 0) {
+            if (threadIdx.x == 0) {
+                while (__hip_atomic_load(&ctl[phase * kSortLine], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < before)
+                    __builtin_amdgcn_s_sleep(1);
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            }
+            __syncthreads();
+        }
+        if (phase == 0)
+            links_body<ND>(H, item, items, u);
+        else if (phase == 1)
+            scan_tile<true, kSortThreads>(H->f_count, H->f_start, H->scan_state, ncells + 1, item, s, s_before);
+        else
+            gather_body<ND, 1>(H, item, items, u, v);
+        // every wavefront's stores have left it, then one release for the block
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            if (phase < 2)
+                __hip_atomic_fetch_add(&ctl[(1 + phase) * kSortLine], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+            s_ticket = atomicAdd(&ctl[0], 1);
+        }
+        __syncthreads();
+    }
 }
 
 
@@ -2168,7 +2274,7 @@ __global__ void __launch_bounds__(kBlock)
         v[k] = fma(b, t, v[k]);
     }
     __syncthreads();  // the block's new u and v are complete
-    if (work && blockIdx.x == 0 && threadIdx.x == 0) work[0] = work[1] = work[2] = 0;
+    if (blockIdx.x == 0) reset_counters(work, H->sort_ctl);
     const int i = i0 + (int)threadIdx.x;
     bool moved = false;  // left its skin
     if (i < nf) {
@@ -2554,23 +2660,21 @@ namespace {
 
 
 // Cell list of n points x (ND doubles per point, caller order) into start / perm, the members
-// of a cell by their index; without `ordered` in the order of the histogram's atomics (the
-// gather that follows orders them).
+// of a cell by their index.
 template <int ND>
 int build_cells(tpsph_handle *h, const int *flag, int n, const double *x, int *cell, int *rank,
-                int *count, int *start, int *perm, bool ordered = true, int *counters = nullptr)
+                int *count, int *start, int *perm)
 {
     // count is zero on entry (cleared at create, and again by k_scatter)
     const int nc = h->P.ncells;
     // (n = 0 too: it clears the scan's state)
     hipLaunchKernelGGL((k_cells<ND>), dim3(gate_blocks(n)), dim3(kBlock), 0, h->stream, h->dev, flag, n, x,
-                       cell, rank, count, counters);
+                       cell, rank, count);
     TRY(launch_check(h, "k_cells"));
     TRY(scan(h, flag, count, start, nc + 1));
     if (n > 0) {
         hipLaunchKernelGGL((k_scatter), dim3(gate_blocks(n)), dim3(kBlock), 0, h->stream, flag, n, cell, rank, start, perm, count);
-        if (ordered)
-            hipLaunchKernelGGL((k_sort_cells), dim3(gate_blocks(nc)), dim3(kBlock), 0, h->stream, flag, nc, start, perm);
+        hipLaunchKernelGGL((k_sort_cells), dim3(gate_blocks(nc)), dim3(kBlock), 0, h->stream, flag, nc, start, perm);
     }
     return launch_check(h, "k_scatter/k_sort_cells");
 }
@@ -2591,11 +2695,22 @@ int update_fluid(tpsph_handle *h, const double *v, const double *u, bool gathere
     {
         TimedScope t(h, TPSPH_TIME_CELL_LIST);
         const bool lists = h->search == TPSPH_SEARCH_LISTS;
-        TRY(build_cells<ND>(h, h->flag, nf, u, h->f_cell, h->f_rank, h->f_count, h->f_start,
-                            h->f_permu, h->f_permu == h->f_perm, lists ? h->counters : nullptr));
-        // the gather orders the members of every cell (where the scatter had an array of its
-        // own; in place k_sort_cells has done it) and, with lists, finds the bricks
-        hipLaunchKernelGGL((k_gather<ND, 1>), dim3(gate_blocks(nf)), dim3(kBlock), 0, h->stream, h->dev, u, v);
+        if (!h->f_head) {
+            TRY(build_cells<ND>(h, h->flag, nf, u, h->f_cell, h->f_rank, h->f_count, h->f_start, h->f_perm));
+            hipLaunchKernelGGL((k_gather<ND, 2>), dim3(gate_blocks(nf)), dim3(kBlock), 0, h->stream, h->dev, u, v);
+        } else if (h->sort_ctl) {
+            const int items = std::min((nf + kSortThreads - 1) / kSortThreads, kSortItems);
+            const int tiles = h->P.ncells / (kSortThreads * kScanItems) + 1;
+            hipLaunchKernelGGL((k_sort<ND>), dim3(std::min(std::max(items, tiles), kSortItems)), dim3(kSortThreads), 0,
+                               h->stream, h->dev, u, v, items, tiles);
+        } else {
+            hipLaunchKernelGGL((k_links<ND>), dim3(gate_blocks(nf)), dim3(kBlock), 0, h->stream, h->dev, u);
+            const int n = h->P.ncells + 1;
+            hipLaunchKernelGGL((k_scan<true>), dim3(scan_words(n) - 1), dim3(kBlock), 0, h->stream, h->flag,
+                               h->f_count, h->f_start, h->scan_state, n);
+            hipLaunchKernelGGL((k_gather<ND, 1>), dim3(gate_blocks(nf)), dim3(kBlock), 0, h->stream, h->dev, u, v);
+        }
+        TRY(launch_check(h, "k_sort / k_gather<1>"));
         if (lists) {
             const int gb = std::max(1, std::min(h->nbricks, 2 * h->n_cu));
             const int gw = (h->nw + kListThreads - 1) / kListThreads;
@@ -2603,7 +2718,6 @@ int update_fluid(tpsph_handle *h, const double *v, const double *u, bool gathere
             TRY(launch_check(h, "k_brick_lists"));
         }
         // the fluid kernel of this kick lowers the flag
-        TRY(launch_check(h, "k_gather<1>"));
     }
     return TPSPH_OK;
 }
@@ -3049,9 +3163,10 @@ int put_handle(tpsph_handle *h)
     d.rec = h->rec; d.vol = h->vol; d.xf = h->xf;
     d.w_start = h->w_start; d.wx = h->wx; d.wy = h->wy; d.wz = h->wz; d.wpos = h->wpos;
     d.wpv = h->wpv; d.wvel = h->wvel; d.wxf = h->wxf; d.pw = h->pw; d.rhow = h->rhow;
-    d.flag = h->flag; d.f_cell = h->f_cell; d.f_permu = h->f_permu; d.iperm = h->iperm;
+    d.flag = h->flag; d.f_head = h->f_head; d.f_next = h->f_rank; d.iperm = h->iperm;
     d.nrebuild = h->nrebuild; d.counters = h->counters; d.scan_state = h->scan_state;
     d.scan_words = scan_words(h->P.ncells + 1);
+    d.f_count = h->f_count; d.sort_ctl = h->sort_ctl;
     d.snap = h->snap; d.mass = h->f_mass; d.wall_near = h->wall_near;
     d.bcount = h->bcount; d.nel = h->nel; d.ord = h->ord; d.tbase = h->tbase; d.uidx = h->uidx;
     d.nbr = h->nbr; d.cnt = h->cnt; d.wnbr = h->wnbr; d.wcnt = h->wcnt; d.wtargets = h->wtargets;
@@ -3204,7 +3319,6 @@ int noalloc_kick(tpsph_handle *h, unsigned char *base, size_t *bytes, const doub
     h->f_cell = L.take<int>(nf);
     h->f_rank = L.take<int>(nf);
     h->f_perm = L.take<int>(nf);
-    h->f_permu = h->f_perm;  // ordered in place (k_sort_cells)
     h->iperm = L.take<int>(nf);
     h->f_count = L.take<int>((size_t)nc + 1);
     h->f_start = L.take<int>((size_t)nc + 1);
@@ -3423,10 +3537,11 @@ int tpsph_create(const tpsph_params *params, int64_t n_fluid, int64_t n_wall,
         P.dyn = h->dyn;
     }
     CTRY(dalloc(h, &h->scan_state, (size_t)scan_words((int)ncells + 1)));
+    if (h->search == TPSPH_SEARCH_LISTS && nf <= kSortMax) CTRY(dalloc(h, &h->sort_ctl, kSortCtl));
     CTRY(dalloc(h, &h->f_cell, nf));
     CTRY(dalloc(h, &h->f_rank, nf));
     CTRY(dalloc(h, &h->f_perm, nf));
-    CTRY(dalloc(h, &h->f_permu, nf));
+    CTRY(dalloc(h, &h->f_head, (size_t)ncells));
     CTRY(dalloc(h, &h->f_count, (size_t)ncells + 1));
     CTRY(dalloc(h, &h->f_start, (size_t)ncells + 1));
     CTRY(dalloc(h, &h->f_mass, nf));
@@ -4031,7 +4146,7 @@ void tpsph_destroy(tpsph_handle *h)
     if (!h) return;
     (void)hipStreamSynchronize(h->stream);
     void *ptrs[] = {h->flag, h->f_cell, h->f_rank, h->f_count, h->f_start, h->f_perm,
-                    h->scan_state, h->f_permu, h->f_mass, h->xs, h->ys, h->zs, h->xf, h->wxf, h->snap, h->rec, h->vol,
+                    h->scan_state, h->sort_ctl, h->f_head, h->f_mass, h->xs, h->ys, h->zs, h->xf, h->wxf, h->snap, h->rec, h->vol,
                     h->w_start, h->w_perm, h->wx, h->wy, h->wz, h->wpos, h->wpv, h->wall_near,
                     h->pw, h->nbr, h->cnt, h->wnbr, h->wcnt, h->anbr, h->acnt, h->ord, h->bcount, h->tbase,
                     h->uidx, h->bhead, h->nel, h->counters, h->wactive, h->bwork, h->nbr16,

@@ -78,7 +78,7 @@ __global__ void k_bcells(DevParams P, const CaseDev *__restrict__ cases,
                          int *__restrict__ cell, int *__restrict__ rank, int *__restrict__ count,
                          unsigned long long *__restrict__ state, int words)
 {
-    clear_scan_state(state, words);
+    clear_scan_state(state, words, blockIdx.x, gridDim.x);
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const CaseDev &cs = cases[pcase[i]];
         DevParams Q = P;

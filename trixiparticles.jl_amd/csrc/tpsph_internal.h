@@ -40,6 +40,11 @@ constexpr int kCellTab = 5120;        // cell offsets of a union in LDS (at most
 constexpr int kGateBlocks = 1024;     // grid-stride kernels behind the rebuild flag: a small
                                       // grid keeps the launch cheap when the flag is down
 constexpr int kCounters = 7;          // tpsph_handle::counters
+constexpr int kSortLine = 32;           // k_sort: ticket and finished items of two phases, a line
+constexpr int kSortCtl = 3 * kSortLine; // of 128 bytes each
+constexpr int kSortThreads = 1024;
+constexpr int kSortItems = 64;          // its blocks
+constexpr int kSortMax = 1 << 17;       // fluids it takes
 constexpr int kPad = 4;               // NaN entries after the SoA coordinate arrays
 
 // message of the last failed tpsph_create (tpsph_last_error(NULL))
@@ -170,9 +175,10 @@ struct DevHandle {
     GlobalPtr<const float4> wxf;
     GlobalPtr<double> pw, rhow;
     // cell list
-    GlobalPtr<int> flag, f_cell, f_permu, iperm, nrebuild, counters;
+    GlobalPtr<int> flag, f_head, f_next, iperm, nrebuild, counters;
     GlobalPtr<unsigned long long> scan_state;
     int scan_words;
+    GlobalPtr<int> f_count, sort_ctl;
     GlobalPtr<double> snap;
     GlobalPtr<const double> mass;
     GlobalPtr<const unsigned char> wall_near;
@@ -758,7 +764,8 @@ namespace tpsph {
 namespace {
 
 // Exclusive scan over the block: an inclusive scan within each wavefront by shuffles, then
-// the wavefront totals through LDS (s holds at least kBlock / 64 ints)
+// the wavefront totals through LDS (s holds at least THREADS / 64 ints)
+template <int THREADS = kBlock>
 __device__ __forceinline__ int block_exclusive_scan(int value, int *s, int &total)
 {
     const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
@@ -773,7 +780,7 @@ __device__ __forceinline__ int block_exclusive_scan(int value, int *s, int &tota
     int below = 0;
     total = 0;
 #pragma unroll
-    for (int w = 0; w < kBlock / 64; w++) {
+    for (int w = 0; w < THREADS / 64; w++) {
         const int t = s[w];
         below += w < wave ? t : 0;
         total += t;
@@ -796,6 +803,19 @@ __device__ __forceinline__ void scan_load(const int *p, int base, int n, bool ve
     } else {
 #pragma unroll
         for (int k = 0; k < kScanItems; k++) v[k] = (base + k < n) ? p[base + k] : 0;
+    }
+}
+
+// zeros in place of what scan_load read
+__device__ __forceinline__ void scan_clear(int *p, int base, int n, bool vec)
+{
+    if (vec && base + kScanItems <= n) {
+#pragma unroll
+        for (int k = 0; k < kScanItems; k += 4) *reinterpret_cast<int4 *>(p + base + k) = make_int4(0, 0, 0, 0);
+    } else {
+#pragma unroll
+        for (int k = 0; k < kScanItems; k++)
+            if (base + k < n) p[base + k] = 0;
     }
 }
 
@@ -827,24 +847,23 @@ __device__ __forceinline__ bool aligned16(const void *p)
 // kick, also when nothing is rebuilt.
 // state[0]: the ticket, state[1 + tile]: {0 nothing, 1 sum, 2 prefix} << 32 | value, all zero on
 // entry (the histogram kernel before it clears them).
-[[maybe_unused]] __global__ void __launch_bounds__(kBlock)
-    k_scan(const int *flag, const int *in, int *out, unsigned long long *state, int n)
+//
+// scan_tile: one tile, of kScanItems ints per thread.  s, s_before: LDS of the block.  CLEAR: `in`
+// is zeroed (the histogram, for the next build).
+template <bool CLEAR, int THREADS = kBlock>
+__device__ __forceinline__ void scan_tile(int *in, int *out, unsigned long long *state, int n,
+                                          int tile, int *s, int &s_before)
 {
-    if (skip(flag)) return;
-    __shared__ int s[kBlock / 64];
-    __shared__ int s_tile, s_before;
-    if (threadIdx.x == 0) s_tile = (int)atomicAdd(&state[0], 1ull);
-    __syncthreads();
-    const int tile = s_tile;
     const bool vec = aligned16(in) && aligned16(out);
-    const int base = tile * kScanTile + (int)threadIdx.x * kScanItems;
+    const int base = (tile * THREADS + (int)threadIdx.x) * kScanItems;
     int v[kScanItems];
     scan_load(in, base, n, vec, v);
+    if constexpr (CLEAR) scan_clear(in, base, n, vec);
     int sum = 0;
 #pragma unroll
     for (int k = 0; k < kScanItems; k++) sum += v[k];
     int total;
-    int run = block_exclusive_scan(sum, s, total);
+    int run = block_exclusive_scan<THREADS>(sum, s, total);
     if (threadIdx.x < 64) {
         const int lane = threadIdx.x;
         auto publish = [&](unsigned long long kind, int value) {
@@ -885,13 +904,25 @@ __device__ __forceinline__ bool aligned16(const void *p)
     scan_store(out, base, n, vec, r);
 }
 
+template <bool CLEAR>
+__global__ void __launch_bounds__(kBlock)
+    k_scan(const int *flag, int *in, int *out, unsigned long long *state, int n)
+{
+    if (skip(flag)) return;
+    __shared__ int s[kBlock / 64];
+    __shared__ int s_tile, s_before;
+    if (threadIdx.x == 0) s_tile = (int)atomicAdd(&state[0], 1ull);
+    __syncthreads();
+    scan_tile<CLEAR>(in, out, state, n, s_tile, s, s_before);
+}
+
 // words of k_scan's state for n ints
 inline int scan_words(int n) { return 1 + (n + kScanTile - 1) / kScanTile; }
 
-// clears them (the histogram kernels call it)
-__device__ __forceinline__ void clear_scan_state(unsigned long long *state, int words)
+// clears them (the histogram kernels call it, as block b of nb)
+__device__ __forceinline__ void clear_scan_state(unsigned long long *state, int words, int b, int nb)
 {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < words; i += gridDim.x * blockDim.x)
+    for (int i = b * (int)blockDim.x + (int)threadIdx.x; i < words; i += nb * (int)blockDim.x)
         state[i] = 0ull;
 }
 
@@ -949,8 +980,11 @@ struct tpsph_handle {
     int *flag = nullptr;  // rebuild of the fluid cell list pending
     // fluid cell list + cell-sorted state
     int *f_cell = nullptr, *f_rank = nullptr, *f_count = nullptr, *f_start = nullptr,
-        *f_perm = nullptr, *f_permu = nullptr;  // f_permu: unordered inside a cell
+        *f_perm = nullptr;
+    // last member of every cell (the others by f_rank, see k_links; nullptr: tpsph_kick_noalloc)
+    int *f_head = nullptr;
     unsigned long long *scan_state = nullptr;  // k_scan
+    int *sort_ctl = nullptr;  // k_sort: ticket and finished items of its phases (nullptr: the four kernels)
     double *f_mass = nullptr;  // caller order
     double *xs = nullptr, *ys = nullptr, *zs = nullptr, *snap = nullptr;
     float4 *xf = nullptr;  // Verlet lists: FP32 positions at the last rebuild (+ kPad NaN)
@@ -1121,9 +1155,9 @@ int derive_params(const tpsph_params *params, int nf, int nw, const double *lo,
 int launch_fluid_brick_mixed(tpsph_handle *h, double *dv);
 
 // Exclusive scan of n ints from in to out on the handle's stream (h->scan_state is clear).
-inline int scan(tpsph_handle *h, const int *flag, const int *in, int *out, int n)
+inline int scan(tpsph_handle *h, const int *flag, int *in, int *out, int n)
 {
-    hipLaunchKernelGGL((k_scan), dim3(scan_words(n) - 1), dim3(kBlock), 0, h->stream, flag, in, out, h->scan_state, n);
+    hipLaunchKernelGGL((k_scan<false>), dim3(scan_words(n) - 1), dim3(kBlock), 0, h->stream, flag, in, out, h->scan_state, n);
     return launch_check(h, "k_scan");
 }
 
