@@ -321,11 +321,12 @@ __global__ void __launch_bounds__(kSortThreads)
 // active wall particles (a non-empty list; active / nactive, built at the rebuild) are
 // visited: the others keep the values the rebuild gave them.  LANES lanes share a wall
 // particle (lane q takes list entries q, q + LANES, ...; the partial sums are added at the
-// end).  A count of -1 (overflow) walks the cells on the first lane.
-template <int ND, int LANES>
+// end).  A count of -1 (overflow) walks the cells, each lane its share of the rows.
+template <int ND>
 __global__ void __launch_bounds__(kBlock)
     k_wall(const DevHandle *__restrict__ H)
 {
+    constexpr int LANES = kWallLanes;
     DevParams P = H->params();
     const FluidView F = H->fluid();
     const double4 *wpos = H->wpos;
@@ -351,9 +352,9 @@ __global__ void __launch_bounds__(kBlock)
                 adami_term<ND>(P, F, xw, j, pressure, volume, vs);
                 j = jn;
             }
-        } else if (q == 0) {
-            Pencils<ND> it;
-            it.init(P, xw.x, xw.y, xw.z, P.hs_fluid);
+        } else {
+            Pencils<ND, LANES> it;
+            it.init(P, xw.x, xw.y, xw.z, P.hs_fluid, q);
             int jb, je;
             while (it.next(P, F.start, jb, je))
                 for (int j = jb; j < je; j++) adami_term<ND>(P, F, xw, j, pressure, volume, vs);
@@ -373,8 +374,8 @@ __global__ void __launch_bounds__(kBlock)
 
 
 // SUM: SummationDensity (the pressure acceleration of pair_fluid<ND, true>, velocity rows
-// of dv only).
-template <int ND, bool SUM = false>
+// of dv only).  ANT: DensityDiffusionAntuono.  Without either the pairs take pair_factored.
+template <int ND, bool SUM = false, bool ANT = false>
 __global__ void __launch_bounds__(kBlock)
     k_fluid(const DevHandle *__restrict__ H, double *__restrict__ dv)
 {
@@ -403,16 +404,22 @@ __global__ void __launch_bounds__(kBlock)
     const double inv_rho_a = 1.0 / rho_a;
     if constexpr (SUM) p_a = p_a / (rho_a * rho_a);  // the target's p / rho^2
     double ga[3] = {0.0, 0.0, 0.0};  // DensityDiffusionAntuono: this particle's gradient
-    if (!SUM && P.ddgrad && active) {
+    if (ANT && active) {
 #pragma unroll
         for (int d = 0; d < ND; d++) ga[d] = P.ddgrad[(size_t)s * ND + d];
     }
 
     double acc[3] = {0.0, 0.0, 0.0}, drho = 0.0;
-    neighbour_sweep<ND, false, kCap, kBlock, SUM>(P, F.start, F.x, F.y, F.z, P.hs_fluid, active,
-                                                  F, Wv, lst, xa, va, rho_a, p_a, inv_rho_a,
-                                                  acc, drho, 0.0,
-                                                  (!SUM && P.ddgrad) ? ga : nullptr);
+    constexpr bool kFactored = !SUM && !ANT;
+    neighbour_sweep<ND, false, kCap, kBlock, SUM, kFactored>(
+        P, F.start, F.x, F.y, F.z, P.hs_fluid, active, F, Wv, lst, xa, va, rho_a, p_a,
+        kFactored ? (P.use_visc ? 2.0 * P.av_c * rho_a : 0.0) : inv_rho_a, acc, drho, 0.0,
+        ANT ? ga : nullptr);
+    if constexpr (kFactored) {
+#pragma unroll
+        for (int d = 0; d < ND; d++) acc[d] *= P.kgrad_c / rho_a;
+        drho *= P.kgrad_c;
+    }
     double accw[3] = {0.0, 0.0, 0.0}, drhow = 0.0;
     if (P.nw > 0) {
         // walls are static: only cells flagged at create can have wall neighbours
@@ -2756,10 +2763,7 @@ int prepare_impl(tpsph_handle *h, const double *v, const double *u, bool gathere
     }
     if (nw > 0) {
         TimedScope t(h, TPSPH_TIME_WALL);
-        if (h->anbr)
-            hipLaunchKernelGGL((k_wall<ND, 4>), dim3(gate_blocks(4 * (int64_t)nw)), dim3(kBlock), 0, h->stream, h->dev);
-        else
-            hipLaunchKernelGGL((k_wall<ND, 1>), dim3(nblocks(nw)), dim3(kBlock), 0, h->stream, h->dev);
+        hipLaunchKernelGGL((k_wall<ND>), dim3(gate_blocks(kWallLanes * (int64_t)nw)), dim3(kBlock), 0, h->stream, h->dev);
         TRY(launch_check(h, "k_wall"));
     }
     return TPSPH_OK;
@@ -2811,7 +2815,8 @@ int kick_impl(tpsph_handle *h, double *dv, const double *v, const double *u, boo
         } else if (h->P.summation) {
             hipLaunchKernelGGL((k_fluid<ND, true>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream, h->dev, dv);
         } else {
-            hipLaunchKernelGGL((k_fluid<ND>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream, h->dev, dv);
+            const auto cells = h->P.ddgrad ? k_fluid<ND, false, true> : k_fluid<ND>;
+            hipLaunchKernelGGL(cells, dim3(nblocks(nf)), dim3(kBlock), 0, h->stream, h->dev, dv);
         }
         TRY(launch_check(h, "k_fluid"));
     }

@@ -8,12 +8,11 @@
 // one after the other (case c owns the global cells cell_off[c] .. cell_off[c] + ncells_c).
 //
 // One kick is one pass of each kernel over the whole ensemble:
-//   k_bcells + scan + k_scatter + k_sort_cells   a counting sort over the global cell index;
-//                                                cases own contiguous cell ranges, so the
-//                                                sorted order keeps every case's particles
-//                                                together and, inside a case, is exactly the
-//                                                order the case sorted alone would have
-//   k_bgather     cell-sorted records with the case's state equation
+//   k_blinks + k_scan + k_bgather   a stable counting sort over the global cell index and the
+//                                   cell-sorted records with the case's state equation; cases own
+//                                   contiguous cell ranges, so the sorted order keeps every case's
+//                                   particles together and, inside a case, is exactly the order
+//                                   the case sorted alone would have
 //   k_bwall       Adami pass of every wall particle over its case's fluid cells
 //   k_bfluid      fused fluid-fluid + fluid-wall interaction + gravity, the cell walk of the
 //                 single-case cell search (k_fluid) on the case's grid and constants
@@ -24,7 +23,7 @@
 // TPSPH_SEARCH_CELLS, skin 0 and the same box.
 //
 // tpsph_batch_solve_ck2n54 captures one step (five kicks and five stages) in a HIP graph and
-// replays it.  Counters and histograms are cleared by kernels (k_scatter clears the cell
+// replays it (the stage kernel also builds the chains of the next kick's sort).  Counters and histograms are cleared by kernels (k_scan clears the cell
 // counts it consumed), so the graph holds no memset node.
 #include "tpsph_internal.h"
 #include "tpsph_batch.h"
@@ -89,18 +88,55 @@ __global__ void k_bcells(DevParams P, const CaseDev *__restrict__ cases,
     }
 }
 
-// cell-sorted records of the fluid state (the fields of k_gather) with the case's state
-// equation; fcase is indexed by the caller's index, whose case ranges the sorted order keeps
+// The fluid's cells as chains (k_links of tpsph.hip): head[g] and next[i], with the cells stored.
+struct BatchLinks {
+    const CaseDev *cases;
+    const int *fcase;
+    int *cell, *next, *head, *count;
+    unsigned long long *state;  // of the scan that follows
+    int words;
+
+    template <int ND>
+    __device__ __forceinline__ void add(const DevParams &P, int i, const double *x) const
+    {
+        const CaseDev &cs = cases[fcase[i]];
+        DevParams Q = P;
+        apply_case(Q, cs);
+        const int g = cs.cell_off + local_cell<ND>(Q, x + (size_t)i * ND);
+        cell[i] = g;
+        atomicAdd(&count[g], 1);
+        next[i] = atomicExch(&head[g], i);
+    }
+};
+
+template <int ND>
+__global__ void k_blinks(DevParams P, BatchLinks L, int n, const double *__restrict__ x)
+{
+    clear_scan_state(L.state, L.words, blockIdx.x, gridDim.x);
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) L.add<ND>(P, i, x);
+}
+
+// cell-sorted records of the fluid state (the fields of k_gather, particle i behind the members
+// of its cell with a smaller index) with the case's state equation; fcase is indexed by the
+// caller's index, whose case ranges the sorted order keeps
 template <int ND>
 __global__ void k_bgather(DevParams P, const CaseDev *__restrict__ cases,
-                          const int *__restrict__ fcase, int nf, const int *__restrict__ perm,
+                          const int *__restrict__ fcase, int nf, const int *__restrict__ cell,
+                          const int *__restrict__ next, const int *__restrict__ head,
+                          const int *__restrict__ start, int *__restrict__ perm,
                           const double *__restrict__ u, const double *__restrict__ v,
                           const double *__restrict__ m, double *__restrict__ xs,
                           double *__restrict__ ys, double *__restrict__ zs,
                           double4 *__restrict__ rec, double2 *__restrict__ vol)
 {
-    for (int s = blockIdx.x * blockDim.x + threadIdx.x; s < nf; s += gridDim.x * blockDim.x) {
-        const int i = perm[s];
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nf; i += gridDim.x * blockDim.x) {
+        const int g = cell[i], members = start[g + 1] - start[g];
+        int s = start[g];
+        for (int k = 0, j = head[g]; k < members; k++) {
+            s += j < i ? 1 : 0;
+            if (k + 1 < members) j = next[j];
+        }
+        perm[s] = i;
         DevParams Q = P;
         apply_case(Q, cases[fcase[i]]);
         double x[3] = {0.0, 0.0, 0.0}, vv[3] = {0.0, 0.0, 0.0};
@@ -110,40 +146,55 @@ __global__ void k_bgather(DevParams P, const CaseDev *__restrict__ cases,
             vv[d] = v[(size_t)i * (ND + 1) + d];
         }
         const double rho = v[(size_t)i * (ND + 1) + ND];
-        xs[s] = x[0];
-        ys[s] = x[1];
-        if constexpr (ND == 3) zs[s] = x[2];
+        if constexpr (ND == 2) {  // {x, y} pairs (see k_bfluid)
+            reinterpret_cast<double2 *>(xs)[s] = make_double2(x[0], x[1]);
+        } else {
+            xs[s] = x[0];
+            ys[s] = x[1];
+            zs[s] = x[2];
+        }
         rec[2 * (size_t)s] = make_double4(x[0], x[1], x[2], rho);
         rec[2 * (size_t)s + 1] = make_double4(vv[0], vv[1], vv[2], state_equation(Q, rho));
         vol[s] = make_double2(m[i] / rho, m[i]);
     }
 }
 
-// Adami pass (k_wall's cell walk) of every wall particle over its case's fluid cells
+// Adami pass (k_wall's cell walk) of every wall particle over its case's fluid cells, four lanes
+// per wall particle: most of the time goes to the cell rows, of which each takes its share
 template <int ND>
 __global__ void __launch_bounds__(kBlock)
     k_bwall(DevParams P, const CaseDev *__restrict__ cases, const int *__restrict__ wcase,
             FluidView F, const double4 *__restrict__ wpos, double *__restrict__ pw,
             double *__restrict__ rhow, double2 *__restrict__ wpv)
 {
-    for (int w = blockIdx.x * blockDim.x + threadIdx.x; w < P.nw; w += gridDim.x * blockDim.x) {
+    constexpr int kLanes = kWallLanes;
+    const int q = threadIdx.x % kLanes;
+    // (the loop bound is uniform per group of lanes, so the partners shuffle together)
+    for (int w = (blockIdx.x * blockDim.x + threadIdx.x) / kLanes; w < P.nw; w += gridDim.x * blockDim.x / kLanes) {
         const CaseDev &cs = cases[wcase[w]];
         DevParams Q = P;
         apply_case(Q, cs);
         const double4 xw = wpos[w];
         double pressure = 0.0, volume = 0.0, vs[3] = {0.0, 0.0, 0.0};
-        Pencils<ND> it;
-        it.init(Q, xw.x, xw.y, xw.z, Q.hs_fluid);
+        Pencils<ND, kLanes> it;
+        it.init(Q, xw.x, xw.y, xw.z, Q.hs_fluid, q);
         const int *start = F.start + cs.cell_off;
         int jb, je;
         while (it.next(Q, start, jb, je))
             for (int j = jb; j < je; j++) adami_term<ND>(Q, F, xw, j, pressure, volume, vs);
-        adami_finish(Q, w, xw.w, pressure, volume, pw, rhow, wpv, vs, nullptr);
+#pragma unroll
+        for (int o = 1; o < kLanes; o <<= 1) {
+            pressure += __shfl_xor(pressure, o);
+            volume += __shfl_xor(volume, o);
+        }
+        if (q == 0) adami_finish(Q, w, xw.w, pressure, volume, pw, rhow, wpv, vs, nullptr);
     }
 }
 
 // Fused fluid-fluid + fluid-wall interaction and gravity (k_fluid) per sorted fluid particle
-// on its case's grid; BLOCK threads per block, CAP list entries per lane in LDS.
+// on its case's grid; BLOCK threads per block, CAP list entries per lane in LDS.  The cases of a
+// wavefront, mostly one, are taken one after the other, so that a case's grid and constants are
+// scalars: as lanes' own values they cost 30 registers and the rows' arithmetic.
 template <int ND, int BLOCK, int CAP>
 __global__ void __launch_bounds__(BLOCK)
     k_bfluid(DevParams P, const CaseDev *__restrict__ cases, const int *__restrict__ fcase,
@@ -155,9 +206,7 @@ __global__ void __launch_bounds__(BLOCK)
     const int s = xcd_tile(blockIdx.x, gridDim.x) * BLOCK + threadIdx.x;
     const bool active = s < P.nf;
     const int sc = active ? s : P.nf - 1;  // an in-bounds particle for the idle lanes
-    const CaseDev &cs = cases[fcase[sc]];
-    DevParams Q = P;
-    apply_case(Q, cs);
+    const int own_case = fcase[sc];
     double xa[3] = {0.0, 0.0, 0.0}, va[3] = {0.0, 0.0, 0.0}, rho_a = 1.0, p_a = 0.0;
     if (active) {
         const double4 a = F.rec[2 * (size_t)s];
@@ -173,18 +222,28 @@ __global__ void __launch_bounds__(BLOCK)
     }
     const double inv_rho_a = 1.0 / rho_a;
     double acc[3] = {0.0, 0.0, 0.0}, drho = 0.0;
-    neighbour_sweep<ND, false, CAP, BLOCK>(Q, F.start + cs.cell_off, F.x, F.y, F.z, Q.hs_fluid,
-                                           active, F, Wv, lst, xa, va, rho_a, p_a, inv_rho_a,
-                                           acc, drho);
     double accw[3] = {0.0, 0.0, 0.0}, drhow = 0.0;
-    if (P.nw > 0) {
-        bool near = false;
-        if (active) near = wall_near[cs.cell_off + local_cell<ND>(Q, xa)] != 0;
-        if (__any(near))
-            neighbour_sweep<ND, true, CAP, BLOCK>(Q, Wv.start + cs.cell_off, Wv.x, Wv.y, Wv.z,
-                                                  Q.hs_wall, near, F, Wv, lst, xa, va, rho_a,
-                                                  p_a, inv_rho_a, accw, drhow);
+    for (unsigned long long todo = __ballot(true); todo != 0;) {
+        const int c = __builtin_amdgcn_readlane(own_case, __ffsll((long long)todo) - 1);
+        const bool mine = own_case == c;
+        todo &= ~__ballot(mine);
+        const CaseDev &cs = cases[c];
+        DevParams Q = P;
+        apply_case(Q, cs);
+        neighbour_sweep<ND, false, CAP, BLOCK, false, true, ND == 2>(
+            Q, F.start + cs.cell_off, F.x, F.y, F.z, Q.hs_fluid, active && mine, F, Wv, lst, xa, va,
+            rho_a, p_a, P.use_visc ? 2.0 * Q.av_c * rho_a : 0.0, acc, drho);
+        if (P.nw > 0) {
+            const bool near = active && mine && wall_near[cs.cell_off + local_cell<ND>(Q, xa)] != 0;
+            if (__any(near))
+                neighbour_sweep<ND, true, CAP, BLOCK>(Q, Wv.start + cs.cell_off, Wv.x, Wv.y, Wv.z,
+                                                      Q.hs_wall, near, F, Wv, lst, xa, va, rho_a,
+                                                      p_a, inv_rho_a, accw, drhow);
+        }
     }
+#pragma unroll
+    for (int d = 0; d < ND; d++) acc[d] *= P.kgrad_c / rho_a;
+    drho *= P.kgrad_c;
     if (!active) return;
     const int i = F.perm[s];
 #pragma unroll
@@ -194,9 +253,10 @@ __global__ void __launch_bounds__(BLOCK)
 
 // One 2N-storage stage of (v, u) with slopes (dv, v) over every case: a block owns kBlock
 // particles and updates their u (with the v of the stage state) before their v.
-template <int ND>
+// LINKS: then what k_blinks does for the next kick.
+template <int ND, bool LINKS>
 __global__ void __launch_bounds__(kBlock)
-    k_bstage(int nf, double *__restrict__ v, double *__restrict__ u, double *__restrict__ tv,
+    k_bstage(DevParams P, BatchLinks L, int nf, double *__restrict__ v, double *__restrict__ u, double *__restrict__ tv,
              double *__restrict__ tu, const double *__restrict__ dv, double a, double b,
              double dt, int first)
 {
@@ -217,6 +277,11 @@ __global__ void __launch_bounds__(kBlock)
         const double t = first ? dt * dv[k] : fma(dt, dv[k], a * tv[k]);
         tv[k] = t;
         v[k] = fma(b, t, v[k]);
+    }
+    if constexpr (LINKS) {
+        clear_scan_state(L.state, L.words, blockIdx.x, gridDim.x);
+        // (the block's new u are complete since the barrier)
+        if ((int)threadIdx.x < np) L.add<ND>(P, i0 + (int)threadIdx.x, u);
     }
 }
 
@@ -295,27 +360,32 @@ int bfail(tpsph_batch *b, int code, const std::string &msg)
     return fail(b ? &b->h : nullptr, code, msg);
 }
 
+BatchLinks batch_links(const tpsph_batch *b)
+{
+    const tpsph_handle *h = &b->h;
+    return {b->cases, b->fcase, h->f_cell, h->f_rank, h->f_head, h->f_count, h->scan_state,
+            scan_words((int)b->ncells_total + 1)};
+}
+
+// linked: the stage kernel has built the chains of u.
 template <int ND>
-int batch_kick(tpsph_batch *b, double *dv, const double *v, const double *u)
+int batch_kick(tpsph_batch *b, double *dv, const double *v, const double *u, bool linked)
 {
     tpsph_handle *h = &b->h;
     const int nf = h->nf, nw = h->nw;
     const int nc = (int)b->ncells_total;
     hipStream_t st = h->stream;
     if (nf == 0) return TPSPH_OK;
-    hipLaunchKernelGGL((k_bcells<ND>), dim3(gate_blocks(nf)), dim3(kBlock), 0, st, h->P, b->cases,
-                       b->fcase, nf, u, h->f_cell, h->f_rank, h->f_count, h->scan_state, scan_words(nc + 1));
-    TRY(launch_check(h, "k_bcells"));
-    TRY(scan(h, nullptr, h->f_count, h->f_start, nc + 1));
-    hipLaunchKernelGGL((k_scatter), dim3(gate_blocks(nf)), dim3(kBlock), 0, st, nullptr, nf, h->f_cell,
-                       h->f_rank, h->f_start, h->f_perm, h->f_count);
-    hipLaunchKernelGGL((k_sort_cells), dim3(gate_blocks(nc)), dim3(kBlock), 0, st, nullptr, nc,
-                       h->f_start, h->f_perm);
-    hipLaunchKernelGGL((k_bgather<ND>), dim3(gate_blocks(nf)), dim3(kBlock), 0, st, h->P, b->cases,
-                       b->fcase, nf, h->f_perm, u, v, h->f_mass, h->xs, h->ys, h->zs, h->rec, h->vol);
+    if (!linked)
+        hipLaunchKernelGGL((k_blinks<ND>), dim3(gate_blocks(nf)), dim3(kBlock), 0, st, h->P, batch_links(b), nf, u);
+    hipLaunchKernelGGL((k_scan<true>), dim3(scan_words(nc + 1) - 1), dim3(kBlock), 0, st, nullptr, h->f_count,
+                       h->f_start, h->scan_state, nc + 1);
+    hipLaunchKernelGGL((k_bgather<ND>), dim3(gate_blocks(nf)), dim3(kBlock), 0, st, h->P, b->cases, b->fcase,
+                       nf, h->f_cell, h->f_rank, h->f_head, h->f_start, h->f_perm, u, v, h->f_mass, h->xs,
+                       h->ys, h->zs, h->rec, h->vol);
     TRY(launch_check(h, "batch cell list"));
     if (nw > 0) {
-        hipLaunchKernelGGL((k_bwall<ND>), dim3(gate_blocks(nw)), dim3(b->wall_block), 0, st, h->P,
+        hipLaunchKernelGGL((k_bwall<ND>), dim3(gate_blocks(kWallLanes * (int64_t)nw)), dim3(b->wall_block), 0, st, h->P,
                            b->cases, b->wcase, h->fluid_view(), h->wpos, h->pw, h->rhow, h->wpv);
         TRY(launch_check(h, "k_bwall"));
     }
@@ -332,9 +402,9 @@ int batch_kick(tpsph_batch *b, double *dv, const double *v, const double *u)
     return launch_check(h, "k_bfluid");
 }
 
-int batch_kick_dispatch(tpsph_batch *b, double *dv, const double *v, const double *u)
+int batch_kick_dispatch(tpsph_batch *b, double *dv, const double *v, const double *u, bool linked = false)
 {
-    return b->h.nd == 2 ? batch_kick<2>(b, dv, v, u) : batch_kick<3>(b, dv, v, u);
+    return b->h.nd == 2 ? batch_kick<2>(b, dv, v, u, linked) : batch_kick<3>(b, dv, v, u, linked);
 }
 
 // one CK2N54 step: five kicks, each followed by its stage update
@@ -351,13 +421,13 @@ int batch_step(tpsph_batch *b, double *v, double *u, double dt)
                                 2277821191437.0 / 14882151754819.0};
     tpsph_handle *h = &b->h;
     for (int i = 0; i < 5; i++) {
-        TRY(batch_kick_dispatch(b, h->sol_dv, v, u));
-        if (h->nd == 2)
-            hipLaunchKernelGGL((k_bstage<2>), dim3(nblocks(h->nf)), dim3(kBlock), 0, h->stream, h->nf, v, u,
-                               h->sol_tv, h->sol_tu, h->sol_dv, A[i], B[i], dt, i == 0);
-        else
-            hipLaunchKernelGGL((k_bstage<3>), dim3(nblocks(h->nf)), dim3(kBlock), 0, h->stream, h->nf, v, u,
-                               h->sol_tv, h->sol_tu, h->sol_dv, A[i], B[i], dt, i == 0);
+        TRY(batch_kick_dispatch(b, h->sol_dv, v, u, i > 0));
+        // the chains of the next kick of the step (one launch less: 14.6 us and 14.8 of the stage
+        // become 25.5 at 64 cases of about 7,400)
+        const auto stage = h->nd == 2 ? (i < 4 ? k_bstage<2, true> : k_bstage<2, false>)
+                                      : (i < 4 ? k_bstage<3, true> : k_bstage<3, false>);
+        hipLaunchKernelGGL(stage, dim3(nblocks(h->nf)), dim3(kBlock), 0, h->stream, h->P, batch_links(b), h->nf,
+                           v, u, h->sol_tv, h->sol_tu, h->sol_dv, A[i], B[i], dt, i == 0);
         TRY(launch_check(h, "k_bstage"));
     }
     return TPSPH_OK;
@@ -494,13 +564,17 @@ int tpsph_batch_create(const tpsph_params *params, int32_t n_cases, const tpsph_
     BTRY(dalloc(h, &h->scan_state, (size_t)scan_words(nc + 1)));
     BTRY(dalloc(h, &h->f_cell, nf));
     BTRY(dalloc(h, &h->f_rank, nf));
+    BTRY(dalloc(h, &h->f_head, (size_t)nc));
     BTRY(dalloc(h, &h->f_perm, nf));
     BTRY(dalloc(h, &h->f_count, (size_t)nc + 1));
     BTRY(dalloc(h, &h->f_start, (size_t)nc + 1));
     BTRY(dalloc(h, &h->f_mass, nf));
-    BTRY(dalloc(h, &h->xs, (size_t)nf + kPad));
-    BTRY(dalloc(h, &h->ys, (size_t)nf + kPad));
-    BTRY(dalloc(h, &h->zs, (size_t)nf + kPad));
+    const size_t nx = (nd == 2 ? 2 : 1) * ((size_t)nf + kPad);  // 2D: {x, y} pairs
+    BTRY(dalloc(h, &h->xs, nx));
+    if (nd == 3) {
+        BTRY(dalloc(h, &h->ys, nx));
+        BTRY(dalloc(h, &h->zs, nx));
+    }
     BTRY(dalloc(h, &h->rec, 2 * (size_t)nf));
     BTRY(dalloc(h, &h->vol, nf));
     BTRY(dalloc(h, &h->w_start, (size_t)nc + 1));
@@ -532,7 +606,8 @@ int tpsph_batch_create(const tpsph_params *params, int32_t n_cases, const tpsph_
             h->last_error = std::string("ensemble set-up: ") + hipGetErrorString(e);
             return cleanup(TPSPH_ERR_HIP);
         }
-        for (double *a : {h->xs, h->ys, h->zs}) BTRY(hip_fill(h, a, (size_t)nf + kPad));
+        for (double *a : {h->xs, h->ys, h->zs})
+            if (a) BTRY(hip_fill(h, a, nx));
         for (double *a : {h->wx, h->wy, h->wz}) BTRY(hip_fill(h, a, (size_t)nw + kPad));
         // static walls: the same counting sort over the global cells, once
         if (nw > 0) {
@@ -663,7 +738,7 @@ void tpsph_batch_destroy(tpsph_batch *b)
     tpsph_handle *h = &b->h;
     (void)hipStreamSynchronize(h->stream);
     drop_graph(b);
-    void *ptrs[] = {b->cases, b->fcase, b->wcase, h->scan_state, h->f_cell, h->f_rank, h->f_perm,
+    void *ptrs[] = {b->cases, b->fcase, b->wcase, h->scan_state, h->f_cell, h->f_rank, h->f_head, h->f_perm,
                     h->f_count, h->f_start, h->f_mass, h->xs, h->ys, h->zs, h->rec, h->vol,
                     h->w_start, h->w_perm, h->wx, h->wy, h->wz, h->wpos, h->wpv, h->pw,
                     h->rhow, h->wall_near, h->sol_dv, h->sol_tv, h->sol_tu};

@@ -20,6 +20,7 @@
 namespace tpsph {
 
 constexpr int kBlock = 256;  // 4 wavefronts of 64
+constexpr int kWallLanes = 4;  // lanes per wall particle of the Adami pass
 constexpr int kCap = 32;     // neighbour-list entries per lane and phase
 constexpr int kScanItems = 16;
 constexpr int kScanTile = kBlock * kScanItems;
@@ -279,14 +280,15 @@ __device__ __forceinline__ T ldo(const T *__restrict__ base, uint32_t byte_off)
     return *(const T *)((const char *)base + byte_off);
 }
 
-// Enumerates the candidate ranges (pencils) around one point, z-outer, y-inner.
-template <int ND>
+// Enumerates the candidate ranges (pencils) around one point, z-outer, y-inner.  LANES > 1: lane q
+// of that many takes every LANES-th of each plane.
+template <int ND, int LANES = 1>
 struct Pencils {
     double xa, ya, za, hs, dz2;
     int y0, y1, z1, iy, iz, rowz;
 
     __device__ __forceinline__ void init(const DevParams &P, double x, double y, double z,
-                                         double hs_)
+                                         double hs_, int q = 0)
     {
         xa = x;
         ya = y;
@@ -295,7 +297,7 @@ struct Pencils {
         dz2 = 0.0;
         rowz = 0;
         const double reach = P.R + hs;
-        y0 = cell_1d(ya - reach, P.lo[1], P.inv_cs[1], P.n[1]);
+        y0 = cell_1d(ya - reach, P.lo[1], P.inv_cs[1], P.n[1]) + q;
         y1 = cell_1d(ya + reach, P.lo[1], P.inv_cs[1], P.n[1]);
         if constexpr (ND == 3) {
             iz = cell_1d(za - reach, P.lo[2], P.inv_cs[2], P.n[2]) - 1;
@@ -321,7 +323,9 @@ struct Pencils {
                 }
                 rowz = P.n[0] * P.n[1] * iz;
             }
-            const int cy = iy++;
+            const int cy = iy;
+            iy += LANES;
+            if (LANES > 1 && cy > y1) continue;
             const double dy = transverse(P, 1, cy, ya, hs);
             const double r2 = P.R2 - fma(dy, dy, dz2);
             if (r2 < 0.0) continue;
@@ -517,6 +521,33 @@ __device__ __forceinline__ void pair_fluid(const DevParams &P, const FluidNbr &n
     drho = fma(n.v.x * kdr, fma(P.dd2, drr, rho_a * vr), drho);
 }
 
+// pair_fluid for a pair in range with the factors common to all pairs of the target left out:
+// acc takes kgrad_c / rho_a and drho kgrad_c afterwards (BrickTarget's form, without density
+// gradients).  visc: 2 alpha c h rho_a, or 0.
+template <int ND>
+__device__ __forceinline__ void pair_factored(const DevParams &P, const FluidNbr &n,
+                                              const double *xa, const double *va, double rho_a,
+                                              double p_a, double visc, double *acc, double &drho)
+{
+    const double p0 = xa[0] - n.a.x, p1 = xa[1] - n.a.y, p2 = (ND == 3) ? xa[2] - n.a.z : 0.0;
+    const double d2 = dist2<ND>(p0, p1, p2);
+    const double w = fma(-0.5 * P.h_inv, sqrt_pos(d2), 1.0);
+    const double Vk = n.v.x * (w * w * w);
+    double vr = (va[0] - n.b.x) * p0 + (va[1] - n.b.y) * p1;
+    if constexpr (ND == 3) vr += (va[2] - n.b.z) * p2;
+    const double rho_b = n.a.w, q = d2 + P.eps_h2, sum_rho = rho_a + rho_b, vn = fmin(vr, 0.0);
+    double f = fma(visc * (rho_b * vn), rcp_pos(q * sum_rho), -(p_a + n.b.w));
+    if (P.use_visc && P.beta != 0.0) {  // uniform
+        const double mu = P.h * vn * rcp_pos(q);
+        f += (rho_a * rho_b) * (2.0 * P.beta * (mu * mu) * rcp_pos(sum_rho));
+    }
+    f *= Vk;
+    acc[0] = fma(f, p0, acc[0]);
+    acc[1] = fma(f, p1, acc[1]);
+    if constexpr (ND == 3) acc[2] = fma(f, p2, acc[2]);
+    drho = fma(Vk, fma(P.dd2, rho_a - rho_b, rho_a * vr), drho);
+}
+
 // The wall viscosity (none without one) acts along r_ab for ArtificialViscosityMonaghan
 // (viscosity.jl:89-132, approaching pairs only) and along v_ab for ViscosityAdami
 // (viscosity.jl:219-280, with eta_a = nu_a rho_a from the fluid's kinematic viscosity and
@@ -646,7 +677,10 @@ __device__ __forceinline__ void pair_fluid_masked(const DevParams &P, const Flui
 // candidates per iteration without branches: the arrays cx/cy/cz carry kPad NaN entries
 // past their end, so reads beyond a range stay in bounds and never pass the test, and every
 // candidate is written to the list while the count only advances on a hit.
-template <int ND, bool WALL, int CAP = kCap, int STRIDE = kBlock, bool SUM = false>
+// FACTORED: fluid pairs by pair_factored, with its visc in the place of inv_rho_a.
+// XY (2D): cx holds {x, y} of every candidate, one load instead of two.
+template <int ND, bool WALL, int CAP = kCap, int STRIDE = kBlock, bool SUM = false, bool FACTORED = false,
+          bool XY = false>
 __device__ __forceinline__ void neighbour_sweep(const DevParams &P, const int *__restrict__ start,
                                                 const double *__restrict__ cx,
                                                 const double *__restrict__ cy,
@@ -673,6 +707,11 @@ __device__ __forceinline__ void neighbour_sweep(const DevParams &P, const int *_
             double d2[4];
 #pragma unroll
             for (int k = 0; k < 4; k++) {
+                if constexpr (XY) {
+                    const double2 c = ldo(reinterpret_cast<const double2 *>(cx), 2u * o + 16u * k);
+                    d2[k] = dist2<ND>(xa[0] - c.x, xa[1] - c.y, 0.0);
+                    continue;
+                }
                 const double p0 = xa[0] - ldo(cx, o + 8u * k);
                 const double p1 = xa[1] - ldo(cy, o + 8u * k);
                 const double p2 = (ND == 3) ? xa[2] - ldo(cz, o + 8u * k) : 0.0;
@@ -699,7 +738,10 @@ __device__ __forceinline__ void neighbour_sweep(const DevParams &P, const int *_
                 FluidNbr cur = load_fluid(F, lst[0]);
                 for (int k = 0; k < cnt; k++) {
                     const FluidNbr nxt = load_fluid(F, lst[min(k + 1, cnt - 1) * STRIDE]);
-                    pair_fluid<ND, SUM>(P, cur, xa, va, rho_a, p_a, inv_rho_a, acc, drho, ga);
+                    if constexpr (FACTORED)
+                        pair_factored<ND>(P, cur, xa, va, rho_a, p_a, inv_rho_a, acc, drho);
+                    else
+                        pair_fluid<ND, SUM>(P, cur, xa, va, rho_a, p_a, inv_rho_a, acc, drho, ga);
                     cur = nxt;
                 }
             }
