@@ -1852,10 +1852,7 @@ __global__ void __launch_bounds__(kBrickThreads)
                     // the candidates are independent chains without branches: two at a time
                     // interleave within the register budget of four waves per SIMD; entries
                     // past the end of the list are the far record's: exact zeros
-                    const int k = list_row_entries(m, r);
-#pragma unroll 1
-                    for (int h2 = 0; h2 < k; h2 += 2) {
-                        const int ea = h2 ? cur4.z : cur4.x, eb = h2 ? cur4.w : cur4.y;
+                    auto two = [&](int ea, int eb) {
                         const BrickRec na = lds_rec<ND>(S, ea);
                         const BrickRec nb = lds_rec<ND>(S, eb);
                         double gna[3], gnb[3];
@@ -1865,7 +1862,9 @@ __global__ void __launch_bounds__(kBrickThreads)
                         }
                         T.add(C, na, acc, drho, gna);
                         T.add(C, nb, acc, drho, gnb);
-                    }
+                    };
+                    two(cur4.x, cur4.y);
+                    if (list_row_entries(m, r) > 2) two(cur4.z, cur4.w);
                     cur4 = nxt4;
                 }
                 T.scale(C, acc, drho);
