@@ -316,60 +316,67 @@ __global__ void __launch_bounds__(kSortThreads)
 }
 
 
-// alist / acnt: the wall particles' Verlet lists of fluid candidates (slot-major, row
-// length lw), or nullptr for the cell walk (every wall particle).  With lists only the
-// active wall particles (a non-empty list; active / nactive, built at the rebuild) are
-// visited: the others keep the values the rebuild gave them.  LANES lanes share a wall
-// particle (lane q takes list entries q, q + LANES, ...; the partial sums are added at the
-// end).  A count of -1 (overflow) walks the cells, each lane its share of the rows.
+// The Adami pass of wall particle w: kWallLanes lanes share it (lane q takes the entries q,
+// q + kWallLanes, ... of its list of n fluid candidates, or for n < 0, an overflowed list or the
+// cell search, its share of the rows of the cell walk; the partial sums are added at the end).
+template <int ND>
+__device__ __forceinline__ void adami_wall(const DevHandle *H, const DevParams &P, const FluidView &F,
+                                           int w, int q, int n)
+{
+    constexpr int LANES = kWallLanes;
+    const double4 xw = H->wpos[w];
+    double pressure = 0.0, volume = 0.0, vs[3] = {0.0, 0.0, 0.0};
+    if (n >= 0) {
+        const int *alist = H->anbr;
+        const int lw = H->lw;
+        // the next list entry is loaded before the current one is evaluated
+        int j = q < n ? alist[(size_t)q * lw + w] : 0;
+        for (int k = q; k < n; k += LANES) {
+            const int jn = alist[(size_t)min(k + LANES, n - 1) * lw + w];
+            adami_term<ND>(P, F, xw, j, pressure, volume, vs);
+            j = jn;
+        }
+    } else {
+        Pencils<ND, LANES> it;
+        it.init(P, xw.x, xw.y, xw.z, P.hs_fluid, q);
+        int jb, je;
+        while (it.next(P, F.start, jb, je))
+            for (int j = jb; j < je; j++) adami_term<ND>(P, F, xw, j, pressure, volume, vs);
+    }
+#pragma unroll
+    for (int o = 1; o < LANES; o <<= 1) {
+        pressure += __shfl_xor(pressure, o);
+        volume += __shfl_xor(volume, o);
+        if (P.visc_w) {
+#pragma unroll
+            for (int d = 0; d < ND; d++) vs[d] += __shfl_xor(vs[d], o);
+        }
+    }
+    if (q == 0) adami_finish(P, w, xw.w, pressure, volume, H->pw, H->rhow, H->wpv, vs, H->wvel);
+}
+
+// The Adami pass of all wall particles, as block bx of nb.  With Verlet lists only the active
+// ones (a non-empty list, listed at the rebuild) are visited: the others keep the values the
+// rebuild gave them.
+template <int ND>
+__device__ __forceinline__ void adami_pass(const DevHandle *H, int bx, int nb)
+{
+    const DevParams P = with_sound(H->params());
+    const FluidView F = H->fluid();
+    const int *active = H->wactive, *acnt = H->acnt;
+    const int na = active ? H->counters[1] : P.nw;
+    // the loop bound is uniform per group of lanes, so the partners shuffle together
+    for (int g = (bx * (int)blockDim.x + (int)threadIdx.x) / kWallLanes; g < na; g += nb * (int)blockDim.x / kWallLanes) {
+        const int w = active ? active[g] : g;
+        adami_wall<ND>(H, P, F, w, threadIdx.x % kWallLanes, active ? acnt[w] : -1);
+    }
+}
+
 template <int ND>
 __global__ void __launch_bounds__(kBlock)
     k_wall(const DevHandle *__restrict__ H)
 {
-    constexpr int LANES = kWallLanes;
-    DevParams P = H->params();
-    const FluidView F = H->fluid();
-    const double4 *wpos = H->wpos;
-    double *pw = H->pw, *rhow = H->rhow, *wvel = H->wvel;
-    double2 *wpv = H->wpv;
-    const int *alist = H->anbr, *acnt = H->acnt, *active = H->wactive, *nactive = H->counters + 1;
-    const int lw = H->lw;
-    P = with_sound(P);
-    const int na = alist ? *nactive : P.nw;
-    const int q = threadIdx.x % LANES;
-    // the loop bound is uniform per LANES lanes, so the partners shuffle together
-    for (int g = (blockIdx.x * blockDim.x + threadIdx.x) / LANES; g < na;
-         g += gridDim.x * blockDim.x / LANES) {
-        const int w = alist ? active[g] : g;
-        const double4 xw = wpos[w];
-        double pressure = 0.0, volume = 0.0, vs[3] = {0.0, 0.0, 0.0};
-        const int n = alist ? acnt[w] : -1;
-        if (n >= 0) {
-            // the next list entry is loaded before the current one is evaluated
-            int j = q < n ? alist[(size_t)q * lw + w] : 0;
-            for (int k = q; k < n; k += LANES) {
-                const int jn = alist[(size_t)min(k + LANES, n - 1) * lw + w];
-                adami_term<ND>(P, F, xw, j, pressure, volume, vs);
-                j = jn;
-            }
-        } else {
-            Pencils<ND, LANES> it;
-            it.init(P, xw.x, xw.y, xw.z, P.hs_fluid, q);
-            int jb, je;
-            while (it.next(P, F.start, jb, je))
-                for (int j = jb; j < je; j++) adami_term<ND>(P, F, xw, j, pressure, volume, vs);
-        }
-#pragma unroll
-        for (int o = 1; o < LANES; o <<= 1) {
-            pressure += __shfl_xor(pressure, o);
-            volume += __shfl_xor(volume, o);
-            if (P.visc_w) {
-#pragma unroll
-                for (int d = 0; d < ND; d++) vs[d] += __shfl_xor(vs[d], o);
-            }
-        }
-        if (q == 0) adami_finish(P, w, xw.w, pressure, volume, pw, rhow, wpv, vs, wvel);
-    }
+    adami_pass<ND>(H, blockIdx.x, gridDim.x);
 }
 
 
@@ -803,40 +810,51 @@ __device__ __forceinline__ void build_list(const DevParams &P, const FluidView &
 }
 
 // Verlet lists of the wall particles (wall-sorted order w) over the fluid: candidates within
-// R + skin/2 of the static wall particle, for the Adami pass.
+// R + skin/2 of the static wall particle, for the Adami pass, which follows with `pass`.  Block
+// bx of gx.
 template <int ND>
-__device__ __forceinline__ void
-    wall_lists_body(int bx, int gx, DevParams P, FluidView F, const double4 *__restrict__ wpos,
-                 int lw, int cap, int *__restrict__ nbr, int *__restrict__ cnt,
-                 int *__restrict__ active, int *__restrict__ nactive, double *__restrict__ pw,
-                 double *__restrict__ rhow, double2 *__restrict__ wpv, double *__restrict__ wvel)
+__device__ __forceinline__ void wall_lists_body(const DevHandle *H, int bx, int gx, bool pass)
 {
-    P = with_sound(P);
-    for (int w = bx * kListThreads + threadIdx.x; w < P.nw; w += gx * kListThreads) {
-        const double4 xw = wpos[w];
-        const float4 xwf = list_f32<ND>(P, xw.x, xw.y, xw.z);
-        Pencils<ND> it;
-        it.init(P, xw.x, xw.y, xw.z, P.hs_list_wall);
-        int n = 0, j, je;
-        while (it.next(P, F.start, j, je)) {
-            for (; j < je; j++) {
-                // what is not surely beyond the list radius (see build_list)
-                const float4 q = F.xf[j];
-                const float ex = xwf.x - q.x, ey = xwf.y - q.y, ez = (ND == 3) ? xwf.z - q.z : 0.f;
-                const float d2f = ex * ex + ey * ey + ez * ez;
-                if (!(d2f > P.wlist_out2)) {
-                    if (n < cap) nbr[(size_t)n * lw + w] = j;
-                    n++;
+    const DevParams P = with_sound(H->params());
+    const FluidView F = H->fluid();
+    const double4 *wpos = H->wpos;
+    const int lw = H->lw, cap = H->cap_a;
+    int *nbr = H->anbr, *cnt = H->acnt, *active = H->wactive, *nactive = H->counters + 1;
+    for (int base = bx * kListThreads; base < P.nw; base += gx * kListThreads) {  // uniform
+        const int w = base + (int)threadIdx.x;
+        if (w < P.nw) {
+            const double4 xw = wpos[w];
+            const float4 xwf = list_f32<ND>(P, xw.x, xw.y, xw.z);
+            Pencils<ND> it;
+            it.init(P, xw.x, xw.y, xw.z, P.hs_list_wall);
+            int n = 0, j, je;
+            while (it.next(P, F.start, j, je)) {
+                for (; j < je; j++) {
+                    // what is not surely beyond the list radius (see build_list)
+                    const float4 q = F.xf[j];
+                    const float ex = xwf.x - q.x, ey = xwf.y - q.y, ez = (ND == 3) ? xwf.z - q.z : 0.f;
+                    const float d2f = ex * ex + ey * ey + ez * ez;
+                    if (!(d2f > P.wlist_out2)) {
+                        if (n < cap) nbr[(size_t)n * lw + w] = j;
+                        n++;
+                    }
                 }
             }
+            cnt[w] = n <= cap ? n : -1;
+            if (n == 0) {  // no fluid within reach until the next rebuild: the values of empty sums
+                const double vs0[3] = {0.0, 0.0, 0.0};
+                adami_finish(P, w, xw.w, 0.0, 0.0, H->pw, H->rhow, H->wpv, vs0, H->wvel);
+            } else {
+                active[atomicAdd(nactive, 1)] = w;
+            }
         }
-        cnt[w] = n <= cap ? n : -1;
-        if (n == 0) {  // no fluid within reach until the next rebuild: the values of empty sums
-            const double vs0[3] = {0.0, 0.0, 0.0};
-            adami_finish(P, w, xw.w, 0.0, 0.0, pw, rhow, wpv, vs0, wvel);
+        if (!pass) continue;  // uniform
+        __syncthreads();  // the block's lists
+        for (int k = threadIdx.x / kWallLanes; k < kListThreads; k += kListThreads / kWallLanes) {
+            const int v = base + k;
+            const int n = v < P.nw ? cnt[v] : 0;
+            if (n != 0) adami_wall<ND>(H, P, F, v, threadIdx.x % kWallLanes, n);
         }
-        else
-            active[atomicAdd(nactive, 1)] = w;
     }
 }
 
@@ -1325,10 +1343,11 @@ __device__ __forceinline__ void brick_int_lists(const DevParams &P, const FluidV
     }
 }
 
-// The rebuild after the cell-sorted gather, in one launch: the first nblocks blocks take the
-// bricks (columns of the targets, union, lists of the targets over the fluid and the walls),
-// the others build the Verlet lists of the wall particles (the Adami pass); both read only
-// the new cell-sorted order.
+// The rebuild after the cell-sorted gather, in one launch: the first nwall blocks build the
+// Verlet lists of the wall particles, the others take the bricks (columns of the targets, union,
+// lists of the targets over the fluid and the walls); both read only the new cell-sorted order.
+// adami: the blocks of the wall particles also run the Adami pass, with the flag down nothing
+// else (one launch of a kick less).
 //
 // The list build is bound by the VALU work of the candidates' tests (1.02M particles: 88k of
 // 146k cycles per brick).  The candidates' FP32 positions come from the staged union (from
@@ -1342,24 +1361,27 @@ __device__ __forceinline__ void brick_int_lists(const DevParams &P, const FluidV
 // Two blocks of 512 threads share a compute unit (76 KB each).
 template <int ND>
 __global__ void __launch_bounds__(kListThreads, 4)
-    k_brick_lists(const DevHandle *__restrict__ H, int nblocks)
+    k_brick_lists(const DevHandle *__restrict__ H, int nwall, bool adami)
 {
-    if (skip(H->flag)) return;
-    const DevParams P = H->params();
-    const FluidView F = H->fluid();
-    if ((int)blockIdx.x >= nblocks) {
-        wall_lists_body<ND>(blockIdx.x - nblocks, gridDim.x - nblocks, P, F, H->wpos, H->lw, H->cap_a,
-                            H->anbr, H->acnt, H->wactive, H->counters + 1, H->pw, H->rhow, H->wpv,
-                            H->wvel);
+    const bool rebuild = !skip(H->flag);
+    if ((int)blockIdx.x < nwall) {
+        if (rebuild)
+            wall_lists_body<ND>(H, blockIdx.x, nwall, adami);
+        else if (adami)
+            adami_pass<ND>(H, blockIdx.x, nwall);
         return;
     }
+    if (!rebuild) return;
+    const DevParams P = H->params();
+    const FluidView F = H->fluid();
+    const int block = (int)blockIdx.x - nwall, nblocks = (int)gridDim.x - nwall;
     const WallView Wv = H->walls();
     const ListsArgs A(*H);
     __shared__ ListsSmem S;
     const int tid = threadIdx.x;
     const int ne = A.nne[0];
     const int nuy = P.bc[1] + 2 * P.ur[1];
-    for (int turn = blockIdx.x;; ) {
+    for (int turn = block;; ) {
         if (turn >= ne) break;  // uniform over the block
         const int b = A.nel[turn];
         const int bx = b % P.nb[0], by = (b / P.nb[0]) % P.nb[1], bz = b / (P.nb[0] * P.nb[1]);
@@ -2686,6 +2708,13 @@ int build_cells(tpsph_handle *h, const int *flag, int n, const double *x, int *c
     return launch_check(h, "k_scatter/k_sort_cells");
 }
 
+// Whether the list kernel also runs the Adami pass: not before the densities are summed, and as a
+// kernel of its own while the kernels are timed.
+bool adami_in_lists(const tpsph_handle *h)
+{
+    return h->search == TPSPH_SEARCH_LISTS && !h->P.summation && !h->timing;
+}
+
 // Fluid cell list (rebuilt only when flagged) + cell-sorted gather of (v, u).
 template <int ND>
 int update_fluid(tpsph_handle *h, const double *v, const double *u, bool gathered,
@@ -2720,8 +2749,9 @@ int update_fluid(tpsph_handle *h, const double *v, const double *u, bool gathere
         TRY(launch_check(h, "k_sort / k_gather<1>"));
         if (lists) {
             const int gb = std::max(1, std::min(h->nbricks, 2 * h->n_cu));
-            const int gw = (h->nw + kListThreads - 1) / kListThreads;
-            hipLaunchKernelGGL((k_brick_lists<ND>), dim3(gb + gw), dim3(kListThreads), 0, h->stream, h->dev, gb);
+            // as many blocks for the walls as the Adami pass has lanes for, at most one turn
+            const int gw = (int)std::min<int64_t>((kWallLanes * (int64_t)h->nw + kListThreads - 1) / kListThreads, 2 * h->n_cu);
+            hipLaunchKernelGGL((k_brick_lists<ND>), dim3(gw + gb), dim3(kListThreads), 0, h->stream, h->dev, gw, adami_in_lists(h));
             TRY(launch_check(h, "k_brick_lists"));
         }
         // the fluid kernel of this kick lowers the flag
@@ -2761,7 +2791,7 @@ int prepare_impl(tpsph_handle *h, const double *v, const double *u, bool gathere
         hipLaunchKernelGGL((k_sum_finish), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream, h->dev);
         TRY(launch_check(h, "k_sum_density"));
     }
-    if (nw > 0) {
+    if (nw > 0 && (nf == 0 || keep_order || !adami_in_lists(h))) {
         TimedScope t(h, TPSPH_TIME_WALL);
         hipLaunchKernelGGL((k_wall<ND>), dim3(gate_blocks(kWallLanes * (int64_t)nw)), dim3(kBlock), 0, h->stream, h->dev);
         TRY(launch_check(h, "k_wall"));
