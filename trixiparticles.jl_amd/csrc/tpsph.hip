@@ -1605,8 +1605,7 @@ struct BrickTarget {
     {
         const double p0 = x[0] - n.x[0], p1 = x[1] - n.x[1];
         const double p2 = (ND == 3) ? x[2] - n.x[2] : 0.0;
-        double d2 = p0 * p0 + p1 * p1;  // (contracted: the clamp below needs no exact bound)
-        if constexpr (ND == 3) d2 += p2 * p2;
+        double d2 = dist2<ND>(p0, p1, p2);
         const double near = __hiloint2double(d2 >= C.az2 ? __double2hiint(d2) : 0x7ff80000,
                                              __double2loint(d2));
         const double w = fmax(fma(C.minus_half_h_inv, sqrt_pos(near), 1.0), 0.0);
