@@ -224,16 +224,15 @@ __global__ void __launch_bounds__(kBrickThreads, 8)
                     const ushort4 nxt4 = l4[(size_t)min(r + 2, rows - 1) * ls + col];
                     float row[3] = {0.0f, 0.0f, 0.0f}, part = 0.0f;
                     // two candidates at a time; entries past the list are the far record's
-                    const int k = list_row_entries(m, r);
-#pragma unroll 1
-                    for (int h2 = 0; h2 < k; h2 += 2) {
-                        const int ea = h2 ? cur4.z : cur4.x, eb = h2 ? cur4.w : cur4.y;
+                    auto two = [&](int ea, int eb) {
                         const float4 a0 = lds_at(S.pa, ea), b0 = lds_at(S.pb, ea);
                         const float4 a1 = lds_at(S.pa, eb), b1 = lds_at(S.pb, eb);
                         const float V0 = lds_at(S.vol, ea), V1 = lds_at(S.vol, eb);
                         T.add(q, a0, b0, V0, row, part);
                         T.add(q, a1, b1, V1, row, part);
-                    }
+                    };
+                    two(cur4.x, cur4.y);
+                    if (list_row_entries(m, r) > 2) two(cur4.z, cur4.w);
 #pragma unroll
                     for (int d = 0; d < ND; d++) acc[d] += row[d];  // (a row at a time: fewer roundings)
                     drho.add(part);
