@@ -610,65 +610,6 @@ inline int visc_mode(const DevParams &P)
     return P.use_visc ? (P.beta != 0.0 ? kViscAlphaBeta : kViscAlpha) : kViscNone;
 }
 
-// pair_fluid without branches, for candidates evaluated in groups: an out-of-range (or
-// invalid) candidate gets kdr = 0 by a select, so its terms are exact zeros whatever the
-// square root of its distance gives (NaN for d2 = 0), and the viscosity acts through
-// min(v_ab.r_ab, 0), which is v_ab.r_ab for approaching pairs and zero otherwise (a zero
-// term added to fac leaves it unchanged).  VISC is visc_mode(P).  For an in-range candidate
-// every operation is the one of pair_fluid, so the sums agree bit for bit (up to the sign
-// of a zero).  Every intermediate of an out-of-range candidate stays finite or is selected
-// away: the far record (coordinates 1e100, zero volume) gives d2 about 1e200, whose
-// reciprocals are normal numbers.
-//
-// ga, gb (DensityDiffusionAntuono only): the renormalised density gradients of the target and
-// the candidate, whose term is pair_fluid's.
-// SUM (SummationDensity): the pressure term -m_b (p_a/rho_a^2 + p_b/rho_b^2) grad W with the
-// target's p/rho^2 in p_a and the candidate's in n.b.w (the brick kernel stages p/rho^2 in
-// the pressure slot), and no density rate.
-template <int ND, int VISC, bool ANT = false, bool SUM = false>
-__device__ __forceinline__ void pair_fluid_masked(const DevParams &P, const FluidNbr &n,
-                                                  bool valid, const double *xa,
-                                                  const double *va, double rho_a, double p_a,
-                                                  double inv_rho_a, double *acc, double &drho,
-                                                  const double *ga = nullptr,
-                                                  const double *gb = nullptr)
-{
-    const double p0 = xa[0] - n.a.x, p1 = xa[1] - n.a.y, p2 = (ND == 3) ? xa[2] - n.a.z : 0.0;
-    const double d2 = dist2<ND>(p0, p1, p2);
-    const bool in = valid & (d2 <= P.R2) & (d2 >= P.az2);
-    const double r = sqrt_pos(d2);
-    const double w = fma(-0.5 * P.h_inv, r, 1.0);
-    const double kdr = in ? P.kgrad_c * (w * w * w) : 0.0;
-    const double v0 = va[0] - n.b.x, v1 = va[1] - n.b.y, v2 = (ND == 3) ? va[2] - n.b.z : 0.0;
-    double vr = v0 * p0 + v1 * p1;
-    if constexpr (ND == 3) vr += v2 * p2;
-    const double rho_b = n.a.w;
-    double fac = SUM ? -n.v.y * (p_a + n.b.w) : -n.v.x * inv_rho_a * (p_a + n.b.w);
-    if constexpr (VISC != kViscNone) {
-        const double q = d2 + P.eps_h2;
-        const double sum_rho = rho_a + rho_b;
-        const double vn = fmin(vr, 0.0);
-        fac = fma(2.0 * P.av_c * n.v.y * vn, rcp_pos(q * sum_rho), fac);
-        if constexpr (VISC == kViscAlphaBeta) {
-            const double mu = P.h * vn * rcp_pos(q);
-            fac += 2.0 * n.v.y * P.beta * (mu * mu) * rcp_pos(sum_rho);
-        }
-    }
-    fac *= kdr;
-    acc[0] = fma(fac, p0, acc[0]);
-    acc[1] = fma(fac, p1, acc[1]);
-    if constexpr (ND == 3) acc[2] = fma(fac, p2, acc[2]);
-    if constexpr (!SUM) {
-        double drr = rho_a - rho_b;
-        if constexpr (ANT) {
-            double gr = (ga[0] + gb[0]) * p0 + (ga[1] + gb[1]) * p1;
-            if constexpr (ND == 3) gr += (ga[2] + gb[2]) * p2;
-            drr = fma(-0.5, gr, drr);
-        }
-        drho = fma(n.v.x * kdr, fma(P.dd2, drr, rho_a * vr), drho);
-    }
-}
-
 // Two-phase sweep over the neighbours of one target: phase 1 runs the exact radius test over
 // the candidates of the pencils and appends hits to a per-lane list in LDS, phase 2 evaluates
 // the pair terms on the dense list; the phases alternate until every lane has exhausted its
