@@ -2740,9 +2740,7 @@ int update_fluid(tpsph_handle *h, const double *v, const double *u, bool gathere
                                h->stream, h->dev, u, v, items, tiles);
         } else {
             hipLaunchKernelGGL((k_links<ND>), dim3(gate_blocks(nf)), dim3(kBlock), 0, h->stream, h->dev, u);
-            const int n = h->P.ncells + 1;
-            hipLaunchKernelGGL((k_scan<true>), dim3(scan_words(n) - 1), dim3(kBlock), 0, h->stream, h->flag,
-                               h->f_count, h->f_start, h->scan_state, n);
+            launch_scan<true>(h->stream, h->flag, h->f_count, h->f_start, h->scan_state, h->P.ncells + 1);
             hipLaunchKernelGGL((k_gather<ND, 1>), dim3(gate_blocks(nf)), dim3(kBlock), 0, h->stream, h->dev, u, v);
         }
         TRY(launch_check(h, "k_sort / k_gather<1>"));

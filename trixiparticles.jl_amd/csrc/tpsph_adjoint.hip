@@ -478,8 +478,8 @@ __device__ __forceinline__ void adj_finish(const DevHandle *handle, const AdjCon
 // wall particles near it, the state equation and gravity.
 // What bounds it: the gathers of the candidates through the L1 (116 bytes of a record, its volume,
 // its weights and its index) at three waves per SIMD.  250k particles in 3D, pullback of one
-// kick: 203 us with the two terms of a pair one after the other, 168 with AdjTarget's; held to
-// 128 registers (four waves) 48 bytes spill and it takes 184.  Candidates from unions staged in
+// kick: 203 us with the two terms of a pair one after the other, 187 with AdjTarget's; held to
+// 128 registers (four waves) 48 bytes spill and it takes 29 us more.  Candidates from unions staged in
 // LDS brick by brick took 239 us (a block of 512 threads, the FP64 chains of two waves per SIMD
 // exposed) and 264 (1,024 threads, which spill). 
 template <int ND, bool ACC>

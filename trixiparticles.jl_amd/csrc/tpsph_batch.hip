@@ -378,8 +378,7 @@ int batch_kick(tpsph_batch *b, double *dv, const double *v, const double *u, boo
     if (nf == 0) return TPSPH_OK;
     if (!linked)
         hipLaunchKernelGGL((k_blinks<ND>), dim3(gate_blocks(nf)), dim3(kBlock), 0, st, h->P, batch_links(b), nf, u);
-    hipLaunchKernelGGL((k_scan<true>), dim3(scan_words(nc + 1) - 1), dim3(kBlock), 0, st, nullptr, h->f_count,
-                       h->f_start, h->scan_state, nc + 1);
+    launch_scan<true>(st, nullptr, h->f_count, h->f_start, h->scan_state, nc + 1);
     hipLaunchKernelGGL((k_bgather<ND>), dim3(gate_blocks(nf)), dim3(kBlock), 0, st, h->P, b->cases, b->fcase,
                        nf, h->f_cell, h->f_rank, h->f_head, h->f_start, h->f_perm, u, v, h->f_mass, h->xs,
                        h->ys, h->zs, h->rec, h->vol);

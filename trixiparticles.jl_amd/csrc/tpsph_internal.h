@@ -887,16 +887,31 @@ __device__ __forceinline__ void scan_tile(int *in, int *out, unsigned long long 
     scan_store(out, base, n, vec, r);
 }
 
-template <bool CLEAR>
-__global__ void __launch_bounds__(kBlock)
+template <bool CLEAR, int THREADS>
+__global__ void __launch_bounds__(THREADS)
     k_scan(const int *flag, int *in, int *out, unsigned long long *state, int n)
 {
     if (skip(flag)) return;
-    __shared__ int s[kBlock / 64];
+    __shared__ int s[THREADS / 64];
     __shared__ int s_tile, s_before;
     if (threadIdx.x == 0) s_tile = (int)atomicAdd(&state[0], 1ull);
     __syncthreads();
-    scan_tile<CLEAR>(in, out, state, n, s_tile, s, s_before);
+    scan_tile<CLEAR, THREADS>(in, out, state, n, s_tile, s, s_before);
+}
+
+// Launches k_scan: tiles of 16,384 ints (1,024 threads) above 2^19.  The prefixes pass from one
+// window of 64 tiles to the next, about 1.5 us each, so the time goes with the number of tiles:
+// 10M cells (1.02M particles in 3D) 128 us in tiles of 4,096, 91 in these (3.5M: 17 and 13); below, the
+// small tiles
+// spread over more compute units.
+template <bool CLEAR>
+inline void launch_scan(hipStream_t st, const int *flag, int *in, int *out, unsigned long long *state, int n)
+{
+    constexpr int kThreads = 1024, kTile = kThreads * kScanItems;
+    if (n > 1 << 19)
+        hipLaunchKernelGGL((k_scan<CLEAR, kThreads>), dim3((n + kTile - 1) / kTile), dim3(kThreads), 0, st, flag, in, out, state, n);
+    else
+        hipLaunchKernelGGL((k_scan<CLEAR, kBlock>), dim3((n + kScanTile - 1) / kScanTile), dim3(kBlock), 0, st, flag, in, out, state, n);
 }
 
 // words of k_scan's state for n ints
@@ -1140,7 +1155,7 @@ int launch_fluid_brick_mixed(tpsph_handle *h, double *dv);
 // Exclusive scan of n ints from in to out on the handle's stream (h->scan_state is clear).
 inline int scan(tpsph_handle *h, const int *flag, int *in, int *out, int n)
 {
-    hipLaunchKernelGGL((k_scan<false>), dim3(scan_words(n) - 1), dim3(kBlock), 0, h->stream, flag, in, out, h->scan_state, n);
+    launch_scan<false>(h->stream, flag, in, out, h->scan_state, n);
     return launch_check(h, "k_scan");
 }
 
