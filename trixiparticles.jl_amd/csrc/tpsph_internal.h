@@ -901,9 +901,8 @@ __global__ void __launch_bounds__(THREADS)
 
 // Launches k_scan: tiles of 16,384 ints (1,024 threads) above 2^19.  The prefixes pass from one
 // window of 64 tiles to the next, about 1.5 us each, so the time goes with the number of tiles:
-// 10M cells (1.02M particles in 3D) 128 us in tiles of 4,096, 91 in these (3.5M: 17 and 13); below, the
-// small tiles
-// spread over more compute units.
+// 10M cells (1.02M particles in 3D) 128 us in tiles of 4,096, 91 in these (3.5M: 17
+// and 13); below, the small tiles spread over more compute units.
 template <bool CLEAR>
 inline void launch_scan(hipStream_t st, const int *flag, int *in, int *out, unsigned long long *state, int n)
 {
