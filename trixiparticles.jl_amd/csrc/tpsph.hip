@@ -148,10 +148,40 @@ __global__ void k_wall_f32(DevParams P, int nw, const double4 *__restrict__ wpos
     wxf[w] = list_f32<ND>(P, x.x, x.y, x.z);
 }
 
+// StateEquationAdaptiveCole: the sound speed of this kick from the nparts block maxima of v.v that
+// k_vmax left, c = min(c_max, max(c_min, sqrt(max v.v) / Ma)), and the constants that depend on
+// it, computed as tpsph_create computes them from a fixed c.  Every block of the gather takes the
+// maximum itself (at most kGateBlocks numbers) and the first one writes dyn for the kernels that
+// follow: a kernel of one block between k_vmax and the gather took 2.2 us and its launch.
+__device__ __forceinline__ void adaptive_sound(const DevHandle *H, DevParams &P, int nparts, bool write)
+{
+    __shared__ double s[kBlock / 64];
+    const double *part = H->vmax_part;
+    double m = 0.0;
+    for (int i = threadIdx.x; i < nparts; i += kBlock) m = fmax(m, part[i]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
+    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = m;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kBlock / 64; w++) m = fmax(m, s[w]);
+    const double c = fmin(P.c_max, fmax(P.c_min, sqrt(m) / P.mach));
+    P.c = c;
+    P.B = P.rho0 * (c * c) / P.gamma;
+    if (write && threadIdx.x == 0) {
+        double *dyn = H->dyn;
+        dyn[0] = c;
+        dyn[1] = P.B;
+        dyn[2] = H->alpha * c * P.h;
+        dyn[3] = P.use_dd ? 2.0 * H->delta * P.h * c : 0.0;
+    }
+}
+
+// nparts: adaptive_sound (MODE 0 with an adaptive sound speed, blocks of kBlock threads), or 0.
 template <int ND, int MODE>
 __device__ __forceinline__ void gather_body(const DevHandle *H, int bx, int nb,
                                             const double *__restrict__ u,
-                                            const double *__restrict__ v)
+                                            const double *__restrict__ v, int nparts = 0)
 {
     DevParams P = H->params();
     int *flag = H->flag, *work = H->bwork, *iperm = H->iperm, *perm = H->f_perm;
@@ -162,7 +192,10 @@ __device__ __forceinline__ void gather_body(const DevHandle *H, int bx, int nb,
     const int *start = H->f_start, *head = H->f_head, *next = H->f_next, *noverflow = H->noverflow;
     int *bcount = H->bcount, *nel = H->nel, *nne = H->counters;
     float4 *xf = H->xf;
-    P = with_sound(P);
+    if (MODE == 0 && nparts > 0)
+        adaptive_sound(H, P, nparts, bx == 0);
+    else
+        P = with_sound(P);
     const int f = *flag;
     // MODE 0 runs first in every kick: it resets the counters of the kernels that follow
     if (MODE == 0 && bx == 0) reset_counters(work, H->sort_ctl);
@@ -249,9 +282,9 @@ __device__ __forceinline__ void gather_body(const DevHandle *H, int bx, int nb,
 
 template <int ND, int MODE>
 __global__ void k_gather(const DevHandle *__restrict__ H, const double *__restrict__ u,
-                         const double *__restrict__ v)
+                         const double *__restrict__ v, int nparts)
 {
-    gather_body<ND, MODE>(H, blockIdx.x, gridDim.x, u, v);
+    gather_body<ND, MODE>(H, blockIdx.x, gridDim.x, u, v, nparts);
 }
 
 // k_links, k_scan and k_gather<1> in one launch, which like theirs returns at once while the flag
@@ -2338,8 +2371,7 @@ __global__ void __launch_bounds__(kBlock)
 // ------------------------------------------------------------------------------------------
 // StateEquationAdaptiveCole: update_speed_of_sound! (wcsph/system.jl:307-320) at the start
 // of every kick.  k_vmax: per-block maxima of v.v over the fluid's current velocities (the
-// caller-order v_ode); k_sound_speed: c = min(c_max, max(c_min, sqrt(max v.v) / Ma)) and the
-// constants that depend on it, computed as tpsph_create computes them from a fixed c.
+// caller-order v_ode), from which the gather takes the sound speed (adaptive_sound).
 // ------------------------------------------------------------------------------------------
 template <int ND>
 __global__ void __launch_bounds__(kBlock)
@@ -2360,31 +2392,6 @@ __global__ void __launch_bounds__(kBlock)
         __syncthreads();
     }
     if (threadIdx.x == 0) part[blockIdx.x] = s[0];
-}
-
-__global__ void __launch_bounds__(kBlock)
-    k_sound_speed(const DevHandle *__restrict__ H, int nparts)
-{
-    const DevParams P = H->params();
-    const double *part = H->vmax_part;
-    double *dyn = H->dyn;
-    const double alpha = H->alpha, delta = H->delta;
-    __shared__ double s[kBlock];
-    double m = 0.0;
-    for (int i = threadIdx.x; i < nparts; i += kBlock) m = fmax(m, part[i]);
-    s[threadIdx.x] = m;
-    __syncthreads();
-    for (int o = kBlock / 2; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) s[threadIdx.x] = fmax(s[threadIdx.x], s[threadIdx.x + o]);
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        const double c = fmin(P.c_max, fmax(P.c_min, sqrt(s[0]) / P.mach));
-        dyn[0] = c;
-        dyn[1] = P.rho0 * (c * c) / P.gamma;
-        dyn[2] = alpha * c * P.h;
-        dyn[3] = P.use_dd ? 2.0 * delta * P.h * c : 0.0;
-    }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2724,7 +2731,8 @@ int update_fluid(tpsph_handle *h, const double *v, const double *u, bool gathere
     if (keep_order) return TPSPH_OK;  // the order and the lists stand, the caller wrote the records
     if (!gathered) {  // else the stage kernel wrote the records of (v, u)
         TimedScope t(h, TPSPH_TIME_GATHER);
-        hipLaunchKernelGGL((k_gather<ND, 0>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream, h->dev, u, v);
+        hipLaunchKernelGGL((k_gather<ND, 0>), dim3(nblocks(nf)), dim3(kBlock), 0, h->stream, h->dev, u, v,
+                           h->dyn ? gate_blocks(nf) : 0);
         TRY(launch_check(h, "k_gather<0>"));
     }
     {
@@ -2732,7 +2740,7 @@ int update_fluid(tpsph_handle *h, const double *v, const double *u, bool gathere
         const bool lists = h->search == TPSPH_SEARCH_LISTS;
         if (!h->f_head) {
             TRY(build_cells<ND>(h, h->flag, nf, u, h->f_cell, h->f_rank, h->f_count, h->f_start, h->f_perm));
-            hipLaunchKernelGGL((k_gather<ND, 2>), dim3(gate_blocks(nf)), dim3(kBlock), 0, h->stream, h->dev, u, v);
+            hipLaunchKernelGGL((k_gather<ND, 2>), dim3(gate_blocks(nf)), dim3(kBlock), 0, h->stream, h->dev, u, v, 0);
         } else if (h->sort_ctl) {
             const int items = std::min((nf + kSortThreads - 1) / kSortThreads, kSortItems);
             const int tiles = h->P.ncells / (kSortThreads * kScanItems) + 1;
@@ -2741,7 +2749,7 @@ int update_fluid(tpsph_handle *h, const double *v, const double *u, bool gathere
         } else {
             hipLaunchKernelGGL((k_links<ND>), dim3(gate_blocks(nf)), dim3(kBlock), 0, h->stream, h->dev, u);
             launch_scan<true>(h->stream, h->flag, h->f_count, h->f_start, h->scan_state, h->P.ncells + 1);
-            hipLaunchKernelGGL((k_gather<ND, 1>), dim3(gate_blocks(nf)), dim3(kBlock), 0, h->stream, h->dev, u, v);
+            hipLaunchKernelGGL((k_gather<ND, 1>), dim3(gate_blocks(nf)), dim3(kBlock), 0, h->stream, h->dev, u, v, 0);
         }
         TRY(launch_check(h, "k_sort / k_gather<1>"));
         if (lists) {
@@ -2770,8 +2778,7 @@ int prepare_impl(tpsph_handle *h, const double *v, const double *u, bool gathere
         TimedScope t(h, TPSPH_TIME_GATHER);
         const int nb = gate_blocks(nf);
         hipLaunchKernelGGL((k_vmax<ND>), dim3(nb), dim3(kBlock), 0, h->stream, nf, h->P.vrows, v, h->vmax_part);
-        hipLaunchKernelGGL((k_sound_speed), dim3(1), dim3(kBlock), 0, h->stream, h->dev, nb);
-        TRY(launch_check(h, "k_vmax/k_sound_speed"));
+        TRY(launch_check(h, "k_vmax"));
         gathered = false;
     }
     TRY(update_fluid<ND>(h, v, u, gathered, keep_order));

@@ -90,7 +90,7 @@ struct DevParams {
     // 3D): a union of up to brick_cap - 1 particles stages, the last record is the far record
     int brick_cap;
     // StateEquationAdaptiveCole: {c, B, av_c, dd2} of the current kick in device memory
-    // (k_sound_speed writes them), or nullptr for the constants above
+    // (the gather writes them), or nullptr for the constants above
     const double *dyn;
     double mach, c_min, c_max;
     // viscosity of the wall model (no-slip): 0 nothing, 1 ArtificialViscosityMonaghan,

@@ -41,7 +41,7 @@ struct BrickSmem32 {
 // What the FP32 pass needs, packed small so that it stays in scalar registers: the pair
 // constants in FP32 and the brick geometry in FP64.  Under StateEquationAdaptiveCole the
 // viscosity and diffusion constants of this kick are read from dyn ({c, B, alpha c h,
-// 2 delta h c}, written by k_sound_speed).
+// 2 delta h c}, written by the gather).
 struct Pair32 {
     float az2, minus_half_h_inv, eps_h2, two_av_c, dd2, rho0;
     int use_visc;
