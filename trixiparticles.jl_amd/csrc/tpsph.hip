@@ -1073,7 +1073,7 @@ struct ListsSmem {
     unsigned short ctab[kCellTab];
     unsigned short near[kBrickCap];  // the targets with walls near their cell
     int row_gb[kBrickMaxRows], row_lds[kBrickMaxRows + 1];
-    short row_x0[kBrickMaxRows], row_x1[kBrickMaxRows];
+    int row_x0[kBrickMaxRows], row_x1[kBrickMaxRows];  // first and last cell along x (a grid has up to 2^20)
     int trow_s[kBrickMaxRows], trow_t[kBrickMaxRows + 1];
     int scan[kListThreads / 64];
     int item, col0, ubase, bad, nnear;
@@ -1213,8 +1213,8 @@ __device__ __forceinline__ int union_list(const DevParams &P, const FluidView &F
                 // conservative half-width: FP32 sqrt, enlarged well past its rounding error
                 const double rx = ((double)(__builtin_amdgcn_sqrtf((float)r2) * 1.000001f) + hs) * P.inv_cs[0];
                 const double last = (double)(P.n[0] - 1);  // cell_1d's clamping
-                const int x0 = max((int)fmin(fmax(xc - rx, 0.0), last), (int)S.row_x0[u]);
-                const int x1 = min((int)fmin(fmax(xc + rx, 0.0), last), (int)S.row_x1[u]);
+                const int x0 = max((int)fmin(fmax(xc - rx, 0.0), last), S.row_x0[u]);
+                const int x1 = min((int)fmin(fmax(xc + rx, 0.0), last), S.row_x1[u]);
                 const unsigned short *ct = S.ctab + u * P.ctab - S.row_x0[u];
                 if (x0 <= x1) {
                     b = ct[x0];
@@ -1469,8 +1469,8 @@ __global__ void __launch_bounds__(kListThreads, 4)
             if (tid < P.maxr) {
                 S.row_gb[tid] = gb;
                 S.row_lds[tid] = lds0;
-                S.row_x0[tid] = (short)x0;
-                S.row_x1[tid] = (short)x1;
+                S.row_x0[tid] = x0;
+                S.row_x1[tid] = x1;
             }
             if (tid == 0) S.row_lds[P.maxr] = tot;
             if (tot > P.brick_cap - 1) tot = INT_MAX;
