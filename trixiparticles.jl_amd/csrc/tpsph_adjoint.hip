@@ -42,10 +42,11 @@ namespace {
 constexpr int kRedBlocks = 256;  // blocks of the deterministic parameter reduction
 constexpr int kAdjLanes = 4;     // lanes per particle of the adjoint passes
 
-// Constants of the parameter derivatives (d dd2 / d delta and the unit gravity direction) and of
-// the fluid pairs: alpha c and beta of the viscosity (zero without) and -1/(2 h), -3/(2 h).
+// Constants of the parameter derivatives (d dd2 / d delta and d (alpha c) / d alpha, zero without
+// the diffusion or the viscosity, and the unit gravity direction) and of the fluid pairs: alpha c
+// and beta of the viscosity (zero without) and -1/(2 h), -3/(2 h).
 struct AdjConsts {
-    double dd2_per_delta;
+    double dd2_per_delta, visc_per_alpha;
     double ghat[3];
     double visc, beta, minus_half_h_inv, minus_3half_h_inv;
 };
@@ -466,7 +467,7 @@ __device__ __forceinline__ void adj_finish(const DevHandle *handle, const AdjCon
     }
     vi[ND] = ACC ? vi[ND] + T.rhob : T.rhob;
     // half of both terms of every pair (see AdjTarget)
-    const double alpha = 0.5 * P.c * T.alpha, delta = 0.5 * K.dd2_per_delta * T.delta;
+    const double alpha = 0.5 * K.visc_per_alpha * T.alpha, delta = 0.5 * K.dd2_per_delta * T.delta;
     ti[0] = ACC ? ti[0] + alpha : alpha;
     ti[1] = ACC ? ti[1] + delta : delta;
     ti[2] = ACC ? ti[2] + gpart : gpart;
@@ -606,6 +607,7 @@ AdjConsts adj_consts(const tpsph_handle *h)
     for (int d = 0; d < 3; d++) g2 += P.g[d] * P.g[d];
     const double g = std::sqrt(g2);
     for (int d = 0; d < 3; d++) K.ghat[d] = g > 0.0 ? P.g[d] / g : 0.0;
+    K.visc_per_alpha = P.use_visc ? P.c : 0.0;
     K.visc = P.use_visc ? P.alpha * P.c : 0.0;
     K.beta = P.use_visc ? P.beta : 0.0;
     K.minus_half_h_inv = -0.5 * P.h_inv;
