@@ -1064,7 +1064,14 @@ struct ListsArgs {
     }
 };
 
+// ND, WIDE: cell rows of a target along y (kRows) and cell offsets of a union (kCellTab).  3D: bricks
+// stage with one or two cell divisions (at most 144 union rows x 42 cells), and, WIDE, with
+// DensityDiffusionAntuono's smaller bricks also with three (256 x 42, and one block per compute
+// unit instead of two); 2D: with one to four (42 x 84).
+template <int ND, bool WIDE>
 struct ListsSmem {
+    static constexpr int kRows = ND == 2 ? 9 : WIDE ? 7 : 5;
+    static constexpr int kCellTab = ND == 2 ? 42 * 84 : WIDE ? 256 * 42 : 144 * 42;
     // the last entries of every thread's list, slot-major: 64 lanes write 64 banks whatever
     // slots they are at (aligned to a wave's ring: the slot is or-ed into the address)
     alignas(kListRing * 128) unsigned short ring[kListThreads / 64][kListRing * 64];
@@ -1104,7 +1111,8 @@ __device__ __forceinline__ int lists_scan(int value, int *s, int &total)
 }
 
 // Target `k` of the brick: its sorted index.
-__device__ __forceinline__ int lists_target(const ListsSmem &S, int nrows, int k)
+template <typename Smem>
+__device__ __forceinline__ int lists_target(const Smem &S, int nrows, int k)
 {
     const int r = bsearch_le(S.trow_t, nrows, k);
     return S.trow_s[r] + (k - S.trow_t[r]);
@@ -1112,9 +1120,9 @@ __device__ __forceinline__ int lists_target(const ListsSmem &S, int nrows, int k
 
 // The FP32 positions and the cell offsets of the union whose rows are in S (n records of the
 // cell-sorted points with cell offsets `start`); uidx: also their sorted indices.
-template <int ND>
+template <int ND, typename Smem>
 __device__ __forceinline__ void stage_union(const DevParams &P, const int *__restrict__ start,
-                                            const float4 *__restrict__ xf, ListsSmem &S, int n,
+                                            const float4 *__restrict__ xf, Smem &S, int n,
                                             int uy0, int uz0, int nuy, int *__restrict__ uidx)
 {
     // four records per thread at a time: their row searches and loads overlap
@@ -1174,13 +1182,13 @@ __device__ __forceinline__ void ring_rows(const unsigned short *ring, int first,
 // to memory when it fills; a wall list is short and goes to memory as it is found), which
 // grows on a hit only.  Returns the number of entries (which may exceed the capacity: the
 // surplus is not written).
-template <int ND, bool WALL>
+template <int ND, bool WALL, typename Smem>
 __device__ __forceinline__ int union_list(const DevParams &P, const FluidView &F,
-                                          const ListsArgs &A, ListsSmem &S, int s, bool active,
+                                          const ListsArgs &A, Smem &S, int s, bool active,
                                           int col, int self, double xa, double ya, double za,
                                           int c1, int c2, int uy0, int uz0, int nuy)
 {
-    constexpr int kRows = ND == 3 ? 5 : 9;  // cell rows along y
+    constexpr int kRows = Smem::kRows;
     const float4 xaf = F.xf[s];
     const double hs = WALL ? P.hs_list_wall : P.hs_list_fluid;
     const float out2 = WALL ? P.wlist_out2 : P.list_out2;
@@ -1279,9 +1287,9 @@ __device__ __forceinline__ int union_list(const DevParams &P, const FluidView &F
 
 // The lists of one brick's targets over the fluid (its union is staged); lists the targets with
 // walls near their cell.  S.bad is set when a list overflowed (the brick then does not stage).
-template <int ND>
+template <int ND, typename Smem>
 __device__ __forceinline__ void brick_lists(const DevParams &P, const FluidView &F,
-                                            const WallView &Wv, const ListsArgs &A, ListsSmem &S,
+                                            const WallView &Wv, const ListsArgs &A, Smem &S,
                                             int ntargets, int nrows, int uy0, int uz0, int nuy)
 {
     for (int base = 0; base < ntargets; base += kListThreads) {
@@ -1313,10 +1321,10 @@ __device__ __forceinline__ void brick_lists(const DevParams &P, const FluidView 
 }
 
 // The wall lists of the targets in S.near, the walls' union staged.
-template <int ND>
+template <int ND, typename Smem>
 __device__ __forceinline__ void brick_wall_lists(const DevParams &P, const FluidView &F,
                                                  const WallView &Wv, const ListsArgs &A,
-                                                 ListsSmem &S, int nrows, int uy0, int uz0,
+                                                 Smem &S, int nrows, int uy0, int uz0,
                                                  int nuy, bool staged)
 {
     for (int base = 0; base < S.nnear; base += kListThreads) {
@@ -1348,10 +1356,10 @@ __device__ __forceinline__ void brick_wall_lists(const DevParams &P, const Fluid
 
 // Int lists of the targets of a brick that does not stage, one thread per target.
 // walls: also their wall lists and headers (not when brick_lists has written them).
-template <int ND>
+template <int ND, typename Smem>
 __device__ __forceinline__ void brick_int_lists(const DevParams &P, const FluidView &F,
                                                 const WallView &Wv, const ListsArgs &A,
-                                                const ListsSmem &S, int ntargets, int nrows,
+                                                const Smem &S, int ntargets, int nrows,
                                                 bool walls)
 {
     for (int k = threadIdx.x; k < ntargets; k += kListThreads) {
@@ -1391,9 +1399,9 @@ __device__ __forceinline__ void brick_int_lists(const DevParams &P, const FluidV
 // entry) is not written any more; the walls of a brick are staged the same way, for the
 // targets near one only (four lanes per target on global memory: 157 us, here 40).  Bricks,
 // unions and lists took 860 us and five launches, four lanes per target 720, this form 495.
-// Two blocks of 512 threads share a compute unit (76 KB each).
-template <int ND>
-__global__ void __launch_bounds__(kListThreads, 4)
+// Two blocks of 512 threads share a compute unit (78 KB each; WIDE: one of 87 KB).
+template <int ND, bool WIDE>
+__global__ void __launch_bounds__(kListThreads, WIDE ? 2 : 4)
     k_brick_lists(const DevHandle *__restrict__ H, int nwall, bool adami)
 {
     const bool rebuild = !skip(H->flag);
@@ -1410,7 +1418,7 @@ __global__ void __launch_bounds__(kListThreads, 4)
     const int block = (int)blockIdx.x - nwall, nblocks = (int)gridDim.x - nwall;
     const WallView Wv = H->walls();
     const ListsArgs A(*H);
-    __shared__ ListsSmem S;
+    __shared__ ListsSmem<ND, WIDE> S;
     const int tid = threadIdx.x;
     const int ne = A.nne[0];
     const int nuy = P.bc[1] + 2 * P.ur[1];
@@ -2721,6 +2729,13 @@ bool adami_in_lists(const tpsph_handle *h)
     return h->search == TPSPH_SEARCH_LISTS && !h->P.summation && !h->timing;
 }
 
+// Whether the bricks stage: the union rows of a brick of full size fit (small fluids have smaller
+// bricks, but whether a call is accepted does not depend on the number of particles).
+bool brick_rows_ok(const DevParams &P) { return P.full_rows <= kBrickMaxRows; }
+
+// Whether the list build needs its larger tables.
+bool wide_lists(const DevParams &P) { return P.nd == 3 && P.lr[1] > 2 && brick_rows_ok(P); }
+
 // Fluid cell list (rebuilt only when flagged) + cell-sorted gather of (v, u).
 template <int ND>
 int update_fluid(tpsph_handle *h, const double *v, const double *u, bool gathered,
@@ -2756,7 +2771,8 @@ int update_fluid(tpsph_handle *h, const double *v, const double *u, bool gathere
             const int gb = std::max(1, std::min(h->nbricks, 2 * h->n_cu));
             // as many blocks for the walls as the Adami pass has lanes for, at most one turn
             const int gw = (int)std::min<int64_t>((kWallLanes * (int64_t)h->nw + kListThreads - 1) / kListThreads, 2 * h->n_cu);
-            hipLaunchKernelGGL((k_brick_lists<ND>), dim3(gw + gb), dim3(kListThreads), 0, h->stream, h->dev, gw, adami_in_lists(h));
+            const auto build = wide_lists(h->P) ? k_brick_lists<ND, ND == 3> : k_brick_lists<ND, false>;
+            hipLaunchKernelGGL(build, dim3(gw + gb), dim3(kListThreads), 0, h->stream, h->dev, gw, adami_in_lists(h));
             TRY(launch_check(h, "k_brick_lists"));
         }
         // the fluid kernel of this kick lowers the flag
@@ -3001,6 +3017,26 @@ int tpsph::derive_params(const tpsph_params *params, int nf, int nw, const doubl
             if (nd == 3 && d == 0) P.bc[d] = std::max(1, P.bc[d] * 11 / 12);
             if (grad && d >= 1) P.bc[d] = std::max(1, P.bc[d] - 1);
         }
+        // union rows: cells within the list radius of the brick box (grown by the margin)
+        const double rl = R + 2.0 * P.half_skin + margin, reach = R + P.hs_list_fluid;
+        auto union_rows = [&] {
+            int rows = 1;
+            for (int d = 1; d < nd; d++) rows *= P.bc[d] + 2 * P.ur[d];
+            return rows;
+        };
+        auto union_cells = [&] { return P.bc[0] + 2 * ((int)std::floor((rl + 4.0 * margin) / P.cs[0]) + 1) + 2; };
+        for (int d = 0; d < 3; d++) {
+            const bool yz = d >= 1 && d < nd;
+            P.ur[d] = yz ? (int)std::ceil(rl / P.cs[d]) + 1 : 0;
+            P.lr[d] = yz ? (int)std::ceil(reach / P.cs[d]) : 0;  // of a target's pencils
+        }
+        P.full_rows = union_rows();
+        // (they do not fit only where the margin is no longer small against a cell: a box more
+        // than 1e12 R from the origin)
+        if (P.full_rows * union_cells() > (nd == 2 ? ListsSmem<2, false>::kCellTab
+                                           : P.lr[1] > 2 ? ListsSmem<3, true>::kCellTab
+                                                         : ListsSmem<3, false>::kCellTab))
+            P.full_rows = INT_MAX;
         // A small fluid in full bricks leaves most of the chip without one: its bricks shrink
         // until they are about as many as the device takes at a time (3/4 of it: the bricks on
         // the surface are not full), down to 50 targets.  Beyond that a second turn costs
@@ -3026,30 +3062,12 @@ int tpsph::derive_params(const tpsph_params *params, int nf, int nw, const doubl
             nb *= P.nb[d];
         }
         nbricks = (int)nb;
-        // union rows: cells within the list radius of the brick box (grown by the margin)
-        const double rl = R + 2.0 * P.half_skin + margin;
-        int rows = 1;
-        for (int d = 0; d < 3; d++) {
-            P.ur[d] = (d >= 1 && d < nd) ? (int)std::ceil(rl / P.cs[d]) + 1 : 0;
-            if (d >= 1 && d < nd) rows *= P.bc[d] + 2 * P.ur[d];
-        }
-        P.maxr = rows;
-        const double reach = R + P.hs_list_fluid;  // of a target's pencils
-        for (int d = 0; d < 3; d++)
-            P.lr[d] = (d >= 1 && d < nd) ? (int)std::ceil(reach / P.cs[d]) : 0;
-        P.ctab = P.bc[0] + 2 * ((int)std::floor((rl + 4.0 * margin) / P.cs[0]) + 1) + 2;
+        P.maxr = union_rows();
+        P.ctab = union_cells();
         P.rl_union2 = (rl + margin) * (rl + margin);
         P.hs_union = margin;
     }
     return TPSPH_OK;
-}
-
-// Whether the bricks stage: the union rows of a brick, their cell offsets and the rows of a
-// target's list fit the tables of the list build.
-static bool brick_rows_ok(const DevParams &P)
-{
-    const int rows = (2 * P.lr[1] + 1) * (P.nd == 3 ? 2 * P.lr[2] + 1 : 1);
-    return P.maxr <= kBrickMaxRows && P.maxr * P.ctab <= kCellTab && rows <= (P.nd == 3 ? 25 : 9);
 }
 
 int tpsph::validate(const tpsph_params *p, int64_t nf, int64_t nw, const double *fm, const double *wx,

@@ -37,7 +37,6 @@ constexpr int kBrickMaxRows = 256;    // union rows per brick (one scan block)
 constexpr int kHeadCount = 11, kHeadCountMask = (1 << 13) - 1, kHeadWalls = 1 << 24;
 constexpr int kListThreads = 512;     // threads of the list build, one per target
 constexpr int kListRing = 32;         // entries a thread of it holds before it writes 16 of them
-constexpr int kCellTab = 5120;        // cell offsets of a union in LDS (at most 121 rows x 40)
 constexpr int kGateBlocks = 1024;     // grid-stride kernels behind the rebuild flag: a small
                                       // grid keeps the launch cheap when the flag is down
 constexpr int kCounters = 7;          // tpsph_handle::counters
@@ -82,7 +81,7 @@ struct DevParams {
     int bc[3], nb[3];
     // union rows of a brick: cells beyond the brick along y and z, rows per brick, and the
     // radius (list radius + margin) and cell growth (margin) of the union
-    int ur[3], maxr;
+    int ur[3], maxr, full_rows;  // full_rows: the rows of a brick of full size
     int lr[3];  // cells within the list radius of a cell along y and z (rows of a target's list)
     int ctab;   // cell offsets per union row (cells of its x-range and one more, at most)
     double rl_union2, hs_union;
