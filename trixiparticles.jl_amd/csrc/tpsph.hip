@@ -3230,7 +3230,9 @@ int put_handle(tpsph_handle *h)
     d.noverflow = h->search == TPSPH_SEARCH_LISTS ? h->counters + 3 : nullptr;
     d.bwork = h->bwork; d.bfall = h->bfall; d.bhead = h->bhead; d.nbr16 = h->nbr16; d.thead = h->thead;
     d.uidx_cap = (int)h->uidx_cap; d.ls = h->ls; d.cap_f = h->cap_f; d.cap_w = h->cap_w;
-    d.anbr = h->anbr; d.acnt = h->acnt; d.wactive = h->wactive; d.lw = h->lw; d.cap_a = h->cap_a;
+    // (without fluid no list is ever built: the walls walk the cells, which are empty)
+    d.wactive = h->nf > 0 ? h->wactive : nullptr;
+    d.anbr = h->anbr; d.acnt = h->acnt; d.lw = h->lw; d.cap_a = h->cap_a;
     d.dyn = h->dyn; d.ddgrad = h->ddgrad; d.vmax_part = h->vmax_part; d.sum_rho = h->sum_rho;
     d.alpha = h->params.alpha; d.delta = h->params.delta;
     hipLaunchKernelGGL((k_put_handle), dim3(1), dim3(1), 0, h->stream, d, h->dev);
@@ -3405,6 +3407,8 @@ int noalloc_kick(tpsph_handle *h, unsigned char *base, size_t *bytes, const doub
     // what must start at zero (or NaN): histograms, the wall-near flags, the SoA padding
     hipLaunchKernelGGL((k_fill_i32), dim3(gate_blocks(nc + 1)), dim3(kBlock), 0, st, h->f_count, 0, nc + 1);
     hipLaunchKernelGGL((k_fill_i32), dim3(gate_blocks(nc + 1)), dim3(kBlock), 0, st, w_count, 0, nc + 1);
+    if (nf == 0)  // no cell list is built then
+        hipLaunchKernelGGL((k_fill_i32), dim3(gate_blocks(nc + 1)), dim3(kBlock), 0, st, h->f_start, 0, nc + 1);
     hipLaunchKernelGGL((k_fill_u8), dim3(gate_blocks(nc)), dim3(kBlock), 0, st, h->wall_near, (unsigned char)0, nc);
     for (double *a : {h->xs, h->ys, h->zs})
         hipLaunchKernelGGL((k_fill_f64), dim3(gate_blocks(nf + kPad)), dim3(kBlock), 0, st, a, nan, nf + kPad);
@@ -3673,6 +3677,10 @@ int tpsph_create(const tpsph_params *params, int64_t n_fluid, int64_t n_wall,
         CTRY(hip_fill(h, a, (size_t)nw + kPad));
     if (hipMemset(h->f_count, 0, ((size_t)ncells + 1) * sizeof(int)) != hipSuccess) {
         h->last_error = "clearing the cell counts failed";
+        return cleanup_fail(TPSPH_ERR_HIP);
+    }
+    if (nf == 0 && hipMemset(h->f_start, 0, ((size_t)ncells + 1) * sizeof(int)) != hipSuccess) {
+        h->last_error = "clearing the cell offsets failed";
         return cleanup_fail(TPSPH_ERR_HIP);
     }
     if (hipMemset(h->wall_near, 0, (size_t)ncells) != hipSuccess) {
