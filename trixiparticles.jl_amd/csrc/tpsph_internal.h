@@ -73,7 +73,7 @@ struct DevParams {
     double half_skin, half_skin2;
     // Verlet lists: squared list radii and the cell growth that makes the pencils reach them
     double rl2_fluid, rl2_wall, hs_list_fluid, hs_list_wall;
-    // FP32 test of the list builds (positions relative to lo inside the grid box box[d]): a
+    // FP32 test of the list builds (positions relative to lo, the grid box is box[d] long): a
     // squared FP32 distance above list_out2 (walls: wlist_out2) is surely beyond the list radius
     double box[3];
     float list_out2, wlist_out2;
