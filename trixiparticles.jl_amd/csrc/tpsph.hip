@@ -293,12 +293,18 @@ __global__ void k_gather(const DevHandle *__restrict__ H, const double *__restri
 // phases only, so the waits end whatever number of blocks the device holds at a time.  What a
 // phase wrote is released by its block at device scope and acquired by the waiting one.
 //
-// A kick without a rebuild saves two launches, a rebuild costs more than by three launches (45k
-// particles in 2D: 29 us against 21, each phase waits for tickets, counts and cold caches).
-// us per pass, three kernels -> this one: kick of 2k in 2D 29.9 -> 24.0, of 48k in 3D 56.9 ->
-// 53.6, two steps of 128k with SummationDensity 1290 -> 1248; two steps of 45k in 2D with a
-// rebuild at four of ten kicks 557 -> 581.  Larger fluids (kSortMax) take the three kernels:
-// their rebuild needs the whole device (1.02M particles: 350 us more with 128 blocks).
+// A kick without a rebuild saves two launches, one with a rebuild is longer than with three kernels
+// (each phase waits for tickets, counts and cold caches, and 64 blocks scan the cells).  us per
+// kick, three kernels -> this one, at rest and rebuilding every time, over the cells of the grid:
+//                      0.2M                     1M            2M            4M            20M
+//   1,800 in 2D    21.2 -> 14.2, 41 -> 48    46 -> 51      50 -> 62      55 -> 84     113 -> 256
+//   45k in 2D      22.1 -> 17.7, 58 -> 67    64 -> 70      66 -> 83      73 -> 105    127 -> 270
+//   48k in 3D      33.5 -> 29.7, 101 -> 111  107 -> 115    122 -> 137    127 -> 158   183 -> 323
+//   125k in 3D     60.9 -> 56.6, 154 -> 167  152 -> 165    155 -> 177    160 -> 198   224 -> 372
+// (at rest the cells do not matter).  The line lies at three turns of the blocks over the scan's
+// tiles, kSortMaxCells: there a rebuild costs what four kicks without one save.  Larger fluids
+// (kSortMax) take the three kernels too: their rebuild needs the whole device (1.02M particles:
+// 350 us more with 128 blocks).
 template <int ND>
 __global__ void __launch_bounds__(kSortThreads)
     k_sort(const DevHandle *__restrict__ H, const double *__restrict__ u,
@@ -3595,7 +3601,8 @@ int tpsph_create(const tpsph_params *params, int64_t n_fluid, int64_t n_wall,
         P.dyn = h->dyn;
     }
     CTRY(dalloc(h, &h->scan_state, (size_t)scan_words((int)ncells + 1)));
-    if (h->search == TPSPH_SEARCH_LISTS && nf <= kSortMax) CTRY(dalloc(h, &h->sort_ctl, kSortCtl));
+    if (h->search == TPSPH_SEARCH_LISTS && nf <= kSortMax && ncells <= kSortMaxCells)
+        CTRY(dalloc(h, &h->sort_ctl, kSortCtl));
     CTRY(dalloc(h, &h->f_cell, nf));
     CTRY(dalloc(h, &h->f_rank, nf));
     CTRY(dalloc(h, &h->f_perm, nf));

@@ -44,7 +44,8 @@ constexpr int kSortLine = 32;           // k_sort: ticket and finished items of 
 constexpr int kSortCtl = 3 * kSortLine; // of 128 bytes each
 constexpr int kSortThreads = 1024;
 constexpr int kSortItems = 64;          // its blocks
-constexpr int kSortMax = 1 << 17;       // fluids it takes
+constexpr int kSortMax = 1 << 17;       // fluids it takes, in grids of at most this many cells
+constexpr int kSortMaxCells = 3 << 20;
 constexpr int kPad = 4;               // NaN entries after the SoA coordinate arrays
 
 // message of the last failed tpsph_create (tpsph_last_error(NULL))
