@@ -3378,6 +3378,8 @@ int noalloc_kick(tpsph_handle *h, unsigned char *base, size_t *bytes, const doub
     const int nc = h->P.ncells;
     ScratchLayout L{base};
     h->flag = L.take<int>(1);
+    // a word per 2,048 cells, which the scan once kept here: the sizes that fit are an interface
+    L.take<int>(((size_t)nc + 1 + 2047) / 2048 + 1);
     h->f_cell = L.take<int>(nf);
     h->f_rank = L.take<int>(nf);
     h->f_perm = L.take<int>(nf);
