@@ -3048,7 +3048,9 @@ int tpsph::derive_params(const tpsph_params *params, int nf, int nw, const doubl
         // 9,537 / 31,250 / 48,778 in 3D 31.6 / 33.3 / 35.7 against 19.5 / 27.6 / 29.0; bricks of
         // half the size at 45,000 and 48,778: 21.0 and 38.5.  The order of every sum is
         // the same whatever the bricks.
-        if (volume > 0.0 && slots > 0) {
+        // (Not for more particles than that many bricks hold: masses that do not fit the spacing
+        // would ask for bricks of single cells, whose unions add up beyond 32 bits.)
+        if (volume > 0.0 && slots > 0 && nf <= 0.75 * slots * P.brick_cap) {
             double cells = 1.0, cell_volume = 1.0;
             for (int d = 0; d < nd; d++) {
                 cells *= P.bc[d];
