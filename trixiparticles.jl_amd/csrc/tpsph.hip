@@ -1828,7 +1828,10 @@ __device__ __forceinline__ int2 union_share(const int *__restrict__ uidx, int fi
 // 299 -> 247 us per launch, and with uidx in place of searches of the union rows, the list
 // layout of list_place and the target headers read ahead 222 us.
 // Bricks: the first gridDim.x in the order of the blocks, then from the work counter (which
-// k_gather<0> and the stage kernel reset).
+// k_gather<0> and the stage kernel reset).  A brick that does not stage takes several times as long
+// as one that does, so its block claims none before it is done: held by their blocks meanwhile,
+// the other bricks made the tail of the launch (128k particles in 3D at h = 1.5 dx, 144 of 396
+// bricks: 282 us per launch with the next ones claimed ahead, 155 so).
 // VISC: visc_mode(P), the viscosity form of the pair loop.  ANT: DensityDiffusionAntuono
 // (P.ddgrad), whose gradients are staged beside the records.  SUM: SummationDensity
 // (pressure slot staged as p / rho^2, no density rate, dv of ND rows).
@@ -1861,6 +1864,7 @@ __global__ void __launch_bounds__(kBrickThreads)
         }
         S.vol[kFarSlot] = 0.0;
     }
+    auto claim = [&] { return (int)gridDim.x + atomicAdd(A.work, 1); };
     auto read_head = [&](int item, int k) {  // lane 0 of wave 0
         S.head[k] = item < ne ? A.bhead[item] : make_int4(-1, -1, 0, 0);
     };
@@ -1869,7 +1873,7 @@ __global__ void __launch_bounds__(kBrickThreads)
     {
         UnionShare<ND, ANT, SUM> share;
         share.load(P, F, union_share(A.uidx, hd.w, nstage));
-        if (tid == 0) read_head((int)gridDim.x < ne ? (int)gridDim.x + atomicAdd(A.work, 1) : ne, 1);
+        if (tid == 0) read_head((int)gridDim.x < ne && hd.z <= kFarSlot ? claim() : ne, 1);
         share.store(S, nstage);
     }
     // Four lanes per target: lane q of target i takes the entries q, q + 4, ... of its list;
@@ -1890,12 +1894,18 @@ __global__ void __launch_bounds__(kBrickThreads)
     ushort4 cur4 = l4[(size_t)q * A.ls + column(hd, hd.x)];
     __syncthreads();
     for (int cur = 0;; cur ^= 1) {
+        const bool staged = hd.z <= kFarSlot;
+        if (!staged) {
+            brick_from_global<ND, SUM>(P, F, A, hd.x, hd.y);
+            if (tid == 0) read_head(claim(), cur ^ 1);
+            __syncthreads();
+        }
         const int4 nx = S.head[cur ^ 1];
         const int nx_stage = nx.z <= kFarSlot ? nx.z : 0;
         const int2 us = union_share(A.uidx, nx.w, nx_stage);
         int item = ne;  // the brick after the next one: its number arrives during the pair loop
-        if (tid == 0 && nx.x >= 0) item = (int)gridDim.x + atomicAdd(A.work, 1);
-        if (hd.z <= kFarSlot) {
+        if (tid == 0 && nx.x >= 0 && nx.z <= kFarSlot) item = claim();
+        if (staged) {
             for (int base = hd.x; base < hd.y; base += kBrickThreads / kL) {
                 const bool active = base + tid / kL < hd.y;
                 const int col = column(hd, base);
@@ -1950,8 +1960,6 @@ __global__ void __launch_bounds__(kBrickThreads)
                     if constexpr (!SUM) o[ND] = drho;
                 }
             }
-        } else {
-            brick_from_global<ND, SUM>(P, F, A, hd.x, hd.y);
         }
         if (nx.x < 0) break;  // uniform: no brick after this one
         // (a load without a branch around it keeps the share in registers; a brick that does
