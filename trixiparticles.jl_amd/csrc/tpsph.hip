@@ -400,7 +400,7 @@ __device__ __forceinline__ void adami_pass(const DevHandle *H, int bx, int nb)
     const DevParams P = with_sound(H->params());
     const FluidView F = H->fluid();
     const int *active = H->wactive, *acnt = H->acnt;
-    const int na = active ? H->counters[1] : P.nw;
+    const int na = active ? H->counters[kCountActive] : P.nw;
     // the loop bound is uniform per group of lanes, so the partners shuffle together
     for (int g = (bx * (int)blockDim.x + (int)threadIdx.x) / kWallLanes; g < na; g += nb * (int)blockDim.x / kWallLanes) {
         const int w = active ? active[g] : g;
@@ -855,7 +855,7 @@ __device__ __forceinline__ void wall_lists_body(const DevHandle *H, int bx, int 
     const FluidView F = H->fluid();
     const double4 *wpos = H->wpos;
     const int lw = H->lw, cap = H->cap_a;
-    int *nbr = H->anbr, *cnt = H->acnt, *active = H->wactive, *nactive = H->counters + 1;
+    int *nbr = H->anbr, *cnt = H->acnt, *active = H->wactive, *nactive = H->counters + kCountActive;
     for (int base = bx * kListThreads; base < P.nw; base += gx * kListThreads) {  // uniform
         const int w = base + (int)threadIdx.x;
         if (w < P.nw) {
@@ -1048,7 +1048,7 @@ __global__ void __launch_bounds__(kBlock)
 // The list build's part of the handle (see tpsph_handle).
 struct ListsArgs {
     const int *nel;
-    int *nne;  // counters: [0] bricks ... [6] work counter
+    int *nne;  // counters (kCountBricks ...)
     int *bcount, *ord, *tbase, *uidx;
     int uidx_cap;
     int4 *bhead;
@@ -1352,7 +1352,7 @@ __device__ __forceinline__ void brick_wall_lists(const DevParams &P, const Fluid
         }
         if (n != 0) {
             A.thead[col].y |= kHeadWalls;
-            if (A.wtargets) A.wtargets[atomicAdd(&A.nne[2], 1)] = col;
+            if (A.wtargets) A.wtargets[atomicAdd(&A.nne[kCountWallTargets], 1)] = col;
         }
     }
 }
@@ -1369,7 +1369,7 @@ __device__ __forceinline__ void brick_int_lists(const DevParams &P, const FluidV
         const int s = lists_target(S, nrows, k), col = S.col0 + k;
         build_list<ND, false>(P, F, Wv, s, col, A.ls, A.cap_f, A.nbr, A.cnt);
         // an overflowed list walks the cells, which need the SoA coordinates every kick
-        if (A.cnt[col] < 0) atomicAdd(&A.nne[3], 1);
+        if (A.cnt[col] < 0) atomicAdd(&A.nne[kCountOverflow], 1);
         A.tbase[col] = -1;
         if (!walls) continue;
         A.ord[col] = s;
@@ -1379,7 +1379,7 @@ __device__ __forceinline__ void brick_int_lists(const DevParams &P, const FluidV
             const int c2 = (ND == 3) ? cell_1d(F.z[s], P.lo[2], P.inv_cs[2], P.n[2]) : 0;
             if (A.wall_near[c0 + P.n[0] * (c1 + P.n[1] * c2)]) {
                 build_list<ND, true>(P, F, Wv, s, col, A.ls, A.cap_w, A.wnbr, A.wcnt);
-                if (A.wtargets && A.wcnt[col] != 0) A.wtargets[atomicAdd(&A.nne[2], 1)] = col;
+                if (A.wtargets && A.wcnt[col] != 0) A.wtargets[atomicAdd(&A.nne[kCountWallTargets], 1)] = col;
             } else {
                 A.wcnt[col] = 0;
             }
@@ -1402,7 +1402,10 @@ __device__ __forceinline__ void brick_int_lists(const DevParams &P, const FluidV
 // entry) is not written any more; the walls of a brick are staged the same way, for the
 // targets near one only (four lanes per target on global memory: 157 us, here 40).  Bricks,
 // unions and lists took 860 us and five launches, four lanes per target 720, this form 495.
-// Two blocks of 512 threads share a compute unit (78 KB each; WIDE: one of 87 KB).
+// Two blocks of 512 threads share a compute unit (78 KB each; WIDE: one of 87 KB).  A brick takes
+// its columns, its part of uidx and the block's next brick from three counters, each on a line of
+// its own: on one line they bounded the build of many bricks of few targets (700k particles in
+// 2D: 96 -> 74 us, with one in a hundred dispersed as spray 235 -> 150).
 template <int ND, bool WIDE>
 __global__ void __launch_bounds__(kListThreads, WIDE ? 2 : 4)
     k_brick_lists(const DevHandle *__restrict__ H, int nwall, bool adami)
@@ -1423,7 +1426,7 @@ __global__ void __launch_bounds__(kListThreads, WIDE ? 2 : 4)
     const ListsArgs A(*H);
     __shared__ ListsSmem<ND, WIDE> S;
     const int tid = threadIdx.x;
-    const int ne = A.nne[0];
+    const int ne = A.nne[kCountBricks];
     const int nuy = P.bc[1] + 2 * P.ur[1];
     for (int turn = block;; ) {
         if (turn >= ne) break;  // uniform over the block
@@ -1488,11 +1491,11 @@ __global__ void __launch_bounds__(kListThreads, WIDE ? 2 : 4)
         }
         if (tid == 0) {
             A.bcount[b] = 0;  // clear for the next rebuild
-            S.col0 = atomicAdd(&A.nne[4], ntargets);
-            S.ubase = tot < INT_MAX ? atomicAdd(&A.nne[5], tot) : 0;
+            S.col0 = atomicAdd(&A.nne[kCountTargets], ntargets);
+            S.ubase = tot < INT_MAX ? atomicAdd(&A.nne[kCountRecords], tot) : 0;
             S.bad = 0;
             S.nnear = 0;
-            S.item = atomicAdd(&A.nne[6], 1);
+            S.item = atomicAdd(&A.nne[kCountClaims], 1);
         }
         __syncthreads();
         const int next = nblocks + S.item;
@@ -2006,7 +2009,7 @@ __global__ void __launch_bounds__(kBlock)
     const DevParams P = with_sound(H->params());
     const FluidView F = H->fluid();
     const WallView Wv = H->walls();
-    const int *ord = H->ord, *wtargets = H->wtargets, *nwtargets = H->counters + 2;
+    const int *ord = H->ord, *wtargets = H->wtargets, *nwtargets = H->counters + kCountWallTargets;
     const int *wnbr = H->wnbr, *wcnt = H->wcnt;
     const int ls = H->ls;
     constexpr int kLanes = 4;
@@ -3240,7 +3243,7 @@ int put_handle(tpsph_handle *h)
     d.snap = h->snap; d.mass = h->f_mass; d.wall_near = h->wall_near;
     d.bcount = h->bcount; d.nel = h->nel; d.ord = h->ord; d.tbase = h->tbase; d.uidx = h->uidx;
     d.nbr = h->nbr; d.cnt = h->cnt; d.wnbr = h->wnbr; d.wcnt = h->wcnt; d.wtargets = h->wtargets;
-    d.noverflow = h->search == TPSPH_SEARCH_LISTS ? h->counters + 3 : nullptr;
+    d.noverflow = h->search == TPSPH_SEARCH_LISTS ? h->counters + kCountOverflow : nullptr;
     d.bwork = h->bwork; d.bfall = h->bfall; d.bhead = h->bhead; d.nbr16 = h->nbr16; d.thead = h->thead;
     d.uidx_cap = (int)h->uidx_cap; d.ls = h->ls; d.cap_f = h->cap_f; d.cap_w = h->cap_w;
     // (without fluid no list is ever built: the walls walk the cells, which are empty)

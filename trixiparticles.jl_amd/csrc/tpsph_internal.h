@@ -39,7 +39,12 @@ constexpr int kListThreads = 512;     // threads of the list build, one per targ
 constexpr int kListRing = 32;         // entries a thread of it holds before it writes 16 of them
 constexpr int kGateBlocks = 1024;     // grid-stride kernels behind the rebuild flag: a small
                                       // grid keeps the launch cheap when the flag is down
-constexpr int kCounters = 7;          // tpsph_handle::counters
+// tpsph_handle::counters, rebuilt with the lists, a line of 128 bytes each: non-empty bricks, active
+// wall particles, fluid particles with wall candidates (wtargets), overflowed lists, and the list
+// build's targets and union records given to bricks and bricks claimed so far
+constexpr int kCountBricks = 0, kCountActive = 32, kCountWallTargets = 64, kCountOverflow = 96,
+              kCountTargets = 128, kCountRecords = 160, kCountClaims = 192, kCounters = 224;
+static_assert(kCounters <= kBlock, "cleared by the threads of a block");
 constexpr int kSortLine = 32;           // k_sort: ticket and finished items of two phases, a line
 constexpr int kSortCtl = 3 * kSortLine; // of 128 bytes each
 constexpr int kSortThreads = 1024;
@@ -1021,9 +1026,7 @@ struct tpsph_handle {
     // Verlet lists of the wall particles over the fluid (Adami pass), active wall particles
     int *anbr = nullptr, *acnt = nullptr, *wactive = nullptr;
     int lw = 0, cap_a = 0;
-    // counters rebuilt with the lists: [0] non-empty bricks, [1] active wall particles,
-    // [2] fluid particles with wall candidates (wtargets), [3] overflowed lists, [4] targets
-    // and [5] union records given to bricks so far, [6] work counter of the list build
+    // counters: see kCounters; wtargets: columns of the fluid particles with wall candidates
     int *counters = nullptr, *wtargets = nullptr;
     int n_cu = 256;  // compute units of the device (grid of the brick kernel)
     // host-mode staging and solver scratch
