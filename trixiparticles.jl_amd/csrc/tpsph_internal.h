@@ -24,8 +24,8 @@ constexpr int kWallLanes = 4;  // lanes per wall particle of the Adami pass
 constexpr int kCap = 32;     // neighbour-list entries per lane and phase
 constexpr int kScanItems = 16;
 constexpr int kScanTile = kBlock * kScanItems;
-constexpr int kBrickThreads = 1024;   // threads of the brick kernel (one block per CU), two
-                                      // per target
+constexpr int kBrickThreads = 1024;   // threads of the brick kernels (one block per CU, four
+                                      // lanes per target; mixed precision two and two)
 constexpr int kBrickCap = 2048;       // LDS records of a brick: the union plus one far record
 constexpr int kBrickCapGrad = 1664;   // the same with DensityDiffusionAntuono's density
                                       // gradients in the records (3D: 96 instead of 72 bytes)
@@ -906,7 +906,7 @@ __global__ void __launch_bounds__(THREADS)
 
 // Launches k_scan: tiles of 16,384 ints (1,024 threads) above 2^19.  The prefixes pass from one
 // window of 64 tiles to the next, about 1.5 us each, so the time goes with the number of tiles:
-// 10M cells (1.02M particles in 3D) 128 us in tiles of 4,096, 91 in these (3.5M: 17
+// 19.9M cells (1.02M particles in 3D) 128 us in tiles of 4,096, 91 in these (3.5M: 17
 // and 13); below, the small tiles spread over more compute units.
 template <bool CLEAR>
 inline void launch_scan(hipStream_t st, const int *flag, int *in, int *out, unsigned long long *state, int n)
@@ -1168,7 +1168,7 @@ int kick_dispatch(tpsph_handle *h, double *dv, const double *v, const double *u,
 // A kick without its fluid pass: the records of (v, u) with the fluid pressures, the rebuild
 // of the cell order and the lists (when a particle left its skin), the Adami pass.
 // keep_order: the caller knows that no particle of (v, u) has left its skin since the last
-// rebuild, so the rebuild launches are left out and the flag is lowered first.
+// rebuild (the flag is down) and has written the records of (v, u), so only the Adami pass is left.
 int prepare_dispatch(tpsph_handle *h, const double *v, const double *u, bool keep_order = false);
 
 // CarpenterKennedy2N54 (williamson_condition = false) coefficients A (A[0] unused) and B
