@@ -1091,6 +1091,9 @@ struct ListsSmem {
     int item, col0, ubase, bad, nnear;
 };
 
+static_assert(sizeof(ListsSmem<2, false>) <= 80 * 1024 && sizeof(ListsSmem<3, false>) <= 80 * 1024,
+              "two blocks per compute unit");
+
 // Exclusive scan over the kListThreads threads of a block.
 __device__ __forceinline__ int lists_scan(int value, int *s, int &total)
 {
@@ -1404,7 +1407,7 @@ __device__ __forceinline__ void brick_int_lists(const DevParams &P, const FluidV
 // entry) is not written any more; the walls of a brick are staged the same way, for the
 // targets near one only (four lanes per target on global memory: 157 us, here 40).  Bricks,
 // unions and lists took 860 us and five launches, four lanes per target 720, this form 495.
-// Two blocks of 512 threads share a compute unit (78 KB each; WIDE: one of 87 KB).  A brick takes
+// Two blocks of 512 threads share a compute unit (80 KB each; WIDE: one of 88 KB).  A brick takes
 // its columns, its part of uidx and the block's next brick from three counters, each on a line of
 // its own: on one line they bounded the build of many bricks of few targets (700k particles in
 // 2D: 96 -> 74 us, with one in a hundred dispersed as spray 235 -> 150).
